@@ -16,8 +16,8 @@
 // exactly the node set of its own recursive walk in the reference
 // (Node.cpp:382-396 visits the children of an opened node; the visiting order
 // differs, which only reorders the sum).  Entries are swept 64 at a time:
-// lane j stages entry j in LDS and every lane computes its interaction with
-// every staged entry it belongs to.
+// lane j stages entry j in LDS, and each lane computes its interactions with
+// the staged entries it belongs to (walk_block: two queues, by lane mask).
 // The opening test decides radius^2 against theta^2 r^2 with a 1e-10 margin
 // and falls back to the reference's correctly rounded radius / sqrt(r^2)
 // inside the margin, so the decision equals the reference's bit for bit.
@@ -59,19 +59,19 @@ struct alignas(16) StackEnt {
     unsigned long long mask;
 };
 
-typedef unsigned u32_alias __attribute__((may_alias));
-
 struct BlockLds {
     StackEnt stk[kStackCap];
-    int32_t ent_node[kEnt];
+    int32_t ent_full[kEnt];              // entries that act on every target (the overflow walk: its pending pairs)
+    int32_t ent_node[kEnt];              // entries under a lane mask
     unsigned long long ent_mask[kEnt];
     union {
-        struct { double cx[64], cy[64], cz[64], m[64]; } d;   // FP64 sweep
+        double4 d[64];                                        // FP64 sweep: centre and G m
         struct { float4 f[64], lo[64]; } s;                   // FP32 sweep: offsets, their remainders
         double acc[4][64];                                    // SPH sums per target lane; mixed-node staging
     } e;
-    uint16_t pairs[128];   // pending SPH pairs: target lane | entry << 8
 };
+// four workgroups of four waves per CU
+static_assert(sizeof(BlockLds) * kWaves * 4 <= 160 * 1024, "the walk's LDS sets its occupancy");
 
 struct WalkArgs {
     int n, nin, nn;
@@ -192,6 +192,56 @@ __device__ inline void sph_pair(double dx, double dy, double dz, double r2, doub
 // the same tree records, on the same L2.
 
 
+// Transpose of a 64 x 64 bit matrix held one row per lane: lane j gives row j
+// (lo: columns 0..31, hi: 32..63) and gets column j.  Halves are exchanged
+// at lane distance 32, 16, .. 1, on the vector unit alone (30 instructions).
+__device__ inline void transpose64(unsigned &lo, unsigned &hi) {
+    const int lane = lane_id();
+    auto s32 = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+    const unsigned a = s32[0], b = s32[1];
+    // 16: both words' low halves in one register, their high halves in another
+    auto s16 = __builtin_amdgcn_permlane16_swap(__builtin_amdgcn_perm(b, a, 0x05040100),
+                                                __builtin_amdgcn_perm(b, a, 0x07060302), false, false);
+    unsigned w[2] = {__builtin_amdgcn_perm(s16[1], s16[0], 0x05040100),
+                     __builtin_amdgcn_perm(s16[1], s16[0], 0x07060302)};
+    const unsigned sel8 = (lane & 8) ? 0x03070105u : 0x06020400u;
+    const unsigned m4 = (lane & 4) ? 0xf0f0f0f0u : 0x0f0f0f0fu, r4 = (lane & 4) ? 4u : 28u;
+    const unsigned m2 = (lane & 2) ? 0xccccccccu : 0x33333333u, r2 = (lane & 2) ? 2u : 30u;
+    const unsigned m1 = (lane & 1) ? 0xaaaaaaaau : 0x55555555u, r1 = (lane & 1) ? 1u : 31u;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        unsigned v = w[k], y;
+        y = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);   // lane ^ 8 (row_ror:8)
+        v = __builtin_amdgcn_perm(y, v, sel8);
+        y = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, true);   // lane ^ 7 (row_half_mirror)
+        y = (unsigned)__builtin_amdgcn_mov_dpp((int)y, 0x1b, 0xf, 0xf, true);    // lane ^ 4
+        v = (v & m4) | (__builtin_amdgcn_alignbit(y, y, r4) & ~m4);
+        y = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);    // lane ^ 2
+        v = (v & m2) | (__builtin_amdgcn_alignbit(y, y, r2) & ~m2);
+        y = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);    // lane ^ 1
+        v = (v & m1) | (__builtin_amdgcn_alignbit(y, y, r1) & ~m1);
+        w[k] = v;
+    }
+    lo = w[0];
+    hi = w[1];
+}
+
+// The set bits of m in ascending order, two at a time: f(j1, j2, both); j2 is
+// j1 again where m has no second bit.  Two entries' loads and arithmetic
+// overlap: one at a time, every pass waits out a chain of about twenty
+// dependent instructions behind an LDS read.
+template <class F>
+__device__ __forceinline__ void bit_pairs(unsigned m, F &&f) {
+    while (m) {
+        const int j1 = __builtin_ctz(m);
+        m &= m - 1;
+        const bool both = m != 0;
+        const int j2 = both ? __builtin_ctz(m) : j1;
+        m &= m - 1;
+        f(j1, j2, both);
+    }
+}
+
 // Group g of 64 targets: particles 64 g .. 64 g + 63 in key order.
 // KIND 0: gravity.  KIND 1: gravity, and every accepted gas node within a
 // margin of 2h of a gas target goes on that target's SPH candidate list
@@ -199,12 +249,27 @@ __device__ inline void sph_pair(double dx, double dy, double dz, double r2, doub
 // split-precision walk found more near pairs than kNearRecs (their results
 // replace that walk's).  KIND 2: the SPH term, inline, for the targets
 // whose list overflowed (groups flagged in gover only; no gravity).
+//
+// An accepted node becomes an entry of one of two queues, each swept 64
+// entries at a time:
+//  - full: every target of the group interacts and none is near; the sweep
+//    has no lane mask at all (a fifth to a third of the entries);
+//  - partial: the 64 lane masks are transposed (transpose64), and each lane
+//    walks the bits of its own word, entry by entry, reading the entry from
+//    LDS.  The loop ends with the busiest lane: on the 1 M disk the partial
+//    masks hold a fifth of the lanes on average, and a lane meets at most
+//    two fifths of a chunk, where a sweep under the masks ran over all of it.
+// The walk is bound by VALU issue (76 % of the SIMDs' cycles): with the two
+// queues, the SPH margin tested in the sweep and two entries in flight per
+// lane it issues 22.6 k vector instructions per wave where one masked sweep
+// issued 28.4 k (1 M disk, FP32), and the kernel takes 0.76 ms against
+// 1.00 ms; the FP64 form 1.24 ms against 1.90 ms.
 template <bool F32, int KIND>
-__device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
+__device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *lds) {
     constexpr bool GAS = KIND == 1 || KIND == 2;
-    if (KIND == 2 && (g >= (a.n + 63) / 64 || !a.gover[g])) return;
-    if (KIND == 3 && (g >= (a.n + 63) / 64 || a.near_cnt[g] <= kNearRecs)) return;
-    __shared__ BlockLds lds[kWaves];
+    if (g >= (a.n + 63) / 64) return;
+    if (KIND == 2 && !a.gover[g]) return;
+    if (KIND == 3 && a.near_cnt[g] <= kNearRecs) return;
     const int wv = threadIdx.x >> 6;
     const int lane = lane_id();
     BlockLds &S = lds[wv];
@@ -212,27 +277,22 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
     const bool valid_t = t < a.n;
     const int q = t;   // particle state is in key order
     const bool act = valid_t && a.active[q] != 0;
-    double px = 0.0, py = 0.0, pz = 0.0, pm = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
+    double px = 0.0, py = 0.0, pz = 0.0, pm = 0.0;
     if (valid_t) {
         px = a.sx[t]; py = a.sy[t]; pz = a.sz[t]; pm = a.sm[t];
-        vx = a.svx[t]; vy = a.svy[t]; vz = a.svz[t];
     }
-    core::Target tg;
-    tg.x = px; tg.y = py; tg.z = pz; tg.m = pm; tg.vx = vx; tg.vy = vy; tg.vz = vz;
-    tg.gas = valid_t && a.stype[t] == 2;
-    tg.h = act ? a.h[q] : 0.0;
-    tg.rho = act ? a.rho[q] : 0.0;
-    tg.P = act ? a.P[q] : 0.0;
-    tg.self = t;
+    const bool tgas = valid_t && a.stype[t] == 2;
+    const double th = act ? a.h[q] : 0.0;
     const unsigned long long amask = __ballot(act && pm != 0.0);
-    bool sph_lane = GAS && ((amask >> lane) & 1ull) && tg.gas && tg.h > 0.0;
+    const bool mine = (amask >> lane) & 1ull;
+    bool sph_lane = GAS && mine && tgas && th > 0.0;
     int slot = -1;
     if (GAS && sph_lane) {
         slot = a.gslot[t];
         if (KIND == 2) sph_lane = a.sph_cnt[slot] > kSphK;
     }
     const unsigned long long sphB = __ballot(sph_lane);
-    const double h2x4 = GAS ? (2.0 * tg.h) * (2.0 * tg.h) : 0.0;   // SPH support (2h)^2
+    const double h2x4 = GAS ? (2.0 * th) * (2.0 * th) : 0.0;   // SPH support (2h)^2
     int lcnt = 0;   // KIND 1: candidates recorded for this target
 
     core::WalkSums s{0, 0, 0, 0, 0, 0, 0};
@@ -245,10 +305,10 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
     // target are too close for FP32 offsets to resolve their direction; they
     // are recorded and evaluated in FP64 after the walk (k_near_pass)
     float r2min = 0.f;
-    double near_a = 0.0;    // uniform: see the near-entry test at staging
-    unsigned lnint = 0u;    // interactions of the fast chunks, counted per staging lane
+    double near_b2 = 0.0;   // uniform: see the full-queue test
+    unsigned lnint = 0u;    // interactions counted per lane
     int nrec = 0;           // uniform: near pairs recorded for k_near_pass
-    bool dfmode = false;    // uniform: this group's sweep carries the offsets' remainders
+    bool dfmode = false;    // uniform: this group's partial chunks carry the offsets' remainders
     float sumx = 0.f, sumy = 0.f, sumz = 0.f, cmpx = 0.f, cmpy = 0.f, cmpz = 0.f;
     const double theta = a.wp.theta, th2 = a.wp.theta * a.wp.theta;
     const double th2lo = th2 * (1.0 - 1e-10), th2hi = th2 * (1.0 + 1e-10);   // group-box accept / open margins
@@ -261,9 +321,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
         // bounding box of the group's active targets (decides whole-group
         // accept / open for most nodes without per-lane tests)
         double lo[3] = {px, py, pz}, hi[3] = {px, py, pz};
-        if (!((amask >> lane) & 1ull)) { lo[0] = lo[1] = lo[2] = 1e308; hi[0] = hi[1] = hi[2] = -1e308; }
+        if (!mine) { lo[0] = lo[1] = lo[2] = 1e308; hi[0] = hi[1] = hi[2] = -1e308; }
         // box of the SPH targets and their largest support 2h
-        double glo[3] = {px, py, pz}, ghi[3] = {px, py, pz}, h2 = sph_lane ? 2.0 * tg.h : 0.0;
+        double glo[3] = {px, py, pz}, ghi[3] = {px, py, pz}, h2 = sph_lane ? 2.0 * th : 0.0;
         if (!sph_lane) { glo[0] = glo[1] = glo[2] = 1e308; ghi[0] = ghi[1] = ghi[2] = -1e308; }
         for (int d = 32; d >= 1; d >>= 1) {
             for (int k = 0; k < 3; k++) {
@@ -296,27 +356,37 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
             double el = a.wp.e0 * invL;
             e2f = uni((float)(el * el));
             // each offset is rounded to 2^-24 of itself, so d carries an error
-            // of about 2^-24 (|target| + |entry|) per component; below 2^-10
+            // of about 2^-24 (|target| + |entry|) per component; below 2^-8
             // of 2 (|x| + |y| + |z|) of the target offset the FP32 direction
-            // could be off by more than 2^-13, and FP32 may round d to zero
+            // could be off by more than 2^-15, and FP32 may round d to zero
             // where the FP64 positions differ (the reference's r == 0 skip is
             // on FP64 r)
-            const float ao = 2.f * (fabsf(xr) + fabsf(yr) + fabsf(zr)) * 0x1p-10f;
-            r2min = ao * ao;
+            // (and a pair needs r^2 (r^2 + e^2)^2 in v_rsq_f32's normal range:
+            // below the floor a group far smaller than the softening length
+            // leaves it)
+            const double fl = 0x1p-123 / ((double)e2f * (double)e2f);
+            const float floor2 = uni((float)(fl < 0x1p-41 ? fl : 0x1p-41));
+            const float off = 2.f * (fabsf(xr) + fabsf(yr) + fabsf(zr));
+            r2min = fmaxf(off * off * 0x1p-16f, floor2);
+            const float ao = sqrtf(r2min);
             // in a chunk with such an entry the sweep forms d from the offsets
             // and their remainders (48 bits: exact difference of the high parts
             // for close pairs by Sterbenz), which resolves the direction down
             // to 2^-34 of the offsets; closer pairs go to the FP64 pass
-            const float adf = ao * 0x1p-24f;
-            r2df = adf * adf;
-            // an entry farther from the targets' box than near_a + near_b
-            // (its offset sum) is beyond every lane's r2min with room for the
-            // FP32 offsets' rounding (2^-23 of target and entry offsets), so
-            // its lanes need no per-lane test
-            float aomax = (amask >> lane) & 1ull ? ao : 0.f;
+            const float adf = off * 0x1p-34f;
+            r2df = fmaxf(adf * adf, floor2);
+            // an entry at distance D from the targets' box, beyond near_a +
+            // 2^-20 of its offset sum, is beyond every lane's r2min with room
+            // for the FP32 offsets' rounding (2^-23 of target and entry
+            // offsets), so its lanes need no per-lane test.  The offset sum is
+            // at most ext + sqrt(3) D, so D (1 - 2^-19) > near_a + 2^-20 ext
+            // is enough.
+            float aomax = mine ? ao : 0.f;
             for (int d = 32; d >= 1; d >>= 1) aomax = fmaxf(aomax, __shfl_xor(aomax, d, 64));
             const double ext = 0.5 * ((hi[0] - lo[0]) + (hi[1] - lo[1]) + (hi[2] - lo[2])) * invL;
-            near_a = uni(4.0 * (double)aomax + 0x1p-20 * ext);
+            const double near_a = uni(4.0 * (double)aomax + 0x1p-20 * ext);
+            const double nb = (near_a + 0x1p-20 * ext) * (1.0 + 0x1p-18) * R;
+            near_b2 = nb * nb;
         }
         // KIND 1: the candidate test on the sweep's own r^2, loose by a
         // margin; k_sph_pairs decides exactly.  In the split form r is
@@ -324,13 +394,13 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
         // most 2^-24 of its size: for a node within 2h (scaled: D) of a target
         // with offset sum A, the computed r exceeds the true one by less than
         // 2^-23 (A + D) + rounding of r^2 itself.
-        const double lim64 = h2x4 * (1.0 + 1e-9);
+        const double lim64 = sph_lane ? h2x4 * (1.0 + 1e-9) : -1.0;
         float lim32 = 0.f;
         if (F32 && KIND == 1) {
-            const double D = 2.0 * tg.h * invL;
+            const double D = 2.0 * th * invL;
             const double A = fabs((double)xr) + fabs((double)yr) + fabs((double)zr);
             const double rl32 = D * (1.0 + 1e-6) + 2.4e-7 * (A + 2.0 * D);
-            lim32 = (float)(rl32 * rl32 * (1.0 + 1e-5));
+            lim32 = sph_lane ? (float)(rl32 * rl32 * (1.0 + 1e-5)) : -1.f;
         }
         int32_t *lbase = (KIND == 1 && slot >= 0) ? a.sph_list + (size_t)slot * kSphK : nullptr;
         // Multi-block pops keep the stack within kStackCap: a pop of up to
@@ -344,7 +414,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
         const int single_above = kStackCap - 64 - growth;
         if (lane == 0) { S.stk[0].first = 0; S.stk[0].count = 1; S.stk[0].mask = amask; }
         int sp = 1;
-        int ni = 0;
+        int nf = 0, ni = 0;   // full and partial entries queued
         unsigned long long n_entries = 0ull, n_tests = 0ull, n_mixed = 0ull;
         while (true) {
             wave_sync_lds();
@@ -374,22 +444,22 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                 // 0 nothing (no node or mass 0)
                 core::TreeNode r;
                 int cls = 0, rnch = 0, rpidx = -1;
-                double rad = 0.0;
+                double rad = 0.0, rmin2 = 0.0;
                 if (in_mask(validB)) {
                     r = a.tree[node];
                     rnch = r.nchild;
                     rpidx = r.pidx;
                     rad = ldexp(R, -(int)r.level);
+                    // nearest and farthest box points from the centre;
+                    // the 1e-10 margins absorb the fused roundings
+                    const double ax = lo[0] - r.cx, bx = r.cx - hi[0];
+                    const double ay = lo[1] - r.cy, by = r.cy - hi[1];
+                    const double az = lo[2] - r.cz, bz = r.cz - hi[2];
+                    const double ex = fmax(fmax(ax, bx), 0.0), ey = fmax(fmax(ay, by), 0.0), ez = fmax(fmax(az, bz), 0.0);
+                    rmin2 = __builtin_fma(ex, ex, __builtin_fma(ey, ey, ez * ez));
                     if (r.mass == 0.0) cls = 0;
                     else if (r.pidx >= 0) cls = 1;
                     else {
-                        // nearest and farthest box points from the centre;
-                        // the 1e-10 margins absorb the fused roundings
-                        const double ax = lo[0] - r.cx, bx = r.cx - hi[0];
-                        const double ay = lo[1] - r.cy, by = r.cy - hi[1];
-                        const double az = lo[2] - r.cz, bz = r.cz - hi[2];
-                        const double ex = fmax(fmax(ax, bx), 0.0), ey = fmax(fmax(ay, by), 0.0), ez = fmax(fmax(az, bz), 0.0);
-                        const double rmin2 = __builtin_fma(ex, ex, __builtin_fma(ey, ey, ez * ez));
                         const double fx = fmax(fabs(ax), fabs(bx)), fy = fmax(fabs(ay), fabs(by)), fz = fmax(fabs(az), fabs(bz));
                         const double rmax2 = __builtin_fma(fx, fx, __builtin_fma(fy, fy, fz * fz));
                         const double rad2 = rad * rad;
@@ -399,18 +469,28 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                     }
                 }
                 n_tests += (unsigned long long)__builtin_popcountll(validB);
-                // whole-mask accepts -> entries (a leaf never acts on itself)
+                // whole-mask accepts -> entries (a leaf never acts on itself:
+                // r == 0, Node.cpp:274-276, so only distinct particles reach
+                // the sweeps' r == 0 and near-pair tests)
                 const unsigned long long c1B = __ballot(cls == 1);
                 const int self = rpidx - g * 64;
                 const bool drop = rpidx >= 0 && (unsigned)self < 64u;   // (its own leaf: a leaf is class 1 or 0)
                 const unsigned long long A = drop ? Mb & ~(1ull << (self & 63)) : Mb;
                 const unsigned long long appB = c1B & __ballot(A != 0ull);
-                if (in_mask(appB)) {
-                    const int slot = ni + mbcnt(appB);
+                unsigned long long fullB = 0ull;
+                if (KIND != 2) {
+                    fullB = appB & __ballot(A == amask);
+                    if (F32) fullB &= __ballot(rmin2 > near_b2);
+                    if (in_mask(fullB)) S.ent_full[nf + mbcnt(fullB)] = node;
+                    nf += __builtin_popcountll(fullB);
+                }
+                const unsigned long long partB = appB & ~fullB;
+                if (in_mask(partB)) {
+                    const int slot = ni + mbcnt(partB);
                     S.ent_node[slot] = node;
                     S.ent_mask[slot] = A;
                 }
-                ni += __builtin_popcountll(appB);
+                ni += __builtin_popcountll(partB);
                 // whole-mask opens -> child blocks
                 const unsigned long long nchB = __ballot(rnch > 0);
                 const unsigned long long pB = __ballot(cls == 2) & nchB;
@@ -426,65 +506,59 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                 if (sp > kStackCap) sp = kStackCap;
                 // per-lane decisions, exactly the reference's test
                 const unsigned long long mixB = __ballot(cls == 3);
-                n_mixed += (unsigned long long)__builtin_popcountll(mixB);
-                // The mixed nodes' centres and thresholds go to the staging
-                // area (free outside the sweep) and are read back at a
-                // uniform address (KIND 2 broadcasts them lane by lane).
-                // A lane accepts a mixed node when r^2 > rad^2 / (theta^2 (1 - 1e-10))
-                // and opens it when r^2 < rad^2 / (theta^2 (1 + 1e-10)): outside
-                // that band the reference's rounded radius / sqrt(r^2) < theta
-                // cannot decide otherwise; inside it, its own expression
-                // decides on its own unfused r^2.  Each node's accept and
-                // open masks are selected into the lane that holds the node,
-                // and its entry and child block are appended after the loop
-                // in lane order (the order the nodes were decided in).
-                const double tacc = rad * rad * inv_th2m;
-                if (KIND != 2 && cls == 3) {
-                    const int slot = mbcnt(mixB);
-                    S.e.acc[0][slot] = r.cx; S.e.acc[1][slot] = r.cy; S.e.acc[2][slot] = r.cz; S.e.acc[3][slot] = tacc;
-                }
-                if (KIND != 2 && mixB) wave_sync_lds();
-                unsigned long long mAA = 0ull, mOO = 0ull;   // decisions on this lane's mixed node
-                int mslot = 0;
-                for (unsigned long long bb = mixB; bb; bb &= bb - 1, mslot++) {
-                    const int kk = __builtin_ctzll(bb);
-                    double ncx, ncy, ncz, Tacc;
-                    if (KIND == 2) {
-                        ncx = rl(r.cx, kk); ncy = rl(r.cy, kk); ncz = rl(r.cz, kk); Tacc = rl(tacc, kk);
-                    } else {
-                        ncx = S.e.acc[0][mslot]; ncy = S.e.acc[1][mslot]; ncz = S.e.acc[2][mslot]; Tacc = S.e.acc[3][mslot];
-                    }
-                    const double Topn = Tacc * open_ratio;
-                    const unsigned long long Mk = rl(Mb, kk);
-                    const double dx = ncx - px, dy = ncy - py, dz = ncz - pz;
-                    const double r2f = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
-                    const unsigned long long live = Mk & __ballot(r2f != 0.0);
-                    unsigned long long AA = live & __ballot(r2f > Tacc);
-                    unsigned long long OO = live & __ballot(r2f < Topn);
-                    const unsigned long long band = live & ~(AA | OO);
-                    if (band) {
-                        const double nrad = rl(rad, kk);
-                        bool a2 = false;
-                        if (in_mask(band)) {
-                            const double r2 = dx * dx + dy * dy + dz * dz;
-                            a2 = (nrad / sqrt(r2)) < theta;
-                        }
-                        const unsigned long long BA = band & __ballot(a2);
-                        AA |= BA;
-                        OO |= band & ~BA;
-                    }
-                    mAA = wl(mAA, AA, kk);
-                    mOO = wl(mOO, OO, kk);
-                }
                 if (mixB) {
-                    const unsigned long long eB = __ballot(mAA != 0ull);
+                    const int nmix = __builtin_popcountll(mixB);
+                    n_mixed += (unsigned long long)nmix;
+                    // The mixed nodes' centres and thresholds go to the staging
+                    // area (free outside the sweep) and are read back at a
+                    // uniform address.  A lane accepts a mixed node when r^2 > rad^2 / (theta^2 (1 - 1e-10)) and opens
+                    // it when r^2 < rad^2 / (theta^2 (1 + 1e-10)): outside
+                    // that band the reference's rounded radius / sqrt(r^2) <
+                    // theta cannot decide otherwise; inside it, its own
+                    // expression decides on its own unfused r^2.  (A centre
+                    // that is NaN is never accepted.)  Each node's accept and
+                    // open masks are selected into the lane that holds the
+                    // node, and its entry and child block are appended after
+                    // the loop in lane order.
+                    const double tacc = rad * rad * inv_th2m;
+                    const int rank = mbcnt(mixB);
+                    if (cls == 3) {
+                        S.e.acc[0][rank] = r.cx; S.e.acc[1][rank] = r.cy; S.e.acc[2][rank] = r.cz; S.e.acc[3][rank] = tacc;
+                    }
+                    wave_sync_lds();
+                    unsigned long long mAA = 0ull, mOO = 0ull;   // decisions on this lane's mixed node
+                    unsigned long long bb = mixB;
+                    for (int at = 0; at < nmix; at++) {
+                        const double ncx = S.e.acc[0][at], ncy = S.e.acc[1][at], ncz = S.e.acc[2][at], Tacc = S.e.acc[3][at];
+                        const double dx = ncx - px, dy = ncy - py, dz = ncz - pz;
+                        const double r2f = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+                        const unsigned long long nz = __ballot(r2f != 0.0);
+                        const unsigned long long ge = __ballot(r2f >= Tacc * open_ratio);
+                        unsigned long long AA = __ballot(r2f > Tacc);
+                        unsigned long long OO = nz & ~ge;
+                        const unsigned long long band = ge & ~AA;
+                        if (band) {
+                            const double nrad = rl(rad, __builtin_ctzll(bb));
+                            const double r2 = dx * dx + dy * dy + dz * dz;
+                            const unsigned long long BA = band & __ballot((nrad / sqrt(r2)) < theta);
+                            AA |= BA;
+                            OO |= band & ~BA;
+                        }
+                        const int kk = __builtin_ctzll(bb);
+                        bb &= bb - 1;
+                        mAA = wl(mAA, AA, kk);
+                        mOO = wl(mOO, OO, kk);
+                    }
+                    mAA &= Mb;
+                    mOO &= Mb;
+                    const unsigned long long eB = mixB & __ballot(mAA != 0ull);
                     if (in_mask(eB)) {
                         const int slot = ni + mbcnt(eB);
                         S.ent_node[slot] = node;
                         S.ent_mask[slot] = mAA;
                     }
                     ni += __builtin_popcountll(eB);
-                    const unsigned long long qB = __ballot(mOO != 0ull) & nchB;
+                    const unsigned long long qB = mixB & __ballot(mOO != 0ull) & nchB;
                     if (in_mask(qB)) {
                         const int slot = sp + mbcnt(qB);
                         if (slot < kStackCap) {
@@ -498,37 +572,27 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                 }
             }
             // ------------------------------------------------- sweep
-            while (ni >= 64 || (sp == 0 && ni > 0)) {
-                const int cnt = ni >= 64 ? 64 : ni;
-                const int e0 = ni - cnt;
+            while (ni >= 64 || nf >= 64 || (sp == 0 && ni + nf > 0)) {
+                const bool part = ni >= 64 || (nf < 64 && ni > 0);   // uniform
+                const int have = part ? ni : nf;
+                const int cnt = have >= 64 ? 64 : have;
+                const int e0 = have - cnt;
+                const int32_t *enode = part ? S.ent_node : S.ent_full;
                 wave_sync_lds();
-                double ecx = 0.0, ecy = 0.0, ecz = 0.0, exd = 0.0, eyd = 0.0, ezd = 0.0;
+                double ecx = 0.0, ecy = 0.0, ecz = 0.0;
                 unsigned long long emask = 0ull;
-                bool cand = false, near = false;
+                bool cand = false;
                 if (lane < cnt) {
-                    const core::TreeNode w = a.tree[S.ent_node[e0 + lane]];
-                    emask = S.ent_mask[e0 + lane];
-                    // a target never meets its own leaf (r == 0, Node.cpp:274-276):
-                    // dropped here, so only distinct particles reach the sweep's
-                    // r == 0 and near-pair tests
-                    const int own = w.pidx - g * 64;
-                    if (w.pidx >= 0 && own >= 0 && own < 64) emask &= ~(1ull << own);
-                    ecx = w.cx; ecy = w.cy; ecz = w.cz;
+                    const core::TreeNode w = a.tree[enode[e0 + lane]];
+                    emask = part ? S.ent_mask[e0 + lane] : amask;
+                    if (KIND == 2) { ecx = w.cx; ecy = w.cy; ecz = w.cz; }
                     if (F32) {
-                        S.ent_mask[e0 + lane] = emask;   // the fast sweep reads its lane's bit from here
-                        exd = (w.cx - gcx) * invL; eyd = (w.cy - gcy) * invL; ezd = (w.cz - gcz) * invL;
+                        const double exd = (w.cx - gcx) * invL, eyd = (w.cy - gcy) * invL, ezd = (w.cz - gcz) * invL;
                         S.e.s.f[lane] = make_float4((float)exd, (float)eyd, (float)ezd, (float)(w.mass * invMu));
                         lnint += (unsigned)__builtin_popcountll(emask);   // less the lanes excluded below
-                        const double bx = fmax(fmax(lo[0] - w.cx, w.cx - hi[0]), 0.0);
-                        const double by = fmax(fmax(lo[1] - w.cy, w.cy - hi[1]), 0.0);
-                        const double bz = fmax(fmax(lo[2] - w.cz, w.cz - hi[2]), 0.0);
-                        const double eoff = (fabs(w.cx - gcx) + fabs(w.cy - gcy) + fabs(w.cz - gcz)) * invL;
-                        const double lim = near_a + 0x1p-20 * eoff;
-                        near = (bx * bx + by * by + bz * bz) * (invL * invL) <= lim * lim;
-                    } else {
+                    } else if (KIND != 2) {
                         // G m staged once per entry (the sweep forms ((G m) rcp) ri, as before)
-                        S.e.d.cx[lane] = w.cx; S.e.d.cy[lane] = w.cy; S.e.d.cz[lane] = w.cz;
-                        S.e.d.m[lane] = a.wp.soft_live ? w.mass : a.wp.G * w.mass;
+                        S.e.d[lane] = make_double4(w.cx, w.cy, w.cz, a.wp.soft_live ? w.mass : a.wp.G * w.mass);
                     }
                     if (GAS && sphB && (emask & sphB)) {
                         // a leaf's gas mass is its mass when it is gas; nodes of
@@ -541,26 +605,29 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                     }
                 }
                 const unsigned long long candB = GAS ? __ballot(cand) : 0ull;
-                const unsigned long long nearB = F32 ? __ballot(near) : 0ull;
-                // remainders of the entry offsets: in LDS for a dfmode sweep, in
-                // the staging lanes' registers for a near chunk's rescan
-                float elx = 0.f, ely = 0.f, elz = 0.f;
-                if (F32 && nearB && !dfmode) {
-                    elx = (float)(exd - (double)(float)exd);
-                    ely = (float)(eyd - (double)(float)eyd);
-                    elz = (float)(ezd - (double)(float)ezd);
-                }
-                if (F32 && dfmode && lane < cnt)
-                    S.e.s.lo[lane] = make_float4((float)(exd - (double)(float)exd), (float)(eyd - (double)(float)eyd),
-                                                 (float)(ezd - (double)(float)ezd), 0.f);
                 wave_sync_lds();
+                unsigned tlo = (unsigned)emask, thi = (unsigned)(emask >> 32);
+                if (KIND != 2 && part) transpose64(tlo, thi);
+                // each half of a lane's word is walked by itself; a full chunk
+                // has every entry
+                const unsigned long long all = cnt == 64 ? ~0ull : (1ull << cnt) - 1;
+                unsigned word[2] = {part ? tlo : (unsigned)all, part ? thi : (unsigned)(all >> 32)};
+                // KIND 1: the entries of each half within the lane's SPH
+                // margin, as the sweep meets them (the r^2 it has anyway; one
+                // compare, select and or per entry, where testing the
+                // candidate entries again after the sweep, all lanes at once,
+                // was a quarter of the walk's instructions), and the entries
+                // resolved or recorded after it
+                const bool spot = KIND == 1 && candB != 0ull;   // uniform
+                unsigned hit[2] = {0u, 0u};
+                unsigned long long hb = 0ull;
+                const bool dfc = F32 && part && dfmode;
                 if (KIND == 2) {
                     // no gravity
                 } else if (F32) {
                     // Three sweeps, counted from the masks at staging:
-                    //  - no entry near a target: every lane of an entry's mask
-                    //    interacts (r2 > r2min > 0 for each);
-                    //  - near entries: lanes within r2min of an entry (FP32
+                    //  - full: every lane interacts (r2 > r2min > 0 for each);
+                    //  - partial: lanes within r2min of an entry (FP32
                     //    offsets cannot resolve the direction) are left out;
                     //  - dfmode (a group that has met such lanes): offsets with
                     //    their FP32 remainders (48 bits; the difference of the
@@ -569,70 +636,85 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                     // with the remainders where they can be, else recorded for
                     // the FP64 pass (and dropped from the count).
                     const float4 *fs = S.e.s.f, *fl = S.e.s.lo;
-                    const bool dfc = dfmode;
                     float cx = 0.f, cy = 0.f, cz = 0.f;
-                    unsigned long long exz = 0ull;   // lanes left out of some entry of this chunk
+                    auto pull = [&](float m, float dx, float dy, float dz, float r2, bool ok) {
+                        const float s2 = r2 + e2f;
+                        float f = m * __builtin_amdgcn_rsqf(r2 * s2 * s2);
+                        f = ok ? f : 0.f;
+                        cx = __builtin_fmaf(f, dx, cx);
+                        cy = __builtin_fmaf(f, dy, cy);
+                        cz = __builtin_fmaf(f, dz, cz);
+                    };
+                    int left = 0;   // this lane was left out of some entry
                     if (dfc) {
-                        for (int j = 0; j < cnt; j++) {
-                            const unsigned long long Mj = rl(emask, j);
-                            const float4 e = fs[j], l = fl[j];
-                            const float dx = (e.x - xr) + (l.x - xlo), dy = (e.y - yr) + (l.y - ylo);
-                            const float dz = (e.z - zr) + (l.z - zlo);
-                            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-                            const float s2 = r2 + e2f;
-                            float f = e.w * __builtin_amdgcn_rsqf(r2 * s2 * s2);
-                            const unsigned long long okB = Mj & __ballot(r2 > r2df);
-                            exz |= Mj & ~okB;
-                            f = in_mask(okB) ? f : 0.f;
-                            cx = __builtin_fmaf(f, dx, cx);
-                            cy = __builtin_fmaf(f, dy, cy);
-                            cz = __builtin_fmaf(f, dz, cz);
+                        if (lane < cnt) {
+                            const core::TreeNode w = a.tree[enode[e0 + lane]];
+                            const double exd = (w.cx - gcx) * invL, eyd = (w.cy - gcy) * invL, ezd = (w.cz - gcz) * invL;
+                            S.e.s.lo[lane] = make_float4((float)(exd - (double)(float)exd), (float)(eyd - (double)(float)eyd),
+                                                         (float)(ezd - (double)(float)ezd), 0.f);
                         }
-                    } else if (!nearB) {
-                        // each lane reads the 32-bit half of entry j's mask that
-                        // holds its bit and sign-extends the bit into an AND
-                        // mask for f (two instructions, against two readlanes
-                        // and a select)
-                        const u32_alias *mh = reinterpret_cast<const u32_alias *>(S.ent_mask + e0) + (lane >> 5);
-                        const int lb = lane & 31;
-                        auto one = [&](int j) {
-                            const float4 e = fs[j];
-                            const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
-                            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-                            const float s2 = r2 + e2f;
-                            float f = e.w * __builtin_amdgcn_rsqf(r2 * s2 * s2);
-                            const int keep = __builtin_amdgcn_sbfe((int)mh[2 * j], lb, 1);
-                            f = __int_as_float(__float_as_int(f) & keep);
-                            cx = __builtin_fmaf(f, dx, cx);
-                            cy = __builtin_fmaf(f, dy, cy);
-                            cz = __builtin_fmaf(f, dz, cz);
+                        wave_sync_lds();
+                        for (int h = 0; h < 2; h++) {
+                            auto one = [&](int j, bool on) {
+                                const float4 e = fs[32 * h + j], l = fl[32 * h + j];
+                                const float dx = (e.x - xr) + (l.x - xlo), dy = (e.y - yr) + (l.y - ylo);
+                                const float dz = (e.z - zr) + (l.z - zlo);
+                                const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                                const bool ok = r2 > r2df;
+                                left = ok ? left : 1;   // (a second entry that is the first again changes nothing)
+                                pull(e.w, dx, dy, dz, r2, ok && on);
+                                if (KIND == 1) hit[h] |= ok && r2 < lim32 ? 1u << j : 0u;
+                            };
+                            bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
+                        }
+                    } else if (part) {
+                        auto sweep = [&](auto spotting) {
+                            for (int h = 0; h < 2; h++) {
+                                auto one = [&](int j, bool on) {
+                                    const float4 e = fs[32 * h + j];
+                                    const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
+                                    const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                                    const bool ok = r2 > r2min;
+                                    left = ok ? left : 1;
+                                    pull(e.w, dx, dy, dz, r2, ok && on);
+                                    if (decltype(spotting)::value) hit[h] |= ok && r2 < lim32 ? 1u << j : 0u;
+                                };
+                                bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
+                            }
                         };
-                        int j = 0;
-                        for (; j + 4 <= cnt; j += 4) { one(j); one(j + 1); one(j + 2); one(j + 3); }
-                        for (; j < cnt; j++) one(j);
+                        if (spot) sweep(std::integral_constant<bool, KIND == 1>{});
+                        else sweep(std::false_type{});
                     } else {
-                        auto one = [&](int j) {
-                            const unsigned long long Mj = rl(emask, j);
-                            const float4 e = fs[j];
-                            const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
-                            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-                            const float s2 = r2 + e2f;
-                            float f = e.w * __builtin_amdgcn_rsqf(r2 * s2 * s2);
-                            const unsigned long long okB = Mj & __ballot(r2 > r2min);
-                            exz |= Mj & ~okB;
-                            f = in_mask(okB) ? f : 0.f;
-                            cx = __builtin_fmaf(f, dx, cx);
-                            cy = __builtin_fmaf(f, dy, cy);
-                            cz = __builtin_fmaf(f, dz, cz);
+                        auto sweep = [&](auto spotting) {
+                            for (int h = 0; h < 2; h++) {
+                                auto one = [&](int j) {
+                                    const float4 e = fs[j];
+                                    const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
+                                    const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                                    pull(e.w, dx, dy, dz, r2, true);
+                                    if (decltype(spotting)::value) hit[h] |= r2 < lim32 ? 1u << (j & 31) : 0u;
+                                };
+                                int j = 32 * h;
+                                const int je = cnt < 32 * h + 32 ? cnt : 32 * h + 32;
+                                for (; j + 4 <= je; j += 4) { one(j); one(j + 1); one(j + 2); one(j + 3); }
+                                for (; j < je; j++) one(j);
+                            }
                         };
-                        int j = 0;
-                        for (; j + 4 <= cnt; j += 4) { one(j); one(j + 1); one(j + 2); one(j + 3); }
-                        for (; j < cnt; j++) one(j);
+                        if (spot) sweep(std::integral_constant<bool, KIND == 1>{});
+                        else sweep(std::false_type{});
                     }
-                    unsigned long long hb = 0ull;   // KIND 1: candidate entries resolved or recorded below
+                    const unsigned long long exz = __ballot(left != 0);   // lanes left out of some entry of this chunk
                     if (exz) {
                         // the left-out lanes, entry by entry (rare: close pairs, or
                         // a group whose box is far wider than its neighbours' gaps)
+                        float elx = 0.f, ely = 0.f, elz = 0.f;
+                        if (!dfc && lane < cnt) {
+                            const core::TreeNode w = a.tree[enode[e0 + lane]];
+                            const double exd = (w.cx - gcx) * invL, eyd = (w.cy - gcy) * invL, ezd = (w.cz - gcz) * invL;
+                            elx = (float)(exd - (double)(float)exd);
+                            ely = (float)(eyd - (double)(float)eyd);
+                            elz = (float)(ezd - (double)(float)ezd);
+                        }
                         for (int jj = 0; jj < cnt; jj++) {
                             const unsigned long long Mj = rl(emask, jj);
                             if (!(Mj & exz)) continue;
@@ -655,86 +737,63 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                             if (!dfc) {
                                 const unsigned long long okD = Z1 & ~Z;
                                 if (okD) {
-                                    const float s2 = r2 + e2f;
-                                    float f = e.w * __builtin_amdgcn_rsqf(r2 * s2 * s2);
-                                    f = in_mask(okD) ? f : 0.f;
-                                    cx = __builtin_fmaf(f, dx, cx);
-                                    cy = __builtin_fmaf(f, dy, cy);
-                                    cz = __builtin_fmaf(f, dz, cz);
-                                    if (KIND == 1 && ((candB >> jj) & 1ull) && in_mask(okD & sphB & __ballot(r2 < lim32)))
-                                        hb |= 1ull << jj;
+                                    pull(e.w, dx, dy, dz, r2, in_mask(okD));
+                                    if (KIND == 1 && in_mask(okD & sphB & __ballot(r2 < lim32))) hb |= 1ull << jj;
                                 }
                             }
                             if (Z) {
                                 if (lane == 0 && nrec < kNearRecs) {
-                                    a.near_node[(size_t)g * kNearRecs + nrec] = S.ent_node[e0 + jj];
+                                    a.near_node[(size_t)g * kNearRecs + nrec] = enode[e0 + jj];
                                     a.near_mask[(size_t)g * kNearRecs + nrec] = Z;
                                 }
                                 nrec++;
                                 nint -= (unsigned long long)__builtin_popcountll(Z);
                                 // as SPH candidates they go on the lists as they are
                                 // (the pair kernel skips r == 0)
-                                if (KIND == 1 && ((candB >> jj) & 1ull) && in_mask(Z & sphB)) hb |= 1ull << jj;
+                                if (KIND == 1 && in_mask(Z & sphB)) hb |= 1ull << jj;
                             }
                         }
-                        dfmode = true;   // the rest of this group's sweep carries the remainders
-                    }
-                    // SPH candidates (KIND 1): the candidate entries within a
-                    // lane's margin on the sweep's own r^2 (and those resolved
-                    // or recorded above), in entry order
-                    if (KIND == 1) {
-                        for (unsigned long long cb = candB; cb; cb &= cb - 1) {
-                            const int j = __builtin_ctzll(cb);
-                            const unsigned long long Mj = rl(emask, j);
-                            const float4 e = fs[j];
-                            float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
-                            if (dfc) {
-                                const float4 l = fl[j];
-                                dx += l.x - xlo; dy += l.y - ylo; dz += l.z - zlo;
-                            }
-                            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-                            const float cut = dfc ? r2df : (nearB ? r2min : -1.f);
-                            const unsigned long long hit = Mj & sphB & __ballot(r2 > cut && r2 < lim32);
-                            if (in_mask(hit) || ((hb >> j) & 1ull)) {
-                                if (lcnt < kSphK) lbase[lcnt] = S.ent_node[e0 + j];
-                                lcnt++;
-                            }
-                        }
+                        dfmode = true;   // the rest of this group's partial chunks carry the remainders
                     }
                     float y = cx - cmpx, tt = sumx + y; cmpx = (tt - sumx) - y; sumx = tt;
                     y = cy - cmpy; tt = sumy + y; cmpy = (tt - sumy) - y; sumy = tt;
                     y = cz - cmpz; tt = sumz + y; cmpz = (tt - sumz) - y; sumz = tt;
                 } else {
-                    for (int j = 0; j < cnt; j++) {
-                        const unsigned long long Mj = rl(emask, j);
-                        double dx = S.e.d.cx[j] - px, dy = S.e.d.cy[j] - py, dz = S.e.d.cz[j] - pz;
-                        double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
-                        bool ok = in_mask(Mj) && r2 != 0.0;
-                        double gx = 0.0, gy = 0.0, gz = 0.0;
-                        if (ok) {
-                            if (a.wp.soft_live) {
-                                ok = core::soft_force(S.e.d.m[j], dx, dy, dz, sqrt(r2), a.wp, &gx, &gy, &gz);
-                            } else {
-                                double ri = rsq64(r2);
-                                double rr = r2 * ri;
-                                double f = S.e.d.m[j] * rcp64(rr * rr + e02) * ri;
-                                gx = f * dx; gy = f * dy; gz = f * dz;
-                                ok = !(gx != gx || gy != gy || gz != gz);
-                            }
-                        }
-                        if (ok) { s.ax += gx; s.ay += gy; s.az += gz; }
-                        nint += (unsigned long long)__builtin_popcountll(__ballot(ok));
-                        if (KIND == 1 && ((candB >> j) & 1ull)) {
-                            const unsigned long long hit = __ballot(ok && sph_lane && r2 < lim64);
-                            if (hit) {
-                                const int nd = S.ent_node[e0 + j];
-                                if (in_mask(hit)) {
-                                    if (lcnt < kSphK) lbase[lcnt] = nd;
-                                    lcnt++;
+                    const double4 *ds4 = S.e.d;
+                    auto sweep = [&](auto spotting) {
+                        for (int h = 0; h < 2; h++) {
+                            auto one = [&](int j, bool on) {
+                                const double4 e = ds4[32 * h + j];
+                                const double dx = e.x - px, dy = e.y - py, dz = e.z - pz;
+                                const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+                                double gx, gy, gz;
+                                bool ok = true;
+                                if (a.wp.soft_live) {
+                                    ok = r2 != 0.0 && core::soft_force(e.w, dx, dy, dz, sqrt(r2), a.wp, &gx, &gy, &gz);
+                                } else {
+                                    // r2 == 0 gives NaN here and is skipped like any NaN
+                                    const double ri = rsq64(r2);
+                                    const double rr = r2 * ri;
+                                    const double f = e.w * rcp64(rr * rr + e02) * ri;
+                                    gx = f * dx; gy = f * dy; gz = f * dz;
+                                    ok = !__builtin_isunordered(gx, gy) && gz == gz;
                                 }
-                            }
+                                ok = ok && on;
+                                if (ok) { s.ax += gx; s.ay += gy; s.az += gz; lnint++; }
+                                if (decltype(spotting)::value) hit[h] |= ok && r2 < lim64 ? 1u << j : 0u;
+                            };
+                            bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
                         }
-                    }
+                    };
+                    if (!part && !mine) word[0] = word[1] = 0u;
+                    if (spot) sweep(std::integral_constant<bool, KIND == 1>{});
+                    else sweep(std::false_type{});
+                }
+                // The candidates found go on their target's list in entry order
+                if (spot) {
+                    unsigned long long hm = ((hit[0] | (unsigned long long)hit[1] << 32) | hb) & candB;
+                    for (; hm; hm &= hm - 1, lcnt++)
+                        if (lcnt < kSphK) lbase[lcnt] = enode[e0 + __builtin_ctzll(hm)];
                 }
                 // SPH term.  Pairs (target lane t, entry j) with r < 2 h_t are
                 // queued in LDS as they are found and evaluated 64 at a time,
@@ -748,10 +807,11 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                 if (KIND == 2 && sphB) {
                     if (candB) {
                         double *acc = &S.e.acc[0][0];
+                        uint16_t *pairs = reinterpret_cast<uint16_t *>(S.ent_full);   // unused by this kind
                         int np = 0;
                         auto run_pairs = [&](int base, int cntp) {
                             wave_sync_lds();
-                            const int pr = lane < cntp ? (int)S.pairs[base + lane] : 0;
+                            const int pr = lane < cntp ? (int)pairs[base + lane] : 0;
                             const int jl = pr >> 8;
                             double wax = 0.0, way = 0.0, waz = 0.0, wdu = 0.0;
                             if (lane < cntp) {
@@ -777,7 +837,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                             acc[lane] = wax; acc[64 + lane] = way; acc[128 + lane] = waz; acc[192 + lane] = wdu;
                             wave_sync_lds();
                             for (int k = 0; k < cntp; k++) {
-                                if (((int)S.pairs[base + k] & 63) == lane) {
+                                if (((int)pairs[base + k] & 63) == lane) {
                                     s.ax += acc[k]; s.ay += acc[64 + k]; s.az += acc[128 + k]; s.du += acc[192 + k];
                                 }
                             }
@@ -797,7 +857,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                                 }
                             }
                             const unsigned long long I = __ballot(inside);
-                            if (inside) S.pairs[np + mbcnt(I)] = (uint16_t)(lane | (j << 8));
+                            if (inside) pairs[np + mbcnt(I)] = (uint16_t)(lane | (j << 8));
                             np += __builtin_popcountll(I);
                             if (np >= 64) {
                                 run_pairs(np - 64, 64);
@@ -808,9 +868,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
                     }
                 }
                 n_entries += (unsigned long long)cnt;
-                ni -= cnt;
+                if (part) ni -= cnt; else nf -= cnt;
             }
-            if (sp == 0 && ni == 0) break;
+            if (sp == 0 && ni + nf == 0) break;
         }
         if (KIND != 2 && lane == 0) {
             bin_add(a.cbins, kCntEntries, g, n_entries);
@@ -828,18 +888,16 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
         if (lane == 0) bin_add(a.cbins, kCntSphPairs, g, cs);
         return;
     }
-    if (act) {
-        double ox, oy, oz;
-        if (F32) {
-            double scale = a.nn > 0 ? a.wp.G * a.tree[0].mass * invL * invL : 0.0;
-            ox = (double)sumx * scale;
-            oy = (double)sumy * scale;
-            oz = (double)sumz * scale;
-        } else {
-            ox = s.ax; oy = s.ay; oz = s.az;
-        }
-        a.ax[q] = ox; a.ay[q] = oy; a.az[q] = oz;
+    double ox, oy, oz;
+    if (F32) {
+        const double scale = a.nn > 0 ? a.wp.G * a.tree[0].mass * invL * invL : 0.0;
+        ox = (double)sumx * scale;
+        oy = (double)sumy * scale;
+        oz = (double)sumz * scale;
+    } else {
+        ox = s.ax; oy = s.ay; oz = s.az;
     }
+    if (act) { a.ax[q] = ox; a.ay[q] = oy; a.az[q] = oz; }
     if (KIND == 1 && slot >= 0) {
         a.sph_cnt[slot] = lcnt;
         if (lcnt > kSphK) a.gover[g] = 1;
@@ -850,9 +908,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g) {
         const unsigned long long ovB = __ballot(slot >= 0 && lcnt > kSphK);
         if (lane == 0) bin_add(a.cbins, kCntSphOver, g, (unsigned long long)__builtin_popcountll(ovB));
     }
+    nint += wave_sum_u64((unsigned long long)lnint);
     if (F32) {
-        nint += wave_sum_u64((unsigned long long)lnint);
-        if (lane == 0 && g < (a.n + 63) / 64) a.near_cnt[g] = nrec;
+        if (lane == 0) a.near_cnt[g] = nrec;
         // a group walked again in FP64 (KIND 3) counts its interactions there
         if (nrec > kNearRecs) nint = 0ull;
     }
@@ -865,28 +923,35 @@ __device__ inline int wave_group() {
 
 // Kernels per precision form: gravity with SPH candidate recording (any gas
 // uploaded) or plain gravity, and the overflow SPH walk (FP64 for both forms).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_block64(WalkArgs a) {
-    walk_block<false, 1>(a, wave_group());
+#define AG2_WALK_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+
+__global__ AG2_WALK_BOUNDS void k_walk_block64(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<false, 1>(a, wave_group(), lds);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_block64_nogas(WalkArgs a) {
-    walk_block<false, 0>(a, wave_group());
+__global__ AG2_WALK_BOUNDS void k_walk_block64_nogas(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<false, 0>(a, wave_group(), lds);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_block32(WalkArgs a) {
-    walk_block<true, 1>(a, wave_group());
+__global__ AG2_WALK_BOUNDS void k_walk_block32(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<true, 1>(a, wave_group(), lds);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_block32_nogas(WalkArgs a) {
-    walk_block<true, 0>(a, wave_group());
+__global__ AG2_WALK_BOUNDS void k_walk_block32_nogas(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<true, 0>(a, wave_group(), lds);
 }
 
 // The overflow walk and the near pass usually touch few groups, but a
 // small opening angle can flag thousands (every SPH list overflowing, many
 // near pairs): one wave per group, exiting at once when its group is not
 // flagged, keeps those walks in parallel.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_sph_overflow(WalkArgs a) {
-    walk_block<false, 2>(a, wave_group());   // exits unless the group is flagged in gover
+__global__ AG2_WALK_BOUNDS void k_walk_sph_overflow(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<false, 2>(a, wave_group(), lds);   // exits unless the group is flagged in gover
 }
 
 // The near pairs of a split-precision walk in FP64 on the FP64 positions,
@@ -928,13 +993,14 @@ __device__ inline void near_fp64_group(const WalkArgs &a, int g, int cnt) {
 
 // The near pass: groups with at most kNearRecs recorded pairs evaluate them
 // in FP64 (near_fp64_group); groups with more are walked again in FP64.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_near_pass(WalkArgs a) {
+__global__ AG2_WALK_BOUNDS void k_near_pass(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
     const int g = wave_group();
     if (g >= (a.n + 63) / 64) return;
     const int cnt = a.near_cnt[g];
     if (cnt > kNearRecs) {
         if (lane_id() == 0) bin_add(a.cbins, kCntNearRedo, g, 1ull);
-        walk_block<false, 3>(a, g);
+        walk_block<false, 3>(a, g, lds);
     } else if (cnt > 0) {
         near_fp64_group(a, g, cnt);
     }
@@ -960,24 +1026,28 @@ __device__ inline int find_job(const JobWalk *jobs, int nj, int G) {
 }
 
 template <bool F32, int KIND>
-__device__ __forceinline__ void walk_jobs(const JobWalk *jobs, int nj, int total) {
+__device__ __forceinline__ void walk_jobs(const JobWalk *jobs, int nj, int total, BlockLds *lds) {
     const int G = wave_group();
     if (G >= total) return;   // whole waves only: nothing below synchronises across waves
     const int j = find_job(jobs, nj, G);
-    walk_block<F32, KIND>(jobs[j].a, G - jobs[j].group0);
+    walk_block<F32, KIND>(jobs[j].a, G - jobs[j].group0, lds);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_jobs64(const JobWalk *jobs, int nj, int total) {
-    walk_jobs<false, 1>(jobs, nj, total);
+__global__ AG2_WALK_BOUNDS void k_walk_jobs64(const JobWalk *jobs, int nj, int total) {
+    __shared__ BlockLds lds[kWaves];
+    walk_jobs<false, 1>(jobs, nj, total, lds);
 }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_jobs64_nogas(const JobWalk *jobs, int nj, int total) {
-    walk_jobs<false, 0>(jobs, nj, total);
+__global__ AG2_WALK_BOUNDS void k_walk_jobs64_nogas(const JobWalk *jobs, int nj, int total) {
+    __shared__ BlockLds lds[kWaves];
+    walk_jobs<false, 0>(jobs, nj, total, lds);
 }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_jobs32(const JobWalk *jobs, int nj, int total) {
-    walk_jobs<true, 1>(jobs, nj, total);
+__global__ AG2_WALK_BOUNDS void k_walk_jobs32(const JobWalk *jobs, int nj, int total) {
+    __shared__ BlockLds lds[kWaves];
+    walk_jobs<true, 1>(jobs, nj, total, lds);
 }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_jobs32_nogas(const JobWalk *jobs, int nj, int total) {
-    walk_jobs<true, 0>(jobs, nj, total);
+__global__ AG2_WALK_BOUNDS void k_walk_jobs32_nogas(const JobWalk *jobs, int nj, int total) {
+    __shared__ BlockLds lds[kWaves];
+    walk_jobs<true, 0>(jobs, nj, total, lds);
 }
 
 
@@ -1261,19 +1331,29 @@ void near_finish(Ctx &c) {
     AG2_HIP(hipGetLastError());
 }
 
+// The gravity walk of one context.
+template <bool F32>
+static void launch_walk(Ctx &c) {
+    const WalkArgs a = walk_args(c);
+    const int groups = (int)((c.n + 63) / 64);
+    const dim3 grid((groups + kWaves - 1) / kWaves), block(64 * kWaves);
+    if (F32) {
+        if (c.sph_active) hipLaunchKernelGGL(k_walk_block32, grid, block, 0, c.stream, a);
+        else hipLaunchKernelGGL(k_walk_block32_nogas, grid, block, 0, c.stream, a);
+    } else {
+        if (c.sph_active) hipLaunchKernelGGL(k_walk_block64, grid, block, 0, c.stream, a);
+        else hipLaunchKernelGGL(k_walk_block64_nogas, grid, block, 0, c.stream, a);
+    }
+}
+
 void forces(Ctx &c, int mode) {
     hipStream_t st = c.stream;
     int n = (int)c.n;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));
     if (mode == 0) {
         sph_prepare(c);
-        WalkArgs a = walk_args(c);
-        int groups = (n + 63) / 64;
         if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[8], st));
-        if (c.sph_active)
-            hipLaunchKernelGGL(k_walk_block64, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
-        else
-            hipLaunchKernelGGL(k_walk_block64_nogas, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
+        launch_walk<false>(c);
         if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[9], st));
         sph_finish(c);
         fold_counters(c);
@@ -1300,16 +1380,10 @@ bool fp32_usable(const Ctx &c) {
 void forces_fp32(Ctx &c, int mode) {
     if (mode != 0) return forces(c, mode);
     hipStream_t st = c.stream;
-    int n = (int)c.n;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));
     sph_prepare(c);
-    WalkArgs a = walk_args(c);
-    int groups = (n + 63) / 64;
     if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[8], st));
-    if (c.sph_active)
-        hipLaunchKernelGGL(k_walk_block32, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
-    else
-        hipLaunchKernelGGL(k_walk_block32_nogas, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
+    launch_walk<true>(c);
     if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[9], st));
     near_finish(c);
     sph_finish(c);

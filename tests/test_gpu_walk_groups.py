@@ -1,0 +1,55 @@
+"""The gravity walk where its queues, groups and chunks have edges: particle
+counts around a group of targets and a chunk of 64 entries, opening angles
+from nearly everything opened (long partial chunks) to wide (short lists), with
+and without gas, in both precision forms, against the oracle's force step.
+
+Counts are exact.  FP64: within 1e-10 of each acceleration, as in the parity
+tests.  Split form: the walk leaves pairs closer than 2^-8 of the FP32 offset
+sum to the FP64 steps, so a pair's offset, rounded to 2^-24 of target and entry,
+is off by at most 2^-15 of the distance per component, sqrt(3) 2^-15 in length,
+and its force by up to four times that (r^-3 and the direction): 2^-12 of the
+sum of the contributions' magnitudes."""
+import numpy as np
+import pytest
+
+from conftest import vec_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def check(ag2, orc, ps, theta, precision, thr=800):
+    E, U = ag2.engine, ag2.units
+    e0, mih = 0.1 * U.KPC, ag2.ics.mass_in_h(ps)
+    with E.Engine(E.make_params(theta=theta, e0=e0, massInH=mih, split_threshold=thr, precision=precision), ps.n) as eng:
+        eng.upload(ps)
+        eng.init_forces()
+        got = eng.download(ps.copy())
+        d = eng.diagnostics()
+    want = ps.copy()
+    scale = np.zeros(ps.n)
+    st = orc.force_step(want, orc.params(theta, e0, mih, thr), scale=scale)
+    assert d["interactions"] == st["interactions"]
+    assert d["sph_pairs"] == st["sph_interactions"]
+    if precision == E.AG2_FP64:
+        err = vec_rel_err(got.ax, got.ay, got.az, want.ax, want.ay, want.az)
+        assert err.max() < 1e-10, err.max()
+    else:
+        off = np.sqrt((got.ax - want.ax) ** 2 + (got.ay - want.ay) ** 2 + (got.az - want.az) ** 2)
+        assert (off <= 2.0 ** -12 * scale).all(), (off / np.where(scale > 0, scale, 1)).max()
+    assert np.array_equal(got.h, want.h)
+    s = np.abs(want.dUdt).max()
+    if s > 0:
+        assert np.abs(got.dUdt - want.dUdt).max() / s < 1e-10
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("theta", [0.05, 0.5, 1.2])
+@pytest.mark.parametrize("n", [5, 64, 65, 127, 129, 700, 4099])
+def test_counts_around_groups_and_chunks(ag2, orc, n, theta, precision):
+    nh, nd = n // 2, n // 4
+    check(ag2, orc, ag2.ics.disk_galaxy(nh, nd, n - nh - nd, seed=n), theta, precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_gas_free_sphere(ag2, orc, precision):
+    check(ag2, orc, ag2.ics.config1_plummer(3001, seed=5), 0.4, precision)
