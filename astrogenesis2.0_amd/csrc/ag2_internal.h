@@ -14,7 +14,7 @@ namespace ag2 {
 
 // Levels: up to core::kDeepest = 126 separate distinct particles (six key
 // words of 21 levels; most builds use two), and bucket members sit one below.
-constexpr int kNearRecs = 32;   // near-pair records per group of 64 targets (split-precision walk)
+constexpr int kNearRecs = 32;   // near-pair records per group of targets (split-precision walk)
 constexpr int kWalkStackCap = 384;                 // pending child blocks per wave of the block walk
 constexpr int kWalkGrowthMax = kWalkStackCap - 1;  // stack growth a tree may need below any point
 constexpr int kSortTile = 2048;   // keys per radix-sort workgroup (256 threads x 8)
@@ -348,6 +348,7 @@ bool fp32_usable(const Ctx &c);          // gravity.hip: e0 / R of the last buil
 void sph_prepare(Ctx &c);                // gravity.hip: SPH list slots before a gravity walk
 void sph_finish(Ctx &c);                 // gravity.hip: SPH candidate evaluation after it
 void near_finish(Ctx &c);                // gravity.hip: FP64 near pairs of a split-precision walk
+int64_t walk_groups_max(int64_t cap);    // gravity.hip: most walk groups any n <= cap makes
 void fold_counters(Ctx &c);              // gravity.hip: walk counters' bins into the DevState
 void kdk_begin(Ctx &c);                  // kdk.hip: time steps, min, first kick + drift
 void kdk_end(Ctx &c);                    // kdk.hip: U update, Hubble, second kick

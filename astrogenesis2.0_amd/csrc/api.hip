@@ -89,7 +89,7 @@ void alloc_all(Ctx &c, int64_t cap) {
         cv(&c.rid, n * 4); cv(&c.rid_alt, n * 4); cv(&c.inv, n * 4);
         cv(&c.gslot, n * 4); cv(&c.gidx, n * 4);
         cv(&c.gtiles, ((n + 1023) / 1024 + 1) * 4); cv(&c.gover, (n + 63) / 64 + 1);
-        const size_t groups = (size_t)(n + 63) / 64 + 1;
+        const size_t groups = (size_t)ag2::walk_groups_max(cap);
         cv(&c.near_cnt, groups * 4);
         cv(&c.near_node, groups * ag2::kNearRecs * 4);
         cv(&c.near_mask, groups * ag2::kNearRecs * 8);
@@ -167,13 +167,13 @@ int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
                     + 4 * 8 + 2 * 4   // keys, sort indices
                     + 3 * 4           // rid, rid copy, inverse
                     + 2 * 4           // c, base
-                    + 2 * 4 + 1       // SPH list slots, targets, group flags
-                    + (4 + ag2::kNearRecs * 12) / 64 + 1;   // near-pair records
+                    + 2 * 4 + 1;      // SPH list slots, targets, group flags
     int64_t per_node = 5 * 4 + 1 + 9 * 8 + (int64_t)sizeof(WalkNode) + 2 * 4 + 1 + 4 +
                        2 * (int64_t)sizeof(core::TreeNode) + 3 * 4 +   // walk and SPH records
                        (int64_t)sizeof(ag2::NodeSums) + 4 +            // node sums, internal-child counts
                        (int64_t)sizeof(ag2::NodeSums) / 64 + 1;        // block sums
     int64_t fixed = 256 * ((n + kSortTile - 1) / kSortTile + 1) * 4 + 8 * 1024 * 8 + (1 << 20) +
+                    walk_groups_max(cap) * (4 + ag2::kNearRecs * 12) +   // near-pair records
                     128 * (4096 + 256);   // the carved buffers' slack and alignment
     return n * per_p + nodes * per_node + fixed + n_gas * (kSphListLen * 4 + 4);
 }

@@ -242,13 +242,18 @@ __device__ __forceinline__ void bit_pairs(unsigned m, F &&f) {
     }
 }
 
-// Group g of 64 targets: particles 64 g .. 64 g + 63 in key order.
+// Group g of TPG targets: particles TPG g .. TPG g + TPG - 1 in key order.
 // KIND 0: gravity.  KIND 1: gravity, and every accepted gas node within a
 // margin of 2h of a gas target goes on that target's SPH candidate list
 // (evaluated by k_sph_pairs).  KIND 3: FP64 gravity again for the groups whose
 // split-precision walk found more near pairs than kNearRecs (their results
 // replace that walk's).  KIND 2: the SPH term, inline, for the targets
 // whose list overflowed (groups flagged in gover only; no gravity).
+//
+// TPG < 64: lane l works for target l % TPG; the NS = 64 / TPG lanes of a
+// target split the opening tests of mixed nodes and the swept entries among
+// them (lane masks of nodes and entries have TPG bits).  See walk_tpg for
+// the choice.
 //
 // An accepted node becomes an entry of one of two queues, each swept 64
 // entries at a time:
@@ -264,16 +269,21 @@ __device__ __forceinline__ void bit_pairs(unsigned m, F &&f) {
 // lane it issues 22.6 k vector instructions per wave where one masked sweep
 // issued 28.4 k (1 M disk, FP32), and the kernel takes 0.76 ms against
 // 1.00 ms; the FP64 form 1.24 ms against 1.90 ms.
-template <bool F32, int KIND>
+template <bool F32, int KIND, int TPG>
 __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *lds) {
+    static_assert(TPG == 64 || TPG == 16 || TPG == 8, "targets per group");
+    static_assert(KIND != 2 || TPG == 64, "overflow flags are per group of 64 targets");
+    constexpr int NS = 64 / TPG;
+    constexpr unsigned long long kAll = TPG == 64 ? ~0ull : (1ull << (TPG & 63)) - 1;
     constexpr bool GAS = KIND == 1 || KIND == 2;
-    if (g >= (a.n + 63) / 64) return;
+    if (g >= (a.n + TPG - 1) / TPG) return;
     if (KIND == 2 && !a.gover[g]) return;
     if (KIND == 3 && a.near_cnt[g] <= kNearRecs) return;
     const int wv = threadIdx.x >> 6;
     const int lane = lane_id();
     BlockLds &S = lds[wv];
-    const int t = g * 64 + lane;
+    const int tl = lane & (TPG - 1), sub = lane / TPG;
+    const int t = g * TPG + tl;
     const bool valid_t = t < a.n;
     const int q = t;   // particle state is in key order
     const bool act = valid_t && a.active[q] != 0;
@@ -283,15 +293,15 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     }
     const bool tgas = valid_t && a.stype[t] == 2;
     const double th = act ? a.h[q] : 0.0;
-    const unsigned long long amask = __ballot(act && pm != 0.0);
-    const bool mine = (amask >> lane) & 1ull;
+    const unsigned long long amask = __ballot(act && pm != 0.0) & kAll;
+    const bool mine = (amask >> tl) & 1ull;
     bool sph_lane = GAS && mine && tgas && th > 0.0;
     int slot = -1;
     if (GAS && sph_lane) {
         slot = a.gslot[t];
         if (KIND == 2) sph_lane = a.sph_cnt[slot] > kSphK;
     }
-    const unsigned long long sphB = __ballot(sph_lane);
+    const unsigned long long sphB = __ballot(sph_lane);   // all NS lanes of a target
     const double h2x4 = GAS ? (2.0 * th) * (2.0 * th) : 0.0;   // SPH support (2h)^2
     int lcnt = 0;   // KIND 1: candidates recorded for this target
 
@@ -325,7 +335,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
         // box of the SPH targets and their largest support 2h
         double glo[3] = {px, py, pz}, ghi[3] = {px, py, pz}, h2 = sph_lane ? 2.0 * th : 0.0;
         if (!sph_lane) { glo[0] = glo[1] = glo[2] = 1e308; ghi[0] = ghi[1] = ghi[2] = -1e308; }
-        for (int d = 32; d >= 1; d >>= 1) {
+        for (int d = TPG / 2; d >= 1; d >>= 1) {
             for (int k = 0; k < 3; k++) {
                 double a1 = __shfl_xor(lo[k], d, 64), b1 = __shfl_xor(hi[k], d, 64);
                 lo[k] = a1 < lo[k] ? a1 : lo[k];
@@ -382,7 +392,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
             // at most ext + sqrt(3) D, so D (1 - 2^-19) > near_a + 2^-20 ext
             // is enough.
             float aomax = mine ? ao : 0.f;
-            for (int d = 32; d >= 1; d >>= 1) aomax = fmaxf(aomax, __shfl_xor(aomax, d, 64));
+            for (int d = TPG / 2; d >= 1; d >>= 1) aomax = fmaxf(aomax, __shfl_xor(aomax, d, 64));
             const double ext = 0.5 * ((hi[0] - lo[0]) + (hi[1] - lo[1]) + (hi[2] - lo[2])) * invL;
             const double near_a = uni(4.0 * (double)aomax + 0x1p-20 * ext);
             const double nb = (near_a + 0x1p-20 * ext) * (1.0 + 0x1p-18) * R;
@@ -473,8 +483,8 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                 // r == 0, Node.cpp:274-276, so only distinct particles reach
                 // the sweeps' r == 0 and near-pair tests)
                 const unsigned long long c1B = __ballot(cls == 1);
-                const int self = rpidx - g * 64;
-                const bool drop = rpidx >= 0 && (unsigned)self < 64u;   // (its own leaf: a leaf is class 1 or 0)
+                const int self = rpidx - g * TPG;
+                const bool drop = rpidx >= 0 && (unsigned)self < (unsigned)TPG;   // (its own leaf: a leaf is class 1 or 0)
                 const unsigned long long A = drop ? Mb & ~(1ull << (self & 63)) : Mb;
                 const unsigned long long appB = c1B & __ballot(A != 0ull);
                 unsigned long long fullB = 0ull;
@@ -510,8 +520,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                     const int nmix = __builtin_popcountll(mixB);
                     n_mixed += (unsigned long long)nmix;
                     // The mixed nodes' centres and thresholds go to the staging
-                    // area (free outside the sweep) and are read back at a
-                    // uniform address.  A lane accepts a mixed node when r^2 > rad^2 / (theta^2 (1 - 1e-10)) and opens
+                    // area (free outside the sweep) and are read back NS at a
+                    // time, one per NS'th of the wave.  A lane accepts a mixed
+                    // node when r^2 > rad^2 / (theta^2 (1 - 1e-10)) and opens
                     // it when r^2 < rad^2 / (theta^2 (1 + 1e-10)): outside
                     // that band the reference's rounded radius / sqrt(r^2) <
                     // theta cannot decide otherwise; inside it, its own
@@ -528,7 +539,8 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                     wave_sync_lds();
                     unsigned long long mAA = 0ull, mOO = 0ull;   // decisions on this lane's mixed node
                     unsigned long long bb = mixB;
-                    for (int at = 0; at < nmix; at++) {
+                    for (int m0 = 0; m0 < nmix; m0 += NS) {
+                        const int at = m0 + sub < nmix ? m0 + sub : nmix - 1;
                         const double ncx = S.e.acc[0][at], ncy = S.e.acc[1][at], ncz = S.e.acc[2][at], Tacc = S.e.acc[3][at];
                         const double dx = ncx - px, dy = ncy - py, dz = ncz - pz;
                         const double r2f = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
@@ -538,19 +550,30 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         unsigned long long OO = nz & ~ge;
                         const unsigned long long band = ge & ~AA;
                         if (band) {
-                            const double nrad = rl(rad, __builtin_ctzll(bb));
+                            // the half-widths of the nodes decided here, from their lanes
+                            unsigned long long mm = bb;
+                            if (TPG < 64) {
+                                mm = mixB;
+                                for (int u = 0; u < at; u++) mm &= mm - 1;
+                            }
+                            const double nrad = shfl_d(rad, __builtin_ctzll(mm));
                             const double r2 = dx * dx + dy * dy + dz * dz;
                             const unsigned long long BA = band & __ballot((nrad / sqrt(r2)) < theta);
                             AA |= BA;
                             OO |= band & ~BA;
                         }
-                        const int kk = __builtin_ctzll(bb);
-                        bb &= bb - 1;
-                        mAA = wl(mAA, AA, kk);
-                        mOO = wl(mOO, OO, kk);
+                        if (TPG == 64) {
+                            const int kk = __builtin_ctzll(bb);
+                            bb &= bb - 1;
+                            mAA = wl(mAA, AA, kk);
+                            mOO = wl(mOO, OO, kk);
+                        } else if (cls == 3 && rank - m0 >= 0 && rank - m0 < NS) {
+                            mAA = AA >> (TPG * (rank - m0));
+                            mOO = OO >> (TPG * (rank - m0));
+                        }
                     }
-                    mAA &= Mb;
-                    mOO &= Mb;
+                    mAA &= Mb & kAll;
+                    mOO &= Mb & kAll;
                     const unsigned long long eB = mixB & __ballot(mAA != 0ull);
                     if (in_mask(eB)) {
                         const int slot = ni + mbcnt(eB);
@@ -580,6 +603,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                 const int32_t *enode = part ? S.ent_node : S.ent_full;
                 wave_sync_lds();
                 double ecx = 0.0, ecy = 0.0, ecz = 0.0;
+                // the staged entry's lane mask; TPG < 64: in the field of the
+                // sub that sweeps it (entries [TPG s, TPG (s + 1)) of a
+                // partial chunk)
                 unsigned long long emask = 0ull;
                 bool cand = false;
                 if (lane < cnt) {
@@ -603,15 +629,25 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         double ez = fmax(fmax(glo[2] - w.cz, w.cz - ghi[2]), 0.0);
                         cand = gasn && ex * ex + ey * ey + ez * ez < reach2;
                     }
+                    if (TPG < 64) emask <<= TPG * (lane / TPG);
                 }
                 const unsigned long long candB = GAS ? __ballot(cand) : 0ull;
                 wave_sync_lds();
                 unsigned tlo = (unsigned)emask, thi = (unsigned)(emask >> 32);
                 if (KIND != 2 && part) transpose64(tlo, thi);
-                // each half of a lane's word is walked by itself; a full chunk
-                // has every entry
-                const unsigned long long all = cnt == 64 ? ~0ull : (1ull << cnt) - 1;
-                unsigned word[2] = {part ? tlo : (unsigned)all, part ? thi : (unsigned)(all >> 32)};
+                // Each half of a lane's word is walked by itself (TPG < 64:
+                // only one half holds bits).
+                constexpr int kHalves = TPG == 64 ? 2 : 1;
+                const int half0 = TPG == 64 ? 0 : (2 * sub) / NS;
+                unsigned word[kHalves];
+                if (part) {
+                    word[0] = half0 ? thi : tlo;
+                    if (kHalves == 2) word[kHalves - 1] = thi;
+                } else {   // a full chunk: every entry of the lane's field
+                    const unsigned long long all = (cnt == 64 ? ~0ull : (1ull << cnt) - 1) & (kAll << (TPG * sub & 63));
+                    word[0] = (unsigned)(all >> (32 * half0));
+                    if (kHalves == 2) word[kHalves - 1] = (unsigned)(all >> 32);
+                }
                 // KIND 1: the entries of each half within the lane's SPH
                 // margin, as the sweep meets them (the r^2 it has anyway; one
                 // compare, select and or per entry, where testing the
@@ -619,7 +655,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                 // was a quarter of the walk's instructions), and the entries
                 // resolved or recorded after it
                 const bool spot = KIND == 1 && candB != 0ull;   // uniform
-                unsigned hit[2] = {0u, 0u};
+                unsigned hit[kHalves] = {};
                 unsigned long long hb = 0ull;
                 const bool dfc = F32 && part && dfmode;
                 if (KIND == 2) {
@@ -654,9 +690,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                                          (float)(ezd - (double)(float)ezd), 0.f);
                         }
                         wave_sync_lds();
-                        for (int h = 0; h < 2; h++) {
+                        for (int h = 0; h < kHalves; h++) {
                             auto one = [&](int j, bool on) {
-                                const float4 e = fs[32 * h + j], l = fl[32 * h + j];
+                                const float4 e = fs[32 * (half0 + h) + j], l = fl[32 * (half0 + h) + j];
                                 const float dx = (e.x - xr) + (l.x - xlo), dy = (e.y - yr) + (l.y - ylo);
                                 const float dz = (e.z - zr) + (l.z - zlo);
                                 const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
@@ -669,9 +705,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         }
                     } else if (part) {
                         auto sweep = [&](auto spotting) {
-                            for (int h = 0; h < 2; h++) {
+                            for (int h = 0; h < kHalves; h++) {
                                 auto one = [&](int j, bool on) {
-                                    const float4 e = fs[32 * h + j];
+                                    const float4 e = fs[32 * (half0 + h) + j];
                                     const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
                                     const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
                                     const bool ok = r2 > r2min;
@@ -686,16 +722,18 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         else sweep(std::false_type{});
                     } else {
                         auto sweep = [&](auto spotting) {
-                            for (int h = 0; h < 2; h++) {
+                            for (int h = 0; h < kHalves; h++) {
                                 auto one = [&](int j) {
-                                    const float4 e = fs[j];
+                                    const float4 e = fs[32 * half0 + j];
                                     const float dx = e.x - xr, dy = e.y - yr, dz = e.z - zr;
                                     const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
                                     pull(e.w, dx, dy, dz, r2, true);
                                     if (decltype(spotting)::value) hit[h] |= r2 < lim32 ? 1u << (j & 31) : 0u;
                                 };
-                                int j = 32 * h;
-                                const int je = cnt < 32 * h + 32 ? cnt : 32 * h + 32;
+                                // the lane's field, or (TPG 64, uniform) this half of the chunk
+                                int j = TPG == 64 ? 32 * h : TPG * sub - 32 * half0;
+                                const int je = TPG == 64 ? (cnt < 32 * h + 32 ? cnt : 32 * h + 32)
+                                                         : (cnt - 32 * half0 < j + TPG ? cnt - 32 * half0 : j + TPG);
                                 for (; j + 4 <= je; j += 4) { one(j); one(j + 1); one(j + 2); one(j + 3); }
                                 for (; j < je; j++) one(j);
                             }
@@ -744,7 +782,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                             if (Z) {
                                 if (lane == 0 && nrec < kNearRecs) {
                                     a.near_node[(size_t)g * kNearRecs + nrec] = enode[e0 + jj];
-                                    a.near_mask[(size_t)g * kNearRecs + nrec] = Z;
+                                    a.near_mask[(size_t)g * kNearRecs + nrec] = TPG == 64 ? Z : Z >> (TPG * (jj / TPG));
                                 }
                                 nrec++;
                                 nint -= (unsigned long long)__builtin_popcountll(Z);
@@ -761,9 +799,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                 } else {
                     const double4 *ds4 = S.e.d;
                     auto sweep = [&](auto spotting) {
-                        for (int h = 0; h < 2; h++) {
+                        for (int h = 0; h < kHalves; h++) {
                             auto one = [&](int j, bool on) {
-                                const double4 e = ds4[32 * h + j];
+                                const double4 e = ds4[32 * (half0 + h) + j];
                                 const double dx = e.x - px, dy = e.y - py, dz = e.z - pz;
                                 const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
                                 double gx, gy, gz;
@@ -785,15 +823,26 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                             bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
                         }
                     };
-                    if (!part && !mine) word[0] = word[1] = 0u;
+                    if (!part && !mine) word[0] = word[kHalves - 1] = 0u;
                     if (spot) sweep(std::integral_constant<bool, KIND == 1>{});
                     else sweep(std::false_type{});
                 }
-                // The candidates found go on their target's list in entry order
+                // The candidates found go on their target's list in entry
+                // order (TPG < 64: the NS lanes of a target one after another)
                 if (spot) {
-                    unsigned long long hm = ((hit[0] | (unsigned long long)hit[1] << 32) | hb) & candB;
-                    for (; hm; hm &= hm - 1, lcnt++)
-                        if (lcnt < kSphK) lbase[lcnt] = enode[e0 + __builtin_ctzll(hm)];
+                    unsigned long long hm = hit[0];
+                    if (kHalves == 2) hm |= (unsigned long long)hit[kHalves - 1] << 32;
+                    else hm <<= 32 * half0;
+                    hm = (hm | hb) & candB;
+                    int at = lcnt, add = __builtin_popcountll(hm);
+                    for (int d = TPG; d < 64; d <<= 1) {
+                        const int o = __shfl_xor(add, d, 64);
+                        if (lane & d) at += o;
+                        add += o;
+                    }
+                    lcnt += add;
+                    for (; hm; hm &= hm - 1, at++)
+                        if (at < kSphK) lbase[at] = enode[e0 + __builtin_ctzll(hm)];
                 }
                 // SPH term.  Pairs (target lane t, entry j) with r < 2 h_t are
                 // queued in LDS as they are found and evaluated 64 at a time,
@@ -897,15 +946,21 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     } else {
         ox = s.ax; oy = s.ay; oz = s.az;
     }
-    if (act) { a.ax[q] = ox; a.ay[q] = oy; a.az[q] = oz; }
-    if (KIND == 1 && slot >= 0) {
+    // the NS lanes of a target in a fixed order
+    for (int d = TPG; d < 64; d <<= 1) {
+        ox += __shfl_xor(ox, d, 64);
+        oy += __shfl_xor(oy, d, 64);
+        oz += __shfl_xor(oz, d, 64);
+    }
+    if (act && sub == 0) { a.ax[q] = ox; a.ay[q] = oy; a.az[q] = oz; }
+    if (KIND == 1 && slot >= 0 && sub == 0) {
         a.sph_cnt[slot] = lcnt;
-        if (lcnt > kSphK) a.gover[g] = 1;
+        if (lcnt > kSphK) a.gover[t >> 6] = 1;
     }
     if (KIND == 1) {
         // targets whose candidate list overflowed (their SPH term comes from
         // the overflow walk)
-        const unsigned long long ovB = __ballot(slot >= 0 && lcnt > kSphK);
+        const unsigned long long ovB = __ballot(slot >= 0 && sub == 0 && lcnt > kSphK);
         if (lane == 0) bin_add(a.cbins, kCntSphOver, g, (unsigned long long)__builtin_popcountll(ovB));
     }
     nint += wave_sum_u64((unsigned long long)lnint);
@@ -921,28 +976,53 @@ __device__ inline int wave_group() {
     return xcd_block(blockIdx.x, gridDim.x) * kWaves + (int)(threadIdx.x >> 6);
 }
 
+// Targets per walk group for a set of n particles.  A group is one wave, and
+// the walk of a small set is one wave's latency: with 64 targets per group a
+// set of 10,000 has 157 waves for the chip's 1,024 SIMDs.  Groups of 8 or 16
+// targets give eight or four times the waves, each with a smaller box (fewer
+// nodes) and its sweep split over the 64 / TPG lanes of a target; the whole
+// walk does more traversal work (2.1 and 1.3 times the node tests per lane of
+// a SIMD), which costs once the SIMDs have waves to overlap.  Walk kernel,
+// microseconds, 8 / 16 / 64 targets: Plummer 10,000 FP32 39 / 51 / 130, FP64
+// 44 / 64 / 184; disk 33,333 FP32 89 / 84 / 170; disk 100,003 FP32 180 / 157 /
+// 226, FP64 - / 193 / 305; disk 200,000 FP32 - / 256 / 243, FP64 - / 330 /
+// 366; disk 1 M FP32 - / 1014 / 759, FP64 - / 1340 / 1239.  The choice
+// depends on the set alone, so a job of a batched walk has the arithmetic of
+// a walk of its own.
+constexpr int kTpg8Max = 24576, kTpg16Max32 = 150000, kTpg16Max64 = 280000;
+inline int walk_tpg(int64_t n, bool f32) {
+    return n <= kTpg8Max ? 8 : n <= (f32 ? kTpg16Max32 : kTpg16Max64) ? 16 : 64;
+}
+
 // Kernels per precision form: gravity with SPH candidate recording (any gas
 // uploaded) or plain gravity, and the overflow SPH walk (FP64 for both forms).
 #define AG2_WALK_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 
 __global__ AG2_WALK_BOUNDS void k_walk_block64(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
-    walk_block<false, 1>(a, wave_group(), lds);
+    walk_block<false, 1, 64>(a, wave_group(), lds);
 }
 
 __global__ AG2_WALK_BOUNDS void k_walk_block64_nogas(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
-    walk_block<false, 0>(a, wave_group(), lds);
+    walk_block<false, 0, 64>(a, wave_group(), lds);
 }
 
 __global__ AG2_WALK_BOUNDS void k_walk_block32(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
-    walk_block<true, 1>(a, wave_group(), lds);
+    walk_block<true, 1, 64>(a, wave_group(), lds);
 }
 
 __global__ AG2_WALK_BOUNDS void k_walk_block32_nogas(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
-    walk_block<true, 0>(a, wave_group(), lds);
+    walk_block<true, 0, 64>(a, wave_group(), lds);
+}
+
+// ... in groups of fewer targets (walk_tpg)
+template <bool F32, int KIND, int TPG>
+__global__ AG2_WALK_BOUNDS void k_walk_small(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<F32, KIND, TPG>(a, wave_group(), lds);
 }
 
 // The overflow walk and the near pass usually touch few groups, but a
@@ -951,16 +1031,17 @@ __global__ AG2_WALK_BOUNDS void k_walk_block32_nogas(WalkArgs a) {
 // flagged, keeps those walks in parallel.
 __global__ AG2_WALK_BOUNDS void k_walk_sph_overflow(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
-    walk_block<false, 2>(a, wave_group(), lds);   // exits unless the group is flagged in gover
+    walk_block<false, 2, 64>(a, wave_group(), lds);   // exits unless the group is flagged in gover
 }
 
 // The near pairs of a split-precision walk in FP64 on the FP64 positions,
 // the reference's law (Node.cpp:337-365; r == 0 skipped, Node.cpp:274-276),
 // added to the walk's results in record order.  Groups with more records
 // than kept are walked again in FP64 instead (k_near_pass).
+template <int TPG>
 __device__ inline void near_fp64_group(const WalkArgs &a, int g, int cnt) {
     const int lane = lane_id();
-    const int t = g * 64 + lane;
+    const int t = g * TPG + lane;   // lanes past TPG are in no record's mask
     double px = 0.0, py = 0.0, pz = 0.0;
     if (t < a.n) { px = a.sx[t]; py = a.sy[t]; pz = a.sz[t]; }
     double fx = 0.0, fy = 0.0, fz = 0.0;
@@ -993,16 +1074,17 @@ __device__ inline void near_fp64_group(const WalkArgs &a, int g, int cnt) {
 
 // The near pass: groups with at most kNearRecs recorded pairs evaluate them
 // in FP64 (near_fp64_group); groups with more are walked again in FP64.
+template <int TPG>
 __global__ AG2_WALK_BOUNDS void k_near_pass(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
     const int g = wave_group();
-    if (g >= (a.n + 63) / 64) return;
+    if (g >= (a.n + TPG - 1) / TPG) return;
     const int cnt = a.near_cnt[g];
     if (cnt > kNearRecs) {
         if (lane_id() == 0) bin_add(a.cbins, kCntNearRedo, g, 1ull);
-        walk_block<false, 3>(a, g, lds);
+        walk_block<false, 3, TPG>(a, g, lds);
     } else if (cnt > 0) {
-        near_fp64_group(a, g, cnt);
+        near_fp64_group<TPG>(a, g, cnt);
     }
 }
 
@@ -1013,7 +1095,7 @@ __global__ AG2_WALK_BOUNDS void k_near_pass(WalkArgs a) {
 struct JobWalk {
     WalkArgs a;
     int group0;
-    int pad;
+    int tpg;   // targets per group (walk_tpg of the job's own n)
 };
 
 __device__ inline int find_job(const JobWalk *jobs, int nj, int G) {
@@ -1030,7 +1112,10 @@ __device__ __forceinline__ void walk_jobs(const JobWalk *jobs, int nj, int total
     const int G = wave_group();
     if (G >= total) return;   // whole waves only: nothing below synchronises across waves
     const int j = find_job(jobs, nj, G);
-    walk_block<F32, KIND>(jobs[j].a, G - jobs[j].group0, lds);
+    const int g = G - jobs[j].group0, tpg = jobs[j].tpg;
+    if (tpg == 64) walk_block<F32, KIND, 64>(jobs[j].a, g, lds);
+    else if (tpg == 16) walk_block<F32, KIND, 16>(jobs[j].a, g, lds);
+    else walk_block<F32, KIND, 8>(jobs[j].a, g, lds);
 }
 
 __global__ AG2_WALK_BOUNDS void k_walk_jobs64(const JobWalk *jobs, int nj, int total) {
@@ -1270,8 +1355,8 @@ void forces_batch(Ctx *const *cs, int nc, hipStream_t st, int f32, void *scratch
     for (int k = 0; k < nc; k++) {
         hj[k].a = walk_args(*cs[k]);
         hj[k].group0 = total;
-        hj[k].pad = 0;
-        total += (int)((cs[k]->n + 63) / 64);
+        hj[k].tpg = walk_tpg(cs[k]->n, f32 != 0);
+        total += (int)((cs[k]->n + hj[k].tpg - 1) / hj[k].tpg);
         gas = gas || cs[k]->sph_active;
     }
     JobWalk *dj = (JobWalk *)scratch_dev;
@@ -1326,23 +1411,46 @@ void sph_finish(Ctx &c) {
 // too many of them walked again in FP64 (both exit at once for other groups).
 void near_finish(Ctx &c) {
     WalkArgs a = walk_args(c);
-    const int groups = (int)((c.n + 63) / 64);
-    hipLaunchKernelGGL(k_near_pass, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, c.stream, a);
+    const int tpg = walk_tpg(c.n, true);
+    const int groups = (int)((c.n + tpg - 1) / tpg);
+    const dim3 grid((groups + kWaves - 1) / kWaves), block(64 * kWaves);
+    if (tpg == 64) hipLaunchKernelGGL(k_near_pass<64>, grid, block, 0, c.stream, a);
+    else if (tpg == 16) hipLaunchKernelGGL(k_near_pass<16>, grid, block, 0, c.stream, a);
+    else hipLaunchKernelGGL(k_near_pass<8>, grid, block, 0, c.stream, a);
     AG2_HIP(hipGetLastError());
 }
 
-// The gravity walk of one context.
+int64_t walk_groups_max(int64_t cap) {
+    int64_t most = cap / 64;
+    const int64_t at[2][2] = {{kTpg8Max, 8}, {kTpg16Max32, 16}};   // the records are the split form's
+    for (const auto &r : at) {
+        const int64_t g = (cap < r[0] ? cap : r[0]) / r[1];
+        most = g > most ? g : most;
+    }
+    return most + 1;
+}
+
+// The gravity walk of one context, in groups of walk_tpg targets.
 template <bool F32>
 static void launch_walk(Ctx &c) {
     const WalkArgs a = walk_args(c);
-    const int groups = (int)((c.n + 63) / 64);
+    const int tpg = walk_tpg(c.n, F32);
+    const int groups = (int)((c.n + tpg - 1) / tpg);
     const dim3 grid((groups + kWaves - 1) / kWaves), block(64 * kWaves);
-    if (F32) {
-        if (c.sph_active) hipLaunchKernelGGL(k_walk_block32, grid, block, 0, c.stream, a);
-        else hipLaunchKernelGGL(k_walk_block32_nogas, grid, block, 0, c.stream, a);
+    hipStream_t st = c.stream;
+    const bool gas = c.sph_active;
+    if (tpg == 8) {
+        if (gas) hipLaunchKernelGGL((k_walk_small<F32, 1, 8>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_walk_small<F32, 0, 8>), grid, block, 0, st, a);
+    } else if (tpg == 16) {
+        if (gas) hipLaunchKernelGGL((k_walk_small<F32, 1, 16>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_walk_small<F32, 0, 16>), grid, block, 0, st, a);
+    } else if (F32) {
+        if (gas) hipLaunchKernelGGL(k_walk_block32, grid, block, 0, st, a);
+        else hipLaunchKernelGGL(k_walk_block32_nogas, grid, block, 0, st, a);
     } else {
-        if (c.sph_active) hipLaunchKernelGGL(k_walk_block64, grid, block, 0, c.stream, a);
-        else hipLaunchKernelGGL(k_walk_block64_nogas, grid, block, 0, c.stream, a);
+        if (gas) hipLaunchKernelGGL(k_walk_block64, grid, block, 0, st, a);
+        else hipLaunchKernelGGL(k_walk_block64_nogas, grid, block, 0, st, a);
     }
 }
 

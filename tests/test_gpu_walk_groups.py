@@ -44,7 +44,7 @@ def check(ag2, orc, ps, theta, precision, thr=800):
 
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("theta", [0.05, 0.5, 1.2])
-@pytest.mark.parametrize("n", [5, 64, 65, 127, 129, 700, 4099])
+@pytest.mark.parametrize("n", [5, 8, 9, 16, 17, 64, 65, 127, 129, 700, 4099])
 def test_counts_around_groups_and_chunks(ag2, orc, n, theta, precision):
     nh, nd = n // 2, n // 4
     check(ag2, orc, ag2.ics.disk_galaxy(nh, nd, n - nh - nd, seed=n), theta, precision)
@@ -53,3 +53,11 @@ def test_counts_around_groups_and_chunks(ag2, orc, n, theta, precision):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_gas_free_sphere(ag2, orc, precision):
     check(ag2, orc, ag2.ics.config1_plummer(3001, seed=5), 0.4, precision)
+
+
+@pytest.mark.parametrize("n,precision", [(24576, 0), (24577, 1), (150000, 1), (150001, 1), (280000, 0), (280001, 0)])
+def test_group_size_limits(ag2, orc, n, precision):
+    """Either side of the particle counts where the walk's groups change size
+    (8, 16, 64 targets)."""
+    nh, nd = n // 2, (3 * n) // 10
+    check(ag2, orc, ag2.ics.disk_galaxy(nh, nd, n - nh - nd, seed=2), 0.5, precision)
