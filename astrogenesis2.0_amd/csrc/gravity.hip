@@ -188,9 +188,22 @@ __device__ inline void sph_pair(double dx, double dy, double dz, double r2, doub
     core::sph_term_hoisted(dx, dy, dz, r2, gas, vx, vy, vz, k, s);
 }
 
-// xcd_block (ag2_internal.h) keeps neighbouring groups, which read mostly
-// the same tree records, on the same L2.
-
+// Workgroups reach the 8 XCDs round robin.  Neighbouring groups read mostly
+// the same tree records and should share one XCD's L2, but one contiguous
+// eighth of the key order per XCD leaves XCDs idle behind the one that holds
+// the longest lists.  So each XCD takes runs of kXcdRun workgroups in turn
+// (the last, incomplete round is split evenly).  Walk kernel, one eighth per
+// XCD / runs of 16: 1 M disk FP32 755 / 709 us, FP64 1,242 / 1,192; 1 M
+// Hernquist 669 / 620; 100,003 disk 158 / 143; 2 M 1,370 / 1,315; 200,000
+// 241 / 244; 3 M 1,947 / 1,966.  Runs of 2, 4, 8 and 32 lie between; of 64,
+// 720 us at 1 M.
+constexpr int kXcdRun = 16;
+__device__ inline int walk_workgroup(int b, int nb) {
+    const int whole = nb / (8 * kXcdRun) * (8 * kXcdRun);
+    if (b >= whole) return whole + xcd_block(b - whole, nb - whole);
+    const int x = b & 7, i = b >> 3;
+    return (i / kXcdRun * 8 + x) * kXcdRun + i % kXcdRun;
+}
 
 // Transpose of a 64 x 64 bit matrix held one row per lane: lane j gives row j
 // (lo: columns 0..31, hi: 32..63) and gets column j.  Halves are exchanged
@@ -973,7 +986,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
 }
 
 __device__ inline int wave_group() {
-    return xcd_block(blockIdx.x, gridDim.x) * kWaves + (int)(threadIdx.x >> 6);
+    return walk_workgroup(blockIdx.x, gridDim.x) * kWaves + (int)(threadIdx.x >> 6);
 }
 
 // Targets per walk group for a set of n particles.  A group is one wave, and
