@@ -88,7 +88,6 @@ struct Ctx {
     double *alt[kStateD] = {};
     uint8_t *type_alt = nullptr, *active_alt = nullptr;
     uint32_t *rid_alt = nullptr;
-    double *stage = nullptr;     // n values: caller-order staging for download
     int32_t *inv = nullptr;      // caller index -> resident slot, built on demand
     double *vd = nullptr;        // visual density in key order, allocated on first use
     double *sfr = nullptr;       // Particle::sfr in caller order (written by the second kick)
@@ -150,6 +149,7 @@ struct Ctx {
     // order (Node.cpp:479, :681).  When every gas particle has the same mass m
     // that sum depends only on the count k: gas_table[k] = fl(gas_table[k-1] + m).
     double *gas_table = nullptr;
+    int64_t gas_table_cap = 0;   // entries it holds (kept for later uploads)
     int gas_equal = 0;
     bool sph_active = false;   // any gas particle uploaded: forces record and evaluate SPH candidates
     int64_t gas_count = 0;     // gas particles uploaded
@@ -366,6 +366,15 @@ void direct_sum_noalloc(Ctx &c, int nt, const int64_t *h_targets, double *ax, do
 void state_fields(Ctx &c, double **f[kStateD]);   // tree_build.hip: the kStateD arrays, in a fixed order
 void build_inverse(Ctx &c);              // tree_build.hip: inv[rid[r]] = r
 void reset_graphs(Ctx &c);               // tree_build.hip: drop the captured build segments
+// transfer.hip: columns between the caller's arrays and the device, through
+// pinned buffers that the device's contexts share (ref / unref: one per
+// context).
+void transfer_ref(int device);
+void transfer_unref(int device);
+void fields_to_host(Ctx &c, int nf, const double *const *src, double *const *host, const uint8_t *type,
+                    uint8_t *htype);
+void fields_to_device(Ctx &c, int nf, double *const *dst, const double *const *host, const double *dflt,
+                      const uint8_t *htype);
 
 // Contexts (api.hip).  ctx_new: stream == nullptr creates the context's own
 // stream, otherwise the context runs on the given one (a serving pool's).

@@ -11,27 +11,6 @@ using ag2::Ctx;
 
 namespace {
 
-__global__ __launch_bounds__(256) void k_fill_f64(int n, double *a, double v) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) a[i] = v;
-}
-
-__global__ __launch_bounds__(256) void k_iota_u32(int n, uint32_t *a) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) a[i] = (uint32_t)i;
-}
-
-// Resident slot r holds caller index rid[r].
-__global__ __launch_bounds__(256) void k_to_caller_f64(int n, const uint32_t *rid, const double *src, double *dst) {
-    int r = blockIdx.x * 256 + threadIdx.x;
-    if (r < n) dst[rid[r]] = src[r];
-}
-
-__global__ __launch_bounds__(256) void k_to_caller_u8(int n, const uint32_t *rid, const uint8_t *src, uint8_t *dst) {
-    int r = blockIdx.x * 256 + threadIdx.x;
-    if (r < n) dst[rid[r]] = src[r];
-}
-
 const char *kNullCtx = "null context";
 
 int fail(Ctx *c, int code, const std::string &msg) {
@@ -75,13 +54,14 @@ void free_all(Ctx &c) {
         if (e) (void)hipEventDestroy(e);
     if (c.ev_counts) (void)hipEventDestroy(c.ev_counts);
     if (c.stream && c.own_stream) (void)hipStreamDestroy(c.stream);
+    ag2::transfer_unref(c.device);
 }
 
 void alloc_all(Ctx &c, int64_t cap) {
     const size_t n = (size_t)cap;
     auto plan = [&](ag2::Carve &cv) {
         double **d[] = {&c.x, &c.y, &c.z, &c.vx, &c.vy, &c.vz, &c.m, &c.U, &c.mu, &c.ax, &c.ay, &c.az, &c.h, &c.rho,
-                        &c.P, &c.T, &c.dUdt, &c.ts, &c.next, &c.pot, &c.stage, &c.sfr};
+                        &c.P, &c.T, &c.dUdt, &c.ts, &c.next, &c.pot, &c.sfr};
         for (double **p : d) cv(p, n * 8);
         for (double *&p : c.alt) cv(&p, n * 8);
         cv(&c.type, n); cv(&c.active, n); cv(&c.gapl, n);
@@ -120,11 +100,6 @@ void alloc_all(Ctx &c, int64_t cap) {
     AG2_HIP(hipEventCreateWithFlags(&c.ev_counts, hipEventDisableTiming));
 }
 
-void upload_field(Ctx &c, double *dst, const double *src, double dflt) {
-    if (src) AG2_HIP(hipMemcpyAsync(dst, src, (size_t)c.n * 8, hipMemcpyHostToDevice, c.stream));
-    else hipLaunchKernelGGL(k_fill_f64, dim3(ag2::grid_for(c.n, 256)), dim3(256), 0, c.stream, (int)c.n, dst, dflt);
-}
-
 // 0 when either event was never recorded (timing_events above 0); the
 // failed query's error is cleared so that later launches do not report it.
 float ev_ms(Ctx &c, int a, int b) {
@@ -161,7 +136,7 @@ int check_params(const ag2_params *p, std::string &why) {
 // arrays at 2 capacity + 64, sort histograms and tiles).
 int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
     int64_t n = cap, nodes = 2 * cap + 64;
-    int64_t per_p = 22 * 8            // state, potential, staging, star-formation rate
+    int64_t per_p = 21 * 8            // state, potential, star-formation rate
                     + kStateD * 8     // permute buffers
                     + 7               // type, active, gap level, their copies, lcp, adjacent key levels
                     + 4 * 8 + 2 * 4   // keys, sort indices
@@ -186,6 +161,7 @@ Ctx *ctx_new(const ag2_params &p, int64_t capacity, hipStream_t stream) {
     c->cap = capacity;
     // captured sort segments keep their passes: graph launches sort every byte
     c->sort_lo = p.graph_launch ? 0 : ag2::kSortLoMax;
+    ag2::transfer_ref(c->device);
     try {
         AG2_HIP(hipSetDevice(c->device));
         // once per device, with the device current: the address of the
@@ -220,18 +196,12 @@ void ctx_upload(Ctx &ctx, const ag2_particles &h) {
     {
         ag2::reset_graphs(*c);   // the particle count is an argument of the captured segments
         c->n = hp->n;
-        upload_field(*c, c->x, hp->x, 0); upload_field(*c, c->y, hp->y, 0); upload_field(*c, c->z, hp->z, 0);
-        upload_field(*c, c->vx, hp->vx, 0); upload_field(*c, c->vy, hp->vy, 0); upload_field(*c, c->vz, hp->vz, 0);
-        upload_field(*c, c->m, hp->m, 0); upload_field(*c, c->U, hp->U, 0); upload_field(*c, c->mu, hp->mu, 0.58);
-        upload_field(*c, c->ax, hp->ax, 0); upload_field(*c, c->ay, hp->ay, 0); upload_field(*c, c->az, hp->az, 0);
-        upload_field(*c, c->h, hp->h, 0); upload_field(*c, c->rho, hp->rho, 0); upload_field(*c, c->P, hp->P, 0);
-        upload_field(*c, c->T, hp->T, 0); upload_field(*c, c->dUdt, hp->dUdt, 0);
-        upload_field(*c, c->ts, nullptr, 0); upload_field(*c, c->next, nullptr, 0);
-        upload_field(*c, c->sfr, nullptr, 0);
-        if (hp->type) AG2_HIP(hipMemcpyAsync(c->type, hp->type, (size_t)c->n, hipMemcpyHostToDevice, c->stream));
-        else AG2_HIP(hipMemsetAsync(c->type, 1, (size_t)c->n, c->stream));
-        ag2::fill_active(*c, 1);
-        hipLaunchKernelGGL(k_iota_u32, dim3(ag2::grid_for(c->n, 256)), dim3(256), 0, c->stream, (int)c->n, c->rid);
+        double *const dst[] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->m, c->U, c->mu, c->ax, c->ay, c->az, c->h,
+                               c->rho, c->P, c->T, c->dUdt, c->ts, c->next, c->sfr};
+        const double *const src[] = {hp->x, hp->y, hp->z, hp->vx, hp->vy, hp->vz, hp->m, hp->U, hp->mu, hp->ax, hp->ay,
+                                     hp->az, hp->h, hp->rho, hp->P, hp->T, hp->dUdt, nullptr, nullptr, nullptr};
+        const double dflt[] = {0, 0, 0, 0, 0, 0, 0, 0, 0.58, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        ag2::fields_to_device(*c, 20, dst, src, dflt, hp->type);
         AG2_HIP(hipMemsetAsync(c->ds, 0, sizeof(ag2::DevState), c->stream));
         // running gas-mass sums of equal-mass gas (see Ctx::gas_table)
         int64_t ng = 0;
@@ -260,12 +230,15 @@ void ctx_upload(Ctx &ctx, const ag2_particles &h) {
             AG2_HIP(hipMalloc(&c->sph_cnt, (size_t)cap * 4));
             c->sph_cap = cap;
         }
-        if (c->gas_table) { AG2_HIP(hipFree(c->gas_table)); c->gas_table = nullptr; }
         if (c->gas_equal) {
             std::vector<double> tab((size_t)ng + 1);
             tab[0] = 0.0;
             for (int64_t k = 1; k <= ng; k++) tab[(size_t)k] = tab[(size_t)k - 1] + mg;
-            AG2_HIP(hipMalloc(&c->gas_table, ((size_t)ng + 1) * 8));
+            if (ng + 1 > c->gas_table_cap) {
+                if (c->gas_table) { AG2_HIP(hipFree(c->gas_table)); c->gas_table = nullptr; c->gas_table_cap = 0; }
+                AG2_HIP(hipMalloc(&c->gas_table, ((size_t)ng + 1) * 8));
+                c->gas_table_cap = ng + 1;
+            }
             AG2_HIP(hipMemcpyAsync(c->gas_table, tab.data(), ((size_t)ng + 1) * 8, hipMemcpyHostToDevice, c->stream));
             AG2_HIP(hipStreamSynchronize(c->stream));
         }
@@ -281,23 +254,16 @@ void ctx_download(Ctx &ctx, ag2_particles &h) {
     ag2_particles *hp = &h;
     Ctx *c = &ctx;
     {
-        struct F { double *h; double *d; } fs[] = {{hp->x, c->x}, {hp->y, c->y}, {hp->z, c->z}, {hp->vx, c->vx},
-            {hp->vy, c->vy}, {hp->vz, c->vz}, {hp->m, c->m}, {hp->U, c->U}, {hp->mu, c->mu}, {hp->ax, c->ax},
-            {hp->ay, c->ay}, {hp->az, c->az}, {hp->h, c->h}, {hp->rho, c->rho}, {hp->P, c->P}, {hp->T, c->T},
-            {hp->dUdt, c->dUdt}};
-        // resident (key) order -> caller order through rid, one field at a
-        // time via the staging buffer (stream order keeps the copies apart)
-        unsigned gb = ag2::grid_for(c->n, 256);
-        for (auto &f : fs)
-            if (f.h) {
-                hipLaunchKernelGGL(k_to_caller_f64, dim3(gb), dim3(256), 0, c->stream, (int)c->n, c->rid, f.d, c->stage);
-                AG2_HIP(hipMemcpyAsync(f.h, c->stage, (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
-            }
-        if (hp->type) {
-            uint8_t *st8 = (uint8_t *)c->stage;
-            hipLaunchKernelGGL(k_to_caller_u8, dim3(gb), dim3(256), 0, c->stream, (int)c->n, c->rid, c->type, st8);
-            AG2_HIP(hipMemcpyAsync(hp->type, st8, (size_t)c->n, hipMemcpyDeviceToHost, c->stream));
-        }
+        double *const hf[] = {hp->x, hp->y, hp->z, hp->vx, hp->vy, hp->vz, hp->m, hp->U, hp->mu, hp->ax, hp->ay,
+                              hp->az, hp->h, hp->rho, hp->P, hp->T, hp->dUdt};
+        const double *const df[] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->m, c->U, c->mu, c->ax, c->ay, c->az,
+                                    c->h, c->rho, c->P, c->T, c->dUdt};
+        const double *src[17];
+        double *dst[17];
+        int nf = 0;
+        for (int f = 0; f < 17; f++)
+            if (hf[f]) { src[nf] = df[f]; dst[nf++] = hf[f]; }
+        ag2::fields_to_host(*c, nf, src, dst, c->type, hp->type);
         AG2_HIP(hipStreamSynchronize(c->stream));
     }
 }
@@ -596,9 +562,9 @@ int ag2_visual_density(void *ctx, double radius, double *out) {
         if (!c->vd) AG2_HIP(hipMalloc(&c->vd, (size_t)c->cap * 8));
         ag2::visual_density(*c, radius > 0.0 ? radius : c->vd_radius0, c->vd);
         if (out) {
-            hipLaunchKernelGGL(k_to_caller_f64, dim3(ag2::grid_for(c->n, 256)), dim3(256), 0, c->stream, (int)c->n,
-                               c->rid, c->vd, c->stage);
-            AG2_HIP(hipMemcpyAsync(out, c->stage, (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
+            const double *src[] = {c->vd};
+            double *dst[] = {out};
+            ag2::fields_to_host(*c, 1, src, dst, nullptr, nullptr);
         }
         AG2_HIP(hipStreamSynchronize(c->stream));
         return AG2_OK;
