@@ -32,14 +32,11 @@ constexpr double kPRTN = 1.6726219e-27;
 constexpr double kKMS = 1.0e3;
 constexpr double kMPC = 3.08567758149137e22;
 
-using core::WalkNode;
-
 // Sums of a node (tree_build.hip k_moments_up): mass, mass-weighted position,
 // gas mass, gas-mass-weighted velocity.
 struct alignas(64) NodeSums {
     double m, sx, sy, sz, g, gx, gy, gz;
 };
-static_assert(sizeof(WalkNode) == 64, "WalkNode must be 64 bytes");
 
 // Scalars that live in device memory so that a step needs no host round trip.
 struct DevState {
@@ -125,8 +122,6 @@ struct Ctx {
     double *n_mass = nullptr;
     double *n_gas = nullptr, *n_gvx = nullptr, *n_gvy = nullptr, *n_gvz = nullptr;
     double *n_cx = nullptr, *n_cy = nullptr, *n_cz = nullptr;
-    WalkNode *wnode = nullptr;   // pre-order records of the potential walk, built on demand
-    bool wnode_valid = false;
     // child-contiguous layout for the block walk
     core::TreeNode *tnode = nullptr;
     core::SphNode *tsph = nullptr;   // SPH records in the walk layout (written when gas is present)
@@ -356,7 +351,6 @@ void kdk_init_steps(Ctx &c);
 void energies(Ctx &c, int with_pot, double out[6]);
 void fill_active(Ctx &c, uint8_t v);
 void alloc_nodes(Ctx &c, int64_t node_cap);
-void pack_walknodes(Ctx &c);             // tree_build.hip: pre-order records for the potential walk
 void direct_sum(Ctx &c, int nt, const int64_t *d_targets, double *d_out, int with_pot);   // direct.hip
 // direct.hip: the device address of the no-allocation scratch on `device`
 // (current), looked up once per device; then the direct sum of host-listed

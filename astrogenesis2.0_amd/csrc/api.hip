@@ -143,7 +143,7 @@ int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
                     + 3 * 4           // rid, rid copy, inverse
                     + 2 * 4           // c, base
                     + 2 * 4 + 1;      // SPH list slots, targets, group flags
-    int64_t per_node = 5 * 4 + 1 + 9 * 8 + (int64_t)sizeof(WalkNode) + 2 * 4 + 1 + 4 +
+    int64_t per_node = 5 * 4 + 1 + 9 * 8 + 2 * 4 + 1 + 4 +
                        2 * (int64_t)sizeof(core::TreeNode) + 3 * 4 +   // walk and SPH records
                        (int64_t)sizeof(ag2::NodeSums) + 4 +            // node sums, internal-child counts
                        (int64_t)sizeof(ag2::NodeSums) / 64 + 1;        // block sums

@@ -38,9 +38,8 @@
 // is m' / sqrt(r'^2 (r'^2 + e'^2)^2) with one v_rsq_f32, each 64-entry chunk
 // is summed plainly and added to the running total with Kahan compensation.
 // The SPH term is FP64 in both forms.
-//
-// k_walk64 (one lane per target, stackless) is kept for the potential.
 #include "ag2_internal.h"
+#include "fp64_math.h"
 
 #include <type_traits>
 
@@ -92,7 +91,7 @@ struct WalkArgs {
     const DevState *ds;
     unsigned long long *cbins;   // spread counters (bin_add), folded into the DevState after the forces
     core::WalkParams wp;
-    double *ax, *ay, *az, *dUdt;
+    double *ax, *ay, *az, *dUdt, *pot;
     DevState *dsw;
     // split-precision walk: near pairs per group (count, then kNearRecs
     // records of node and lane mask), evaluated in FP64 by k_near_pass
@@ -262,6 +261,7 @@ __device__ __forceinline__ void bit_pairs(unsigned m, F &&f) {
 // split-precision walk found more near pairs than kNearRecs (their results
 // replace that walk's).  KIND 2: the SPH term, inline, for the targets
 // whose list overflowed (groups flagged in gover only; no gravity).
+// KIND 4: the FP64 potential of every target (active or not).
 //
 // TPG < 64: lane l works for target l % TPG; the NS = 64 / TPG lanes of a
 // target split the opening tests of mixed nodes and the swept entries among
@@ -299,13 +299,13 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     const int t = g * TPG + tl;
     const bool valid_t = t < a.n;
     const int q = t;   // particle state is in key order
-    const bool act = valid_t && a.active[q] != 0;
+    const bool act = valid_t && (KIND == 4 || a.active[q] != 0);
     double px = 0.0, py = 0.0, pz = 0.0, pm = 0.0;
     if (valid_t) {
         px = a.sx[t]; py = a.sy[t]; pz = a.sz[t]; pm = a.sm[t];
     }
     const bool tgas = valid_t && a.stype[t] == 2;
-    const double th = act ? a.h[q] : 0.0;
+    const double th = KIND != 4 && act ? a.h[q] : 0.0;
     const unsigned long long amask = __ballot(act && pm != 0.0) & kAll;
     const bool mine = (amask >> tl) & 1ull;
     bool sph_lane = GAS && mine && tgas && th > 0.0;
@@ -631,7 +631,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         lnint += (unsigned)__builtin_popcountll(emask);   // less the lanes excluded below
                     } else if (KIND != 2) {
                         // G m staged once per entry (the sweep forms ((G m) rcp) ri, as before)
-                        S.e.d[lane] = make_double4(w.cx, w.cy, w.cz, a.wp.soft_live ? w.mass : a.wp.G * w.mass);
+                        S.e.d[lane] = make_double4(w.cx, w.cy, w.cz, KIND == 4 || a.wp.soft_live ? w.mass : a.wp.G * w.mass);
                     }
                     if (GAS && sphB && (emask & sphB)) {
                         // a leaf's gas mass is its mass when it is gas; nodes of
@@ -817,6 +817,15 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                 const double4 e = ds4[32 * (half0 + h) + j];
                                 const double dx = e.x - px, dy = e.y - py, dz = e.z - pz;
                                 const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+                                if (KIND == 4) {
+                                    // -(G / e0) m (pi/2 - atan(r / e0)), scaled at the end
+                                    if (r2 != 0.0 && on) {
+                                        const double ir = rsq_full(r2);
+                                        s.pot = __builtin_fma(e.w, softened_angle(a.wp.e0, r2 * ir, ir), s.pot);
+                                        lnint++;
+                                    }
+                                    return;
+                                }
                                 double gx, gy, gz;
                                 bool ok = true;
                                 if (a.wp.soft_live) {
@@ -934,7 +943,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
             }
             if (sp == 0 && ni + nf == 0) break;
         }
-        if (KIND != 2 && lane == 0) {
+        if (KIND != 2 && KIND != 4 && lane == 0) {
             bin_add(a.cbins, kCntEntries, g, n_entries);
             bin_add(a.cbins, kCntTests, g, n_tests);
             bin_add(a.cbins, kCntMixed, g, n_mixed);
@@ -948,6 +957,16 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
         }
         unsigned long long cs = wave_sum_u64((unsigned long long)s.nsph);
         if (lane == 0) bin_add(a.cbins, kCntSphPairs, g, cs);
+        return;
+    }
+    if (KIND == 4) {
+        double ph = s.pot;
+        int any = lnint != 0u;
+        for (int d = TPG; d < 64; d <<= 1) {
+            ph += __shfl_xor(ph, d, 64);
+            any |= __shfl_xor(any, d, 64);
+        }
+        if (valid_t && sub == 0) a.pot[q] = any ? -(a.wp.G / a.wp.e0) * ph : 0.0;
         return;
     }
     double ox, oy, oz;
@@ -1036,6 +1055,16 @@ template <bool F32, int KIND, int TPG>
 __global__ AG2_WALK_BOUNDS void k_walk_small(WalkArgs a) {
     __shared__ BlockLds lds[kWaves];
     walk_block<F32, KIND, TPG>(a, wave_group(), lds);
+}
+
+// The potential (energy diagnostics): the same walk, the softened potential
+// in place of the force.  One lane per target walking the pre-order nodes by
+// itself took 3.58 ms on the 1 M disk (uncoalesced records, a square root, a
+// quotient and the library's atan per pair); this takes 1.20 ms.
+template <int TPG>
+__global__ AG2_WALK_BOUNDS void k_walk_potential(WalkArgs a) {
+    __shared__ BlockLds lds[kWaves];
+    walk_block<false, 4, TPG>(a, wave_group(), lds);
 }
 
 // The overflow walk and the near pass usually touch few groups, but a
@@ -1295,48 +1324,6 @@ __global__ void k_zero_job_counters(const JobWalk *jobs, int nj) {
     ds->near_redo = 0ull;
 }
 
-// One lane per target, stackless pre-order walk (core::walk_fp64); used for
-// the potential diagnostic.
-__global__ __launch_bounds__(256) void k_walk64(int n, int nin, int nn, const WalkNode *__restrict__ wn,
-                                                const double *__restrict__ sx,
-                                                const double *__restrict__ sy, const double *__restrict__ sz,
-                                                const double *__restrict__ sm, const uint8_t *__restrict__ stype,
-                                                const double *__restrict__ svx, const double *__restrict__ svy,
-                                                const double *__restrict__ svz, const double *__restrict__ mvx,
-                                                const double *__restrict__ mvy, const double *__restrict__ mvz,
-                                                const double *__restrict__ h, const double *__restrict__ rho,
-                                                const double *__restrict__ P, const uint8_t *__restrict__ active,
-                                                core::WalkParams wp, int mode, double *ax, double *ay, double *az,
-                                                double *dUdt, double *pot, DevState *ds) {
-    int t = blockIdx.x * 256 + threadIdx.x;
-    core::WalkSums s{0, 0, 0, 0, 0, 0, 0};
-    if (t < n) {
-        int q = t;
-        bool act = mode == 1 || active[q];
-        if (act) {
-            core::Target tg;
-            tg.x = sx[t]; tg.y = sy[t]; tg.z = sz[t]; tg.m = sm[t];
-            tg.vx = svx[t]; tg.vy = svy[t]; tg.vz = svz[t];
-            tg.h = h[q]; tg.rho = rho[q]; tg.P = P[q];
-            tg.gas = stype[t] == 2;
-            tg.self = t < nin ? t : -1;
-            core::walk_fp64(wn, nn, tg, svx, svy, svz, stype, mvx, mvy, mvz, wp, mode, &s);
-            if (mode == 0) {
-                ax[q] = s.ax; ay[q] = s.ay; az[q] = s.az;
-                dUdt[q] += s.du;
-            } else {
-                pot[q] = s.pot;
-            }
-        }
-    }
-    unsigned long long a = wave_sum_u64((unsigned long long)s.nint);
-    unsigned long long b = wave_sum_u64((unsigned long long)s.nsph);
-    if (lane_id() == 0 && mode == 0) {
-        if (a) atomicAdd(&ds->interactions, a);
-        if (b) atomicAdd(&ds->sph_pairs, b);
-    }
-}
-
 WalkArgs walk_args(Ctx &c) {
     WalkArgs a;
     a.n = (int)c.n; a.nin = c.nin; a.nn = c.n_nodes;
@@ -1349,7 +1336,7 @@ WalkArgs walk_args(Ctx &c) {
     a.h = c.h; a.rho = c.rho; a.P = c.P; a.active = c.active;
     a.ds = c.ds;
     a.wp = core::WalkParams{c.p.theta, c.p.e0, c.p.G, core::soft_branch_live(c.p.e0)};
-    a.ax = c.ax; a.ay = c.ay; a.az = c.az; a.dUdt = c.dUdt;
+    a.ax = c.ax; a.ay = c.ay; a.az = c.az; a.dUdt = c.dUdt; a.pot = c.pot;
     a.dsw = c.ds;
     a.cbins = c.cbins;
     a.near_cnt = c.near_cnt; a.near_node = c.near_node; a.near_mask = c.near_mask;
@@ -1469,7 +1456,6 @@ static void launch_walk(Ctx &c) {
 
 void forces(Ctx &c, int mode) {
     hipStream_t st = c.stream;
-    int n = (int)c.n;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));
     if (mode == 0) {
         sph_prepare(c);
@@ -1479,11 +1465,13 @@ void forces(Ctx &c, int mode) {
         sph_finish(c);
         fold_counters(c);
     } else {
-        core::WalkParams wp{c.p.theta, c.p.e0, c.p.G, core::soft_branch_live(c.p.e0)};
-        pack_walknodes(c);
-        hipLaunchKernelGGL(k_walk64, dim3(grid_for(n, 256)), dim3(256), 0, st, n, c.nin, c.n_nodes, c.wnode,
-                           c.x, c.y, c.z, c.m, c.type, c.vx, c.vy, c.vz, c.n_gvx, c.n_gvy, c.n_gvz, c.h,
-                           c.rho, c.P, c.active, wp, mode, c.ax, c.ay, c.az, c.dUdt, c.pot, c.ds);
+        const WalkArgs a = walk_args(c);
+        const int tpg = walk_tpg(c.n, false);
+        const int groups = (int)((c.n + tpg - 1) / tpg);
+        const dim3 grid((groups + kWaves - 1) / kWaves), block(64 * kWaves);
+        if (tpg == 8) hipLaunchKernelGGL(k_walk_potential<8>, grid, block, 0, st, a);
+        else if (tpg == 16) hipLaunchKernelGGL(k_walk_potential<16>, grid, block, 0, st, a);
+        else hipLaunchKernelGGL(k_walk_potential<64>, grid, block, 0, st, a);
     }
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[5], st));
     AG2_HIP(hipGetLastError());

@@ -1016,23 +1016,6 @@ __global__ __launch_bounds__(256) void k_iscan_apply(int n, const int32_t *in, c
     }
 }
 
-// Pre-order walk records (core::WalkNode) for the one-lane-per-target
-// potential walk; built only when the potential is asked for.
-__global__ __launch_bounds__(256) void k_pack_walknode(int nn, const DevState *ds, const int32_t *skip,
-                                                       const int32_t *pidx, const int8_t *level, const double *m,
-                                                       const double *gas, const double *cx, const double *cy,
-                                                       const double *cz, WalkNode *wn) {
-    int nd = blockIdx.x * 256 + threadIdx.x;
-    if (nd >= nn) return;
-    double R = __longlong_as_double((long long)ds->Rbits);
-    WalkNode w;
-    w.cx = cx[nd]; w.cy = cy[nd]; w.cz = cz[nd]; w.mass = m[nd];
-    w.radius = ldexp(R, -(int)level[nd]);
-    w.gas = gas[nd];
-    w.skip = skip[nd]; w.pidx = pidx[nd]; w.level = level[nd]; w.flags = 0;
-    wn[nd] = w;
-}
-
 // ------------------------------------------------------------ deep refinement
 // Distinct particles that agree on every key word so far, and tie runs too
 // long for k_tie_rank, are refined word by word: the particles tied on words
@@ -1193,7 +1176,6 @@ void alloc_nodes(Ctx &c, int64_t cap) {
         cv(&c.n_pidx, n * 4); cv(&c.n_level, n);
         double **d8[] = {&c.n_mass, &c.n_gas, &c.n_gvx, &c.n_gvy, &c.n_gvz, &c.n_cx, &c.n_cy, &c.n_cz, &c.g_rho};
         for (double **p : d8) cv(p, n * 8);
-        cv(&c.wnode, n * sizeof(WalkNode));
         cv(&c.g_first, n * 4); cv(&c.g_list, (n + 256) * 4);
         cv(&c.g_fired, n); cv(&c.g_final, n * 4);
         cv(&c.tnode, n * sizeof(core::TreeNode));
@@ -1636,7 +1618,6 @@ void build_tree_b(Ctx &c) {
             }
         }
     }
-    c.wnode_valid = false;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[3], st));
     AG2_HIP(hipGetLastError());
     c.tree_valid = true;
@@ -1646,14 +1627,6 @@ void build_tree(Ctx &c) {
     build_tree_a(c);
     AG2_HIP(hipEventSynchronize(c.ev_counts));
     build_tree_b(c);
-}
-
-void pack_walknodes(Ctx &c) {
-    if (c.wnode_valid || c.n_nodes <= 0) return;
-    hipLaunchKernelGGL(k_pack_walknode, dim3(grid_for(c.n_nodes, 256)), dim3(256), 0, c.stream, c.n_nodes, c.ds,
-                       c.n_skip, c.n_pidx, c.n_level, c.n_mass, c.n_gas, c.n_cx, c.n_cy, c.n_cz, c.wnode);
-    AG2_HIP(hipGetLastError());
-    c.wnode_valid = true;
 }
 
 }  // namespace ag2

@@ -61,3 +61,19 @@ def test_group_size_limits(ag2, orc, n, precision):
     (8, 16, 64 targets)."""
     nh, nd = n // 2, (3 * n) // 10
     check(ag2, orc, ag2.ics.disk_galaxy(nh, nd, n - nh - nd, seed=2), 0.5, precision)
+
+
+@pytest.mark.parametrize("n", [3000, 25000, 280001])
+def test_potential_in_every_group_size(ag2, n):
+    """The tree potential with every node opened is the direct sum's: 0.5 sum
+    m phi, all terms of one sign, so both are within n 2^-53 of it (each target
+    adds its n terms), in groups of 8, 16 and 64 targets."""
+    ps = ag2.ics.config1_plummer(n, seed=3)
+    E = ag2.engine
+    with E.Engine(E.make_params(theta=0.0, e0=0.05 * ag2.units.KPC, massInH=1.0, split_threshold=800), n) as eng:
+        eng.upload(ps)
+        eng.build_tree()
+        tree = eng.energy(with_potential=True)["potential"]
+        phi = eng.direct_sum(np.arange(n), with_potential=True)[3]
+    want = 0.5 * np.sum(ps.m.astype(np.longdouble) * phi)
+    assert abs(tree - want) <= 2 * n * 2.0 ** -53 * abs(want)
