@@ -22,6 +22,7 @@ constexpr int kSortLoMax = 2;     // low bytes of word 0 the radix passes may le
 constexpr int kSortRunLong = 64;  // a longest run above this sorts every byte in the next build
 constexpr int kStateD = 19;        // FP64 per-particle state arrays carried across steps
 constexpr int kSphListLen = 256;   // SPH candidates recorded per gas target (gravity.hip kSphK)
+constexpr int kSphMore = 7;        // spill chunks a list may go on in, kSphListLen candidates each
 constexpr size_t kCounterBinBytes = 8 * 256 * 64;   // counters x bins x one 64-byte line (gravity.hip)
 
 // Reference constants (Constants.h:7-18, Units.h).
@@ -59,6 +60,7 @@ struct DevState {
                           // in a deep tree the largest sum of (internal children - 1) along a path, + 8
     int32_t deep_m;       // particles in tie runs at the current word of the deep refinement
     int32_t walk_err;     // a walk's stack overflowed (never expected; kept until the next upload)
+    int32_t spill_next;   // SPH spill chunks taken by the last forces
     int32_t any_bucket;   // this build has adjacent particles at one position (bucket nodes)
     double red[8];   // energy reductions
 };
@@ -153,7 +155,11 @@ struct Ctx {
     int64_t sph_reserve = 0;   // the SPH lists are allocated for at least this many targets
     int32_t *gslot = nullptr, *gidx = nullptr, *gtiles = nullptr;   // target -> list slot, slot -> target
     int32_t *sph_list = nullptr, *sph_cnt = nullptr;                 // candidate lists (kSphListLen per slot)
-    uint8_t *gover = nullptr;                                        // per group: a list overflowed
+    uint8_t *gover = nullptr;                                        // per group of 64: a list found no room
+    // spill chunks of lists past kSphListLen, and their numbers per slot
+    // (allocated for small opening angles, sph_spill_chunks)
+    int32_t *sph_spill = nullptr, *sph_more = nullptr;
+    int64_t spill_cap = 0, spill_refused = 0;
     // split-precision walk: (node, lane mask) pairs whose targets lie within
     // the FP32 offsets' resolution, evaluated in FP64 after the walk
     // (kNearRecs per group; a group with more is walked again in FP64)
@@ -340,6 +346,8 @@ void visual_density(Ctx &c, double rvd, double *vd);   // visual_density.hip: ke
 void forces(Ctx &c, int mode);           // gravity.hip  (mode 0 forces, 1 potential)
 void forces_fp32(Ctx &c, int mode);      // gravity.hip  (split-precision FP32 forces)
 bool fp32_usable(const Ctx &c);          // gravity.hip: e0 / R of the last build suits the FP32 sweep
+int64_t sph_spill_bytes(int64_t n_gas, double theta);   // gravity.hip: device bytes of the spill chunks
+void reserve_spill(Ctx &c);              // gravity.hip: allocate them for the context's theta and gas
 void sph_prepare(Ctx &c);                // gravity.hip: SPH list slots before a gravity walk
 void sph_finish(Ctx &c);                 // gravity.hip: SPH candidate evaluation after it
 void near_finish(Ctx &c);                // gravity.hip: FP64 near pairs of a split-precision walk

@@ -41,7 +41,7 @@ void free_all(Ctx &c) {
     if (c.slab) (void)hipFree(c.slab);
     if (c.node_slab) (void)hipFree(c.node_slab);
     // allocated on demand
-    void *ptrs[] = {c.sph_list, c.sph_cnt, c.gas_table, c.vd};
+    void *ptrs[] = {c.sph_list, c.sph_cnt, c.sph_spill, c.sph_more, c.gas_table, c.vd};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (uint64_t *p : c.kdeep)
@@ -229,7 +229,12 @@ void ctx_upload(Ctx &ctx, const ag2_particles &h) {
             AG2_HIP(hipMalloc(&c->sph_list, (size_t)cap * kSphListLen * 4));
             AG2_HIP(hipMalloc(&c->sph_cnt, (size_t)cap * 4));
             c->sph_cap = cap;
+            // (the chunk numbers are per slot)
+            if (c->sph_spill) { AG2_HIP(hipFree(c->sph_spill)); c->sph_spill = nullptr; }
+            if (c->sph_more) { AG2_HIP(hipFree(c->sph_more)); c->sph_more = nullptr; }
+            c->spill_cap = c->spill_refused = 0;
         }
+        ag2::reserve_spill(*c);
         if (c->gas_equal) {
             std::vector<double> tab((size_t)ng + 1);
             tab[0] = 0.0;

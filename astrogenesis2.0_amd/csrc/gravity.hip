@@ -25,10 +25,11 @@
 // SPH (the term the reference adds at every accepted gas node within 2 h of
 // a gas target): the gravity walk (KIND 1) records, per active gas target,
 // the accepted gas nodes within a loose margin of 2 h in a list of kSphK
-// node records; k_sph_pairs then evaluates the lists, eight lanes per
-// target, with the exact r < 2 h test and the reference's self skip.  A
-// group whose list filled sets a flag, and the overflow walk (KIND 2) walks
-// only those groups again with the SPH term inline.  Gas-free uploads use
+// node records, going on in spill chunks where a small opening angle accepts
+// more; k_sph_pairs then evaluates the lists, eight lanes per target, with the
+// exact r < 2 h test and the reference's self skip.  Where the chunks ran out,
+// the overflow walk (KIND 2) walks the groups of those targets again with the
+// SPH term inline.  Gas-free uploads use
 // the KIND 0 kernels, which carry no SPH code.
 //
 // FP64 sweep: the reference's softened law G m / (r^2 + e0^2) d / r.
@@ -49,7 +50,7 @@ namespace {
 constexpr int kWaves = 4;
 constexpr int kStackCap = kWalkStackCap;   // pending child blocks per wave
 constexpr int kEnt = 128;        // batch entries: < 64 left after a sweep + <= 64 added per iteration
-constexpr int kSphK = kSphListLen;   // recorded SPH candidates per gas target (more: the overflow walk)
+constexpr int kSphK = kSphListLen;   // recorded SPH candidates per gas target (more: spill chunks, then the overflow walk)
 
 // A pending block of siblings: nodes first .. first+count-1, opened by the
 // lanes in mask.
@@ -77,10 +78,13 @@ struct WalkArgs {
     const core::TreeNode *__restrict__ tree;
     const core::SphNode *__restrict__ tsph;
     // SPH candidate lists: gslot[t] = list slot of key-order target t (-1:
-    // none), sph_list[slot * kSphK + k], sph_cnt[slot], gover[group] = 1 if a
-    // list of the group overflowed
+    // none), sph_list[slot * kSphK + k], sph_cnt[slot]; past kSphK candidates a
+    // list goes on in spill chunks of kSphK (their numbers in sph_more[slot *
+    // kSphMore + ..]; spill_cap chunks, taken with a counter) and sets
+    // gover[group of 64]: see list_overflowed
     const int32_t *__restrict__ gslot;
-    int32_t *sph_list, *sph_cnt;
+    int32_t *sph_list, *sph_cnt, *sph_spill, *sph_more;
+    int spill_cap;
     uint8_t *gover;
     const double *__restrict__ sx, *__restrict__ sy, *__restrict__ sz, *__restrict__ sm;
     const uint8_t *__restrict__ stype;
@@ -254,6 +258,13 @@ __device__ __forceinline__ void bit_pairs(unsigned m, F &&f) {
     }
 }
 
+// Is a target with cnt candidates left to the overflow walk?  When the spill
+// chunks ran out, every target past its list is, so that which of them got a
+// chunk (a matter of timing) decides nothing.
+__device__ inline bool list_overflowed(const WalkArgs &a, int cnt) {
+    return cnt > kSphK * (1 + kSphMore) || (cnt > kSphK && (a.spill_cap == 0 || a.ds->spill_next > a.spill_cap));
+}
+
 // Group g of TPG targets: particles TPG g .. TPG g + TPG - 1 in key order.
 // KIND 0: gravity.  KIND 1: gravity, and every accepted gas node within a
 // margin of 2h of a gas target goes on that target's SPH candidate list
@@ -312,9 +323,10 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     int slot = -1;
     if (GAS && sph_lane) {
         slot = a.gslot[t];
-        if (KIND == 2) sph_lane = a.sph_cnt[slot] > kSphK;
+        if (KIND == 2) sph_lane = list_overflowed(a, a.sph_cnt[slot]);
     }
     const unsigned long long sphB = __ballot(sph_lane);   // all NS lanes of a target
+    if (KIND == 2 && !sphB) return;
     const double h2x4 = GAS ? (2.0 * th) * (2.0 * th) : 0.0;   // SPH support (2h)^2
     int lcnt = 0;   // KIND 1: candidates recorded for this target
 
@@ -425,7 +437,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
             const double rl32 = D * (1.0 + 1e-6) + 2.4e-7 * (A + 2.0 * D);
             lim32 = sph_lane ? (float)(rl32 * rl32 * (1.0 + 1e-5)) : -1.f;
         }
-        int32_t *lbase = (KIND == 1 && slot >= 0) ? a.sph_list + (size_t)slot * kSphK : nullptr;
+        int32_t *lbase = (KIND == 1 && slot >= 0) ? a.sph_list + (size_t)slot * kSphK : nullptr;   // current chunk
         // Multi-block pops keep the stack within kStackCap: a pop of up to
         // 64 nodes pushes at most 64 blocks, and above `single_above` the walk
         // pops one block at a time; from any point the stack then grows by at
@@ -862,9 +874,32 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                         if (lane & d) at += o;
                         add += o;
                     }
-                    lcnt += add;
-                    for (; hm; hm &= hm - 1, at++)
-                        if (at < kSphK) lbase[at] = enode[e0 + __builtin_ctzll(hm)];
+                    if (a.spill_cap == 0) {   // uniform
+                        for (; hm; hm &= hm - 1, at++)
+                            if (at < kSphK) lbase[at] = enode[e0 + __builtin_ctzll(hm)];
+                        lcnt += add;
+                    } else {
+                        // a step adds at most 64, so it enters one new chunk at most
+                        const int chunk = lcnt > 0 ? (lcnt - 1) / kSphK : 0;
+                        lcnt += add;
+                        int32_t *nbase = lbase;
+                        const bool full = add > 0 && (lcnt - 1) / kSphK > chunk;
+                        if (__any(full)) {
+                            int c = -1;
+                            if (full && sub == 0 && chunk < kSphMore && lbase) {
+                                c = atomicAdd(&a.dsw->spill_next, 1);
+                                if (c >= a.spill_cap) c = -1;
+                                else a.sph_more[(size_t)slot * kSphMore + chunk] = c;
+                            }
+                            c = shfl_i(c, tl);
+                            if (full) nbase = c >= 0 ? a.sph_spill + (size_t)c * kSphK : nullptr;
+                        }
+                        for (; hm; hm &= hm - 1, at++) {
+                            int32_t *to = at / kSphK == chunk ? lbase : nbase;
+                            if (to) to[at % kSphK] = enode[e0 + __builtin_ctzll(hm)];
+                        }
+                        lbase = nbase;
+                    }
                 }
                 // SPH term.  Pairs (target lane t, entry j) with r < 2 h_t are
                 // queued in LDS as they are found and evaluated 64 at a time,
@@ -990,8 +1025,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
         if (lcnt > kSphK) a.gover[t >> 6] = 1;
     }
     if (KIND == 1) {
-        // targets whose candidate list overflowed (their SPH term comes from
-        // the overflow walk)
+        // targets whose candidates did not fit their list alone
         const unsigned long long ovB = __ballot(slot >= 0 && sub == 0 && lcnt > kSphK);
         if (lane == 0) bin_add(a.cbins, kCntSphOver, g, (unsigned long long)__builtin_popcountll(ovB));
     }
@@ -1183,8 +1217,9 @@ __global__ AG2_WALK_BOUNDS void k_walk_jobs32_nogas(const JobWalk *jobs, int nj,
 // pass also clears gslot and the groups' overflow flags.
 __global__ __launch_bounds__(256) void k_sph_count(int n, const uint8_t *type, const double *h,
                                                    const uint8_t *active, const double *m, int32_t *tiles,
-                                                   int32_t *gslot, uint8_t *gover) {
+                                                   int32_t *gslot, uint8_t *gover, DevState *ds) {
     __shared__ int scr[4];
+    if (blockIdx.x == 0 && threadIdx.x == 0) ds->spill_next = 0;
     int b0 = blockIdx.x * 1024 + threadIdx.x * 4;
     int c = 0;
     for (int k = 0; k < 4; k++) {
@@ -1231,6 +1266,8 @@ __global__ __launch_bounds__(256) void k_sph_scatter(int n, const uint8_t *type,
 // walk.
 constexpr int kPairLanes = 8;
 
+// SPILL: lists may go on in spill chunks (the context has some).
+template <bool SPILL>
 __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gidx, const int32_t *cnts) {
     const int lane = lane_id();
     const int sub = lane & (kPairLanes - 1);
@@ -1242,7 +1279,7 @@ __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gi
     int t = -1, c = 0;
     if (slot < nsph) {
         c = cnts[slot];
-        if (c <= kSphK) t = gidx[slot];
+        if (!list_overflowed(a, c)) t = gidx[slot];
         else c = 0;
     }
     if (t >= 0) {
@@ -1251,21 +1288,26 @@ __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gi
         tg.h = a.h[t]; tg.rho = a.rho[t]; tg.P = a.P[t];
         const double vx = a.svx[t], vy = a.svy[t], vz = a.svz[t];
         const core::SphConst sk = core::sph_const(tg);
+        // kSphK candidates of the list itself, then of its spill chunks
         const int32_t *lst = a.sph_list + (size_t)slot * kSphK;
-        // one candidate ahead: the next record's load overlaps this pair
-        core::SphNode wn{};
-        if (sub < c) wn = a.tsph[lst[sub]];
-        for (int k = sub; k < c; k += kPairLanes) {
-            const core::SphNode w = wn;
-            if (k + kPairLanes < c) wn = a.tsph[lst[k + kPairLanes]];
-            if (w.pidx == t) continue;
-            const double dx = tg.x - w.cx, dy = tg.y - w.cy, dz = tg.z - w.cz;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 == 0.0) continue;
-            bool inside = r2 < sk.h2x4 * (1.0 - 1e-12);
-            if (!inside && !(r2 > sk.h2x4 * (1.0 + 1e-12))) inside = sqrt(r2) < sk.h * 2;
-            if (!inside) continue;
-            sph_pair(dx, dy, dz, r2, w.gas, vx - w.vx, vy - w.vy, vz - w.vz, sk, &s);
+        for (int c0 = 0; c0 < (SPILL ? c : 1); c0 += kSphK) {
+            if (SPILL && c0 > 0) lst = a.sph_spill + (size_t)a.sph_more[(size_t)slot * kSphMore + c0 / kSphK - 1] * kSphK;
+            const int here = !SPILL || c - c0 < kSphK ? c - c0 : kSphK;
+            // one candidate ahead: the next record's load overlaps this pair
+            core::SphNode wn{};
+            if (sub < here) wn = a.tsph[lst[sub]];
+            for (int k = sub; k < here; k += kPairLanes) {
+                const core::SphNode w = wn;
+                if (k + kPairLanes < here) wn = a.tsph[lst[k + kPairLanes]];
+                if (w.pidx == t) continue;
+                const double dx = tg.x - w.cx, dy = tg.y - w.cy, dz = tg.z - w.cz;
+                const double r2 = dx * dx + dy * dy + dz * dz;
+                if (r2 == 0.0) continue;
+                bool inside = r2 < sk.h2x4 * (1.0 - 1e-12);
+                if (!inside && !(r2 > sk.h2x4 * (1.0 + 1e-12))) inside = sqrt(r2) < sk.h * 2;
+                if (!inside) continue;
+                sph_pair(dx, dy, dz, r2, w.gas, vx - w.vx, vy - w.vy, vz - w.vz, sk, &s);
+            }
         }
     }
     for (int d = kPairLanes / 2; d >= 1; d >>= 1) {
@@ -1330,6 +1372,7 @@ WalkArgs walk_args(Ctx &c) {
     a.tree = c.tnode;
     a.tsph = c.tsph;
     a.gslot = c.gslot; a.sph_list = c.sph_list; a.sph_cnt = c.sph_cnt; a.gover = c.gover;
+    a.sph_spill = c.sph_spill; a.sph_more = c.sph_more; a.spill_cap = (int)c.spill_cap;
     a.sx = c.x; a.sy = c.y; a.sz = c.z; a.sm = c.m; a.stype = c.type;
     a.svx = c.vx; a.svy = c.vy; a.svz = c.vz;
     a.mvx = c.n_gvx; a.mvy = c.n_gvy; a.mvz = c.n_gvz;
@@ -1379,15 +1422,57 @@ void fold_counters(Ctx &c) {
     AG2_HIP(hipGetLastError());
 }
 
+// Spill chunks for n_gas targets at this opening angle.  Within 2h a target
+// meets about 75 gas nodes at theta 0.5, 570 at 0.15 (the 200,000 disk), and
+// their number grows as theta^-1.75 up to the particles themselves; half as
+// many again are provided, over three quarters of the list (so from theta
+// 0.37 down: noting the chunks costs the walk 3 % where no list needs them).
+// At theta 0.15 the overflow walk of the lists that did not fit took 5.26 ms
+// of a force evaluation of 9.1 ms; with the chunks it has nothing to do, and
+// the evaluation takes 3.9 ms.
+int64_t sph_spill_chunks(int64_t n_gas, double theta) {
+    const double t = theta > 0.05 ? theta : 0.05;
+    double per = 1.5 * 75.0 * pow(0.5 / t, 1.75) / kSphK - 0.75;
+    if (!(per > 0.0) || n_gas <= 0) return 0;
+    if (per > kSphMore) per = kSphMore;
+    const double want = per * (double)n_gas + 64.0;
+    return want < 0x7fffffff ? (int64_t)want : 0x7fffffff;
+}
+
+int64_t sph_spill_bytes(int64_t n_gas, double theta) {
+    const int64_t chunks = sph_spill_chunks(n_gas, theta);
+    return chunks > 0 ? chunks * kSphK * 4 + n_gas * kSphMore * 4 : 0;
+}
+
+// Where there is no memory for the chunks the overflow walk does their work.
+void reserve_spill(Ctx &c) {
+    const int64_t want = sph_spill_chunks(c.sph_cap, c.p.theta);
+    if (!c.sph_active || c.spill_cap >= want || c.spill_refused == want) return;
+    AG2_HIP(hipStreamSynchronize(c.stream));
+    if (c.sph_spill) { (void)hipFree(c.sph_spill); c.sph_spill = nullptr; }
+    if (c.sph_more) { (void)hipFree(c.sph_more); c.sph_more = nullptr; }
+    c.spill_cap = 0;
+    if (hipMalloc(&c.sph_spill, (size_t)want * kSphK * 4) != hipSuccess ||
+        hipMalloc(&c.sph_more, (size_t)c.sph_cap * kSphMore * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        if (c.sph_spill) { (void)hipFree(c.sph_spill); c.sph_spill = nullptr; }
+        c.sph_more = nullptr;
+        c.spill_refused = want;
+        return;
+    }
+    c.spill_cap = want;
+}
+
 // SPH candidate lists for a step: slots for the active SPH targets (before
 // the gravity walk, which fills the lists) ...
 void sph_prepare(Ctx &c) {
     if (!c.sph_active) return;
+    reserve_spill(c);   // (a smaller theta than at the upload)
     hipStream_t st = c.stream;
     int n = (int)c.n;
     int nt = (n + 1023) / 1024;
     hipLaunchKernelGGL(k_sph_count, dim3(nt), dim3(256), 0, st, n, c.type, c.h, c.active, c.m, c.gtiles, c.gslot,
-                       c.gover);
+                       c.gover, c.ds);
     hipLaunchKernelGGL(k_sph_scatter, dim3(nt), dim3(256), 0, st, n, c.type, c.h, c.active, c.m, c.gtiles, c.gidx,
                        c.gslot, c.ds);
     AG2_HIP(hipGetLastError());
@@ -1401,7 +1486,8 @@ void sph_finish(Ctx &c) {
     WalkArgs a = walk_args(c);
     int64_t lanes = c.gas_count * kPairLanes;
     int nb = (int)((lanes + 255) / 256);
-    if (nb > 0) hipLaunchKernelGGL(k_sph_pairs, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
+    if (nb > 0 && c.spill_cap > 0) hipLaunchKernelGGL(k_sph_pairs<true>, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
+    else if (nb > 0) hipLaunchKernelGGL(k_sph_pairs<false>, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
     const int groups = (int)((c.n + 63) / 64);
     hipLaunchKernelGGL(k_walk_sph_overflow, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
     AG2_HIP(hipGetLastError());

@@ -210,6 +210,11 @@ int64_t pow2_at_least(int64_t v) {
     return p;
 }
 
+// Device bytes of a context's SPH spill chunks.
+int64_t spill_bytes(const Ctx &c) {
+    return c.spill_cap > 0 ? c.spill_cap * ag2::kSphListLen * 4 + c.sph_cap * ag2::kSphMore * 4 : 0;
+}
+
 // A context for job j: the smallest spare one that is large enough, else a
 // new one if the budget allows (dropping spare contexts to make room).  New
 // contexts are sized in classes (particles and gas targets rounded up to a
@@ -220,7 +225,9 @@ Ctx *take_context(Pool &P, Job &j, hipStream_t st) {
     Ctx *best = nullptr;
     size_t bi = 0;
     for (size_t i = 0; i < P.spare.size(); i++)
-        if (P.spare[i]->cap >= j.n && P.spare[i]->sph_cap >= j.n_gas && (!best || P.spare[i]->cap < best->cap)) {
+        if (P.spare[i]->cap >= j.n && P.spare[i]->sph_cap >= j.n_gas &&
+            spill_bytes(*P.spare[i]) >= ag2::sph_spill_bytes(j.n_gas > 0 ? P.spare[i]->sph_cap : 0, j.p.theta) &&
+            (!best || P.spare[i]->cap < best->cap)) {
             best = P.spare[i];
             bi = i;
         }
@@ -231,16 +238,16 @@ Ctx *take_context(Pool &P, Job &j, hipStream_t st) {
     }
     int64_t cap = pow2_at_least(j.n > (1 << 14) ? j.n : (1 << 14));
     int64_t gcap = j.n_gas > 0 ? pow2_at_least(j.n_gas > (1 << 12) ? j.n_gas : (1 << 12)) : 0;
-    int64_t need = ag2::ctx_footprint(cap, gcap);
+    int64_t need = ag2::ctx_footprint(cap, gcap) + ag2::sph_spill_bytes(gcap, j.p.theta);
     if (P.used + need > P.budget) {
         cap = j.n;
         gcap = j.n_gas;
-        need = ag2::ctx_footprint(cap, gcap);
+        need = ag2::ctx_footprint(cap, gcap) + ag2::sph_spill_bytes(gcap, j.p.theta);
     }
     while (P.used + need > P.budget && !P.spare.empty()) {
         Ctx *c = P.spare.back();
         P.spare.pop_back();
-        P.used -= ag2::ctx_footprint(c->cap, c->sph_cap);
+        P.used -= ag2::ctx_footprint(c->cap, c->sph_cap) + spill_bytes(*c);
         ag2::ctx_delete(c);
     }
     if (P.used + need > P.budget) return nullptr;
@@ -432,7 +439,7 @@ int ag2_job_submit(void *pool, const ag2_params *params, const ag2_particles *h,
         if (h->n < 1) return pfail(P, AG2_ERR_ARG, "n must be >= 1");
         if (h->n > 0x7fffff00LL / 2) return pfail(P, AG2_ERR_CAPACITY, "n too large");
         if (steps < 0) return pfail(P, AG2_ERR_ARG, "steps must be >= 0");
-        if (ag2::ctx_footprint(h->n, ngas_of(*h)) > P->budget) return pfail(P, AG2_ERR_CAPACITY, "job exceeds the pool's memory budget");
+        if (ag2::ctx_footprint(h->n, ngas_of(*h)) + ag2::sph_spill_bytes(ngas_of(*h), params->theta) > P->budget) return pfail(P, AG2_ERR_CAPACITY, "job exceeds the pool's memory budget");
         Job *j = new Job();
         j->id = P->next_id++;
         j->p = *params;

@@ -105,8 +105,9 @@ typedef struct ag2_diag {
                                 the last upload (a caller can time many steps and
                                 read the count once)                             */
     int64_t sph_overflow;    /* gas targets of the last forces with more SPH
-                                candidates than their list holds (256): their SPH
-                                term came from the overflow walk                 */
+                                candidates than their list holds (256): the rest
+                                went to spill chunks, or their SPH term came from
+                                the overflow walk                                */
     int64_t fp64_fallback;   /* 1: the last forces of an AG2_FP32_SPLIT context ran
                                 the FP64 sweep, because the softening length was
                                 below 2^-24 of the root half-width (FP32 cannot

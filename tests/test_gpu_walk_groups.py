@@ -40,6 +40,7 @@ def check(ag2, orc, ps, theta, precision, thr=800):
     s = np.abs(want.dUdt).max()
     if s > 0:
         assert np.abs(got.dUdt - want.dUdt).max() / s < 1e-10
+    return got, d
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -77,3 +78,16 @@ def test_potential_in_every_group_size(ag2, n):
         phi = eng.direct_sum(np.arange(n), with_potential=True)[3]
     want = 0.5 * np.sum(ps.m.astype(np.longdouble) * phi)
     assert abs(tree - want) <= 2 * n * 2.0 ** -53 * abs(want)
+
+
+@pytest.mark.parametrize("n,precision", [(9000, 0), (60000, 1), (200000, 1)])
+def test_long_sph_lists(ag2, orc, n, precision):
+    """A small opening angle accepts more SPH candidates than a target's list
+    holds (256): they go on in spill chunks, in every group size.  Two
+    evaluations are bit-identical, whichever chunk a target got."""
+    ps = ag2.ics.disk_galaxy(n // 4, n // 4, n - 2 * (n // 4), seed=8)
+    a, da = check(ag2, orc, ps, 0.2, precision)
+    b, _ = check(ag2, orc, ps, 0.2, precision)
+    assert da["sph_overflow"] > 0
+    for f in ("ax", "ay", "az", "dUdt"):
+        assert np.array_equal(getattr(a, f), getattr(b, f)), f
