@@ -273,6 +273,12 @@ __device__ inline unsigned long long lanes_below() {
     return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
+// Orders the wave's LDS accesses (one wave's lanes exchanging through LDS).
+__device__ inline void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Inclusive wave scan of an int (64 lanes).
 __device__ inline int wave_incl_scan(int v) {
     for (int d = 1; d < 64; d <<= 1) {

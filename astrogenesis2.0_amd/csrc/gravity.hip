@@ -179,11 +179,6 @@ __device__ inline int mbcnt(unsigned long long b) {
 }
 // Lane-mask -> per-lane bool with no vector work (the mask is the condition).
 __device__ inline bool in_mask(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
-__device__ inline void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // The SPH term with the target's constants hoisted (core::sph_term_hoisted:
 // the reference's arithmetic bit for bit).
 __device__ inline void sph_pair(double dx, double dy, double dz, double r2, double gas, double vx, double vy,

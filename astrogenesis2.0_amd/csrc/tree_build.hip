@@ -270,6 +270,172 @@ __global__ __launch_bounds__(256) void k_rs_scatter(int n, const uint64_t *__res
     rs_scatter_tile<SMALL>(n, kin, vin, kout, vout, shift, hist, dtotal, nblk, blockIdx.x);
 }
 
+// ------------------------------------------------------------ merge sort
+// Two launches for a set of a few tiles, where the radix passes are launches
+// and little else (six bytes are 12 or 18 launches of 4-7 us).  k_ms_tile
+// sorts each tile of TILE keys by itself in LDS (stable radix passes over
+// the bytes the build sorts, bound by their barriers and LDS round trips:
+// 2.5 us each); k_ms_merge gives each key its place: its
+// position in its own tile plus, for every other tile, the number of keys
+// that come before it, by binary search (equal keys in tile order, so the
+// sort is stable).  A tile whose range leaves out a whole wave's keys is not
+// searched: particles move little between steps, so most are.
+constexpr int kMsThreads = 1024;
+constexpr int kMsWaves = kMsThreads / 64;
+// Sort phase in microseconds, radix passes against tiles of 2048 / 4096 / 8192
+// (first build after an upload, in caller order; later builds are 1-5 us
+// below): 10,000 69 against 33 / 36 / 51; 20,000 73 against 36 / 43 / 55;
+// 33,333 86 against 42 / 46 / 63; 65,000 87 against 66 / 53 / 65; 100,003 89
+// against 142 / 95 / 81; 200,000 94 against 467 / 273 / 186 (the searches grow
+// with the tiles' number for every key).
+constexpr int kMsSmall = 40000, kMsMax = 80000;     // up to here kMsTile0, kMsTile1
+constexpr int kMsTile0 = 2048, kMsTile1 = 4096;
+
+template <int TILE>
+__device__ __forceinline__ void ms_tile(int n, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                        uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int lo, int tile) {
+    constexpr int kMsItems = TILE / kMsThreads;
+    __shared__ uint64_t sk[TILE];
+    __shared__ uint32_t sv[TILE];
+    __shared__ int wcnt[kMsWaves][256];
+    __shared__ int wtot[4];
+    const int tid = threadIdx.x, w = tid >> 6, lane = lane_id();
+    const int t0 = tile * TILE;
+    const int len = n - t0 < TILE ? n - t0 : TILE;
+    // item j of lane l of wave w: tile position (w kMsItems + j) 64 + l
+    const int base = w * (64 * kMsItems) + lane;
+    uint64_t k[kMsItems];
+    uint32_t v[kMsItems];
+#pragma unroll
+    for (int j = 0; j < kMsItems; j++) {
+        const int p = base + j * 64;
+        // past the end: the largest key, which stays behind (the sort is stable)
+        k[j] = p < len ? kin[t0 + p] : ~0ull;
+        v[j] = p < len ? vin[t0 + p] : 0u;
+    }
+    const unsigned long long below = lanes_below();
+    for (int pass = lo; pass < 8; pass++) {
+        for (int d = lane; d < 256; d += 64) wcnt[w][d] = 0;
+        wave_sync_lds();
+        int loc[kMsItems], dig[kMsItems];
+#pragma unroll
+        for (int j = 0; j < kMsItems; j++) {
+            const int d = (int)((k[j] >> (8 * pass)) & 255);
+            unsigned long long peers = ~0ull;
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const int bit = (d >> b) & 1;
+                const unsigned long long bm = __ballot(bit);
+                peers &= bit ? bm : ~bm;
+            }
+            const int cur = wcnt[w][d];
+            wave_sync_lds();
+            if ((peers & below) == 0ull) wcnt[w][d] = cur + __popcll(peers);
+            wave_sync_lds();
+            loc[j] = cur + __popcll(peers & below);
+            dig[j] = d;
+        }
+        __syncthreads();
+        // digit d's first place: the keys of smaller digits, then of earlier waves
+        int inc = 0, tot = 0;
+        if (tid < 256) {
+            for (int u = 0; u < kMsWaves; u++) tot += wcnt[u][tid];
+            inc = wave_incl_scan(tot);
+            if (lane == 63) wtot[w] = inc;
+        }
+        __syncthreads();
+        if (tid < 256) {
+            int at = inc - tot;
+            for (int u = 0; u < w; u++) at += wtot[u];
+            for (int u = 0; u < kMsWaves; u++) { const int c = wcnt[u][tid]; wcnt[u][tid] = at; at += c; }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kMsItems; j++) {
+            const int to = wcnt[w][dig[j]] + loc[j];
+            sk[to] = k[j];
+            sv[to] = v[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kMsItems; j++) { k[j] = sk[base + j * 64]; v[j] = sv[base + j * 64]; }
+        // (the next pass writes sk only after two more barriers)
+    }
+#pragma unroll
+    for (int j = 0; j < kMsItems; j++) {
+        const int p = base + j * 64;
+        if (p < len) { kout[t0 + p] = k[j]; vout[t0 + p] = v[j]; }
+    }
+}
+
+// Element i of the tile-sorted keys to its place: kMsLanes neighbouring lanes
+// per element share the other tiles, four at a time each, searched side by
+// side (one lane for all of them waits out every search in turn).
+constexpr int kMsLanes = 4;
+constexpr int kMsPer = 256 / kMsLanes;   // elements per workgroup
+
+template <int TILE>
+__device__ __forceinline__ void ms_merge(int n, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                         uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int lo, int i) {
+    constexpr int kG = 4;
+    const bool on = i < n;
+    const int e = on ? i : n - 1;
+    const int shift = 8 * lo;
+    const uint64_t k = kin[e], q = k >> shift;
+    const int own = e / TILE, tiles = (n + TILE - 1) / TILE;
+    const int share = threadIdx.x & (kMsLanes - 1);
+    int at = share == 0 ? e - own * TILE : 0;
+    for (int t0 = 0; t0 < tiles; t0 += kG * kMsLanes) {
+        const int t = t0 + share * kG;
+        int len[kG], pos[kG];
+        bool need = false;
+#pragma unroll
+        for (int u = 0; u < kG; u++) {
+            const int b = (t + u) * TILE;
+            len[u] = t + u < tiles && t + u != own ? (n - b < TILE ? n - b : TILE) : 0;
+            pos[u] = 0;
+            if (len[u] > 0) {
+                const uint64_t first = kin[b] >> shift, last = kin[b + len[u] - 1] >> shift;
+                const bool before = t + u < own;   // equal keys there come first
+                const bool all = before ? last <= q : last < q, none = before ? first > q : first >= q;
+                pos[u] = all ? len[u] : 0;
+                need |= !all && !none;
+            }
+        }
+        if (__any(need)) {
+#pragma unroll
+            for (int u = 0; u < kG; u++) pos[u] = 0;
+            for (int step = TILE; step; step >>= 1)
+#pragma unroll
+                for (int u = 0; u < kG; u++) {
+                    const int p = pos[u] + step;
+                    if (p <= len[u]) {
+                        const uint64_t o = kin[(t + u) * TILE + p - 1] >> shift;
+                        if (t + u < own ? o <= q : o < q) pos[u] = p;
+                    }
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < kG; u++) at += pos[u];
+    }
+    for (int d = kMsLanes / 2; d >= 1; d >>= 1) at += __shfl_xor(at, d, 64);
+    if (on && share == 0) { kout[at] = k; vout[at] = vin[e]; }
+}
+
+template <int TILE>
+__global__ __launch_bounds__(kMsThreads) void k_ms_tile(int n, const uint64_t *__restrict__ kin,
+                                                        const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
+                                                        uint32_t *__restrict__ vout, int lo) {
+    ms_tile<TILE>(n, kin, vin, kout, vout, lo, blockIdx.x);
+}
+
+template <int TILE>
+__global__ __launch_bounds__(256) void k_ms_merge(int n, const uint64_t *__restrict__ kin,
+                                                  const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
+                                                  uint32_t *__restrict__ vout, int lo) {
+    ms_merge<TILE>(n, kin, vin, kout, vout, lo, blockIdx.x * kMsPer + threadIdx.x / kMsLanes);
+}
+
 // Batched sort of several contexts (a serving round): job j's tiles are the
 // workgroups [tile0, tile0 + nblk) of one launch per kernel and pass, found
 // by binary search; each job keeps its own buffers, so its result is that of
@@ -293,6 +459,21 @@ __device__ inline int find_sort_job(const SortJob *jobs, int nj, int b) {
 __global__ __launch_bounds__(256) void k_rsb_hist(const SortJob *jobs, int nj, int pass) {
     const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x)];
     rs_hist_tile(J.n, (pass & 1) ? J.key_alt : J.key, 8 * pass, J.hist, J.nblk, (int)blockIdx.x - J.tile0);
+}
+
+template <int TILE>
+__global__ __launch_bounds__(kMsThreads) void k_msb_tile(const SortJob *jobs, int nj, int lo) {
+    const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x)];
+    ms_tile<TILE>(J.n, J.key, J.idx, J.key_alt, J.idx_alt, lo, (int)blockIdx.x - J.tile0);
+}
+
+template <int TILE>
+__global__ __launch_bounds__(256) void k_msb_merge(const SortJob *jobs, int nj, int lo) {
+    constexpr int kPer = TILE / kMsPer;   // workgroups per tile
+    const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x / kPer)];
+    const int b = (int)blockIdx.x - J.tile0 * kPer;
+    if (b * kMsPer < J.n)
+        ms_merge<TILE>(J.n, J.key_alt, J.idx_alt, J.key, J.idx, lo, b * kMsPer + (int)threadIdx.x / kMsLanes);
 }
 
 __global__ __launch_bounds__(256) void k_rsb_scan(const SortJob *jobs) {
@@ -1263,19 +1444,24 @@ static void radix_sort(Ctx &c, int n) {
     int nblk = (n + kSortTile - 1) / kSortTile;
     uint64_t *kin = c.key, *kout = c.key_alt;
     uint32_t *vin = c.idx, *vout = c.idx_alt;
-    const bool small = nblk <= kSortSmallTiles;
+    if (n <= kMsMax) {
+        const dim3 gt(grid_for(n, n <= kMsSmall ? kMsTile0 : kMsTile1)), gm(grid_for(n, kMsPer));
+        if (n <= kMsSmall) {
+            hipLaunchKernelGGL(k_ms_tile<kMsTile0>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo);
+            hipLaunchKernelGGL(k_ms_merge<kMsTile0>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
+        } else {
+            hipLaunchKernelGGL(k_ms_tile<kMsTile1>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo);
+            hipLaunchKernelGGL(k_ms_merge<kMsTile1>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
+        }
+        return;
+    }
     // bytes sort_lo .. 7 (an even number of passes)
     for (int pass = c.sort_lo; pass < 8; pass++) {
         int shift = pass * 8;
         hipLaunchKernelGGL(k_rs_hist, dim3(nblk), dim3(256), 0, c.stream, n, kin, shift, c.hist, nblk);
-        if (small) {
-            hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nblk), dim3(256), 0, c.stream, n, kin, vin, kout, vout, shift,
-                               c.hist, c.dtotal, nblk);
-        } else {
-            hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, c.stream, nblk, c.hist, c.dtotal);
-            hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nblk), dim3(256), 0, c.stream, n, kin, vin, kout, vout, shift,
-                               c.hist, c.dtotal, nblk);
-        }
+        hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, c.stream, nblk, c.hist, c.dtotal);
+        hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nblk), dim3(256), 0, c.stream, n, kin, vin, kout, vout, shift,
+                           c.hist, c.dtotal, nblk);
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
@@ -1386,20 +1572,38 @@ size_t sort_job_bytes() { return sizeof(SortJob); }
 void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void *scratch_host) {
     if (nc <= 0) return;
     SortJob *hj = (SortJob *)scratch_host;
+    // the bytes every job sorts (an even number of passes ends in key / idx),
+    // and by which sort: each job's order is that of its own sort either way
+    int lo = kSortLoMax;
+    int64_t most = 0;
+    for (int k = 0; k < nc; k++) {
+        lo = cs[k]->sort_lo < lo ? cs[k]->sort_lo : lo;
+        most = cs[k]->n > most ? cs[k]->n : most;
+    }
+    const int tile = most > kMsMax ? kSortTile : most > kMsSmall ? kMsTile1 : kMsTile0;
     int total = 0;
     for (int k = 0; k < nc; k++) {
         Ctx &c = *cs[k];
         const int n = (int)c.n;
-        const int nblk = (n + kSortTile - 1) / kSortTile;
+        const int nblk = (n + tile - 1) / tile;
         hj[k] = SortJob{n, nblk, total, 0, c.key, c.key_alt, c.idx, c.idx_alt, c.hist, c.dtotal};
         total += nblk;
     }
     if (total < 1) return;
     SortJob *dj = (SortJob *)scratch_dev;
     AG2_HIP(hipMemcpyAsync(dj, hj, sizeof(SortJob) * (size_t)nc, hipMemcpyHostToDevice, st));
-    // the bytes every job sorts (an even number of passes ends in key / idx)
-    int lo = kSortLoMax;
-    for (int k = 0; k < nc; k++) lo = cs[k]->sort_lo < lo ? cs[k]->sort_lo : lo;
+    if (most <= kMsMax) {
+        const dim3 gm((unsigned)(total * (tile / kMsPer)));
+        if (tile == kMsTile0) {
+            hipLaunchKernelGGL(k_msb_tile<kMsTile0>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo);
+            hipLaunchKernelGGL(k_msb_merge<kMsTile0>, gm, dim3(256), 0, st, dj, nc, lo);
+        } else {
+            hipLaunchKernelGGL(k_msb_tile<kMsTile1>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo);
+            hipLaunchKernelGGL(k_msb_merge<kMsTile1>, gm, dim3(256), 0, st, dj, nc, lo);
+        }
+        AG2_HIP(hipGetLastError());
+        return;
+    }
     for (int pass = lo; pass < 8; pass++) {
         hipLaunchKernelGGL(k_rsb_hist, dim3(total), dim3(256), 0, st, dj, nc, pass);
         hipLaunchKernelGGL(k_rsb_scan, dim3(256 * nc), dim3(256), 0, st, dj);
