@@ -33,7 +33,7 @@ constexpr double kPRTN = 1.6726219e-27;
 constexpr double kKMS = 1.0e3;
 constexpr double kMPC = 3.08567758149137e22;
 
-// Sums of a node (tree_build.hip k_moments_up): mass, mass-weighted position,
+// Sums of a node or of a block of particles (tree_build.hip): mass, mass-weighted position,
 // gas mass, gas-mass-weighted velocity.
 struct alignas(64) NodeSums {
     double m, sx, sy, sz, g, gx, gy, gz;
@@ -137,10 +137,7 @@ struct Ctx {
     int32_t *g_final = nullptr;
     double *g_rho = nullptr;
 
-    // moments: each node's sums, built bottom-up (one arrival counter per
-    // node; internal-children counts bound the walk's stack in deep trees)
-    NodeSums *nsum = nullptr;
-    int32_t *n_ichild = nullptr;
+    int32_t *n_ichild = nullptr;   // internal children (they bound the walk's stack in deep trees)
     NodeSums *nsum_tile = nullptr;   // sums of aligned 64- and 4096-particle blocks (node sums)
     // The reference sums a node's gas mass one particle at a time in array
     // order (Node.cpp:479, :681).  When every gas particle has the same mass m

@@ -145,7 +145,7 @@ int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
                     + 2 * 4 + 1;      // SPH list slots, targets, group flags
     int64_t per_node = 5 * 4 + 1 + 9 * 8 + 2 * 4 + 1 + 4 +
                        2 * (int64_t)sizeof(core::TreeNode) + 3 * 4 +   // walk and SPH records
-                       (int64_t)sizeof(ag2::NodeSums) + 4 +            // node sums, internal-child counts
+                       4 +                                             // internal-child counts
                        (int64_t)sizeof(ag2::NodeSums) / 64 + 1;        // block sums
     int64_t fixed = 256 * ((n + kSortTile - 1) / kSortTile + 1) * 4 + 8 * 1024 * 8 + (1 << 20) +
                     walk_groups_max(cap) * (4 + ag2::kNearRecs * 12) +   // near-pair records

@@ -833,34 +833,82 @@ struct PVals {
     const uint8_t *stype;
 };
 
-__device__ inline void add_particle(NodeSums &s, int p, const PVals &v) {
-    const double m = v.sm[p];
-    s.m += m;
-    s.sx += v.sx[p] * m;
-    s.sy += v.sy[p] * m;
-    s.sz += v.sz[p] * m;
-    if (v.stype[p] == 2) {
-        s.g += m;
-        s.gx += v.svx[p] * m;
-        s.gy += v.svy[p] * m;
-        s.gz += v.svz[p] * m;
+// Butterflies over the wave (lane distances 32, 16, .. 1) of several sums at
+// once, in halving form: at each distance a pair of lanes exchanges half of
+// its sums and each adds the other half, so that a sum takes one exchange in
+// all instead of six per lane.  Every sum adds the same terms in the same
+// order as a plain butterfly.  The exchanges stay on the vector unit: the 96
+// LDS permutes per eight sums of the plain form were what bounded the node
+// sums (k_tile_sums at 10,000 particles, whose three workgroups sit on three
+// CUs: 21.5 -> 5.5 us; 1,000,000: 29 -> 15 us).
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+__device__ inline double lane_xor8(double v) { return dpp_f64<0x128>(v); }                 // row_ror:8
+__device__ inline double lane_xor4(double v) { return dpp_f64<0x1b>(dpp_f64<0x141>(v)); }   // ^ 7, then ^ 3
+__device__ inline double lane_xor2(double v) { return dpp_f64<0x4e>(v); }
+__device__ inline double lane_xor1(double v) { return dpp_f64<0xb1>(v); }
+
+// Lanes with bit 5 (4) clear get a's sum over the lane pair at distance 32
+// (16), the others b's.
+template <int D>
+__device__ inline double halve_swap(double a, double b) {
+    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a);
+    const unsigned long long ub = __builtin_bit_cast(unsigned long long, b);
+    unsigned long long x, y;
+    if (D == 32) {
+        auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+        auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        x = (unsigned long long)hi[0] << 32 | lo[0];
+        y = (unsigned long long)hi[1] << 32 | lo[1];
+    } else {
+        auto lo = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+        auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        x = (unsigned long long)hi[0] << 32 | lo[0];
+        y = (unsigned long long)hi[1] << 32 | lo[1];
     }
+    return __builtin_bit_cast(double, x) + __builtin_bit_cast(double, y);
+}
+__device__ inline double halve8(double a, double b) {
+    const bool up = (lane_id() & 8) != 0;
+    return (up ? b : a) + lane_xor8(up ? a : b);
+}
+__device__ inline double halve4(double a, double b) {
+    const bool up = (lane_id() & 4) != 0;
+    return (up ? b : a) + lane_xor4(up ? a : b);
+}
+__device__ inline double halve2(double a, double b) {
+    const bool up = (lane_id() & 2) != 0;
+    return (up ? b : a) + lane_xor2(up ? a : b);
 }
 
-__device__ inline void add_sums(NodeSums &s, const NodeSums &t) {
-    s.m += t.m; s.sx += t.sx; s.sy += t.sy; s.sz += t.sz;
-    s.g += t.g; s.gx += t.gx; s.gy += t.gy; s.gz += t.gz;
+// Eight sums over the wave: lane l gets sum l >> 3.
+__device__ inline double wave_sums8(const double (&v)[8]) {
+    double r[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) r[j] = halve_swap<32>(v[j], v[j + 4]);
+    double s = halve8(halve_swap<16>(r[0], r[2]), halve_swap<16>(r[1], r[3]));
+    s += lane_xor4(s);
+    s += lane_xor2(s);
+    s += lane_xor1(s);
+    return s;
 }
 
-__device__ inline NodeSums shfl_sums(const NodeSums &s, int d) {
-    return NodeSums{__shfl_xor(s.m, d, 64), __shfl_xor(s.sx, d, 64), __shfl_xor(s.sy, d, 64),
-                    __shfl_xor(s.sz, d, 64), __shfl_xor(s.g, d, 64), __shfl_xor(s.gx, d, 64),
-                    __shfl_xor(s.gy, d, 64), __shfl_xor(s.gz, d, 64)};
-}
-
-// Butterfly over the wave; every lane ends with a sum, lane 0's is the one used.
-__device__ inline NodeSums wave_sums(NodeSums s) {
-    for (int d = 32; d >= 1; d >>= 1) add_sums(s, shfl_sums(s, d));
+// Thirty-two sums over the wave: lane l gets sum l >> 1.
+__device__ inline double wave_sums32(const double (&v)[32]) {
+    double r[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) r[j] = halve_swap<32>(v[j], v[j + 16]);
+#pragma unroll
+    for (int j = 0; j < 8; j++) r[j] = halve_swap<16>(r[j], r[j + 8]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) r[j] = halve8(r[j], r[j + 4]);
+    double s = halve2(halve4(r[0], r[2]), halve4(r[1], r[3]));
+    s += lane_xor1(s);
     return s;
 }
 
@@ -869,27 +917,47 @@ __device__ inline NodeSums wave_sums(NodeSums s) {
 // hold zeros.  The grid covers all n particles: the launch does not wait
 // for the host to learn nin.
 __global__ __launch_bounds__(1024) void k_tile_sums(const DevState *ds, PVals v, NodeSums *blk1, NodeSums *blk2) {
-    __shared__ NodeSums sb[64];
+    static_assert(sizeof(NodeSums) == 64, "a block's sums are written as eight doubles");
+    __shared__ double sb[8][64 + 1];
     const int nin = ds->nin;
     const int w = threadIdx.x >> 6, lane = lane_id();
     const int b0 = blockIdx.x * 64 + w * 4;   // first 64-block of this wave
-    NodeSums t[4];
+    double m[4], t[32];
+    bool gas[4];
+#pragma unroll
     for (int u = 0; u < 4; u++) {
-        t[u] = NodeSums{0, 0, 0, 0, 0, 0, 0, 0};
         const int p = (b0 + u) * kBlk1 + lane;
-        if (p < nin) add_particle(t[u], p, v);
+        const bool in = p < nin;
+        const int q = in ? p : 0;   // n > 0: particle 0 is there
+        m[u] = in ? v.sm[q] : 0.0;
+        const double x = v.sx[q], y = v.sy[q], z = v.sz[q];
+        gas[u] = in && v.stype[q] == 2;
+        t[8 * u] = m[u];
+        t[8 * u + 1] = in ? x * m[u] : 0.0;
+        t[8 * u + 2] = in ? y * m[u] : 0.0;
+        t[8 * u + 3] = in ? z * m[u] : 0.0;
     }
+#pragma unroll
     for (int u = 0; u < 4; u++) {
-        const NodeSums r = wave_sums(t[u]);
-        if (lane == 0) {
-            blk1[b0 + u] = r;
-            sb[w * 4 + u] = r;
-        }
+        const int p = (b0 + u) * kBlk1 + lane;
+        t[8 * u + 4] = gas[u] ? m[u] : 0.0;
+        t[8 * u + 5] = gas[u] ? v.svx[p] * m[u] : 0.0;
+        t[8 * u + 6] = gas[u] ? v.svy[p] * m[u] : 0.0;
+        t[8 * u + 7] = gas[u] ? v.svz[p] * m[u] : 0.0;
+    }
+    const double r = wave_sums32(t);
+    if ((lane & 1) == 0) {
+        const int j = lane >> 1;   // block b0 + (j >> 3), sum j & 7
+        ((double *)(blk1 + b0))[j] = r;
+        sb[j & 7][w * 4 + (j >> 3)] = r;
     }
     __syncthreads();
     if (w == 0) {
-        const NodeSums r = wave_sums(sb[lane]);
-        if (lane == 0) blk2[blockIdx.x] = r;
+        double f[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) f[j] = sb[j][lane];
+        const double q = wave_sums8(f);
+        if ((lane & 7) == 0) ((double *)(blk2 + blockIdx.x))[lane >> 3] = q;
     }
 }
 
@@ -929,91 +997,30 @@ __device__ inline Cover make_cover(int s, int e, int nin, int nout) {
     return c;
 }
 
-__device__ inline void add_piece(NodeSums &acc, const Cover &c, int k, const PVals &v, const NodeSums *blk1,
-                                 const NodeSums *blk2) {
-    if (k < c.k1) add_particle(acc, c.s + k, v);
-    else if (k < c.k2) add_sums(acc, blk1[c.p1 / kBlk1 + (k - c.k1)]);
-    else if (k < c.k3) add_sums(acc, blk2[c.p2 / kBlk2 + (k - c.k2)]);
-    else if (k < c.k4) add_sums(acc, blk1[c.p3 / kBlk1 + (k - c.k3)]);
-    else if (k < c.k5) add_particle(acc, c.p4 + (k - c.k4), v);
-    else add_particle(acc, c.nin + (k - c.k5), v);
-}
-
-struct StagedP {
-    double m, x, y, z, vx, vy, vz;
-    int gas;
-};
-
-__global__ __launch_bounds__(256) void k_sums_direct(int nn, int nin, int n, int proot, const int32_t *first,
-                                                     const int32_t *count, const int32_t *pidx, PVals v,
-                                                     const NodeSums *blk1, const NodeSums *blk2,
-                                                     NodeSums *nsum) {
-    __shared__ double st_m[kStage], st_x[kStage], st_y[kStage], st_z[kStage];
-    __shared__ double st_vx[kStage], st_vy[kStage], st_vz[kStage];
-    __shared__ uint8_t st_g[kStage];
-    // nodes in XCD ranges: neighbours in pre-order share particles
-    const int b = xcd_block(blockIdx.x, gridDim.x);
-    const int nd0 = b * 256;
-    const int last = nd0 + 255 < nn ? nd0 + 255 : nn - 1;
-    // every particle between the first particles of two nodes has its leaf
-    // between them in pre-order, so the span is at most 255 + kSumSmall
-    const int P0 = first[nd0];
-    int P1 = first[last] + kSumSmall;
-    P1 = P1 < nin ? P1 : nin;
-    for (int k = threadIdx.x; k < P1 - P0; k += 256) {
-        const int p = P0 + k;
-        const double m = v.sm[p];
-        st_m[k] = m; st_x[k] = v.sx[p]; st_y[k] = v.sy[p]; st_z[k] = v.sz[p];
-        const bool g = v.stype[p] == 2;
-        st_g[k] = g ? 1 : 0;
-        if (g) { st_vx[k] = v.svx[p]; st_vy[k] = v.svy[p]; st_vz[k] = v.svz[p]; }
-    }
-    __syncthreads();
-    const int nd = nd0 + (int)threadIdx.x;
-    int s = 0, c = 0;
-    bool small = false, wide = false;
-    if (nd < nn && pidx[nd] < 0) {
-        s = first[nd];
-        c = count[nd];
-        wide = (nd == 0 && proot) || c > kSumSmall;
-        small = !wide;
-    }
-    if (small) {
-        NodeSums t{0, 0, 0, 0, 0, 0, 0, 0};
-        for (int k = s - P0; k < s - P0 + c; k++) {
-            const double m = st_m[k];
-            t.m += m;
-            t.sx += st_x[k] * m;
-            t.sy += st_y[k] * m;
-            t.sz += st_z[k] * m;
-            if (st_g[k]) {
-                t.g += m;
-                t.gx += st_vx[k] * m;
-                t.gy += st_vy[k] * m;
-                t.gz += st_vz[k] * m;
-            }
-        }
-        nsum[nd] = t;
-    }
-    unsigned long long wb = __ballot(wide);
-    while (wb) {
-        const int l = __builtin_ctzll(wb);
-        wb &= wb - 1;
-        const int ws = __shfl(s, l, 64), wc = __shfl(c, l, 64), wn = __shfl(nd, l, 64);
-        const Cover cv = make_cover(ws, ws + wc, nin, (wn == 0 && proot) ? n - nin : 0);
-        NodeSums t{0, 0, 0, 0, 0, 0, 0, 0};
-        for (int k = lane_id(); k < cv.total; k += 64) add_piece(t, cv, k, v, blk1, blk2);
-        t = wave_sums(t);
-        if (lane_id() == 0) nsum[wn] = t;
-    }
-}
-
-// A tree with no particle inside the root cube: the parallel root's sums are
-// those of the particles outside it.
-__global__ void k_moments_root_only(int n, PVals v, NodeSums *nsum) {
-    NodeSums s{0, 0, 0, 0, 0, 0, 0, 0};
-    for (int q = 0; q < n; q++) add_particle(s, q, v);
-    nsum[0] = s;
+// The eight terms of piece k of a cover.  A particle and a block of sums are
+// read through selected addresses, not on two branches, so a wave whose lanes
+// hold both waits for memory once.
+__device__ inline void load_piece(double (&f)[8], const Cover &c, int k, const PVals &v, const NodeSums *blk1,
+                                  const NodeSums *blk2) {
+    const bool part = k < c.k1 || k >= c.k4;
+    const int p = k < c.k1 ? c.s + k : k < c.k5 ? c.p4 + (k - c.k4) : c.nin + (k - c.k5);
+    const NodeSums *b = k < c.k2   ? blk1 + (c.p1 / kBlk1 + (k - c.k1))
+                        : k < c.k3 ? blk2 + (c.p2 / kBlk2 + (k - c.k2))
+                                   : blk1 + (c.p3 / kBlk1 + (k - c.k3));
+    const int q = part ? p : 0;
+    const double m = *(part ? v.sm + q : &b->m), g = *(part ? v.sm + q : &b->g);
+    const double x = *(part ? v.sx + q : &b->sx), y = *(part ? v.sy + q : &b->sy), z = *(part ? v.sz + q : &b->sz);
+    const double gx = *(part ? v.svx + q : &b->gx), gy = *(part ? v.svy + q : &b->gy),
+                 gz = *(part ? v.svz + q : &b->gz);
+    const bool gas = v.stype[q] == 2;
+    f[0] = m;
+    f[1] = part ? x * m : x;
+    f[2] = part ? y * m : y;
+    f[3] = part ? z * m : z;
+    f[4] = part && !gas ? 0.0 : g;
+    f[5] = part ? (gas ? gx * m : 0.0) : gx;
+    f[6] = part ? (gas ? gy * m : 0.0) : gy;
+    f[7] = part ? (gas ? gz * m : 0.0) : gz;
 }
 
 struct NodeMoments {
@@ -1069,9 +1076,19 @@ __global__ __launch_bounds__(256) void k_child_count(int nn, const int32_t *pidx
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-// Every node at once: sums over its key range (the parallel root also
+// Every node at once: the sums over its key range (the parallel root also
 // counts the particles outside its cube, Node.cpp:477-499), centre of mass,
 // gas-weighted velocity, and the walk record at the node's layout place.
+//
+// 256 nodes per workgroup, in XCD ranges (neighbours in pre-order share
+// particles and blocks).  The particles of the workgroup's small nodes and
+// leaves are staged in LDS once; the internal nodes are listed as small (up
+// to kSumTiny particles, or more) and wide, so that the lanes of a wave loop
+// over nodes of like size and the four waves share the wide ones; the sums
+// pass to the nodes' own threads through LDS.  At 1,000,000 particles this is
+// bound by memory (the node arrays and records, 230 bytes a node): sums and
+// moments as two kernels, every node's lane looping over its own particles,
+// took 65 + 110 us (17 + 5 us at 10,000), this one 107 (11).
 //
 // Zero masses (zm, set when any particle has m == 0): the serial insert's
 // running centre of mass (Node.cpp:692-697) divides by the node's mass after
@@ -1079,32 +1096,131 @@ __global__ __launch_bounds__(256) void k_child_count(int nn, const int32_t *pidx
 // index in it, since particles are inserted in array order) has m == 0, that
 // is 0/0 and the node's centre stays NaN for good.  Such a node is never
 // accepted (radius / NaN < theta is false), so the walk opens it.
-__global__ __launch_bounds__(256) void k_node_moments(int nn, int n, int proot, int64_t thr, int zm,
+constexpr int kSumTiny = 8;
+
+__global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, int proot, int64_t thr, int zm,
                                                       const uint32_t *rid, const DevState *ds,
                                                       const int32_t *first, const int32_t *count,
                                                       const int32_t *parent, const int32_t *pidx,
-                                                      const int8_t *level, const NodeSums *nsum,
+                                                      const int8_t *level, const NodeSums *blk1,
+                                                      const NodeSums *blk2,
                                                       const double *gas_table, int gas_equal, int64_t ngas, PVals v,
                                                       const int32_t *nchild, const int32_t *rank,
                                                       const int32_t *cstart, NodeMoments o,
                                                       core::TreeNode *tree, core::SphNode *tsph,
                                                       int32_t *group_first, uint8_t *group_fired) {
-    // nodes in XCD ranges: neighbours in pre-order read neighbouring prefix
-    // sums and particles
-    int nd = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    __shared__ double st_m[kStage], st_x[kStage], st_y[kStage], st_z[kStage];
+    __shared__ double st_vx[kStage], st_vy[kStage], st_vz[kStage];
+    __shared__ uint8_t st_g[kStage];
+    __shared__ double sum[8][256];
+    __shared__ int l_first[256], l_count[256];
+    __shared__ uint8_t list[3][256];   // tiny, small and wide nodes of this workgroup
+    __shared__ int part[3][4];
+    const int nd0 = xcd_block(blockIdx.x, gridDim.x) * 256;
+    const int last = nd0 + 255 < nn ? nd0 + 255 : nn - 1;
+    const int lane = lane_id(), wv = threadIdx.x >> 6;
+    const int nd = nd0 + (int)threadIdx.x;
+    // every particle between the first particles of two nodes has its leaf
+    // between them in pre-order, so the span is at most 255 + kSumSmall
+    const int P0 = first[nd0];
+    int P1 = first[last] + kSumSmall;
+    P1 = P1 < nin ? P1 : nin;
+    int s = 0, cn = 0, p = -1;
+    if (nd < nn) {
+        s = first[nd];
+        cn = count[nd];
+        p = pidx[nd];
+    }
+    for (int k = threadIdx.x; k < P1 - P0; k += 256) {
+        const int q = P0 + k;
+        const bool g = v.stype[q] == 2;
+        st_m[k] = v.sm[q]; st_x[k] = v.sx[q]; st_y[k] = v.sy[q]; st_z[k] = v.sz[q];
+        st_g[k] = g ? 1 : 0;
+        if (g) { st_vx[k] = v.svx[q]; st_vy[k] = v.svy[q]; st_vz[k] = v.svz[q]; }
+    }
+    const bool inner = nd < nn && p < 0;
+    const bool wide = inner && ((nd == 0 && proot) || cn > kSumSmall);
+    const bool tiny = inner && !wide && cn <= kSumTiny;
+    const unsigned long long bal[3] = {__ballot(tiny), __ballot(inner && !wide && !tiny), __ballot(wide)};
+    if (lane < 3) part[lane][wv] = __popcll(lane == 0 ? bal[0] : lane == 1 ? bal[1] : bal[2]);
+    l_first[threadIdx.x] = s;
+    l_count[threadIdx.x] = cn;
+    __syncthreads();
+    int len[3];
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+        int at = 0;
+        len[u] = 0;
+        for (int k = 0; k < 4; k++) {
+            const int h = part[u][k];
+            at += k < wv ? h : 0;
+            len[u] += h;
+        }
+        if (bal[u] >> lane & 1) list[u][at + __popcll(bal[u] & lanes_below())] = (uint8_t)threadIdx.x;
+    }
+    __syncthreads();
+    // tiny and small nodes a lane each, in rows of 64
+    const int rows0 = (len[0] + 63) / 64, rows = rows0 + (len[1] + 63) / 64;
+    for (int r = wv; r < rows; r += 4) {
+        const int u = r < rows0 ? 0 : 1;
+        const int at = (r - (u ? rows0 : 0)) * 64 + lane;
+        if (at < len[u]) {
+            const int t = list[u][at];
+            const int k0 = l_first[t] - P0, k1 = k0 + l_count[t];
+            NodeSums a{0, 0, 0, 0, 0, 0, 0, 0};
+            for (int k = k0; k < k1; k++) {
+                const double m = st_m[k];
+                a.m += m;
+                a.sx += st_x[k] * m;
+                a.sy += st_y[k] * m;
+                a.sz += st_z[k] * m;
+                if (st_g[k]) {
+                    a.g += m;
+                    a.gx += st_vx[k] * m;
+                    a.gy += st_vy[k] * m;
+                    a.gz += st_vz[k] * m;
+                }
+            }
+            sum[0][t] = a.m; sum[1][t] = a.sx; sum[2][t] = a.sy; sum[3][t] = a.sz;
+            sum[4][t] = a.g; sum[5][t] = a.gx; sum[6][t] = a.gy; sum[7][t] = a.gz;
+        }
+    }
+    // wide nodes a wave each, the waves without rows first
+    for (int j = 3 - wv; j < len[2]; j += 4) {
+        const int t = list[2][j];
+        const int ws = l_first[t];
+        const bool root = nd0 + t == 0 && proot;
+        const Cover cv = make_cover(ws, ws + l_count[t], nin, root ? n - nin : 0);
+        double a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        // two pieces in flight, added in order
+        for (int k = lane; k < cv.total; k += 128) {
+            const bool two = k + 64 < cv.total;
+            double f[8], h[8];
+            load_piece(f, cv, k, v, blk1, blk2);
+            load_piece(h, cv, two ? k + 64 : k, v, blk1, blk2);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                a[i] += f[i];
+                a[i] = two ? a[i] + h[i] : a[i];
+            }
+        }
+        const double r = wave_sums8(a);
+        if ((lane & 7) == 0) sum[lane >> 3][t] = r;
+    }
+    __syncthreads();
     if (nd >= nn) return;
     // cleared group state for the density phase (Node.cpp:722-796)
     group_first[nd] = kGroupNone;
     group_fired[nd] = 0;
-    int p = pidx[nd];
     int par = parent[nd];
     double M, g, cx, cy, cz, mvx = 0.0, mvy = 0.0, mvz = 0.0;
     const core::Pos pos{v.sx, v.sy, v.sz};
     // buckets exist only where k_lcp met adjacent particles at one position
     const bool buckets = ds->any_bucket != 0;
     if (p >= 0) {
-        M = v.sm[p];
-        g = v.stype[p] == 2 ? M : 0.0;
+        const int k = p - P0;
+        M = st_m[k];
+        g = st_g[k] ? M : 0.0;
         bool vec = par < 0 ? (n == 1) : core::parallel_node(count, parent, par, n, thr);
         if (par >= 0 && !vec && buckets) {
             // members of a bucket sit exactly at their position
@@ -1112,14 +1228,15 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int n, int proot, 
             const int pe = (par == 0 && proot) ? n : first[par] + count[par];
             vec = core::is_bucket(pos, ps, pe);
         }
-        cx = core::leaf_com(v.sx[p], M, vec);
-        cy = core::leaf_com(v.sy[p], M, vec);
-        cz = core::leaf_com(v.sz[p], M, vec);
+        cx = core::leaf_com(st_x[k], M, vec);
+        cy = core::leaf_com(st_y[k], M, vec);
+        cz = core::leaf_com(st_z[k], M, vec);
     } else {
-        int s = first[nd], e = first[nd] + count[nd];
+        int e = s + cn;
         if (nd == 0 && proot) { s = 0; e = n; }
-        const NodeSums ns = nsum[nd];
-        const double S[8] = {ns.m, ns.sx, ns.sy, ns.sz, ns.g, ns.gx, ns.gy, ns.gz};
+        double S[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) S[j] = sum[j][threadIdx.x];
         M = S[0];
         // equal gas masses: the reference's running sum, bit for bit (its
         // group selection compares gas masses and can sit on exact ties).
@@ -1135,7 +1252,7 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int n, int proot, 
         else { cx = cy = cz = 0.0; }
         if (zm && !(nd == 0 && proot) && !core::parallel_node(count, parent, nd, n, thr)) {
             uint32_t first_any = 0xffffffffu, first_pos = 0xffffffffu;
-            for (int j = first[nd]; j < first[nd] + count[nd]; j++) {
+            for (int j = s; j < s + cn; j++) {
                 const uint32_t q = rid[j];
                 first_any = q < first_any ? q : first_any;
                 if (v.sm[j] != 0.0) first_pos = q < first_pos ? q : first_pos;
@@ -1164,7 +1281,7 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int n, int proot, 
     if (tsph && g > 0.0) {   // only gas nodes are ever SPH candidates
         core::SphNode w;
         w.cx = cx; w.cy = cy; w.cz = cz; w.gas = g;
-        if (p >= 0) { w.vx = v.svx[p]; w.vy = v.svy[p]; w.vz = v.svz[p]; }
+        if (p >= 0) { w.vx = st_vx[p - P0]; w.vy = st_vy[p - P0]; w.vz = st_vz[p - P0]; }
         else { w.vx = mvx; w.vy = mvy; w.vz = mvz; }
         w.pidx = p;
         w.pad = 0;
@@ -1364,7 +1481,6 @@ void alloc_nodes(Ctx &c, int64_t cap) {
         cv(&c.n_nchild, n * 4); cv(&c.n_rank, n * 4); cv(&c.n_cstart, n * 4);
         cv(&c.n_ichild, n * 4);
         cv(&c.nsum_tile, (pcap / kBlk2 + 1) * (kBlk2 / kBlk1 + 1) * sizeof(NodeSums));
-        cv(&c.nsum, n * sizeof(NodeSums));
         cv(&c.n_bsum, (n / 1024 + 2) * 4);
     };
     Carve size;
@@ -1781,28 +1897,23 @@ void build_tree_b(Ctx &c) {
                                    c.n_int, kw, c.lcp, c.base, c.n_cstart, o);
         }
         PVals pv{c.x, c.y, c.z, c.m, c.vx, c.vy, c.vz, c.type};
-        // child counts, node sums bottom-up, the child-place scan, then
-        // moments and walk records
+        // child counts, the child-place scan, then node sums, moments and
+        // walk records
         int gn = grid_for(nn, 256);
         int nbn = (nn + 1023) / 1024;
         hipLaunchKernelGGL(k_child_count, dim3(nbn), dim3(256), 0, st, nn, c.n_pidx, c.n_level, c.n_count, c.n_skip,
                            c.n_nchild, c.n_rank, c.n_ichild, gl, part, part + kLeafBlocks, c.ds, c.n_bsum);
-        if (nin > 0) {
-            // the block sums from build_order are stale after a refinement
-            // re-ordered the particles or the node arrays grew
-            if (!tiles_current) launch_tile_sums(c);
-            NodeSums *blk1, *blk2;
-            tile_sum_buffers(c, &blk1, &blk2);
-            hipLaunchKernelGGL(k_sums_direct, dim3(gn), dim3(256), 0, st, nn, nin, n, proot, c.n_first, c.n_count,
-                               c.n_pidx, pv, blk1, blk2, c.nsum);
-        } else if (proot)
-            hipLaunchKernelGGL(k_moments_root_only, dim3(1), dim3(1), 0, st, n, pv, c.nsum);
+        // the block sums from build_order are stale after a refinement
+        // re-ordered the particles or the node arrays grew
+        if (nin > 0 && !tiles_current) launch_tile_sums(c);
+        NodeSums *blk1, *blk2;
+        tile_sum_buffers(c, &blk1, &blk2);
         hipLaunchKernelGGL(k_iscan_apply, dim3(nbn), dim3(256), 0, st, nn, c.n_nchild, c.n_bsum, c.n_cstart);
         NodeMoments nm{c.n_mass, c.n_gas, c.n_cx, c.n_cy, c.n_cz, c.n_gvx, c.n_gvy, c.n_gvz};
-        hipLaunchKernelGGL(k_node_moments, dim3(gn), dim3(256), 0, st, nn, n, proot, c.p.split_threshold,
+        hipLaunchKernelGGL(k_node_moments, dim3(gn), dim3(256), 0, st, nn, nin, n, proot, c.p.split_threshold,
                            c.zero_mass > 0 ? 1 : 0, c.rid, c.ds,
-                           c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_level, c.nsum, c.gas_table, c.gas_equal,
-                           c.gas_count, pv,
+                           c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_level, blk1, blk2, c.gas_table,
+                           c.gas_equal, c.gas_count, pv,
                            c.n_nchild, c.n_rank, c.n_cstart, nm, c.tnode,
                            c.sph_active ? c.tsph : nullptr, c.g_first, c.g_fired);
         c.groups_cleared = true;
