@@ -112,13 +112,14 @@ struct Ctx {
     bool fp64_fallback = false;  // the last forces of a split-precision context ran the FP64 sweep
     uint32_t *hist = nullptr, *dtotal = nullptr;
     // topology over particles in key order
-    int8_t *lcp = nullptr;
-    int8_t *lk = nullptr;   // key levels particles i and i + 1 share (-1 after the last one inside)
+    uint8_t *lcp = nullptr;    // levels that particles i and i + 1 share, + 1 (0 after the last one inside)
+    uint8_t *lmin = nullptr;   // the least of them in each tile of 1024
+    int32_t *leaf_part = nullptr;   // per tile: deepest leaf level | gaps << 8
     int32_t *cnt = nullptr, *base = nullptr, *bsum = nullptr;
 
     // nodes (pre-order)
     int64_t node_cap = 0;
-    int32_t *n_first = nullptr, *n_count = nullptr, *n_skip = nullptr, *n_parent = nullptr;
+    int32_t *n_first = nullptr, *n_count = nullptr, *n_parent = nullptr;
     int32_t *n_pidx = nullptr;
     int8_t *n_level = nullptr;
     double *n_mass = nullptr;
@@ -137,7 +138,6 @@ struct Ctx {
     int32_t *g_final = nullptr;
     double *g_rho = nullptr;
 
-    int32_t *n_ichild = nullptr;   // internal children (they bound the walk's stack in deep trees)
     NodeSums *nsum_tile = nullptr;   // sums of aligned 64- and 4096-particle blocks (node sums)
     // The reference sums a node's gas mass one particle at a time in array
     // order (Node.cpp:479, :681).  When every gas particle has the same mass m

@@ -65,7 +65,9 @@ void alloc_all(Ctx &c, int64_t cap) {
         for (double **p : d) cv(p, n * 8);
         for (double *&p : c.alt) cv(&p, n * 8);
         cv(&c.type, n); cv(&c.active, n); cv(&c.gapl, n);
-        cv(&c.type_alt, n); cv(&c.active_alt, n); cv(&c.lcp, n); cv(&c.lk, n + 1);
+        cv(&c.type_alt, n); cv(&c.active_alt, n);
+        // whole tiles of 1024, and what a search reads past the last particle's
+        cv(&c.lcp, n + 1024 + 128); cv(&c.lmin, (n + 1023) / 1024 + 2048);
         cv(&c.rid, n * 4); cv(&c.rid_alt, n * 4); cv(&c.inv, n * 4);
         cv(&c.gslot, n * 4); cv(&c.gidx, n * 4);
         cv(&c.gtiles, ((n + 1023) / 1024 + 1) * 4); cv(&c.gover, (n + 63) / 64 + 1);
@@ -79,7 +81,7 @@ void alloc_all(Ctx &c, int64_t cap) {
         const size_t nblk = (n + ag2::kSortTile - 1) / ag2::kSortTile + 1;
         cv(&c.hist, 256 * nblk * 4); cv(&c.dtotal, 256 * 4);
         cv(&c.cnt, (n + 1) * 4); cv(&c.base, (n + 1) * 4);
-        cv(&c.bsum, ((n + 1023) / 1024 + 1) * 4);
+        cv(&c.bsum, ((n + 1023) / 1024 + 1) * 4); cv(&c.leaf_part, ((n + 1023) / 1024 + 1) * 4);
         cv(&c.partials, 8 * 1024 * 8);
         cv(&c.ds, sizeof(ag2::DevState));
         cv(&c.cbins, ag2::kCounterBinBytes);
@@ -138,14 +140,13 @@ int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
     int64_t n = cap, nodes = 2 * cap + 64;
     int64_t per_p = 21 * 8            // state, potential, star-formation rate
                     + kStateD * 8     // permute buffers
-                    + 7               // type, active, gap level, their copies, lcp, adjacent key levels
+                    + 6               // type, active, gap level, their copies, adjacent levels
                     + 4 * 8 + 2 * 4   // keys, sort indices
                     + 3 * 4           // rid, rid copy, inverse
                     + 2 * 4           // c, base
                     + 2 * 4 + 1;      // SPH list slots, targets, group flags
-    int64_t per_node = 5 * 4 + 1 + 9 * 8 + 2 * 4 + 1 + 4 +
+    int64_t per_node = 4 * 4 + 1 + 9 * 8 + 2 * 4 + 1 + 4 +
                        2 * (int64_t)sizeof(core::TreeNode) + 3 * 4 +   // walk and SPH records
-                       4 +                                             // internal-child counts
                        (int64_t)sizeof(ag2::NodeSums) / 64 + 1;        // block sums
     int64_t fixed = 256 * ((n + kSortTile - 1) / kSortTile + 1) * 4 + 8 * 1024 * 8 + (1 << 20) +
                     walk_groups_max(cap) * (4 + ag2::kNearRecs * 12) +   // near-pair records

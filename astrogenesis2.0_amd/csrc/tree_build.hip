@@ -658,22 +658,31 @@ __global__ __launch_bounds__(256) void k_inverse(int n, const uint32_t *rid, int
     if (r < n) inv[rid[r]] = r;
 }
 
-// L[i] and c[i] = max(0, L[i] - L[i-1]), over the key words of this build
-// (nw of them) and the positions in key order (runs at one position are
-// buckets).  A distinct pair that agrees on every word sets ds->tie_deep:
-// the build refines it with deeper words (refine_ties), or fails past
-// kDeepest levels.
+// lv[i] = L[i] + 1 (0 .. 127; L: the levels particles i and i + 1 share, -1
+// after the last one inside) and c[i] = max(0, L[i] - L[i-1]), over the key
+// words of this build (nw of them) and the positions in key order (runs at
+// one position are buckets).  A distinct pair that agrees on every word sets
+// ds->tie_deep: the build refines it with deeper words (refine_ties), or
+// fails past kDeepest levels.
 // Four particles per thread (a 1024-particle scan tile per workgroup); the
-// tile's sum of c goes to bsum for k_scan_apply.
+// tile's sum of c goes to bsum for k_scan_apply, the least lv of the tile
+// (0 past the last particle) to lmin for the cell searches.
+constexpr int kLevTile = 1024;
+
 __global__ __launch_bounds__(256) void k_lcp(int n, core::KeyWords kw, int nw, core::Pos pos, DevState *ds,
-                                             int parallel_root, int8_t *L, int8_t *Lk, int32_t *c, int32_t *bsum) {
-    __shared__ int scr[4];
+                                             int parallel_root, uint8_t *lv, uint8_t *lmin, int32_t *c,
+                                             int32_t *bsum) {
+    __shared__ int scr[4], wmin[4];
     const int nin = ds->nin;
     const bool proot = parallel_root != 0, splits = proot && nin < n;
-    int tile = 0;
+    int tile = 0, least = 127;
     for (int k = 0; k < 4; k++) {
-        const int i = blockIdx.x * 1024 + k * 256 + threadIdx.x;
-        if (i >= nin) continue;
+        const int i = blockIdx.x * kLevTile + k * 256 + threadIdx.x;
+        if (i >= nin) {
+            lv[i] = 0;
+            least = 0;
+            continue;
+        }
         int li = core::pair_lcp(kw, pos, i, nin, proot, splits);
         int lp = i == 0 ? -1 : core::pair_lcp(kw, pos, i - 1, nin, proot, splits);
         // a coincident pair's level is its bucket's (pair_lcp), whatever the key words say
@@ -682,16 +691,24 @@ __global__ __launch_bounds__(256) void k_lcp(int n, core::KeyWords kw, int nw, c
         if (i + 1 < nin && li >= 21 * nw && !coincident) ds->tie_deep = 1;
         if (li > core::kDeepest) { li = core::kDeepest; ds->tie_deep = 1; }
         if (lp > core::kDeepest) lp = core::kDeepest;
-        L[i] = (int8_t)li;
-        // the keys' own adjacent levels, for the cell searches (buckets share every level)
-        Lk[i] = i + 1 < nin ? (int8_t)core::shared_levels(kw, i, i + 1) : (int8_t)-1;
+        lv[i] = (uint8_t)(li + 1);
+        least = li + 1 < least ? li + 1 : least;
         const int v = li - lp > 0 ? li - lp : 0;
         c[i] = v;
         tile += v;
     }
+    for (int d = 32; d >= 1; d >>= 1) {
+        const int t = __shfl_xor(least, d, 64);
+        least = t < least ? t : least;
+    }
+    if (lane_id() == 0) wmin[threadIdx.x >> 6] = least;
     int tot;
     block256_excl_scan(tile, scr, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) {
+        bsum[blockIdx.x] = tot;
+        for (int w = 1; w < 4; w++) least = wmin[w] < least ? wmin[w] : least;
+        lmin[blockIdx.x] = (uint8_t)least;
+    }
 }
 
 // The exclusive scan of c into base over tiles of 1024 (256 threads x 4):
@@ -721,89 +738,288 @@ __global__ __launch_bounds__(256) void k_scan_apply(const int32_t *c, const int3
 }
 
 // ------------------------------------------------------------ nodes
-// One thread per internal node.  The internal nodes, numbered q = 0 .. n_int
-// - 1 in pre-order, are those of particle i for base[i] <= q < base[i] + c[i]
-// (k_make_leaf lists own[q] = i); node q of particle i sits at pre-order
-// index i + q, at level L[i-1] + 1 + (q - base[i]).  A particle can start a
-// chain of many nested cells, each needing a galloping search for its last
-// particle; giving every cell its own thread keeps those searches from
-// running one after another in a single lane, and listing only internal
-// nodes keeps every lane of a wave searching.
-__global__ __launch_bounds__(256) void k_make_internal(int nin, int nn, int n_int, core::KeyWords kw,
-                                                       const int8_t *L, const int32_t *base, const int32_t *own,
-                                                       core::NodeOut o) {
-    int q = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-    if (q >= n_int) return;
-    int i = own[q];
-    int l = core::lcp_prev(L, i) + 1 + (q - base[i]);
-    core::make_internal(kw, L, base, i, l, nin, nn, o);
+// The tree from the levels alone.  A particle starts c[i] internal nodes, of
+// levels L[i-1] + 1 .. L[i], then its leaf; the internal nodes, numbered q =
+// 0 .. n_int - 1 in pre-order, are those of particle i for base[i] <= q <
+// base[i] + c[i] (k_make_leaf lists own[q] = i), and node q of particle i
+// sits at pre-order index i + q.  The level-l node from particle i on ends
+// with the first j >= i whose L[j] < l, and every j before that with L[j] ==
+// l ends one child: the next starts at particle j + 1, as its first node.  So
+// the end, the children and their ranks come out of one search for levels <=
+// l, with no look at the keys.  (Members of a bucket, whose L is the bucket's
+// level, come out as its children.)
+struct NodeArrays {
+    int32_t *first, *count, *parent, *pidx, *nchild, *rank;
+    int8_t *level;
+};
+
+// The bytes of x below t (bytes 0 .. 127, t 1 .. 128 in every byte of t4), as
+// 4 bits scaled by 128, shifted up by 4 with HI.
+template <bool HI>
+__device__ inline unsigned below4(unsigned x, unsigned t4, unsigned acc) {
+    const unsigned less = ~((x | 0x80808080u) - t4) & 0x80808080u;
+    return (unsigned)__builtin_amdgcn_udot4(less, HI ? 0x80402010u : 0x08040201u, acc, false);
 }
 
-__global__ __launch_bounds__(256) void k_make_root_only(core::NodeOut o) {
-    o.first[0] = 0; o.count[0] = 0; o.skip[0] = 1; o.parent[0] = -1; o.pidx[0] = -1; o.level[0] = 0;
+typedef unsigned levels16 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Which of 16 bytes are below t, 16 bits.
+__device__ inline unsigned below16(const levels16 &x, unsigned t4) {
+    const unsigned a = below4<true>(x[1], t4, below4<false>(x[0], t4, 0u));
+    const unsigned b = below4<true>(x[3], t4, below4<false>(x[2], t4, 0u));
+    return a >> 7 | b << 1;
 }
 
-// Grid-stride over a fixed grid (at most kLeafBlocks workgroups), so the
-// deepest level and the gap count cost one pair of atomics per workgroup.
-constexpr int kLeafBlocks = 1024;
+// Which of the 64 levels from particle i on are below t; x: the 68 bytes from
+// i & ~3 on.
+__device__ inline unsigned long long below64(const levels16 (&x)[4], unsigned x4, int sh, unsigned t4) {
+    unsigned long long m = 0ull;
+#pragma unroll
+    for (int k = 0; k < 4; k++) m |= (unsigned long long)below16(x[k], t4) << (16 * k);
+    const unsigned long long up = below4<false>(x4, t4, 0u) >> 7;
+    return sh ? m >> sh | up << (64 - sh) : m;
+}
 
-__global__ __launch_bounds__(256) void k_make_leaf(int nin, core::KeyWords kw,
-                                                   const int8_t *L, const int8_t *Lk, const int32_t *base,
-                                                   const int32_t *c,
-                                                   core::NodeOut o, const uint32_t *idx, const uint8_t *gapl,
-                                                   int32_t *own, unsigned long long *part_lv,
-                                                   unsigned long long *part_gap) {
+// The boundaries among the 16 levels of each lane (bit b of le: the particle
+// after p0 + b starts a child), as children run + 1, run + 2, .. of node nd;
+// returns their number.
+__device__ inline int emit_children(unsigned le, int p0, int nd, int run, const int32_t *base, const NodeArrays &o) {
+    const unsigned long long any = __ballot(le != 0);
+    int r = run + __popcll(any & lanes_below()), total = __popcll(any);
+    if (__ballot((le & (le - 1)) != 0)) {   // more than one in some lane
+        const int k = __popc(le);
+        const int inc = wave_incl_scan(k);
+        r = run + inc - k;
+        total = __shfl(inc, 63, 64);
+    }
+    while (le) {
+        const int p = p0 + __builtin_ctz(le) + 1;
+        le &= le - 1;
+        const int ch = p + base[p];
+        o.parent[ch] = nd;
+        o.rank[ch] = ++r;
+    }
+    return total;
+}
+
+// 1024 levels from s on (a multiple of 16) for a node: every boundary from i
+// on in them, up to the node's end if that is here (returned; -1: the node
+// goes on).
+__device__ inline int scan_levels(const uint8_t *lv, int s, int i, unsigned lt4, unsigned le4, int nd, int *run,
+                                const int32_t *base, const NodeArrays &o) {
+    const int p0 = s + lane_id() * 16;
+    const levels16 x = *(const levels16 *)(lv + p0);
+    const int cut = i - p0;
+    const unsigned from = cut <= 0 ? 0xffffu : cut >= 16 ? 0u : 0xffffu << cut & 0xffffu;
+    const unsigned lt = below16(x, lt4) & from;
+    unsigned le = below16(x, le4) & from;
+    const unsigned long long f = __ballot(lt != 0);
+    int end = -1;
+    if (f) {
+        const int fl = __builtin_ctzll(f);
+        const int at = __builtin_ctz(__shfl(lt, fl, 64));
+        end = s + fl * 16 + at;
+        le = lane_id() < fl ? le : lane_id() == fl ? le & ((1u << at) - 1) : 0u;
+    }
+    if (__ballot(le != 0)) *run += emit_children(le, p0, nd, *run, base, o);
+    return end;
+}
+
+// One thread per internal node.  A node whose end is among the 64 levels from
+// its first particle on (and that has at most 8 children) is found by its
+// thread, in one read; the others, a few in a hundred, are listed and shared by
+// the workgroup's waves: the 1024 levels from the first particle on, the rest
+// of the tile they end in, then the tiles' least levels, then the tiles that hold a child's end, a read each.  tsum
+// (zeroed by k_make_leaf) gets the children of every 1024 nodes for
+// k_iscan_apply.
+// Galloping searches over the keys for each node's end and its parent's
+// start, then a pass that followed the children by their skip links, were
+// chains of 10 to 50 dependent reads: make_leaf, make_internal and
+// child_count took 14 + 17 + 11 us at 10,000 particles and 37 + 39 + 17 us at
+// 1,000,000; now make_leaf and make_internal 6.5 + 9.5 and 16 + 30.
+template <int PER>
+__global__ __launch_bounds__(256) void k_make_internal(int nin, int n_int, const uint8_t *lv, const uint8_t *lmin,
+                                                       const int32_t *base, const int32_t *own, NodeArrays o,
+                                                       int32_t *tsum) {
+    __shared__ int w_i[PER], w_l[PER], w_nd[PER], n_wide;
+    if (threadIdx.x == 0) n_wide = 0;
+    __syncthreads();
+    const int q = xcd_block(blockIdx.x, gridDim.x) * PER + threadIdx.x;
+    const bool have = (int)threadIdx.x < PER && q < n_int;
+    int nch = 0, nd = 0;
+    if (have) {
+        const int i = own[q];
+        const int l = (i > 0 ? (int)lv[i - 1] : 0) + (q - base[i]);
+        nd = i + q;
+        levels16 x[4];
+        const uint8_t *w = lv + (i & ~3);
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = *(const levels16 *)(w + 16 * k);
+        const unsigned x4 = *(const unsigned *)(w + 64);
+        const unsigned long long lt = below64(x, x4, i & 3, (unsigned)(l + 1) * 0x01010101u);
+        unsigned long long le = below64(x, x4, i & 3, (unsigned)(l + 2) * 0x01010101u);
+        o.first[nd] = i;
+        o.pidx[nd] = -1;
+        o.level[nd] = (int8_t)l;
+        if (nd == 0) o.parent[0] = -1;
+        o.parent[nd + 1] = nd;
+        o.rank[nd + 1] = 0;
+        // a tree of one particle under a root that always splits has no level below the root's
+        int e = lt ? __builtin_ctzll(lt) : 64;
+        e = i + e > nin - 1 ? nin - 1 - i : e;
+        le &= e < 64 ? (1ull << e) - 1 : ~0ull;
+        const int more = __popcll(le);
+        if (e < 64 && more <= 7) {
+            o.count[nd] = e + 1;
+            o.nchild[nd] = nch = more + 1;
+            int p[7], b[7];
+#pragma unroll
+            for (int k = 0; k < 7; k++) {
+                p[k] = le ? i + __builtin_ctzll(le) + 1 : i;
+                le &= le - 1;
+            }
+#pragma unroll
+            for (int k = 0; k < 7; k++) b[k] = base[p[k]];
+#pragma unroll
+            for (int k = 0; k < 7; k++)
+                if (k < more) {
+                    o.parent[p[k] + b[k]] = nd;
+                    o.rank[p[k] + b[k]] = k + 1;
+                }
+        } else {
+            const int at = atomicAdd(&n_wide, 1);
+            w_i[at] = i;
+            w_l[at] = l;
+            w_nd[at] = nd;
+        }
+    }
+    // the children of the threads' own nodes (1 .. 8 each), by tile of nodes
+    unsigned long long left = __ballot(nch > 0);
+    while (left) {
+        const int f = __builtin_ctzll(left);
+        const int t = __shfl(nd >> 10, f, 64);
+        const bool in = nch > 0 && (nd >> 10) == t;
+        int s = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s += __popcll(__ballot(in && (nch >> k & 1))) << k;
+        if (lane_id() == f) atomicAdd(&tsum[t], s);
+        left &= ~__ballot(in);
+    }
+    __syncthreads();
+    const int nw = n_wide;
+    for (int k = threadIdx.x >> 6; k < nw; k += 4) {
+        const int i = w_i[k], l = w_l[k], node = w_nd[k];
+        const unsigned lt4 = (unsigned)(l + 1) * 0x01010101u, le4 = (unsigned)(l + 2) * 0x01010101u;
+        int run = 0;
+        const int s = i & ~15, tile = (s + 2 * kLevTile - 1) / kLevTile;   // the first tile all past s + 1023
+        int end = scan_levels(lv, s, i, lt4, le4, node, &run, base, o);
+        if (end < 0 && s % kLevTile)
+            end = scan_levels(lv, (tile - 1) * kLevTile, s + kLevTile, lt4, le4, node, &run, base, o);
+        for (int t0 = tile & ~15, from = tile; end < 0; t0 += kLevTile, from = t0) {
+            // the tile of particle nin - 1 holds a level below every l, so
+            // the search ends there at the latest
+            const int p0 = t0 + lane_id() * 16;
+            const levels16 x = *(const levels16 *)(lmin + p0);
+            const int cut = from - p0;
+            const unsigned in = cut <= 0 ? 0xffffu : cut >= 16 ? 0u : 0xffffu << cut & 0xffffu;
+            // tiles with a child's end or the node's, in order
+            unsigned le = below16(x, le4) & in;
+            unsigned long long b = __ballot(le != 0);
+            while (b && end < 0) {
+                const int f = __builtin_ctzll(b);
+                b &= b - 1;
+                unsigned m = __shfl(le, f, 64);
+                while (m && end < 0) {
+                    end = scan_levels(lv, (t0 + f * 16 + __builtin_ctz(m)) * kLevTile, i, lt4, le4, node, &run, base, o);
+                    m &= m - 1;
+                }
+            }
+        }
+        if (lane_id() == 0) {
+            o.count[node] = end - i + 1;
+            o.nchild[node] = run + 1;
+            atomicAdd(&tsum[node >> 10], run + 1);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_make_root_only(NodeArrays o, int32_t *tsum) {
+    if (threadIdx.x == 0) {
+        o.first[0] = 0; o.count[0] = 0; o.parent[0] = -1; o.pidx[0] = -1; o.level[0] = 0;
+        o.nchild[0] = 0; o.rank[0] = 0;
+        tsum[0] = 0;
+    }
+}
+
+// The leaves (one per particle), the list of the particles that start the
+// internal nodes, and per tile of 1024 particles the deepest leaf level and
+// the number of gaps (part: level | gaps << 8).  It needs nothing of the host,
+// so it runs while the host waits for the counts; when the nodes are more
+// than the room (ds->err) it writes nothing, and the host launches it again
+// after making room.
+__global__ __launch_bounds__(256) void k_make_leaf(const DevState *ds, const uint8_t *lv, const int32_t *base,
+                                                   const int32_t *c, NodeArrays o, const uint32_t *idx,
+                                                   const uint8_t *gapl, int32_t *own, int32_t *tsum, int32_t *part) {
     __shared__ int wl[4], wg[4];
-    int lv = 0, gp = 0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < nin; i += gridDim.x * 256) {
-        int li = 0;
-        core::make_leaf(kw, L, Lk, base, c, i, o, &li);
-        // particle i starts internal nodes base[i] .. base[i] + c[i] - 1
+    if (ds->err) return;
+    const int nin = ds->nin;
+    for (int k = blockIdx.x * 256 + threadIdx.x; k <= ds->n_nodes / 1024; k += gridDim.x * 256) tsum[k] = 0;
+    int deep = 0, gp = 0;
+    for (int k = 0; k < 4; k++) {
+        const int i = blockIdx.x * kLevTile + k * 256 + threadIdx.x;
+        if (i >= nin) continue;
+        const int a = i > 0 ? lv[i - 1] : 0, b = lv[i];
+        const int li = a > b ? a : b;   // one level below the deeper neighbour pair
         const int b0 = base[i], ci = c[i];
-        for (int k = 0; k < ci; k++) own[b0 + k] = i;
-        lv = li > lv ? li : lv;
-        int g = gapl[idx[i]];
+        const int g = gapl[idx[i]];
+        const int nd = i + b0 + ci;
+        o.first[nd] = i;
+        o.count[nd] = 1;
+        o.pidx[nd] = i;
+        o.level[nd] = (int8_t)li;
+        o.nchild[nd] = 0;
+        if (nd == 0) o.parent[0] = -1;
+        // particle i starts internal nodes base[i] .. base[i] + c[i] - 1
+        for (int u = 0; u < ci; u++) own[b0 + u] = i;
+        deep = li > deep ? li : deep;
         gp += (g > 0 && g <= li) ? 1 : 0;
     }
     for (int d = 32; d >= 1; d >>= 1) {
-        int t = __shfl_xor(lv, d, 64);
-        lv = t > lv ? t : lv;
+        const int t = __shfl_xor(deep, d, 64);
+        deep = t > deep ? t : deep;
         gp += __shfl_xor(gp, d, 64);
     }
-    if (lane_id() == 0) { wl[threadIdx.x >> 6] = lv; wg[threadIdx.x >> 6] = gp; }
+    if (lane_id() == 0) { wl[threadIdx.x >> 6] = deep; wg[threadIdx.x >> 6] = gp; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int bl = wl[0], bg = wg[0];
-        for (int w = 1; w < 4; w++) { bl = wl[w] > bl ? wl[w] : bl; bg += wg[w]; }
-        part_lv[blockIdx.x] = (unsigned long long)bl;
-        part_gap[blockIdx.x] = (unsigned long long)bg;
+        for (int w = 1; w < 4; w++) { deep = wl[w] > deep ? wl[w] : deep; gp += wg[w]; }
+        part[blockIdx.x] = deep | gp << 8;
     }
 }
 
-// Deepest leaf level and gap count from make_leaf's per-block partials
-// (one workgroup of 256; run by the first workgroup of k_child_count).
-__device__ inline void leaf_fold(int nb, const unsigned long long *part_lv, const unsigned long long *part_gap,
-                                 DevState *ds) {
-    __shared__ unsigned long long wl[4], wg[4];
-    unsigned long long lv = 0ull, gp = 0ull;
+// Deepest leaf level and gap count from make_leaf's per-tile partials
+// (one workgroup of 256; run by the first workgroup of k_iscan_apply).
+__device__ inline void leaf_fold(int nb, const int32_t *part, DevState *ds) {
+    __shared__ int wl[4], wg[4];
+    int lv = 0, gp = 0;
     for (int k = threadIdx.x; k < nb; k += 256) {
-        lv = part_lv[k] > lv ? part_lv[k] : lv;
-        gp += part_gap[k];
+        const int p = part[k];
+        lv = (p & 0xff) > lv ? p & 0xff : lv;
+        gp += p >> 8;
     }
     for (int o = 32; o >= 1; o >>= 1) {
-        unsigned long long q = __shfl_xor(lv, o, 64);
+        const int q = __shfl_xor(lv, o, 64);
         lv = q > lv ? q : lv;
         gp += __shfl_xor(gp, o, 64);
     }
     if (lane_id() == 0) { wl[threadIdx.x >> 6] = lv; wg[threadIdx.x >> 6] = gp; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long l = wl[0], g = wg[0];
-        for (int w = 1; w < 4; w++) { l = wl[w] > l ? wl[w] : l; g += wg[w]; }
-        ds->max_level = (int32_t)l;
+        for (int w = 1; w < 4; w++) { lv = wl[w] > lv ? wl[w] : lv; gp += wg[w]; }
+        ds->max_level = lv;
         // stack growth bound: at most 7 blocks per level below
-        ds->walk_depth = 7 * ((int32_t)l + 3);
-        ds->gap = g;
+        ds->walk_depth = 7 * (lv + 3);
+        ds->gap = (unsigned long long)gp;
     }
 }
 
@@ -1029,52 +1245,10 @@ struct NodeMoments {
 
 // Child-contiguous layout for the block walk (core::TreeNode): the root at 0,
 // the children of node p at [1 + cstart[p], 1 + cstart[p] + nchild[p]) in
-// octant order, cstart being the exclusive scan of nchild in pre-order.  Every node
-// follows its children's skip links (pull, no atomics): it counts them and
-// gives each its rank among its siblings, which in pre-order is its octant
-// order.  A bucket (particles at one position) holds its member leaves, the
-// next count nodes, as children.
-__global__ __launch_bounds__(256) void k_child_count(int nn, const int32_t *pidx, const int8_t *level,
-                                                     const int32_t *count, const int32_t *skip, int32_t *nchild,
-                                                     int32_t *rank, int32_t *ichild, int nleaf_blocks,
-                                                     const unsigned long long *part_lv,
-                                                     const unsigned long long *part_gap, DevState *ds,
-                                                     int32_t *bsum) {
-    __shared__ int scr[4];
-    if (blockIdx.x == 0) leaf_fold(nleaf_blocks, part_lv, part_gap, ds);
-    // four nodes per thread (a 1024-node scan tile per workgroup); the tile's
-    // sum of nchild goes to bsum for k_iscan_apply
-    // The four nodes' child chains are followed side by side, so their skip
-    // loads are in flight together.  A bucket's members are consecutive
-    // leaves: the same loop ranks them.
-    int ch[4], end[4], nc[4], ni[4];
-    for (int k = 0; k < 4; k++) {
-        const int p = blockIdx.x * 1024 + k * 256 + threadIdx.x;
-        nc[k] = ni[k] = 0;
-        ch[k] = p + 1;
-        end[k] = (p < nn && pidx[p] < 0) ? skip[p] : 0;
-    }
-    while (ch[0] < end[0] || ch[1] < end[1] || ch[2] < end[2] || ch[3] < end[3]) {
-        for (int k = 0; k < 4; k++) {
-            if (ch[k] < end[k]) {
-                rank[ch[k]] = nc[k]++;
-                ni[k] += pidx[ch[k]] < 0 ? 1 : 0;
-                ch[k] = skip[ch[k]];
-            }
-        }
-    }
-    int tile = 0;
-    for (int k = 0; k < 4; k++) {
-        const int p = blockIdx.x * 1024 + k * 256 + threadIdx.x;
-        if (p >= nn) continue;
-        nchild[p] = nc[k];
-        ichild[p] = ni[k];
-        tile += nc[k];
-    }
-    int tot;
-    block256_excl_scan(tile, scr, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
+// octant order (rank, which in pre-order is the order of the children's first
+// particles), cstart being the exclusive scan of nchild in pre-order.  A
+// bucket (particles at one position) holds its member leaves, the next count
+// nodes, as children.
 
 // Every node at once: the sums over its key range (the parallel root also
 // counts the particles outside its cube, Node.cpp:477-499), centre of mass,
@@ -1300,8 +1474,12 @@ __global__ __launch_bounds__(256) void k_iscan_tiles(int n, const int32_t *in, i
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(256) void k_iscan_apply(int n, const int32_t *in, const int32_t *bsum, int32_t *out) {
+// In a build's scan of the children (ds given) the first workgroup also folds
+// the leaves' partials.
+__global__ __launch_bounds__(256) void k_iscan_apply(int n, const int32_t *in, const int32_t *bsum, int32_t *out,
+                                                     int nleaf_tiles, const int32_t *leaf_part, DevState *ds) {
     __shared__ int scr[4];
+    if (ds && blockIdx.x == 0) leaf_fold(nleaf_tiles, leaf_part, ds);
     int b0 = blockIdx.x * 1024 + threadIdx.x * 4;
     int v[4];
     int s = 0;
@@ -1423,7 +1601,18 @@ __global__ void k_reset_tie_flags(DevState *ds) {
     ds->tie_deep = 0;
 }
 
-__global__ void k_reset_walk_depth(DevState *ds) { ds->walk_depth = 0; }
+// Internal children of every node, for k_branch_depth (zeroed, then counted).
+__global__ __launch_bounds__(256) void k_zero_inner(int nn, int32_t *ichild, DevState *ds) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < nn) ichild[p] = 0;
+    if (p == 0) ds->walk_depth = 0;
+}
+
+__global__ __launch_bounds__(256) void k_count_inner(int nn, const int32_t *pidx, const int32_t *parent,
+                                                     int32_t *ichild) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < nn && pidx[p] < 0 && parent[p] >= 0) atomicAdd(&ichild[parent[p]], 1);
+}
 
 // Stack growth bound of the block walk in a deep tree.  Taking one block of
 // siblings off the stack pushes one block per sibling opened, and only
@@ -1469,7 +1658,7 @@ void alloc_nodes(Ctx &c, int64_t cap) {
     // block sums for every particle slot (launch_tile_sums covers all c.n <= c.cap)
     const size_t pcap = (size_t)c.cap > n ? (size_t)c.cap : n;
     auto plan = [&](Carve &cv) {
-        cv(&c.n_first, n * 4); cv(&c.n_count, n * 4); cv(&c.n_skip, n * 4);
+        cv(&c.n_first, n * 4); cv(&c.n_count, n * 4);
         cv(&c.n_parent, n * 4);
         cv(&c.n_pidx, n * 4); cv(&c.n_level, n);
         double **d8[] = {&c.n_mass, &c.n_gas, &c.n_gvx, &c.n_gvy, &c.n_gvz, &c.n_cx, &c.n_cy, &c.n_cz, &c.g_rho};
@@ -1479,7 +1668,6 @@ void alloc_nodes(Ctx &c, int64_t cap) {
         cv(&c.tnode, n * sizeof(core::TreeNode));
         cv(&c.tsph, n * sizeof(core::SphNode));
         cv(&c.n_nchild, n * 4); cv(&c.n_rank, n * 4); cv(&c.n_cstart, n * 4);
-        cv(&c.n_ichild, n * 4);
         cv(&c.nsum_tile, (pcap / kBlk2 + 1) * (kBlk2 / kBlk1 + 1) * sizeof(NodeSums));
         cv(&c.n_bsum, (n / 1024 + 2) * 4);
     };
@@ -1622,7 +1810,8 @@ static void seg_order(Ctx &c) {
     core::Pos pos{c.alt[0], c.alt[1], c.alt[2]};
     int nb = (n + 1023) / 1024;
     if (nb < 1) nb = 1;
-    hipLaunchKernelGGL(k_lcp, dim3(nb), dim3(256), 0, st, n, kw, 2, pos, c.ds, proot, c.lcp, c.lk, c.cnt, c.bsum);
+    hipLaunchKernelGGL(k_lcp, dim3(nb), dim3(256), 0, st, n, kw, 2, pos, c.ds, proot, c.lcp, c.lmin, c.cnt,
+                       c.bsum);
     hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, st, c.cnt, c.bsum, c.ds, proot, c.node_cap, c.base);
     AG2_HIP(hipMemcpyAsync(c.hs_pinned, c.ds, sizeof(DevState), hipMemcpyDeviceToHost, st));
 }
@@ -1746,8 +1935,35 @@ static void launch_tile_sums(Ctx &c) {
     hipLaunchKernelGGL(k_tile_sums, dim3(ntile), dim3(1024), 0, c.stream, c.ds, pv, blk1, blk2);
 }
 
+static NodeArrays node_arrays(const Ctx &c) {
+    return NodeArrays{c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_nchild, c.n_rank, c.n_level};
+}
+
+// n_cstart lists the internal nodes' particles until the child-place scan
+// overwrites it.
+static void launch_leaves(Ctx &c) {
+    const int nb = ((int)c.n + kLevTile - 1) / kLevTile;
+    if (nb < 1) return;
+    hipLaunchKernelGGL(k_make_leaf, dim3(nb), dim3(256), 0, c.stream, c.ds, c.lcp, c.base, c.cnt, node_arrays(c),
+                       c.idx_alt, c.gapl, c.n_cstart, c.n_bsum, c.leaf_part);
+}
+
+// Up to 65536 internal nodes (1024 workgroups of 64, four a CU) fewer nodes
+// per workgroup spread the listed nodes over more waves: 10,000 particles 9.5
+// us against 11.0 with 256 nodes, 100,000 12.7 against 13.5; 1,000,000 35
+// against 30.
+constexpr int kInternalSpread = 65536;
+
+static void launch_internal(Ctx &c, const NodeArrays &o) {
+    if (c.n_int <= kInternalSpread)
+        hipLaunchKernelGGL(k_make_internal<64>, dim3(grid_for(c.n_int, 64)), dim3(256), 0, c.stream, c.nin, c.n_int,
+                           c.lcp, c.lmin, c.base, c.n_cstart, o, c.n_bsum);
+    else
+        hipLaunchKernelGGL(k_make_internal<256>, dim3(grid_for(c.n_int, 256)), dim3(256), 0, c.stream, c.nin,
+                           c.n_int, c.lcp, c.lmin, c.base, c.n_cstart, o, c.n_bsum);
+}
+
 void build_order(Ctx &c) {
-    int n = (int)c.n;
     hipStream_t st = c.stream;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[2], st));
     // poisoned until this build's counts overwrite it (checked in build_tree_b)
@@ -1755,10 +1971,11 @@ void build_order(Ctx &c) {
     run_segment(c, 2, seg_order);
     swap_state(c);
     AG2_HIP(hipEventRecord(c.ev_counts, st));
-    // the block sums need only the particles in key order: they run while
-    // the host waits for the counts
+    // the leaves and the block sums need only the particles in key order:
+    // they run while the host waits for the counts
+    launch_leaves(c);
     launch_tile_sums(c);
-    (void)n;
+    AG2_HIP(hipGetLastError());
 }
 
 core::KeyWords key_words(const Ctx &c) {
@@ -1803,7 +2020,8 @@ static void refine_ties(Ctx &c) {
         const core::KeyWords kw = key_words(c);   // words 0 .. w-1 are present
         hipLaunchKernelGGL(k_deep_flag, dim3(g), dim3(256), 0, st, c.ds, kw, w, c.cnt);
         hipLaunchKernelGGL(k_iscan_tiles, dim3(nb), dim3(256), 0, st, nin, c.cnt, c.bsum);
-        hipLaunchKernelGGL(k_iscan_apply, dim3(nb), dim3(256), 0, st, nin, c.cnt, c.bsum, c.base);
+        hipLaunchKernelGGL(k_iscan_apply, dim3(nb), dim3(256), 0, st, nin, c.cnt, c.bsum, c.base, 0,
+                           (const int32_t *)nullptr, (DevState *)nullptr);
         hipLaunchKernelGGL(k_deep_compact, dim3(g), dim3(256), 0, st, c.ds, c.cnt, c.base, c.spos, &c.ds->deep_m);
         AG2_HIP(hipMemcpyAsync(&c.hs_pinned->deep_m, &c.ds->deep_m, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         AG2_HIP(hipStreamSynchronize(st));
@@ -1829,7 +2047,7 @@ static void refine_ties(Ctx &c) {
     const core::Pos pos{c.alt[0], c.alt[1], c.alt[2]};
     const int nbn = (n + 1023) / 1024 < 1 ? 1 : (n + 1023) / 1024;
     hipLaunchKernelGGL(k_lcp, dim3(nbn), dim3(256), 0, st, n, key_words(c), c.kw_used, pos, c.ds,
-                       proot, c.lcp, c.lk, c.cnt, c.bsum);
+                       proot, c.lcp, c.lmin, c.cnt, c.bsum);
     hipLaunchKernelGGL(k_scan_apply, dim3(nbn), dim3(256), 0, st, c.cnt, c.bsum, c.ds, proot, c.node_cap, c.base);
     swap_state(c);
     AG2_HIP(hipMemcpyAsync(c.hs_pinned, c.ds, sizeof(DevState), hipMemcpyDeviceToHost, st));
@@ -1878,37 +2096,26 @@ void build_tree_b(Ctx &c) {
     if (c.vd_radius0 == 0.0) c.vd_radius0 = __builtin_bit_cast(double, c.hs.Rbits) / 100000;
     c.n_nodes = c.hs.n_nodes;
     int nin = c.nin, nn = c.n_nodes;
-    const core::KeyWords kw = key_words(c);
-    core::NodeOut o{c.n_first, c.n_count, c.n_skip, c.n_parent, c.n_pidx, c.n_level};
+    const NodeArrays o = node_arrays(c);
     if (nn > 0) {
-        // make_leaf's per-block partials (deepest level, gap count), folded by k_child_count
-        unsigned long long *part = (unsigned long long *)c.partials;
-        int gl = 0;
-        if (nin == 0) {
-            hipLaunchKernelGGL(k_make_root_only, dim3(1), dim3(1), 0, st, o);
-        } else {
-            int gi = grid_for(nin, 256);
-            gl = gi < kLeafBlocks ? gi : kLeafBlocks;
-            // n_cstart lists the internal nodes' particles until the child-place scan overwrites it
-            hipLaunchKernelGGL(k_make_leaf, dim3(gl), dim3(256), 0, st, nin, kw, c.lcp, c.lk, c.base, c.cnt, o,
-                               c.idx_alt, c.gapl, c.n_cstart, part, part + kLeafBlocks);
-            if (c.n_int > 0)
-                hipLaunchKernelGGL(k_make_internal, dim3(grid_for(c.n_int, 256)), dim3(256), 0, st, nin, nn,
-                                   c.n_int, kw, c.lcp, c.base, c.n_cstart, o);
-        }
         PVals pv{c.x, c.y, c.z, c.m, c.vx, c.vy, c.vz, c.type};
-        // child counts, the child-place scan, then node sums, moments and
-        // walk records
+        // internal nodes with every node's parent and rank, the child-place
+        // scan, then node sums, moments and walk records
         int gn = grid_for(nn, 256);
         int nbn = (nn + 1023) / 1024;
-        hipLaunchKernelGGL(k_child_count, dim3(nbn), dim3(256), 0, st, nn, c.n_pidx, c.n_level, c.n_count, c.n_skip,
-                           c.n_nchild, c.n_rank, c.n_ichild, gl, part, part + kLeafBlocks, c.ds, c.n_bsum);
-        // the block sums from build_order are stale after a refinement
-        // re-ordered the particles or the node arrays grew
-        if (nin > 0 && !tiles_current) launch_tile_sums(c);
+        // the leaves and block sums from build_order are stale after a
+        // refinement re-ordered the particles or the node arrays grew
+        if (nin > 0 && !tiles_current) {
+            launch_leaves(c);
+            launch_tile_sums(c);
+        }
+        if (nin == 0) hipLaunchKernelGGL(k_make_root_only, dim3(1), dim3(64), 0, st, o, c.n_bsum);
+        else if (c.n_int > 0)
+            launch_internal(c, o);
         NodeSums *blk1, *blk2;
         tile_sum_buffers(c, &blk1, &blk2);
-        hipLaunchKernelGGL(k_iscan_apply, dim3(nbn), dim3(256), 0, st, nn, c.n_nchild, c.n_bsum, c.n_cstart);
+        hipLaunchKernelGGL(k_iscan_apply, dim3(nbn), dim3(256), 0, st, nn, c.n_nchild, c.n_bsum, c.n_cstart,
+                           (nin + kLevTile - 1) / kLevTile, c.leaf_part, c.ds);
         NodeMoments nm{c.n_mass, c.n_gas, c.n_cx, c.n_cy, c.n_cz, c.n_gvx, c.n_gvy, c.n_gvz};
         hipLaunchKernelGGL(k_node_moments, dim3(gn), dim3(256), 0, st, nn, nin, n, proot, c.p.split_threshold,
                            c.zero_mass > 0 ? 1 : 0, c.rid, c.ds,
@@ -1919,9 +2126,11 @@ void build_tree_b(Ctx &c) {
         c.groups_cleared = true;
         if (deep && nin > 0) {
             // the walk's stack bound comes from the branching depth here
-            hipLaunchKernelGGL(k_reset_walk_depth, dim3(1), dim3(1), 0, st, c.ds);
+            // (n_cstart is free again: the walk records hold the places)
+            hipLaunchKernelGGL(k_zero_inner, dim3(gn), dim3(256), 0, st, nn, c.n_cstart, c.ds);
+            hipLaunchKernelGGL(k_count_inner, dim3(gn), dim3(256), 0, st, nn, c.n_pidx, c.n_parent, c.n_cstart);
             hipLaunchKernelGGL(k_branch_depth, dim3(grid_for(nin, 256)), dim3(256), 0, st, nin, c.base, c.cnt,
-                               c.n_parent, c.n_ichild, c.ds);
+                               c.n_parent, c.n_cstart, c.ds);
             AG2_HIP(hipMemcpyAsync(&c.hs_pinned->walk_depth, &c.ds->walk_depth, sizeof(int32_t),
                                    hipMemcpyDeviceToHost, st));
             AG2_HIP(hipStreamSynchronize(st));
