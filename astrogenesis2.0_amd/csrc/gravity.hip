@@ -186,6 +186,72 @@ __device__ inline void sph_pair(double dx, double dy, double dz, double r2, doub
     core::sph_term_hoisted(dx, dy, dz, r2, gas, vx, vy, vz, k, s);
 }
 
+// The same term, value for value, with the square root and the four quotients
+// in short correctly rounded forms: one estimate and its Newton steps serve
+// the root and the quotient by r, 1 / h (ih) is formed once per target, and
+// each quotient ends with one step on its exact remainder.  The compiler's
+// general forms scale their operands against overflow and fix up special
+// values on every call; plain_support and plain_pair stand for that here
+// (every intermediate and remainder far inside the normal range), and what
+// lies outside takes sph_pair.  Compared with / and sqrt over 2e8 random
+// operands, the estimates off by their full 5.3e-8: no result differs.
+__device__ inline bool plain_support(double h) { return h > 0x1p-100 && h < 0x1p100; }
+
+// r2 = |d|^2 > 0, vd = v . d, hv = h vd (which the term divides where vd < 0)
+__device__ inline bool plain_pair(double r2, double vd, double hv) {
+    return r2 > 0x1p-300 && !(vd < 0.0 && !(hv < -0x1p-500 && hv > -0x1p500));
+}
+
+// sqrt(x), and 1 / sqrt(x) to the last bit or so.
+__device__ inline double root_plain(double x, double *inv) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, hy = 0.5 * y;
+    const double e = __builtin_fma(-hy, g, 0.5);
+    hy = __builtin_fma(hy, e, hy);
+    g = __builtin_fma(g, e, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), hy, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), hy, g);
+    const double i = hy + hy;
+    *inv = __builtin_fma(__builtin_fma(-g, i, 1.0), i, i);
+    return g;
+}
+
+// a / b from y = 1 / b.
+__device__ inline double quot_plain(double a, double b, double y) {
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+}
+
+// The term of a pair within 2 h: r = sqrt(r2), ir = 1 / r.
+__device__ inline void sph_pair_plain(double dx, double dy, double dz, double r, double ir, double gas, double vx,
+                                      double vy, double vz, double vd, double hv, const core::SphConst &k, double ih,
+                                      double *sx, double *sy, double *sz, double *su) {
+    const double q = quot_plain(r, k.h, ih);
+    const double near = -3.0 * q + 2.25 * q * q, far = -0.75 * ((2 - q) * (2 - q));
+    const double poly = q < 1.0 ? near : far;
+    const double gsc = quot_plain(quot_plain(k.a3 * poly, k.h, ih), r, ir);
+    const double gx = dx * gsc, gy = dy * gsc, gz = dz * gsc;
+    const double den = r * r + k.eta_h2;
+    double z = __builtin_amdgcn_rcp(den);
+    z = __builtin_fma(__builtin_fma(-den, z, 1.0), z, z);
+    z = __builtin_fma(__builtin_fma(-den, z, 1.0), z, z);
+    const double mu = quot_plain(hv, den, z);
+    const double MU = vd < 0 ? -0.5 * k.cij * mu + 1.0 * (mu * mu) : 0.0;
+    const double fp = -gas * k.pr, fv = -gas * MU;
+    double ax = fp * gx, ay = fp * gy, az = fp * gz;
+    ax += fv * gx;
+    ay += fv * gy;
+    az += fv * gz;
+    *su += 0.5 * gas * (k.pr + MU) * (vx * gx + vy * gy + vz * gz);
+    const bool bad = ax != ax || ay != ay || az != az;
+    if (__any(bad)) {
+        ax = bad ? 0.0 : ax;
+        ay = bad ? 0.0 : ay;
+        az = bad ? 0.0 : az;
+    }
+    *sx += ax; *sy += ay; *sz += az;
+}
+
 // Workgroups reach the 8 XCDs round robin.  Neighbouring groups read mostly
 // the same tree records and should share one XCD's L2, but one contiguous
 // eighth of the key order per XCD leaves XCDs idle behind the one that holds
@@ -1259,13 +1325,38 @@ __global__ __launch_bounds__(256) void k_sph_scatter(int n, const uint8_t *type,
 // reference: on r^2 with a margin, exactly inside it), r != 0 and the node is
 // not the target's own leaf.  Lists that overflowed are left to the overflow
 // walk.
+//
+// Four neighbouring lanes read one record together, 16 bytes each, and hand
+// the pieces to their owners through LDS: a lane that reads its own 64-byte
+// record alone makes every load of the wave touch 64 cache lines, and the
+// L1's tag lookups (256 cycles per 64 records) bounded the kernel.  With that
+// and the short root and quotients (sph_pair_plain) 14.1 M pairs of the 1 M
+// disk take 117 us where they took 136, 200,000 disk at opening angle 0.15
+// 196 us for 224; the shared reads alone 124 and 212.  What is left is the
+// vector unit (about half of the time), and four waves per SIMD to wait with:
+// holding the registers to five or six spills (325 and 541 us).
 constexpr int kPairLanes = 8;
+constexpr int kQuadBytes = 4 * 64 + 64;   // records of a quad's four lanes, and room to spread the banks
+
+// Piece j (16 bytes) of the record of lane i of quad q: the pieces of a
+// record are permuted by i, so that eight lanes reading the same piece of
+// their records meet no bank twice.
+__device__ inline int piece_at(int q, int i, int j) { return q * kQuadBytes + i * 64 + (j ^ i) * 16; }
+
+template <int I>
+__device__ inline int quad_bcast(int v) {
+    return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true);
+}
 
 // SPILL: lists may go on in spill chunks (the context has some).
 template <bool SPILL>
 __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gidx, const int32_t *cnts) {
+    static_assert(sizeof(core::SphNode) == 64, "a record is four pieces of 16 bytes");
+    __shared__ __align__(16) char stage[4][16 * kQuadBytes];
     const int lane = lane_id();
     const int sub = lane & (kPairLanes - 1);
+    char *mine = stage[threadIdx.x >> 6];
+    const int qd = lane >> 2, qi = lane & 3;
     // targets in key order, in XCD ranges: neighbouring targets share most
     // of their candidate records, which then come from one L2
     const int slot = (int)((xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x) / kPairLanes);
@@ -1277,32 +1368,82 @@ __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gi
         if (!list_overflowed(a, c)) t = gidx[slot];
         else c = 0;
     }
+    core::Target tg{};
+    double vx = 0.0, vy = 0.0, vz = 0.0;
+    core::SphConst sk{};
+    double ih = 0.0, h2 = 0.0;
+    bool plain = false;
+    unsigned np = 0u;   // pairs counted on the short path
     if (t >= 0) {
-        core::Target tg;
         tg.x = a.sx[t]; tg.y = a.sy[t]; tg.z = a.sz[t];
         tg.h = a.h[t]; tg.rho = a.rho[t]; tg.P = a.P[t];
-        const double vx = a.svx[t], vy = a.svy[t], vz = a.svz[t];
-        const core::SphConst sk = core::sph_const(tg);
-        // kSphK candidates of the list itself, then of its spill chunks
-        const int32_t *lst = a.sph_list + (size_t)slot * kSphK;
-        for (int c0 = 0; c0 < (SPILL ? c : 1); c0 += kSphK) {
-            if (SPILL && c0 > 0) lst = a.sph_spill + (size_t)a.sph_more[(size_t)slot * kSphMore + c0 / kSphK - 1] * kSphK;
-            const int here = !SPILL || c - c0 < kSphK ? c - c0 : kSphK;
-            // one candidate ahead: the next record's load overlaps this pair
-            core::SphNode wn{};
-            if (sub < here) wn = a.tsph[lst[sub]];
-            for (int k = sub; k < here; k += kPairLanes) {
-                const core::SphNode w = wn;
-                if (k + kPairLanes < here) wn = a.tsph[lst[k + kPairLanes]];
-                if (w.pidx == t) continue;
-                const double dx = tg.x - w.cx, dy = tg.y - w.cy, dz = tg.z - w.cz;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 == 0.0) continue;
-                bool inside = r2 < sk.h2x4 * (1.0 - 1e-12);
-                if (!inside && !(r2 > sk.h2x4 * (1.0 + 1e-12))) inside = sqrt(r2) < sk.h * 2;
-                if (!inside) continue;
-                sph_pair(dx, dy, dz, r2, w.gas, vx - w.vx, vy - w.vy, vz - w.vz, sk, &s);
+        vx = a.svx[t]; vy = a.svy[t]; vz = a.svz[t];
+        sk = core::sph_const(tg);
+        ih = 1.0 / tg.h;
+        plain = plain_support(tg.h);
+        h2 = tg.h * 2;
+    }
+    // candidate k of the list: kSphK in the list itself, then spill chunks
+    const int32_t *lst = a.sph_list + (size_t)slot * kSphK;
+    auto candidate = [&](int k) -> int {
+        if (k >= c) return 0;   // (a record of no use; record 0 is there)
+        if (SPILL && k >= kSphK)
+            return a.sph_spill[(size_t)a.sph_more[(size_t)slot * kSphMore + k / kSphK - 1] * kSphK + k % kSphK];
+        return lst[k];
+    };
+    int most = c;
+    for (int d = 32; d >= kPairLanes; d >>= 1) {
+        const int o = __shfl_xor(most, d, 64);
+        most = o > most ? o : most;
+    }
+    most = __builtin_amdgcn_readfirstlane(most);
+    // piece qi of the quad's four records, one round ahead; the list entry
+    // two rounds ahead
+    uint4 p0{}, p1{}, p2{}, p3{};
+    auto fetch = [&](int rec) {
+        const char *base = (const char *)a.tsph + 16 * qi;
+        p0 = *(const uint4 *)(base + (size_t)quad_bcast<0>(rec) * 64);
+        p1 = *(const uint4 *)(base + (size_t)quad_bcast<1>(rec) * 64);
+        p2 = *(const uint4 *)(base + (size_t)quad_bcast<2>(rec) * 64);
+        p3 = *(const uint4 *)(base + (size_t)quad_bcast<3>(rec) * 64);
+    };
+    int next = 0;
+    if (most > 0) {
+        fetch(candidate(sub));
+        next = candidate(sub + kPairLanes);
+    }
+    for (int k0 = 0; k0 < most; k0 += kPairLanes) {
+        *(uint4 *)(mine + piece_at(qd, 0, qi)) = p0;
+        *(uint4 *)(mine + piece_at(qd, 1, qi)) = p1;
+        *(uint4 *)(mine + piece_at(qd, 2, qi)) = p2;
+        *(uint4 *)(mine + piece_at(qd, 3, qi)) = p3;
+        wave_sync_lds();
+        if (k0 + kPairLanes < most) {
+            fetch(next);
+            next = candidate(k0 + 2 * kPairLanes + sub);
+        }
+        const double2 cxy = *(const double2 *)(mine + piece_at(qd, qi, 0));
+        const double2 czg = *(const double2 *)(mine + piece_at(qd, qi, 1));
+        const double2 vxy = *(const double2 *)(mine + piece_at(qd, qi, 2));
+        const double2 vzp = *(const double2 *)(mine + piece_at(qd, qi, 3));
+        wave_sync_lds();
+        const int pidx = (int)(unsigned)__builtin_bit_cast(unsigned long long, vzp.y);
+        const double dx = tg.x - cxy.x, dy = tg.y - cxy.y, dz = tg.z - czg.x;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double ux = vx - vxy.x, uy = vy - vxy.y, uz = vz - vzp.x;
+        const double vd = ux * dx + uy * dy + uz * dz, hv = tg.h * vd;
+        const bool cand = k0 + sub < c && pidx != t;
+        const bool fast = plain && plain_pair(r2, vd, hv);
+        if (cand && fast) {
+            double ir;
+            const double r = root_plain(r2, &ir);
+            if (r < h2) {   // the reference's test itself
+                sph_pair_plain(dx, dy, dz, r, ir, czg.y, ux, uy, uz, vd, hv, sk, ih, &s.ax, &s.ay, &s.az, &s.du);
+                np++;
             }
+        }
+        if (__any(cand && !fast)) {
+            if (cand && !fast && r2 != 0.0 && sqrt(r2) < sk.h * 2) sph_pair(dx, dy, dz, r2, czg.y, ux, uy, uz, sk, &s);
         }
     }
     for (int d = kPairLanes / 2; d >= 1; d >>= 1) {
@@ -1315,7 +1456,7 @@ __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gi
         a.ax[t] += s.ax; a.ay[t] += s.ay; a.az[t] += s.az;
         a.dUdt[t] += s.du;
     }
-    unsigned long long cs = wave_sum_u64((unsigned long long)s.nsph);
+    unsigned long long cs = wave_sum_u64((unsigned long long)s.nsph + np);
     if (lane == 0) bin_add(a.cbins, kCntSphPairs, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), cs);
 }
 
