@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(int n, const uint64_t *__res
 
 // ------------------------------------------------------------ merge sort
 // Two launches for a set of a few tiles, where the radix passes are launches
-// and little else (six bytes are 12 or 18 launches of 4-7 us).  k_ms_tile
+// and little else (six bytes are 18 launches of 4-7 us).  k_ms_tile
 // sorts each tile of TILE keys by itself in LDS (stable radix passes over
 // the bytes the build sorts, bound by their barriers and LDS round trips:
 // 2.5 us each); k_ms_merge gives each key its place: its
@@ -282,44 +282,70 @@ __global__ __launch_bounds__(256) void k_rs_scatter(int n, const uint64_t *__res
 // searched: particles move little between steps, so most are.
 constexpr int kMsThreads = 1024;
 constexpr int kMsWaves = kMsThreads / 64;
-// Sort phase in microseconds, radix passes against tiles of 2048 / 4096 / 8192
-// (first build after an upload, in caller order; later builds are 1-5 us
-// below): 10,000 69 against 33 / 36 / 51; 20,000 73 against 36 / 43 / 55;
-// 33,333 86 against 42 / 46 / 63; 65,000 87 against 66 / 53 / 65; 100,003 89
-// against 142 / 95 / 81; 200,000 94 against 467 / 273 / 186 (the searches grow
-// with the tiles' number for every key).
-constexpr int kMsSmall = 40000, kMsMax = 80000;     // up to here kMsTile0, kMsTile1
+// Sort phase in microseconds (first build after an upload, in caller order;
+// later builds are 1-5 us below), radix passes / merge with tiles of 2048 /
+// of 4096 / sample sort:
+//    10,000   69 / 33 / 36 / 51        100,003   89 / 142 / 95 / 58
+//    20,000   73 / 36 / 43 / 51        200,000   94 / 467 / 273 / 69
+//    33,333   86 / 42 / 46 / 52        520,000  112 / - / - / 84
+//    45,000   87 / 52 / 48 / 52      1,000,000  146 / - / - / 108
+//    65,000   87 / 66 / 55 / 53      1,500,000  178 / - / - / 185
+// The merge's searches grow with the tiles' number for every key; the sample
+// sort runs out of CUs above 256 tiles (a workgroup's sort fills one).
+constexpr int kMsSmall = 40000, kMsMax = 60000;       // merge: up to here kMsTile0, kMsTile1
 constexpr int kMsTile0 = 2048, kMsTile1 = 4096;
+constexpr int kBsMax = 256 * kMsTile1;                // sample sort up to here, radix passes above
+constexpr int kBsTiles = kBsMax / kMsTile0;           // most tiles of a set (a thread each)
 
-template <int TILE>
-__device__ __forceinline__ void ms_tile(int n, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                        uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int lo, int tile) {
-    constexpr int kMsItems = TILE / kMsThreads;
-    __shared__ uint64_t sk[TILE];
-    __shared__ uint32_t sv[TILE];
-    __shared__ int wcnt[kMsWaves][256];
-    __shared__ int wtot[4];
+// The first sample of a tile: its number's bits reversed, within the step.
+__device__ inline int sample_phase(int tile, int step) {
+    return (int)(__brev((unsigned)tile) >> (__builtin_clz((unsigned)step) + 1)) & (step - 1);
+}
+
+// Stable sort of len keys by one workgroup in LDS, on the bytes lo .. 7 in
+// which they differ at all.  Item j of lane l of wave w holds position
+// (w it + j) 64 + l before and after (it: items in use, 1024 it >= len).
+template <int ITEMS>
+struct SortLds {
+    uint64_t k[ITEMS * kMsThreads];
+    uint32_t v[ITEMS * kMsThreads];
+    int wcnt[kMsWaves][256];
+    int wtot[4];
+    unsigned long long red[kMsWaves];
+};
+
+template <int ITEMS>
+__device__ __forceinline__ void lds_sort(SortLds<ITEMS> &S, uint64_t (&k)[ITEMS], uint32_t (&v)[ITEMS], int it,
+                                         int len, int lo) {
     const int tid = threadIdx.x, w = tid >> 6, lane = lane_id();
-    const int t0 = tile * TILE;
-    const int len = n - t0 < TILE ? n - t0 : TILE;
-    // item j of lane l of wave w: tile position (w kMsItems + j) 64 + l
-    const int base = w * (64 * kMsItems) + lane;
-    uint64_t k[kMsItems];
-    uint32_t v[kMsItems];
+    const int base = w * (64 * it) + lane;
+    // the bits in which the keys differ; unused positions get a key with all
+    // of them set, which stays behind (the sort is stable)
+    if (tid == 0) S.red[0] = k[0];
+    __syncthreads();
+    const unsigned long long k0 = S.red[0];
+    unsigned long long diff = 0ull;
 #pragma unroll
-    for (int j = 0; j < kMsItems; j++) {
-        const int p = base + j * 64;
-        // past the end: the largest key, which stays behind (the sort is stable)
-        k[j] = p < len ? kin[t0 + p] : ~0ull;
-        v[j] = p < len ? vin[t0 + p] : 0u;
-    }
+    for (int j = 0; j < ITEMS; j++)
+        if (j < it && base + j * 64 < len) diff |= k[j] ^ k0;
+    for (int d = 32; d >= 1; d >>= 1) diff |= __shfl_xor(diff, d, 64);
+    __syncthreads();
+    if (lane == 0) S.red[w] = diff;
+    __syncthreads();
+    diff = 0ull;
+    for (int u = 0; u < kMsWaves; u++) diff |= S.red[u];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++)
+        if (j < it && base + j * 64 >= len) { k[j] = k0 | diff; v[j] = 0u; }
     const unsigned long long below = lanes_below();
     for (int pass = lo; pass < 8; pass++) {
-        for (int d = lane; d < 256; d += 64) wcnt[w][d] = 0;
+        if ((diff >> (8 * pass) & 255) == 0) continue;
+        for (int d = lane; d < 256; d += 64) S.wcnt[w][d] = 0;
         wave_sync_lds();
-        int loc[kMsItems], dig[kMsItems];
+        int loc[ITEMS], dig[ITEMS];
 #pragma unroll
-        for (int j = 0; j < kMsItems; j++) {
+        for (int j = 0; j < ITEMS; j++) {
+            if (j >= it) break;
             const int d = (int)((k[j] >> (8 * pass)) & 255);
             unsigned long long peers = ~0ull;
 #pragma unroll
@@ -328,9 +354,9 @@ __device__ __forceinline__ void ms_tile(int n, const uint64_t *__restrict__ kin,
                 const unsigned long long bm = __ballot(bit);
                 peers &= bit ? bm : ~bm;
             }
-            const int cur = wcnt[w][d];
+            const int cur = S.wcnt[w][d];
             wave_sync_lds();
-            if ((peers & below) == 0ull) wcnt[w][d] = cur + __popcll(peers);
+            if ((peers & below) == 0ull) S.wcnt[w][d] = cur + __popcll(peers);
             wave_sync_lds();
             loc[j] = cur + __popcll(peers & below);
             dig[j] = d;
@@ -339,32 +365,62 @@ __device__ __forceinline__ void ms_tile(int n, const uint64_t *__restrict__ kin,
         // digit d's first place: the keys of smaller digits, then of earlier waves
         int inc = 0, tot = 0;
         if (tid < 256) {
-            for (int u = 0; u < kMsWaves; u++) tot += wcnt[u][tid];
+            for (int u = 0; u < kMsWaves; u++) tot += S.wcnt[u][tid];
             inc = wave_incl_scan(tot);
-            if (lane == 63) wtot[w] = inc;
+            if (lane == 63) S.wtot[w] = inc;
         }
         __syncthreads();
         if (tid < 256) {
             int at = inc - tot;
-            for (int u = 0; u < w; u++) at += wtot[u];
-            for (int u = 0; u < kMsWaves; u++) { const int c = wcnt[u][tid]; wcnt[u][tid] = at; at += c; }
+            for (int u = 0; u < w; u++) at += S.wtot[u];
+            for (int u = 0; u < kMsWaves; u++) { const int c = S.wcnt[u][tid]; S.wcnt[u][tid] = at; at += c; }
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kMsItems; j++) {
-            const int to = wcnt[w][dig[j]] + loc[j];
-            sk[to] = k[j];
-            sv[to] = v[j];
+        for (int j = 0; j < ITEMS; j++) {
+            if (j >= it) break;
+            const int to = S.wcnt[w][dig[j]] + loc[j];
+            S.k[to] = k[j];
+            S.v[to] = v[j];
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kMsItems; j++) { k[j] = sk[base + j * 64]; v[j] = sv[base + j * 64]; }
-        // (the next pass writes sk only after two more barriers)
+        for (int j = 0; j < ITEMS; j++) {
+            if (j >= it) break;
+            k[j] = S.k[base + j * 64];
+            v[j] = S.v[base + j * 64];
+        }
+        // (the next pass writes S.k only after two more barriers)
     }
+}
+
+template <int TILE>
+__device__ __forceinline__ void ms_tile(int n, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                        uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int lo, int tile,
+                                        uint64_t *__restrict__ samp, int step) {
+    constexpr int kMsItems = TILE / kMsThreads;
+    __shared__ SortLds<kMsItems> S;
+    const int t0 = tile * TILE;
+    const int len = n - t0 < TILE ? n - t0 : TILE;
+    const int base = (threadIdx.x >> 6) * (64 * kMsItems) + lane_id();
+    uint64_t k[kMsItems];
+    uint32_t v[kMsItems];
 #pragma unroll
     for (int j = 0; j < kMsItems; j++) {
         const int p = base + j * 64;
-        if (p < len) { kout[t0 + p] = k[j]; vout[t0 + p] = v[j]; }
+        k[j] = p < len ? kin[t0 + p] : 0ull;
+        v[j] = p < len ? vin[t0 + p] : 0u;
+    }
+    lds_sort<kMsItems>(S, k, v, kMsItems, len, lo);
+    const int phase = step ? sample_phase(tile, step) : 0;
+#pragma unroll
+    for (int j = 0; j < kMsItems; j++) {
+        const int p = base + j * 64;
+        if (p < len) {
+            kout[t0 + p] = k[j];
+            vout[t0 + p] = v[j];
+            if (step && (p & (step - 1)) == phase) samp[tile * (TILE / step) + p / step] = k[j] >> (8 * lo);
+        }
     }
 }
 
@@ -422,11 +478,198 @@ __device__ __forceinline__ void ms_merge(int n, const uint64_t *__restrict__ kin
     if (on && share == 0) { kout[at] = k; vout[at] = vin[e]; }
 }
 
+// ------------------------------------------------------------ sample sort
+// Three launches for a set between the merge sort's range and that of the
+// radix passes (18 launches, bandwidth only in the millions): k_ms_tile leaves every step-th key of its sorted tile as a
+// sample; k_bs_split ranks the samples among all of them and keeps every 64th
+// as a splitter;
+// k_bs_bucket finds one bucket's piece of every tile, gathers the pieces in
+// tile order and sorts them in LDS.  Splitters are single elements (key,
+// tile, position), so equal keys part in the stable order and long runs of
+// them split like any others.
+// The samples of tile t stand at t's own phase of the step (its number with
+// the bits reversed): samples at the same quantiles of tiles that hold like
+// mixtures of keys (any order but a sorted one) would fall in clusters, with
+// hardly a splitter between them.  A bucket holds 64 steps on average and
+// strays by an eighth of that (one standard deviation, for a random order);
+// the room is twice the average, and k_bs_bucket ranks the keys of a larger
+// one singly.
+constexpr int kBsPer = 64;   // samples per bucket
+
+struct Splitter {
+    uint64_t q;       // key from the lowest sorted bit on
+    int tile, pos;
+};
+
+__device__ inline int sample_count(int n, int TILE, int tile, int step) {
+    const int len = n - tile * TILE < TILE ? n - tile * TILE : TILE;
+    const int ph = sample_phase(tile, step);
+    return len > ph ? (len - ph - 1) / step + 1 : 0;
+}
+
+// Elements of tile u that come before q of tile t (t != u): its sorted keys
+// below q, and those equal to q if u comes first.
+__device__ inline bool before(uint64_t o, uint64_t q, bool first) { return first ? o <= q : o < q; }
+
+// The samples of one tile, a lane each: their ranks, and the splitters among
+// them.  The workgroup's waves share the other tiles, whose samples they
+// search in LDS, four lists side by side.
+template <int TILE>
+__device__ __forceinline__ void bs_split(int n, int step, const uint64_t *__restrict__ samp, Splitter *split,
+                                         int own) {
+    constexpr int kG = 4;
+    __shared__ uint64_t list[kG * kMsThreads];
+    __shared__ int part[kMsThreads];
+    const int S = TILE / step, groups = S / 64;       // waves that hold the tile's samples
+    const int tiles = (n + TILE - 1) / TILE;
+    const int w = threadIdx.x >> 6, mine = w % groups, slot = w / groups, slots = kMsWaves / groups;
+    const int j = mine * 64 + lane_id();
+    const bool on = j < sample_count(n, TILE, own, step);
+    const uint64_t q = on ? samp[(size_t)own * S + j] : 0ull;
+    int at = 0;
+    for (int t0 = 0; t0 < tiles; t0 += slots * kG) {
+        const int t = t0 + slot * kG;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kG; u++)
+            if (t + u < tiles) list[(slot * kG + u) * S + j] = samp[(size_t)(t + u) * S + j];
+        __syncthreads();
+        int len[kG], pos[kG];
+#pragma unroll
+        for (int u = 0; u < kG; u++) {
+            len[u] = t + u < tiles && t + u != own ? sample_count(n, TILE, t + u, step) : 0;
+            pos[u] = 0;
+        }
+        for (int d = S; d; d >>= 1)
+#pragma unroll
+            for (int u = 0; u < kG; u++) {
+                const int p = pos[u] + d;
+                if (p <= len[u] && before(list[(slot * kG + u) * S + p - 1], q, t + u < own)) pos[u] = p;
+            }
+#pragma unroll
+        for (int u = 0; u < kG; u++) at += pos[u];
+    }
+    part[threadIdx.x] = at;
+    __syncthreads();
+    if (slot > 0 || !on) return;
+    at = j;
+    for (int k = 0; k < slots; k++) at += part[(k * groups + mine) * 64 + lane_id()];
+    if (at > 0 && at % kBsPer == 0)
+        split[at / kBsPer - 1] = Splitter{q, own, j * step + sample_phase(own, step)};
+}
+
+// Elements of tile u before a splitter.
+template <int TILE>
+__device__ inline int split_tile(const uint64_t *__restrict__ kin, int n, int u, const Splitter &s, int shift) {
+    const int len = n - u * TILE < TILE ? n - u * TILE : TILE;
+    if (u == s.tile) return s.pos;
+    int p = 0;
+    for (int d = TILE; d; d >>= 1)
+        if (p + d <= len && before(kin[(size_t)u * TILE + p + d - 1] >> shift, s.q, u < s.tile)) p += d;
+    return p;
+}
+
+// Bucket b of a set: pieces, gather, sort.
+template <int TILE, int ITEMS>
+__device__ __forceinline__ void bs_bucket(int n, int step, const uint64_t *__restrict__ kin,
+                                          const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
+                                          uint32_t *__restrict__ vout, int lo, const Splitter *__restrict__ split,
+                                          int b) {
+    __shared__ SortLds<ITEMS> S;
+    __shared__ int from[kBsTiles], off[kBsTiles];
+    __shared__ int scr[kMsWaves], low[kMsWaves];
+    const int tid = threadIdx.x, w = tid >> 6, lane = lane_id(), shift = 8 * lo;
+    const int tiles = (n + TILE - 1) / TILE;
+    int samples = (tiles - 1) * (TILE / step) + sample_count(n, TILE, tiles - 1, step);
+    const int buckets = samples > 0 ? (samples - 1) / kBsPer + 1 : 1;
+    if (b >= buckets) return;
+    // one tile per thread
+    int l = 0, h = 0;
+    if (tid < tiles) {
+        h = n - tid * TILE < TILE ? n - tid * TILE : TILE;
+        if (b > 0) l = split_tile<TILE>(kin, n, tid, split[b - 1], shift);
+        if (b < buckets - 1) h = split_tile<TILE>(kin, n, tid, split[b], shift);
+    }
+    const int inc = wave_incl_scan(h - l);
+    int lsum = l;
+    for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
+    if (lane == 63) { scr[w] = inc; low[w] = lsum; }
+    __syncthreads();
+    int at = inc - (h - l), size = 0, first = 0;
+    for (int u = 0; u < kMsWaves; u++) {
+        at += u < w ? scr[u] : 0;
+        size += scr[u];
+        first += low[u];
+    }
+    if (tid < tiles) { from[tid] = tid * TILE + l; off[tid] = at; }
+    __syncthreads();
+    // element i of the bucket: the last tile whose piece starts at or before it
+    int top = 1;
+    while (top < tiles) top <<= 1;
+    auto source = [&](int i) -> int {
+        int t = 0;
+        for (int d = top >> 1; d; d >>= 1)
+            if (t + d < tiles && off[t + d] <= i) t += d;
+        return from[t] + (i - off[t]);
+    };
+    if (size > ITEMS * kMsThreads) {
+        // larger than the room: every key's place by searches in all tiles
+        for (int i = tid; i < size; i += kMsThreads) {
+            const int g = source(i);
+            const uint64_t k = kin[g];
+            const Splitter me{k >> shift, g / TILE, g % TILE};
+            int r = 0;
+            for (int u = 0; u < tiles; u++) r += split_tile<TILE>(kin, n, u, me, shift);
+            kout[r] = k;
+            vout[r] = vin[g];
+        }
+        return;
+    }
+    const int it = (size + kMsThreads - 1) / kMsThreads;
+    const int base = w * (64 * it) + lane;
+    uint64_t k[ITEMS];
+    uint32_t v[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        k[j] = 0ull;
+        v[j] = 0u;
+        if (j < it && base + j * 64 < size) {
+            const int g = source(base + j * 64);
+            k[j] = kin[g];
+            v[j] = vin[g];
+        }
+    }
+    lds_sort<ITEMS>(S, k, v, it, size, lo);
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int p = base + j * 64;
+        if (j < it && p < size) { kout[first + p] = k[j]; vout[first + p] = v[j]; }
+    }
+}
+
+// The samples' step for n keys (64 steps: a bucket's average).
+static int bs_step(int64_t n) { return n <= 262144 ? 16 : n <= 524288 ? 32 : 64; }
+
+template <int TILE>
+__global__ __launch_bounds__(kMsThreads) void k_bs_split(int n, int step, const uint64_t *__restrict__ samp,
+                                                         Splitter *split) {
+    bs_split<TILE>(n, step, samp, split, blockIdx.x);
+}
+
+template <int TILE, int ITEMS>
+__global__ __launch_bounds__(kMsThreads) void k_bs_bucket(int n, int step, const uint64_t *__restrict__ kin,
+                                                          const uint32_t *__restrict__ vin,
+                                                          uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                          int lo, const Splitter *__restrict__ split) {
+    bs_bucket<TILE, ITEMS>(n, step, kin, vin, kout, vout, lo, split, blockIdx.x);
+}
+
 template <int TILE>
 __global__ __launch_bounds__(kMsThreads) void k_ms_tile(int n, const uint64_t *__restrict__ kin,
                                                         const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
-                                                        uint32_t *__restrict__ vout, int lo) {
-    ms_tile<TILE>(n, kin, vin, kout, vout, lo, blockIdx.x);
+                                                        uint32_t *__restrict__ vout, int lo,
+                                                        uint64_t *__restrict__ samp, int step) {
+    ms_tile<TILE>(n, kin, vin, kout, vout, lo, blockIdx.x, samp, step);
 }
 
 template <int TILE>
@@ -445,6 +688,7 @@ struct SortJob {
     uint64_t *key, *key_alt;
     uint32_t *idx, *idx_alt;
     uint32_t *hist, *dtotal;
+    uint64_t *samp;   // key2, which is written after the sort: samples, then splitters
 };
 
 __device__ inline int find_sort_job(const SortJob *jobs, int nj, int b) {
@@ -462,9 +706,24 @@ __global__ __launch_bounds__(256) void k_rsb_hist(const SortJob *jobs, int nj, i
 }
 
 template <int TILE>
-__global__ __launch_bounds__(kMsThreads) void k_msb_tile(const SortJob *jobs, int nj, int lo) {
+__global__ __launch_bounds__(kMsThreads) void k_msb_tile(const SortJob *jobs, int nj, int lo, int step) {
     const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x)];
-    ms_tile<TILE>(J.n, J.key, J.idx, J.key_alt, J.idx_alt, lo, (int)blockIdx.x - J.tile0);
+    ms_tile<TILE>(J.n, J.key, J.idx, J.key_alt, J.idx_alt, lo, (int)blockIdx.x - J.tile0, J.samp, step);
+}
+
+// (64 samples a tile in a batch: one bucket's worth)
+template <int TILE>
+__global__ __launch_bounds__(kMsThreads) void k_bsb_split(const SortJob *jobs, int nj) {
+    const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x)];
+    bs_split<TILE>(J.n, TILE / kBsPer, J.samp, (Splitter *)(J.samp + (size_t)J.nblk * kBsPer),
+                   (int)blockIdx.x - J.tile0);
+}
+
+template <int TILE, int ITEMS>
+__global__ __launch_bounds__(kMsThreads) void k_bsb_bucket(const SortJob *jobs, int nj, int lo) {
+    const SortJob &J = jobs[find_sort_job(jobs, nj, blockIdx.x)];
+    bs_bucket<TILE, ITEMS>(J.n, TILE / kBsPer, J.key_alt, J.idx_alt, J.key, J.idx, lo,
+                           (const Splitter *)(J.samp + (size_t)J.nblk * kBsPer), (int)blockIdx.x - J.tile0);
 }
 
 template <int TILE>
@@ -1744,6 +2003,18 @@ static void radix_pairs(Ctx &c, int n, uint64_t *kin, uint64_t *kout, uint32_t *
     }
 }
 
+template <int TILE, int ITEMS>
+static void sample_sort(Ctx &c, int n, int step) {
+    // samples and splitters in key2, which is written after the sort
+    const int tiles = grid_for(n, TILE), S = TILE / step;
+    Splitter *split = (Splitter *)(c.key2 + (size_t)tiles * S);
+    hipLaunchKernelGGL(k_ms_tile<TILE>, dim3(tiles), dim3(kMsThreads), 0, c.stream, n, c.key, c.idx, c.key_alt,
+                       c.idx_alt, c.sort_lo, c.key2, step);
+    hipLaunchKernelGGL(k_bs_split<TILE>, dim3(tiles), dim3(kMsThreads), 0, c.stream, n, step, c.key2, split);
+    hipLaunchKernelGGL((k_bs_bucket<TILE, ITEMS>), dim3(tiles * S / kBsPer), dim3(kMsThreads), 0, c.stream, n, step,
+                       c.key_alt, c.idx_alt, c.key, c.idx, c.sort_lo, split);
+}
+
 static void radix_sort(Ctx &c, int n) {
     int nblk = (n + kSortTile - 1) / kSortTile;
     uint64_t *kin = c.key, *kout = c.key_alt;
@@ -1751,12 +2022,21 @@ static void radix_sort(Ctx &c, int n) {
     if (n <= kMsMax) {
         const dim3 gt(grid_for(n, n <= kMsSmall ? kMsTile0 : kMsTile1)), gm(grid_for(n, kMsPer));
         if (n <= kMsSmall) {
-            hipLaunchKernelGGL(k_ms_tile<kMsTile0>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo);
+            hipLaunchKernelGGL(k_ms_tile<kMsTile0>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo,
+                               (uint64_t *)nullptr, 0);
             hipLaunchKernelGGL(k_ms_merge<kMsTile0>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
         } else {
-            hipLaunchKernelGGL(k_ms_tile<kMsTile1>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo);
+            hipLaunchKernelGGL(k_ms_tile<kMsTile1>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo,
+                               (uint64_t *)nullptr, 0);
             hipLaunchKernelGGL(k_ms_merge<kMsTile1>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
         }
+        return;
+    }
+    if (n <= kBsMax) {
+        const int step = bs_step(n);
+        if (step == 16) sample_sort<kMsTile0, 2>(c, n, step);
+        else if (step == 32) sample_sort<kMsTile0, 4>(c, n, step);
+        else sample_sort<kMsTile1, 8>(c, n, step);
         return;
     }
     // bytes sort_lo .. 7 (an even number of passes)
@@ -1885,13 +2165,13 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
         lo = cs[k]->sort_lo < lo ? cs[k]->sort_lo : lo;
         most = cs[k]->n > most ? cs[k]->n : most;
     }
-    const int tile = most > kMsMax ? kSortTile : most > kMsSmall ? kMsTile1 : kMsTile0;
+    const int tile = most > kBsMax ? kSortTile : most > kMsMax || most <= kMsSmall ? kMsTile0 : kMsTile1;
     int total = 0;
     for (int k = 0; k < nc; k++) {
         Ctx &c = *cs[k];
         const int n = (int)c.n;
         const int nblk = (n + tile - 1) / tile;
-        hj[k] = SortJob{n, nblk, total, 0, c.key, c.key_alt, c.idx, c.idx_alt, c.hist, c.dtotal};
+        hj[k] = SortJob{n, nblk, total, 0, c.key, c.key_alt, c.idx, c.idx_alt, c.hist, c.dtotal, c.key2};
         total += nblk;
     }
     if (total < 1) return;
@@ -1900,12 +2180,20 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
     if (most <= kMsMax) {
         const dim3 gm((unsigned)(total * (tile / kMsPer)));
         if (tile == kMsTile0) {
-            hipLaunchKernelGGL(k_msb_tile<kMsTile0>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo);
+            hipLaunchKernelGGL(k_msb_tile<kMsTile0>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo, 0);
             hipLaunchKernelGGL(k_msb_merge<kMsTile0>, gm, dim3(256), 0, st, dj, nc, lo);
         } else {
-            hipLaunchKernelGGL(k_msb_tile<kMsTile1>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo);
+            hipLaunchKernelGGL(k_msb_tile<kMsTile1>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo, 0);
             hipLaunchKernelGGL(k_msb_merge<kMsTile1>, gm, dim3(256), 0, st, dj, nc, lo);
         }
+        AG2_HIP(hipGetLastError());
+        return;
+    }
+    if (most <= kBsMax) {
+        const dim3 g(total), b(kMsThreads);
+        hipLaunchKernelGGL(k_msb_tile<kMsTile0>, g, b, 0, st, dj, nc, lo, kMsTile0 / kBsPer);
+        hipLaunchKernelGGL(k_bsb_split<kMsTile0>, g, b, 0, st, dj, nc);
+        hipLaunchKernelGGL((k_bsb_bucket<kMsTile0, 4>), g, b, 0, st, dj, nc, lo);
         AG2_HIP(hipGetLastError());
         return;
     }

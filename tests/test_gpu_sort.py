@@ -51,3 +51,50 @@ def test_order(ag2, n):
         for _ in range(3):
             eng.step()
             check_order(ag2, eng, n)
+
+
+@pytest.mark.parametrize("n", [59999, 60000, 60001, 262144, 262145, 524288, 524289, 1048576, 1048577])
+def test_order_sample_sort(ag2, n):
+    """Either side of the sample sort's range and of its steps."""
+    E = ag2.engine
+    ps = ag2.ics.shuffled(ag2.ics.hernquist(n, seed=n), n)
+    with E.Engine(E.make_params(theta=0.7, e0=0.05 * ag2.units.KPC, split_threshold=800), n) as eng:
+        for order in (slice(None), slice(None, None, -1)):
+            for a in (ps.x, ps.y, ps.z):
+                a[:] = a[order].copy()
+            eng.upload(ps)
+            eng.build_tree()
+            check_order(ag2, eng, n)
+
+
+def test_order_overfull_bucket(ag2):
+    """128 tiles of 2048 particles on a line, each with 15 particles between
+    two of its samples in one and the same stretch: more than a bucket holds."""
+    E, tiles, tile, step = ag2.engine, 128, 2048, 16
+    n = tiles * tile
+    ps = ag2.ics.plummer(n, 1e10, 1.0, 20.0, seed=3)
+    g = np.random.default_rng(7)
+    for t in range(tiles):
+        first = int(f"{t % step:04b}"[::-1], 2) + 1024   # this tile's sample below the stretch
+        x = np.concatenate([g.uniform(0.1, 0.5, first + 1), g.uniform(0.5, 0.5001, step - 1),
+                            g.uniform(0.5001, 0.9, tile - first - step)])
+        ps.x[t * tile:(t + 1) * tile] = g.permutation(x) * ag2.units.KPC
+    ps.y[:] = ps.z[:] = 0.3 * ag2.units.KPC
+    with E.Engine(E.make_params(theta=0.7, e0=0.05 * ag2.units.KPC, split_threshold=800), n) as eng:
+        eng.upload(ps)
+        eng.build_tree()
+        check_order(ag2, eng, n)
+        perm = eng.order()[0]
+        assert (np.diff(ps.x[perm]) >= 0).all() and len(perm) == n
+
+
+def test_batch_with_large_job(ag2):
+    """A serving round whose largest job is past the merge sort's range."""
+    from test_gpu_serving import close, run_pool, solo
+    dt = 0.1 * ag2.units.MYR
+    prm = ag2.engine.make_params(theta=0.7, e0=0.05 * ag2.units.KPC, split_threshold=800, min_dt=dt, max_dt=dt)
+    jobs = [(ag2.ics.plummer(n, 1e10, 1.0, 20.0, seed=n), prm, 2) for n in (2, 63, 2049, 60001, 130000)]
+    res, _ = run_pool(ag2, jobs, max_jobs=8)
+    assert len(res) == len(jobs)
+    for i, (ps, prm, steps) in enumerate(jobs):
+        assert close(res[i], solo(ag2, ps, prm, steps)) is None, i
