@@ -504,7 +504,7 @@ struct Splitter {
 __device__ inline int sample_count(int n, int TILE, int tile, int step) {
     const int len = n - tile * TILE < TILE ? n - tile * TILE : TILE;
     const int ph = sample_phase(tile, step);
-    return len > ph ? (len - ph - 1) / step + 1 : 0;
+    return len > ph ? ((len - ph - 1) >> (__builtin_ctz((unsigned)step))) + 1 : 0;
 }
 
 // Elements of tile u that come before q of tile t (t != u): its sorted keys
@@ -513,7 +513,10 @@ __device__ inline bool before(uint64_t o, uint64_t q, bool first) { return first
 
 // The samples of one tile, a lane each: their ranks, and the splitters among
 // them.  The workgroup's waves share the other tiles, whose samples they
-// search in LDS, four lists side by side.
+// search in LDS, four lists side by side (7 us at 100,000 disk particles, 14
+// at 1,000,000, once lists that lie wholly to one side are left out; 12 and
+// 22 with every list searched, up to 99 where each sample searched the lists
+// in memory).
 template <int TILE>
 __device__ __forceinline__ void bs_split(int n, int step, const uint64_t *__restrict__ samp, Splitter *split,
                                          int own) {
@@ -535,17 +538,28 @@ __device__ __forceinline__ void bs_split(int n, int step, const uint64_t *__rest
             if (t + u < tiles) list[(slot * kG + u) * S + j] = samp[(size_t)(t + u) * S + j];
         __syncthreads();
         int len[kG], pos[kG];
+        bool need = false;
 #pragma unroll
         for (int u = 0; u < kG; u++) {
             len[u] = t + u < tiles && t + u != own ? sample_count(n, TILE, t + u, step) : 0;
             pos[u] = 0;
-        }
-        for (int d = S; d; d >>= 1)
-#pragma unroll
-            for (int u = 0; u < kG; u++) {
-                const int p = pos[u] + d;
-                if (p <= len[u] && before(list[(slot * kG + u) * S + p - 1], q, t + u < own)) pos[u] = p;
+            if (len[u] > 0) {
+                const uint64_t *l = list + (slot * kG + u) * S;
+                const bool f = t + u < own, all = before(l[len[u] - 1], q, f), none = !before(l[0], q, f);
+                pos[u] = all ? len[u] : 0;
+                need |= on && !all && !none;
             }
+        }
+        if (__any(need)) {   // (tiles of one order mostly stand apart)
+#pragma unroll
+            for (int u = 0; u < kG; u++) pos[u] = 0;
+            for (int d = S; d; d >>= 1)
+#pragma unroll
+                for (int u = 0; u < kG; u++) {
+                    const int p = pos[u] + d;
+                    if (p <= len[u] && before(list[(slot * kG + u) * S + p - 1], q, t + u < own)) pos[u] = p;
+                }
+        }
 #pragma unroll
         for (int u = 0; u < kG; u++) at += pos[u];
     }
@@ -923,49 +937,54 @@ __global__ __launch_bounds__(256) void k_inverse(int n, const uint32_t *rid, int
 // one position are buckets).  A distinct pair that agrees on every word sets
 // ds->tie_deep: the build refines it with deeper words (refine_ties), or
 // fails past kDeepest levels.
-// Four particles per thread (a 1024-particle scan tile per workgroup); the
-// tile's sum of c goes to bsum for k_scan_apply, the least lv of the tile
-// (0 past the last particle) to lmin for the cell searches.
+// One particle per thread, a 1024-particle scan tile per workgroup (four per
+// thread of 256 waited for each one's loads in turn: 7.5 us at 10,000
+// particles, now 4.6); the tile's sum of c goes to bsum for k_scan_apply, the
+// least lv of the tile (0 past the last particle) to lmin for the cell
+// searches.
 constexpr int kLevTile = 1024;
 
-__global__ __launch_bounds__(256) void k_lcp(int n, core::KeyWords kw, int nw, core::Pos pos, DevState *ds,
-                                             int parallel_root, uint8_t *lv, uint8_t *lmin, int32_t *c,
-                                             int32_t *bsum) {
-    __shared__ int scr[4], wmin[4];
+__global__ __launch_bounds__(kLevTile) void k_lcp(int n, core::KeyWords kw, int nw, core::Pos pos, DevState *ds,
+                                                  int parallel_root, uint8_t *lv, uint8_t *lmin, int32_t *c,
+                                                  int32_t *bsum) {
+    __shared__ int level[kLevTile], wsum[kLevTile / 64], wmin[kLevTile / 64];
     const int nin = ds->nin;
     const bool proot = parallel_root != 0, splits = proot && nin < n;
-    int tile = 0, least = 127;
-    for (int k = 0; k < 4; k++) {
-        const int i = blockIdx.x * kLevTile + k * 256 + threadIdx.x;
-        if (i >= nin) {
-            lv[i] = 0;
-            least = 0;
-            continue;
-        }
-        int li = core::pair_lcp(kw, pos, i, nin, proot, splits);
-        int lp = i == 0 ? -1 : core::pair_lcp(kw, pos, i - 1, nin, proot, splits);
+    const int i = blockIdx.x * kLevTile + threadIdx.x;
+    int li = -1, v = 0;
+    if (i < nin) {
+        li = core::pair_lcp(kw, pos, i, nin, proot, splits);
         // a coincident pair's level is its bucket's (pair_lcp), whatever the key words say
         const bool coincident = i + 1 < nin && core::same_pos(pos, i, i + 1);
         if (coincident) ds->any_bucket = 1;
         if (i + 1 < nin && li >= 21 * nw && !coincident) ds->tie_deep = 1;
         if (li > core::kDeepest) { li = core::kDeepest; ds->tie_deep = 1; }
-        if (lp > core::kDeepest) lp = core::kDeepest;
-        lv[i] = (uint8_t)(li + 1);
-        least = li + 1 < least ? li + 1 : least;
-        const int v = li - lp > 0 ? li - lp : 0;
-        c[i] = v;
-        tile += v;
     }
+    lv[i] = (uint8_t)(li + 1);
+    level[threadIdx.x] = li;
+    __syncthreads();
+    if (i < nin) {
+        int lp = -1;
+        if (threadIdx.x > 0) lp = level[threadIdx.x - 1];
+        else if (i > 0) lp = core::pair_lcp(kw, pos, i - 1, nin, proot, splits);
+        if (lp > core::kDeepest) lp = core::kDeepest;
+        v = li - lp > 0 ? li - lp : 0;
+        c[i] = v;
+    }
+    int least = li + 1;
     for (int d = 32; d >= 1; d >>= 1) {
         const int t = __shfl_xor(least, d, 64);
         least = t < least ? t : least;
+        v += __shfl_xor(v, d, 64);
     }
-    if (lane_id() == 0) wmin[threadIdx.x >> 6] = least;
-    int tot;
-    block256_excl_scan(tile, scr, &tot);
+    if (lane_id() == 0) { wsum[threadIdx.x >> 6] = v; wmin[threadIdx.x >> 6] = least; }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        bsum[blockIdx.x] = tot;
-        for (int w = 1; w < 4; w++) least = wmin[w] < least ? wmin[w] : least;
+        for (int w = 1; w < kLevTile / 64; w++) {
+            v += wsum[w];
+            least = wmin[w] < least ? wmin[w] : least;
+        }
+        bsum[blockIdx.x] = v;
         lmin[blockIdx.x] = (uint8_t)least;
     }
 }
@@ -1095,7 +1114,7 @@ __device__ inline int scan_levels(const uint8_t *lv, int s, int i, unsigned lt4,
 // start, then a pass that followed the children by their skip links, were
 // chains of 10 to 50 dependent reads: make_leaf, make_internal and
 // child_count took 14 + 17 + 11 us at 10,000 particles and 37 + 39 + 17 us at
-// 1,000,000; now make_leaf and make_internal 6.5 + 9.5 and 16 + 30.
+// 1,000,000; now make_leaf and make_internal 4.4 + 9.5 and 15 + 30.
 template <int PER>
 __global__ __launch_bounds__(256) void k_make_internal(int nin, int n_int, const uint8_t *lv, const uint8_t *lmin,
                                                        const int32_t *base, const int32_t *own, NodeArrays o,
@@ -1216,17 +1235,16 @@ __global__ __launch_bounds__(256) void k_make_root_only(NodeArrays o, int32_t *t
 // so it runs while the host waits for the counts; when the nodes are more
 // than the room (ds->err) it writes nothing, and the host launches it again
 // after making room.
-__global__ __launch_bounds__(256) void k_make_leaf(const DevState *ds, const uint8_t *lv, const int32_t *base,
-                                                   const int32_t *c, NodeArrays o, const uint32_t *idx,
-                                                   const uint8_t *gapl, int32_t *own, int32_t *tsum, int32_t *part) {
-    __shared__ int wl[4], wg[4];
+__global__ __launch_bounds__(kLevTile) void k_make_leaf(const DevState *ds, const uint8_t *lv, const int32_t *base,
+                                                        const int32_t *c, NodeArrays o, const uint32_t *idx,
+                                                        const uint8_t *gapl, int32_t *own, int32_t *tsum,
+                                                        int32_t *part) {
+    __shared__ int wl[kLevTile / 64], wg[kLevTile / 64];
     if (ds->err) return;
-    const int nin = ds->nin;
-    for (int k = blockIdx.x * 256 + threadIdx.x; k <= ds->n_nodes / 1024; k += gridDim.x * 256) tsum[k] = 0;
+    const int i = blockIdx.x * kLevTile + threadIdx.x;
+    for (int k = i; k <= ds->n_nodes / 1024; k += gridDim.x * kLevTile) tsum[k] = 0;
     int deep = 0, gp = 0;
-    for (int k = 0; k < 4; k++) {
-        const int i = blockIdx.x * kLevTile + k * 256 + threadIdx.x;
-        if (i >= nin) continue;
+    if (i < ds->nin) {
         const int a = i > 0 ? lv[i - 1] : 0, b = lv[i];
         const int li = a > b ? a : b;   // one level below the deeper neighbour pair
         const int b0 = base[i], ci = c[i];
@@ -1240,8 +1258,8 @@ __global__ __launch_bounds__(256) void k_make_leaf(const DevState *ds, const uin
         if (nd == 0) o.parent[0] = -1;
         // particle i starts internal nodes base[i] .. base[i] + c[i] - 1
         for (int u = 0; u < ci; u++) own[b0 + u] = i;
-        deep = li > deep ? li : deep;
-        gp += (g > 0 && g <= li) ? 1 : 0;
+        deep = li;
+        gp = (g > 0 && g <= li) ? 1 : 0;
     }
     for (int d = 32; d >= 1; d >>= 1) {
         const int t = __shfl_xor(deep, d, 64);
@@ -1251,7 +1269,7 @@ __global__ __launch_bounds__(256) void k_make_leaf(const DevState *ds, const uin
     if (lane_id() == 0) { wl[threadIdx.x >> 6] = deep; wg[threadIdx.x >> 6] = gp; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; w++) { deep = wl[w] > deep ? wl[w] : deep; gp += wg[w]; }
+        for (int w = 1; w < kLevTile / 64; w++) { deep = wl[w] > deep ? wl[w] : deep; gp += wg[w]; }
         part[blockIdx.x] = deep | gp << 8;
     }
 }
@@ -2090,7 +2108,7 @@ static void seg_order(Ctx &c) {
     core::Pos pos{c.alt[0], c.alt[1], c.alt[2]};
     int nb = (n + 1023) / 1024;
     if (nb < 1) nb = 1;
-    hipLaunchKernelGGL(k_lcp, dim3(nb), dim3(256), 0, st, n, kw, 2, pos, c.ds, proot, c.lcp, c.lmin, c.cnt,
+    hipLaunchKernelGGL(k_lcp, dim3(nb), dim3(kLevTile), 0, st, n, kw, 2, pos, c.ds, proot, c.lcp, c.lmin, c.cnt,
                        c.bsum);
     hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, st, c.cnt, c.bsum, c.ds, proot, c.node_cap, c.base);
     AG2_HIP(hipMemcpyAsync(c.hs_pinned, c.ds, sizeof(DevState), hipMemcpyDeviceToHost, st));
@@ -2232,7 +2250,7 @@ static NodeArrays node_arrays(const Ctx &c) {
 static void launch_leaves(Ctx &c) {
     const int nb = ((int)c.n + kLevTile - 1) / kLevTile;
     if (nb < 1) return;
-    hipLaunchKernelGGL(k_make_leaf, dim3(nb), dim3(256), 0, c.stream, c.ds, c.lcp, c.base, c.cnt, node_arrays(c),
+    hipLaunchKernelGGL(k_make_leaf, dim3(nb), dim3(kLevTile), 0, c.stream, c.ds, c.lcp, c.base, c.cnt, node_arrays(c),
                        c.idx_alt, c.gapl, c.n_cstart, c.n_bsum, c.leaf_part);
 }
 
@@ -2334,7 +2352,7 @@ static void refine_ties(Ctx &c) {
     const int proot = (c.n >= 2 && c.n >= c.p.split_threshold) ? 1 : 0;
     const core::Pos pos{c.alt[0], c.alt[1], c.alt[2]};
     const int nbn = (n + 1023) / 1024 < 1 ? 1 : (n + 1023) / 1024;
-    hipLaunchKernelGGL(k_lcp, dim3(nbn), dim3(256), 0, st, n, key_words(c), c.kw_used, pos, c.ds,
+    hipLaunchKernelGGL(k_lcp, dim3(nbn), dim3(kLevTile), 0, st, n, key_words(c), c.kw_used, pos, c.ds,
                        proot, c.lcp, c.lmin, c.cnt, c.bsum);
     hipLaunchKernelGGL(k_scan_apply, dim3(nbn), dim3(256), 0, st, c.cnt, c.bsum, c.ds, proot, c.node_cap, c.base);
     swap_state(c);
