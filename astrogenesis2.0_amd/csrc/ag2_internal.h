@@ -165,6 +165,7 @@ struct Ctx {
 
     // reductions
     double *partials = nullptr;
+    bool tw_partials = false;   // the drift left the tree width's partials in it
     // the particle buffers and the node buffers are each carved from one
     // device allocation (Carve)
     void *slab = nullptr, *node_slab = nullptr;
@@ -331,6 +332,60 @@ __device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
     return v;
 }
 
+// Counters that every wave adds to go through kCountBins bins, each on its
+// own 64-byte line, picked by the wave's group: a single address would
+// serialise tens of thousands of atomics.  fold_counter_bins sums the bins.
+enum { kCntInteractions = 0, kCntSphPairs, kCntEntries, kCntTests, kCntMixed, kCntSphOver, kCntNear, kCntNearRedo,
+       kCounters };
+constexpr int kCountBins = 256;
+static_assert((size_t)kCounters * kCountBins * 64 <= kCounterBinBytes, "counter bins exceed their buffer");
+
+// Each counter of the force phase is the sum of its bins (set, not added, so
+// the DevState needs no clearing beforehand); the bins are cleared.
+// One workgroup of 256, a thread per bin: k_fold_counters after a force phase
+// of its own, in a step the extra workgroup of the second kick.
+__device__ inline void fold_counter_bins(unsigned long long *bins, DevState *ds) {
+    __shared__ unsigned long long part[kCounters][4];
+    // every bin's loads first: one round trip for all counters
+    unsigned long long v[kCounters];
+    for (int c = 0; c < kCounters; c++) v[c] = bins[((size_t)c * kCountBins + threadIdx.x) * 8];
+    for (int c = 0; c < kCounters; c++) {
+        bins[((size_t)c * kCountBins + threadIdx.x) * 8] = 0ull;
+        const unsigned long long w = wave_sum_u64(v[c]);
+        if (lane_id() == 0) part[c][threadIdx.x >> 6] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long t[kCounters];
+        for (int c = 0; c < kCounters; c++) t[c] = part[c][0] + part[c][1] + part[c][2] + part[c][3];
+        ds->interactions = t[kCntInteractions];
+        ds->interactions_total += t[kCntInteractions];
+        ds->sph_pairs = t[kCntSphPairs];
+        ds->walk_entries = t[kCntEntries];
+        ds->walk_tests = t[kCntTests];
+        ds->walk_mixed = t[kCntMixed];
+        ds->sph_overflow = t[kCntSphOver];
+        ds->near_pairs = t[kCntNear];
+        ds->near_redo = t[kCntNearRedo];
+    }
+}
+
+// A workgroup's partial sums of |x| and |x|^2 for the tree width: waves in
+// order, the fixed grid's partials in order after them.
+constexpr int kTwBlocks = 512;   // fixed grid: fixed reduction order for R
+__device__ inline void tw_block_sums(double s, double q, double *part) {
+    s = wave_sum(s);
+    q = wave_sum(q);
+    __shared__ double ls[4], lq[4];
+    const int w = threadIdx.x >> 6;
+    if (lane_id() == 0) { ls[w] = s; lq[w] = q; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = ((ls[0] + ls[1]) + ls[2]) + ls[3];
+        part[2 * blockIdx.x + 1] = ((lq[0] + lq[1]) + lq[2]) + lq[3];
+    }
+}
+
 // --------------------------------------------------------- host wrappers
 void build_tree(Ctx &c);                 // tree_build.hip: build_tree_a, stream sync, build_tree_b
 void build_tree_a(Ctx &c);               // tree_build.hip: up to the node count (async)
@@ -346,8 +401,9 @@ void build_tree_b(Ctx &c);               // tree_build.hip: nodes, moments, layo
 core::KeyWords key_words(const Ctx &c);  // tree_build.hip: the key words of the last build
 void gas_density(Ctx &c);                // sph_density.hip
 void visual_density(Ctx &c, double rvd, double *vd);   // visual_density.hip: key order into vd
-void forces(Ctx &c, int mode);           // gravity.hip  (mode 0 forces, 1 potential)
-void forces_fp32(Ctx &c, int mode);      // gravity.hip  (split-precision FP32 forces)
+// gravity.hip (mode 0 forces, 1 potential; fold: the counters too, else kdk_end does)
+void forces(Ctx &c, int mode, bool fold = true);
+void forces_fp32(Ctx &c, int mode, bool fold = true);   // (split-precision FP32 forces)
 bool fp32_usable(const Ctx &c);          // gravity.hip: e0 / R of the last build suits the FP32 sweep
 int64_t sph_spill_bytes(int64_t n_gas, double theta);   // gravity.hip: device bytes of the spill chunks
 void reserve_spill(Ctx &c);              // gravity.hip: allocate them for the context's theta and gas
@@ -357,7 +413,7 @@ void near_finish(Ctx &c);                // gravity.hip: FP64 near pairs of a sp
 int64_t walk_groups_max(int64_t cap);    // gravity.hip: most walk groups any n <= cap makes
 void fold_counters(Ctx &c);              // gravity.hip: walk counters' bins into the DevState
 void kdk_begin(Ctx &c);                  // kdk.hip: time steps, min, first kick + drift
-void kdk_end(Ctx &c);                    // kdk.hip: U update, Hubble, second kick
+void kdk_end(Ctx &c);                    // kdk.hip: U update, Hubble, second kick, the walk counters
 void kdk_init_steps(Ctx &c);
 void energies(Ctx &c, int with_pot, double out[6]);
 void fill_active(Ctx &c, uint8_t v);

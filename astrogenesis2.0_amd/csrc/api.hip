@@ -363,10 +363,10 @@ int ag2_gas_density(void *ctx) {
     });
 }
 
-static void run_forces(Ctx &c, int mode) {
+static void run_forces(Ctx &c, int mode, bool fold = true) {
     c.fp64_fallback = c.p.precision == AG2_FP32_SPLIT && !ag2::fp32_usable(c);
-    if (c.p.precision == AG2_FP32_SPLIT && !c.fp64_fallback) ag2::forces_fp32(c, mode);
-    else ag2::forces(c, mode);
+    if (c.p.precision == AG2_FP32_SPLIT && !c.fp64_fallback) ag2::forces_fp32(c, mode, fold);
+    else ag2::forces(c, mode, fold);
 }
 
 int ag2_forces(void *ctx) {
@@ -411,7 +411,7 @@ int ag2_step(void *ctx) {
             ag2::build_tree(*c);
         }
         ag2::gas_density(*c);
-        run_forces(*c, 0);
+        run_forces(*c, 0, false);
         ag2::kdk_end(*c);
         if (c->timing >= 2) AG2_HIP(hipEventRecord(c->ev[7], c->stream));
         c->steps++;

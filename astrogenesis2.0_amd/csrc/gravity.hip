@@ -162,13 +162,6 @@ __device__ inline double shfl_d(double v, int src) {
     unsigned hi = (unsigned)__shfl((int)(b >> 32), src, 64);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
-// Counters that every wave adds to go through kCountBins bins, each on its
-// own 64-byte line, picked by the wave's group: a single address would
-// serialise tens of thousands of atomics.  k_fold_counters sums the bins.
-enum { kCntInteractions = 0, kCntSphPairs, kCntEntries, kCntTests, kCntMixed, kCntSphOver, kCntNear, kCntNearRedo,
-       kCounters };
-constexpr int kCountBins = 256;
-static_assert((size_t)kCounters * kCountBins * 64 <= kCounterBinBytes, "counter bins exceed their buffer");
 __device__ inline void bin_add(unsigned long long *bins, int counter, int bin, unsigned long long v) {
     if (v) atomicAdd(&bins[((size_t)counter * kCountBins + (bin & (kCountBins - 1))) * 8], v);
 }
@@ -1460,32 +1453,8 @@ __global__ __launch_bounds__(256) void k_sph_pairs(WalkArgs a, const int32_t *gi
     if (lane == 0) bin_add(a.cbins, kCntSphPairs, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), cs);
 }
 
-// Each counter of the force phase is the sum of its bins (set, not added, so
-// the DevState needs no clearing beforehand); the bins are cleared.
 __global__ __launch_bounds__(256) void k_fold_counters(unsigned long long *bins, DevState *ds) {
-    __shared__ unsigned long long part[kCounters][4];
-    // every bin's loads first: one round trip for all counters
-    unsigned long long v[kCounters];
-    for (int c = 0; c < kCounters; c++) v[c] = bins[((size_t)c * kCountBins + threadIdx.x) * 8];
-    for (int c = 0; c < kCounters; c++) {
-        bins[((size_t)c * kCountBins + threadIdx.x) * 8] = 0ull;
-        const unsigned long long w = wave_sum_u64(v[c]);
-        if (lane_id() == 0) part[c][threadIdx.x >> 6] = w;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long t[kCounters];
-        for (int c = 0; c < kCounters; c++) t[c] = part[c][0] + part[c][1] + part[c][2] + part[c][3];
-        ds->interactions = t[kCntInteractions];
-        ds->interactions_total += t[kCntInteractions];
-        ds->sph_pairs = t[kCntSphPairs];
-        ds->walk_entries = t[kCntEntries];
-        ds->walk_tests = t[kCntTests];
-        ds->walk_mixed = t[kCntMixed];
-        ds->sph_overflow = t[kCntSphOver];
-        ds->near_pairs = t[kCntNear];
-        ds->near_redo = t[kCntNearRedo];
-    }
+    fold_counter_bins(bins, ds);
 }
 
 __global__ void k_zero_job_counters(const JobWalk *jobs, int nj) {
@@ -1676,7 +1645,7 @@ static void launch_walk(Ctx &c) {
     }
 }
 
-void forces(Ctx &c, int mode) {
+void forces(Ctx &c, int mode, bool fold) {
     hipStream_t st = c.stream;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));
     if (mode == 0) {
@@ -1685,7 +1654,7 @@ void forces(Ctx &c, int mode) {
         launch_walk<false>(c);
         if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[9], st));
         sph_finish(c);
-        fold_counters(c);
+        if (fold) fold_counters(c);
     } else {
         const WalkArgs a = walk_args(c);
         const int tpg = walk_tpg(c.n, false);
@@ -1708,7 +1677,7 @@ bool fp32_usable(const Ctx &c) {
     return !(R > 0.0) || c.p.e0 >= ldexp(R, -24);
 }
 
-void forces_fp32(Ctx &c, int mode) {
+void forces_fp32(Ctx &c, int mode, bool fold) {
     if (mode != 0) return forces(c, mode);
     hipStream_t st = c.stream;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));
@@ -1718,7 +1687,7 @@ void forces_fp32(Ctx &c, int mode) {
     if (c.timing >= 1) AG2_HIP(hipEventRecord(c.ev[9], st));
     near_finish(c);
     sph_finish(c);
-    fold_counters(c);
+    if (fold) fold_counters(c);
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[5], st));
     AG2_HIP(hipGetLastError());
 }

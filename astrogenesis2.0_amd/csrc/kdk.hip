@@ -84,31 +84,45 @@ __device__ inline unsigned long long min_next_fold(int nb, const unsigned long l
 }
 
 // Simulation.cpp:256-272: globalTime = min next; active particles kick + drift.
+// TW: also the tree width's partials over the new positions, one particle per
+// thread in at most kTwBlocks workgroups: those of k_tw_partial bit for bit,
+// and one launch fewer (3.3 us at 10,000 particles).
+template <bool TW>
 __global__ __launch_bounds__(256) void k_kick_drift(int n, int nb, const unsigned long long *part, DevState *ds,
                                                     const double *ts, const double *next,
                                                     double *x, double *y, double *z, double *vx, double *vy,
                                                     double *vz, const double *ax, const double *ay, const double *az,
-                                                    uint8_t *active) {
+                                                    uint8_t *active, double *tw) {
     const unsigned long long mb = min_next_fold(nb, part);
     int i = blockIdx.x * 256 + threadIdx.x;
     double gt = __longlong_as_double((long long)mb);
     if (i == 0) { ds->min_next_bits = mb; ds->gtime = gt; }
-    if (i >= n) return;
-    bool a = gt == next[i];
-    active[i] = a ? 1 : 0;
-    if (!a) return;
-    double dt = ts[i];
-    double gx = ax[i], gy = ay[i], gz = az[i];
-    if (!(gx != gx || gy != gy || gz != gz)) {
-        vx[i] = vx[i] + gx * dt / 2;
-        vy[i] = vy[i] + gy * dt / 2;
-        vz[i] = vz[i] + gz * dt / 2;
-    } else {
-        atomicAdd(&ds->nan_kicks, 1ull);
+    if (!TW && i >= n) return;
+    const bool in = i < n, a = in && gt == next[i];
+    if (in) active[i] = a ? 1 : 0;
+    if (a) {
+        double dt = ts[i];
+        double gx = ax[i], gy = ay[i], gz = az[i];
+        if (!(gx != gx || gy != gy || gz != gz)) {
+            vx[i] = vx[i] + gx * dt / 2;
+            vy[i] = vy[i] + gy * dt / 2;
+            vz[i] = vz[i] + gz * dt / 2;
+        } else {
+            atomicAdd(&ds->nan_kicks, 1ull);
+        }
+        x[i] = x[i] + vx[i] * dt;
+        y[i] = y[i] + vy[i] * dt;
+        z[i] = z[i] + vz[i] * dt;
     }
-    x[i] = x[i] + vx[i] * dt;
-    y[i] = y[i] + vy[i] * dt;
-    z[i] = z[i] + vz[i] * dt;
+    if (TW) {
+        double s = 0.0, q = 0.0;
+        if (in) {
+            const double d = sqrt(x[i] * x[i] + y[i] * y[i] + z[i] * z[i]);
+            s += d;
+            q += d * d;
+        }
+        tw_block_sums(s, q, tw);
+    }
 }
 
 // Simulation.cpp:295-341: U update for gas, Hubble scaling, second kick.
@@ -141,7 +155,12 @@ __global__ __launch_bounds__(256) void k_kick2(int n, const uint8_t *active, uin
                                                double *next, double *x, double *y, double *z, double *vx,
                                                double *vy, double *vz, const double *ax, const double *ay,
                                                const double *az, double *U, double *dUdt, double H0, DevState *ds,
-                                               GasSources gs) {
+                                               GasSources gs, unsigned long long *bins) {
+    // the last workgroup: the walk's counters (a launch of its own takes 4.6 us)
+    if (blockIdx.x == gridDim.x - 1) {
+        fold_counter_bins(bins, ds);
+        return;
+    }
     int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n || !active[i]) return;
     double dt = ts[i];
@@ -247,19 +266,28 @@ void kdk_begin(Ctx &c) {
     hipStream_t st = c.stream;
     unsigned sb = grid_for(n, 256);
     sb = sb < (unsigned)kStepBlocks ? (sb ? sb : 1u) : (unsigned)kStepBlocks;
-    unsigned long long *part = (unsigned long long *)c.partials;
+    // past the tree width's partials and maxima, which k_kick_drift may write
+    unsigned long long *part = (unsigned long long *)(c.partials + 4 * 1024);
     hipLaunchKernelGGL(k_steps, dim3(sb), dim3(256), 0, st, n, c.ax, c.ay, c.az, c.p.eta, c.p.e0,
                        c.p.min_dt, c.p.max_dt, c.ts, c.next, c.ds, part);
-    hipLaunchKernelGGL(k_kick_drift, dim3(grid_for(n, 256)), dim3(256), 0, st, n, (int)sb, part, c.ds, c.ts, c.next,
-                       c.x, c.y, c.z, c.vx, c.vy, c.vz, c.ax, c.ay, c.az, c.active);
+    // (a captured build keeps its own launch of the partials)
+    const int g = grid_for(n, 256);
+    const bool tw = g <= kTwBlocks && !c.p.graph_launch;
+    if (tw)
+        hipLaunchKernelGGL(k_kick_drift<true>, dim3(g), dim3(256), 0, st, n, (int)sb, part, c.ds, c.ts, c.next, c.x,
+                           c.y, c.z, c.vx, c.vy, c.vz, c.ax, c.ay, c.az, c.active, c.partials);
+    else
+        hipLaunchKernelGGL(k_kick_drift<false>, dim3(g), dim3(256), 0, st, n, (int)sb, part, c.ds, c.ts, c.next, c.x,
+                           c.y, c.z, c.vx, c.vy, c.vz, c.ax, c.ay, c.az, c.active, c.partials);
     AG2_HIP(hipGetLastError());
+    c.tw_partials = tw;   // the build that follows uses them
 }
 
 void kdk_end(Ctx &c) {
     int n = (int)c.n;
     GasSources gs{c.p.cooling != 0, c.p.star_formation != 0, c.p.sfr_seed, c.steps, c.rid, c.rho, c.T, c.sfr};
-    hipLaunchKernelGGL(k_kick2, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n, c.active, c.type, c.ts, c.next,
-                       c.x, c.y, c.z, c.vx, c.vy, c.vz, c.ax, c.ay, c.az, c.U, c.dUdt, c.p.H0, c.ds, gs);
+    hipLaunchKernelGGL(k_kick2, dim3(grid_for(n, 256) + 1), dim3(256), 0, c.stream, n, c.active, c.type, c.ts, c.next,
+                       c.x, c.y, c.z, c.vx, c.vy, c.vz, c.ax, c.ay, c.az, c.U, c.dUdt, c.p.H0, c.ds, gs, c.cbins);
     AG2_HIP(hipGetLastError());
 }
 

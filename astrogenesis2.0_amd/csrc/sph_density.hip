@@ -161,7 +161,8 @@ void gas_density(Ctx &c) {
         if (n > 0 && c.sph_active)
             hipLaunchKernelGGL(k_group_init, dim3(grid_for(n, 256)), dim3(256), 0, st, n, c.type, c.h, 0, c.g_first,
                                c.g_fired);
-        hipLaunchKernelGGL(k_zero_groups, dim3(1), dim3(1), 0, st, c.ds);
+        // (without gas the node kernel of the build cleared the count)
+        if (c.sph_active || nn <= 0) hipLaunchKernelGGL(k_zero_groups, dim3(1), dim3(1), 0, st, c.ds);
     }
     c.h_cleared = c.groups_cleared = false;
     if (c.timing >= 2) AG2_HIP(hipEventRecord(c.ev[4], st));

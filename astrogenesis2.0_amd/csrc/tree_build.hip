@@ -7,10 +7,11 @@
 namespace ag2 {
 namespace {
 
-constexpr int kTwBlocks = 512;   // fixed grid: fixed reduction order for R
 constexpr unsigned long long kOut = ~0ull;
 
 // ------------------------------------------------------------ tree width
+// (k_kick_drift forms the same partials in a step of up to 256 kTwBlocks
+// particles.)
 __global__ __launch_bounds__(256) void k_tw_partial(int n, const double *__restrict__ x,
                                                     const double *__restrict__ y,
                                                     const double *__restrict__ z, double *part) {
@@ -20,16 +21,7 @@ __global__ __launch_bounds__(256) void k_tw_partial(int n, const double *__restr
         s += d;
         q += d * d;
     }
-    s = wave_sum(s);
-    q = wave_sum(q);
-    __shared__ double ls[4], lq[4];
-    int w = threadIdx.x >> 6;
-    if (lane_id() == 0) { ls[w] = s; lq[w] = q; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = ((ls[0] + ls[1]) + ls[2]) + ls[3];
-        part[2 * blockIdx.x + 1] = ((lq[0] + lq[1]) + lq[2]) + lq[3];
-    }
+    tw_block_sums(s, q, part);
 }
 
 // Tree::calcTreeWidth (Tree.cpp:86-117): cut = mean + 10 sigma of |x|,
@@ -1550,7 +1542,7 @@ struct NodeMoments {
 constexpr int kSumTiny = 8;
 
 __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, int proot, int64_t thr, int zm,
-                                                      const uint32_t *rid, const DevState *ds,
+                                                      const uint32_t *rid, DevState *ds,
                                                       const int32_t *first, const int32_t *count,
                                                       const int32_t *parent, const int32_t *pidx,
                                                       const int8_t *level, const NodeSums *blk1,
@@ -1663,6 +1655,7 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, in
     // cleared group state for the density phase (Node.cpp:722-796)
     group_first[nd] = kGroupNone;
     group_fired[nd] = 0;
+    if (!tsph && nd == 0) ds->final_count = 0;   // no gas: no group in effect
     int par = parent[nd];
     double M, g, cx, cy, cz, mvx = 0.0, mvy = 0.0, mvz = 0.0;
     const core::Pos pos{v.sx, v.sy, v.sz};
@@ -2083,7 +2076,8 @@ static void seg_keys(Ctx &c) {
     int twb = g < kTwBlocks ? (g > 0 ? g : 1) : kTwBlocks;
     // partials: the sums at [0, 2 twb), the maxima after them
     unsigned long long *rmax = (unsigned long long *)(c.partials + 2 * kTwBlocks);
-    hipLaunchKernelGGL(k_tw_partial, dim3(twb), dim3(256), 0, st, n, c.x, c.y, c.z, c.partials);
+    if (!c.tw_partials) hipLaunchKernelGGL(k_tw_partial, dim3(twb), dim3(256), 0, st, n, c.x, c.y, c.z, c.partials);
+    c.tw_partials = false;
     hipLaunchKernelGGL(k_tw_max, dim3(twb), dim3(256), 0, st, n, c.x, c.y, c.z, twb, c.partials, c.ds, rmax);
     hipLaunchKernelGGL(k_keygen, dim3(g), dim3(256), 0, st, n, c.x, c.y, c.z, twb, rmax, c.ds, c.key, c.idx,
                        c.gapl);
