@@ -385,6 +385,35 @@ AG2_HD bool octant_path(double px, double py, double pz, double R, int levels, u
     return true;
 }
 
+// The bits of an 11-bit number, three places apart.
+AG2_HD uint32_t spread11(uint32_t v) {
+    v = (v | v << 16) & 0x070000FFu;
+    v = (v | v << 8) & 0x0700F00Fu;
+    v = (v | v << 4) & 0x430C30C3u;
+    return (v | v << 2) & 0x49249249u;
+}
+
+// Word 0 of the octant path (levels 1 .. 21) from the position in units of
+// the finest cell, for a particle inside the root cube; scale = 2^20 / R.
+// The descent compares with centres that carry roundings of up to 2^-28
+// cells, the scaled position one of 2^-31: a coordinate farther than 2^-20
+// cells from every cell face decides all 21 comparisons alike and keeps the
+// particle strictly inside its nodes' bounds (no gap).  False where one is
+// nearer, or nothing is known (R zero or not finite).
+AG2_HD bool octant_word0_apart(double px, double py, double pz, double scale, uint64_t *key) {
+    const double ux = px * scale + 1048576.0, uy = py * scale + 1048576.0, uz = pz * scale + 1048576.0;
+    const double fx = floor(ux), fy = floor(uy), fz = floor(uz);
+    const double ax = fabs(ux - fx - 0.5), ay = fabs(uy - fy - 0.5), az = fabs(uz - fz - 0.5);
+    if (!(ax < 0.5 - 0x1p-20 && ay < 0.5 - 0x1p-20 && az < 0.5 - 0x1p-20)) return false;
+    if (!(fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < 2097152.0 && fy < 2097152.0 && fz < 2097152.0)) return false;
+    const uint32_t ix = (uint32_t)(int32_t)fx, iy = (uint32_t)(int32_t)fy, iz = (uint32_t)(int32_t)fz;
+    const uint32_t lo = spread11(ix & 1023u) | spread11(iy & 1023u) << 1 | spread11(iz & 1023u) << 2;
+    const uint64_t hi = (uint64_t)spread11(ix >> 10) | (uint64_t)spread11(iy >> 10) << 1 |
+                        (uint64_t)spread11(iz >> 10) << 2;
+    *key = hi << 30 | lo;
+    return true;
+}
+
 // Word w of the octant path (levels 21 w + 1 .. 21 w + 21) of a particle
 // inside the root cube, by the descent of octant_path; *gap as there, over
 // levels 1 .. 21 w + 21.
