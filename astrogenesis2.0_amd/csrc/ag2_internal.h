@@ -122,9 +122,7 @@ struct Ctx {
     int32_t *n_first = nullptr, *n_count = nullptr, *n_parent = nullptr;
     int32_t *n_pidx = nullptr;
     int8_t *n_level = nullptr;
-    double *n_mass = nullptr;
-    double *n_gas = nullptr, *n_gvx = nullptr, *n_gvy = nullptr, *n_gvz = nullptr;
-    double *n_cx = nullptr, *n_cy = nullptr, *n_cz = nullptr;
+    double *n_gas = nullptr;   // gas mass (sets with gas; every other moment is in the walk records)
     // child-contiguous layout for the block walk
     core::TreeNode *tnode = nullptr;
     core::SphNode *tsph = nullptr;   // SPH records in the walk layout (written when gas is present)

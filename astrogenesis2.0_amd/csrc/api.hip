@@ -145,7 +145,7 @@ int64_t ctx_footprint(int64_t cap, int64_t n_gas) {
                     + 3 * 4           // rid, rid copy, inverse
                     + 2 * 4           // c, base
                     + 2 * 4 + 1;      // SPH list slots, targets, group flags
-    int64_t per_node = 4 * 4 + 1 + 9 * 8 + 2 * 4 + 1 + 4 +
+    int64_t per_node = 4 * 4 + 1 + 2 * 8 + 2 * 4 + 1 + 4 +
                        2 * (int64_t)sizeof(core::TreeNode) + 3 * 4 +   // walk and SPH records
                        (int64_t)sizeof(ag2::NodeSums) / 64 + 1;        // block sums
     int64_t fixed = 256 * ((n + kSortTile - 1) / kSortTile + 1) * 4 + 8 * 1024 * 8 + (1 << 20) +
@@ -616,26 +616,35 @@ int ag2_get_tree(void *ctx, int64_t cap, int32_t *level, int64_t *first, int64_t
         if ((int64_t)nn > cap) return fail(c, AG2_ERR_CAPACITY, "cap is smaller than the node count");
         std::vector<int8_t> lv(nn);
         std::vector<int32_t> f(nn), k(nn);
-        std::vector<double> cx(nn), cy(nn), cz(nn), vx(nn), vy(nn), vz(nn);
+        // the moments are in the walk records, whose pre-order index they hold;
+        // a node's gas velocity in its SPH record (sets with gas)
+        const bool sph = c->sph_active && mvel != nullptr;
+        std::vector<ag2::core::TreeNode> rec(nn);
+        std::vector<ag2::core::SphNode> srec(sph ? nn : 0);
         if (nn) {
             AG2_HIP(hipMemcpy(lv.data(), c->n_level, nn, hipMemcpyDeviceToHost));
             AG2_HIP(hipMemcpy(f.data(), c->n_first, nn * 4, hipMemcpyDeviceToHost));
             AG2_HIP(hipMemcpy(k.data(), c->n_count, nn * 4, hipMemcpyDeviceToHost));
-            if (mass) AG2_HIP(hipMemcpy(mass, c->n_mass, nn * 8, hipMemcpyDeviceToHost));
-            if (gas) AG2_HIP(hipMemcpy(gas, c->n_gas, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(cx.data(), c->n_cx, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(cy.data(), c->n_cy, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(cz.data(), c->n_cz, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(vx.data(), c->n_gvx, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(vy.data(), c->n_gvy, nn * 8, hipMemcpyDeviceToHost));
-            AG2_HIP(hipMemcpy(vz.data(), c->n_gvz, nn * 8, hipMemcpyDeviceToHost));
+            AG2_HIP(hipMemcpy(rec.data(), c->tnode, nn * sizeof(rec[0]), hipMemcpyDeviceToHost));
+            if (sph) AG2_HIP(hipMemcpy(srec.data(), c->tsph, nn * sizeof(srec[0]), hipMemcpyDeviceToHost));
         }
         for (size_t i = 0; i < nn; i++) {
             if (level) level[i] = lv[i];
             if (first) first[i] = f[i];
             if (count) count[i] = k[i];
-            if (com) { com[3 * i] = cx[i]; com[3 * i + 1] = cy[i]; com[3 * i + 2] = cz[i]; }
-            if (mvel) { mvel[3 * i] = vx[i]; mvel[3 * i + 1] = vy[i]; mvel[3 * i + 2] = vz[i]; }
+        }
+        for (size_t j = 0; j < nn; j++) {
+            const ag2::core::TreeNode &r = rec[j];
+            const size_t i = (size_t)r.pre;
+            if (mass) mass[i] = r.mass;
+            if (gas) gas[i] = r.gas;
+            if (com) { com[3 * i] = r.cx; com[3 * i + 1] = r.cy; com[3 * i + 2] = r.cz; }
+            const bool v = sph && r.pidx < 0 && r.gas > 0.0;   // (leaves report none)
+            if (mvel) {
+                mvel[3 * i] = v ? srec[j].vx : 0.0;
+                mvel[3 * i + 1] = v ? srec[j].vy : 0.0;
+                mvel[3 * i + 2] = v ? srec[j].vz : 0.0;
+            }
         }
         return AG2_OK;
     });

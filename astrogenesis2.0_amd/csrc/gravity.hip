@@ -89,7 +89,6 @@ struct WalkArgs {
     const double *__restrict__ sx, *__restrict__ sy, *__restrict__ sz, *__restrict__ sm;
     const uint8_t *__restrict__ stype;
     const double *__restrict__ svx, *__restrict__ svy, *__restrict__ svz;
-    const double *__restrict__ mvx, *__restrict__ mvy, *__restrict__ mvz;
     const double *__restrict__ h, *__restrict__ rho, *__restrict__ P;
     const uint8_t *__restrict__ active;
     const DevState *ds;
@@ -981,11 +980,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                 const double tvx = a.svx[ti], tvy = a.svy[ti], tvz = a.svz[ti];
                                 core::Target tt;
                                 tt.h = a.h[ti]; tt.rho = a.rho[ti]; tt.P = a.P[ti];
-                                const core::TreeNode nj = a.tree[S.ent_node[e0 + jl]];
+                                const core::SphNode nj = a.tsph[S.ent_node[e0 + jl]];   // (a candidate has gas)
                                 const double jx = nj.cx, jy = nj.cy, jz = nj.cz, jg = nj.gas;
-                                double jvx, jvy, jvz;
-                                if (nj.pidx >= 0) { jvx = a.svx[nj.pidx]; jvy = a.svy[nj.pidx]; jvz = a.svz[nj.pidx]; }
-                                else { jvx = a.mvx[nj.pre]; jvy = a.mvy[nj.pre]; jvz = a.mvz[nj.pre]; }
+                                const double jvx = nj.vx, jvy = nj.vy, jvz = nj.vz;
                                 const core::SphConst k = core::sph_const(tt);
                                 core::WalkSums w{0, 0, 0, 0, 0, 0, 0};
                                 const double ddx = tx - jx, ddy = ty - jy, ddz = tz - jz;
@@ -1480,7 +1477,6 @@ WalkArgs walk_args(Ctx &c) {
     a.sph_spill = c.sph_spill; a.sph_more = c.sph_more; a.spill_cap = (int)c.spill_cap;
     a.sx = c.x; a.sy = c.y; a.sz = c.z; a.sm = c.m; a.stype = c.type;
     a.svx = c.vx; a.svy = c.vy; a.svz = c.vz;
-    a.mvx = c.n_gvx; a.mvy = c.n_gvy; a.mvz = c.n_gvz;
     a.h = c.h; a.rho = c.rho; a.P = c.P; a.active = c.active;
     a.ds = c.ds;
     a.wp = core::WalkParams{c.p.theta, c.p.e0, c.p.G, core::soft_branch_live(c.p.e0)};

@@ -54,10 +54,12 @@ __global__ __launch_bounds__(256) void k_group_fire(int nn, const int32_t *paren
 
 // Groups in effect: fired nodes with no fired ancestor.  Each workgroup
 // lists its own in LDS and writes them to its slice of the list (256 entries
-// per workgroup, at most one per node) with their count, so no counter is
+// per workgroup, at most one per node; place: their walk records) with their
+// count, so no counter is
 // shared between workgroups.
 __global__ __launch_bounds__(256) void k_group_top(int nn, const int32_t *parent, const uint8_t *fired,
-                                                   int32_t *list, int32_t *bcount) {
+                                                   const int32_t *cstart, const int32_t *rank, int32_t *list,
+                                                   int32_t *place, int32_t *bcount) {
     __shared__ int cnt;
     if (threadIdx.x == 0) cnt = 0;
     __syncthreads();
@@ -66,7 +68,11 @@ __global__ __launch_bounds__(256) void k_group_top(int nn, const int32_t *parent
         bool top = true;
         for (int a = parent[nd]; a >= 0; a = parent[a])
             if (fired[a]) { top = false; break; }
-        if (top) list[blockIdx.x * 256 + atomicAdd(&cnt, 1)] = nd;
+        if (top) {
+            const int at = blockIdx.x * 256 + atomicAdd(&cnt, 1);
+            list[at] = nd;
+            place[at] = core::node_place(nd, parent[nd], cstart, rank);
+        }
     }
     __syncthreads();
     if (threadIdx.x == 0) bcount[blockIdx.x] = cnt;
@@ -85,10 +91,10 @@ __device__ inline void group_count(int nb, const int32_t *bcount, DevState *ds) 
 // One wave per group in effect, in a fixed lane-strided order with a
 // butterfly sum (deterministic); the wave then writes h, rho, P, T of every
 // gas particle in the group's range (Node.cpp:757-795).
-__global__ __launch_bounds__(256) void k_group_rho(int nb, const int32_t *list, const int32_t *bcount,
+__global__ __launch_bounds__(256) void k_group_rho(int nb, const int32_t *list, const int32_t *place,
+                                                   const int32_t *bcount, const core::TreeNode *tree,
                                                    const int32_t *first, const int32_t *count, const int8_t *level,
-                                                   const int32_t *parent, const double *cx, const double *cy,
-                                                   const double *cz, const double *sx, const double *sy,
+                                                   const int32_t *parent, const double *sx, const double *sy,
                                                    const double *sz, const double *sm, const uint8_t *stype,
                                                    const double *U, const double *mu, int64_t N, int64_t thr,
                                                    DevState *ds, double *g_rho, double *h, double *rho,
@@ -103,7 +109,8 @@ __global__ __launch_bounds__(256) void k_group_rho(int nb, const int32_t *list, 
         for (int k = w; k < nf; k += 4) {
             int F = list[b * 256 + k];
             double hh = ldexp(R, -(int)level[F]) * 2;
-            double gx = cx[F], gy = cy[F], gz = cz[F];
+            const core::TreeNode &rec = tree[place[b * 256 + k]];
+            double gx = rec.cx, gy = rec.cy, gz = rec.cz;
             int j0 = first[F], j1 = first[F] + count[F];
             double s = 0.0;
             for (int j = j0 + lane_id(); j < j1; j += 64) {
@@ -150,12 +157,13 @@ void gas_density(Ctx &c) {
                            c.n_gas, c.p.massInH, c.rid, c.g_first);
         hipLaunchKernelGGL(k_group_fire, dim3(grid_for(nn, 256)), dim3(256), 0, st, nn, c.n_parent, c.g_first,
                            c.g_fired);
-        // g_final holds the per-workgroup group counts
+        // g_final holds the per-workgroup group counts; g_first, read by now,
+        // the places of the groups listed
         int nb = grid_for(nn, 256);
-        hipLaunchKernelGGL(k_group_top, dim3(nb), dim3(256), 0, st, nn, c.n_parent, c.g_fired, c.g_list, c.g_final);
-        hipLaunchKernelGGL(k_group_rho, dim3(nb), dim3(256), 0, st, nb, c.g_list,
-                           c.g_final, c.n_first, c.n_count, c.n_level, c.n_parent, c.n_cx, c.n_cy, c.n_cz, c.x, c.y,
-                           c.z, c.m, c.type, c.U, c.mu, c.n, c.p.split_threshold, c.ds, c.g_rho, c.h, c.rho, c.P,
+        hipLaunchKernelGGL(k_group_top, dim3(nb), dim3(256), 0, st, nn, c.n_parent, c.g_fired, c.n_cstart,
+                           c.n_rank, c.g_list, c.g_first, c.g_final);
+        hipLaunchKernelGGL(k_group_rho, dim3(nb), dim3(256), 0, st, nb, c.g_list, c.g_first,
+                           c.g_final, c.tnode, c.n_first, c.n_count, c.n_level, c.n_parent, c.x, c.y, c.z, c.m, c.type, c.U, c.mu, c.n, c.p.split_threshold, c.ds, c.g_rho, c.h, c.rho, c.P,
                            c.T);
     } else {
         if (n > 0 && c.sph_active)

@@ -1514,10 +1514,6 @@ __device__ inline void load_piece(double (&f)[8], const Cover &c, int k, const P
     f[7] = part ? (gas ? gz * m : 0.0) : gz;
 }
 
-struct NodeMoments {
-    double *m, *gas, *cx, *cy, *cz, *mvx, *mvy, *mvz;
-};
-
 // Child-contiguous layout for the block walk (core::TreeNode): the root at 0,
 // the children of node p at [1 + cstart[p], 1 + cstart[p] + nchild[p]) in
 // octant order (rank, which in pre-order is the order of the children's first
@@ -1555,7 +1551,7 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, in
                                                       const NodeSums *blk2,
                                                       const double *gas_table, int gas_equal, int64_t ngas, PVals v,
                                                       const int32_t *nchild, const int32_t *rank,
-                                                      const int32_t *cstart, NodeMoments o,
+                                                      const int32_t *cstart, double *gas_mass,
                                                       core::TreeNode *tree, core::SphNode *tsph,
                                                       int32_t *group_first, uint8_t *group_fired) {
     __shared__ double st_m[kStage], st_x[kStage], st_y[kStage], st_z[kStage];
@@ -1712,10 +1708,8 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, in
         if (g > 0) { mvx = S[5] / g; mvy = S[6] / g; mvz = S[7] / g; }
         if (buckets && core::is_bucket(pos, s, e)) { cx = v.sx[s]; cy = v.sy[s]; cz = v.sz[s]; }
     }
-    o.m[nd] = M; o.gas[nd] = g;
-    o.cx[nd] = cx; o.cy[nd] = cy; o.cz[nd] = cz;
-    o.mvx[nd] = mvx; o.mvy[nd] = mvy; o.mvz[nd] = mvz;
-    const int place = par < 0 ? 0 : 1 + cstart[par] + rank[nd];
+    if (tsph) gas_mass[nd] = g;   // (pre-order: the density phase climbs it)
+    const int place = core::node_place(nd, par, cstart, rank);
     const int kc = nchild[nd];
     core::TreeNode t;
     t.cx = cx; t.cy = cy; t.cz = cz; t.mass = M; t.gas = g;
@@ -1937,8 +1931,7 @@ void alloc_nodes(Ctx &c, int64_t cap) {
         cv(&c.n_first, n * 4); cv(&c.n_count, n * 4);
         cv(&c.n_parent, n * 4);
         cv(&c.n_pidx, n * 4); cv(&c.n_level, n);
-        double **d8[] = {&c.n_mass, &c.n_gas, &c.n_gvx, &c.n_gvy, &c.n_gvz, &c.n_cx, &c.n_cy, &c.n_cz, &c.g_rho};
-        for (double **p : d8) cv(p, n * 8);
+        cv(&c.n_gas, n * 8); cv(&c.g_rho, n * 8);
         cv(&c.g_first, n * 4); cv(&c.g_list, (n + 256) * 4);
         cv(&c.g_fired, n); cv(&c.g_final, n * 4);
         cv(&c.tnode, n * sizeof(core::TreeNode));
@@ -2422,21 +2415,20 @@ void build_tree_b(Ctx &c) {
         tile_sum_buffers(c, &blk1, &blk2);
         hipLaunchKernelGGL(k_iscan_apply, dim3(nbn), dim3(256), 0, st, nn, c.n_nchild, c.n_bsum, c.n_cstart,
                            (nin + kLevTile - 1) / kLevTile, c.leaf_part, c.ds);
-        NodeMoments nm{c.n_mass, c.n_gas, c.n_cx, c.n_cy, c.n_cz, c.n_gvx, c.n_gvy, c.n_gvz};
         hipLaunchKernelGGL(k_node_moments, dim3(gn), dim3(256), 0, st, nn, nin, n, proot, c.p.split_threshold,
                            c.zero_mass > 0 ? 1 : 0, c.rid, c.ds,
                            c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_level, blk1, blk2, c.gas_table,
                            c.gas_equal, c.gas_count, pv,
-                           c.n_nchild, c.n_rank, c.n_cstart, nm, c.tnode,
+                           c.n_nchild, c.n_rank, c.n_cstart, c.n_gas, c.tnode,
                            c.sph_active ? c.tsph : nullptr, c.g_first, c.g_fired);
         c.groups_cleared = true;
         if (deep && nin > 0) {
             // the walk's stack bound comes from the branching depth here
-            // (n_cstart is free again: the walk records hold the places)
-            hipLaunchKernelGGL(k_zero_inner, dim3(gn), dim3(256), 0, st, nn, c.n_cstart, c.ds);
-            hipLaunchKernelGGL(k_count_inner, dim3(gn), dim3(256), 0, st, nn, c.n_pidx, c.n_parent, c.n_cstart);
+            // (g_list is free until the density phase)
+            hipLaunchKernelGGL(k_zero_inner, dim3(gn), dim3(256), 0, st, nn, c.g_list, c.ds);
+            hipLaunchKernelGGL(k_count_inner, dim3(gn), dim3(256), 0, st, nn, c.n_pidx, c.n_parent, c.g_list);
             hipLaunchKernelGGL(k_branch_depth, dim3(grid_for(nin, 256)), dim3(256), 0, st, nin, c.base, c.cnt,
-                               c.n_parent, c.n_cstart, c.ds);
+                               c.n_parent, c.g_list, c.ds);
             AG2_HIP(hipMemcpyAsync(&c.hs_pinned->walk_depth, &c.ds->walk_depth, sizeof(int32_t),
                                    hipMemcpyDeviceToHost, st));
             AG2_HIP(hipStreamSynchronize(st));

@@ -263,6 +263,12 @@ struct alignas(64) TreeNode {
     int32_t pad1;
 };
 
+// Place of node nd (pre-order; par: its parent) in the child-contiguous
+// layout.
+AG2_HD int node_place(int nd, int par, const int32_t *cstart, const int32_t *rank) {
+    return par < 0 ? 0 : 1 + cstart[par] + rank[nd];
+}
+
 // SPH view of a node in the walk layout (same index as its TreeNode): centre
 // of mass, gas mass, gas velocity (a leaf: its particle's velocity; a node:
 // the gas-mass-weighted mean), particle of a leaf.  64 bytes.

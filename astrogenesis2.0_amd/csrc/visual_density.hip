@@ -26,7 +26,9 @@ __global__ __launch_bounds__(256) void k_visual_density(int n, int nin, const in
                                                         const int32_t *__restrict__ cnt,
                                                         const int32_t *__restrict__ parent,
                                                         const int8_t *__restrict__ level,
-                                                        const double *__restrict__ nmass, const DevState *ds,
+                                                        const int32_t *__restrict__ cstart,
+                                                        const int32_t *__restrict__ rank,
+                                                        const core::TreeNode *__restrict__ tree, const DevState *ds,
                                                         double rvd, double *__restrict__ vd) {
     int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
@@ -47,7 +49,7 @@ __global__ __launch_bounds__(256) void k_visual_density(int n, int nin, const in
             // Node.cpp:855-860
             double r = ldexp(R, -(int)level[a]);
             double vol = r * r * r;
-            double m = nmass[a];
+            double m = tree[core::node_place(a, parent[a], cstart, rank)].mass;
             if (vol != 0.0 && m != 0.0) {
                 double d = m / vol;
                 if (d != 0.0 && d != INFINITY) out = d;
@@ -63,7 +65,7 @@ void visual_density(Ctx &c, double rvd, double *vd) {
     int n = (int)c.n;
     if (n < 1) return;
     hipLaunchKernelGGL(k_visual_density, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n, c.nin, c.base, c.cnt,
-                       c.n_parent, c.n_level, c.n_mass, c.ds, rvd, vd);
+                       c.n_parent, c.n_level, c.n_cstart, c.n_rank, c.tnode, c.ds, rvd, vd);
     AG2_HIP(hipGetLastError());
 }
 
