@@ -106,6 +106,7 @@ struct WalkArgs {
 // most 5.3e-8 and 4.5e-8 relative error over 1e-60 .. 1e60, measured on
 // gfx950) and one Newton step, which leaves at most 4.2e-15 and 2.2e-15 --
 // four orders of magnitude inside the 1e-10 parity bound of the force sums.
+// (A force takes the root alone, 4.2e-15, where it took both, 6.4e-15.)
 __device__ inline double rsq64(double x) {
     double y = __builtin_amdgcn_rsq(x);
     double hx = 0.5 * x;
@@ -344,8 +345,8 @@ __device__ inline bool list_overflowed(const WalkArgs &a, int cnt) {
 // The walk is bound by VALU issue (76 % of the SIMDs' cycles): with the two
 // queues, the SPH margin tested in the sweep and two entries in flight per
 // lane it issues 22.6 k vector instructions per wave where one masked sweep
-// issued 28.4 k (1 M disk, FP32), and the kernel takes 0.76 ms against
-// 1.00 ms; the FP64 form 1.24 ms against 1.90 ms.
+// issued 28.4 k (1 M disk, FP32), and the kernel takes 0.71 ms against
+// 1.00 ms; the FP64 form 0.99 ms against 1.90 ms.
 template <bool F32, int KIND, int TPG>
 __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *lds) {
     static_assert(TPG == 64 || TPG == 16 || TPG == 8, "targets per group");
@@ -892,22 +893,69 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                     return;
                                 }
                                 double gx, gy, gz;
-                                bool ok = true;
-                                if (a.wp.soft_live) {
-                                    ok = r2 != 0.0 && core::soft_force(e.w, dx, dy, dz, sqrt(r2), a.wp, &gx, &gy, &gz);
-                                } else {
-                                    // r2 == 0 gives NaN here and is skipped like any NaN
-                                    const double ri = rsq64(r2);
-                                    const double rr = r2 * ri;
-                                    const double f = e.w * rcp64(rr * rr + e02) * ri;
-                                    gx = f * dx; gy = f * dy; gz = f * dz;
-                                    ok = !__builtin_isunordered(gx, gy) && gz == gz;
-                                }
-                                ok = ok && on;
+                                const bool ok = on && r2 != 0.0 &&
+                                                core::soft_force(e.w, dx, dy, dz, sqrt(r2), a.wp, &gx, &gy, &gz);
                                 if (ok) { s.ax += gx; s.ay += gy; s.az += gz; lnint++; }
                                 if (decltype(spotting)::value) hit[h] |= ok && r2 < lim64 ? 1u << j : 0u;
                             };
-                            bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
+                            if (KIND == 4 || a.wp.soft_live) {
+                                bit_pairs(word[h], [&](int j1, int j2, bool both) { one(j1, true); one(j2, both); });
+                                continue;
+                            }
+                            // Two entries side by side, with nothing between
+                            // them but the rare case: f = m / ((r^2 + e^2) r) as
+                            // one reciprocal root of r^2 (r^2 + e^2)^2.  (A root
+                            // and a quotient took half as many instructions
+                            // again: the 1 M disk's walk 1,192 us, now 991; one
+                            // entry at a time, with the rare case between
+                            // two, 1,236.)
+                            auto two = [&](int j1, int j2, bool both) {
+                                const double4 e1 = ds4[32 * (half0 + h) + j1], e2 = ds4[32 * (half0 + h) + j2];
+                                double dx1 = e1.x - px, dy1 = e1.y - py, dz1 = e1.z - pz;
+                                double dx2 = e2.x - px, dy2 = e2.y - py, dz2 = e2.z - pz;
+                                const double q1 = __builtin_fma(dx1, dx1, __builtin_fma(dy1, dy1, dz1 * dz1));
+                                const double q2 = __builtin_fma(dx2, dx2, __builtin_fma(dy2, dy2, dz2 * dz2));
+                                const double s1 = q1 + e02, s2 = q2 + e02;
+                                const double x1 = (q1 * s1) * s1, x2 = (q2 * s2) * s2;
+                                double f1 = e1.w * rsq64(x1), f2 = e2.w * rsq64(x2);
+                                bool ok1 = x1 > 0x1p-900 && fabs(f1) < 0x1p1000;
+                                bool ok2 = x2 > 0x1p-900 && fabs(f2) < 0x1p1000;
+                                if (__any(!(ok1 && ok2))) {
+                                    // coincident, NaN, or far outside the scales
+                                    // of a simulation: r2 == 0 gives NaN and is
+                                    // skipped like any NaN
+                                    auto rare = [&](double m, double r2, double &dx, double &dy, double &dz, double &f,
+                                                    bool &ok) {
+                                        if (ok) return;
+                                        const double ri = rsq64(r2), rr = r2 * ri;
+                                        f = m * rcp64(rr * rr + e02) * ri;
+                                        ok = !__builtin_isunordered(f * dx, f * dy) && f * dz == f * dz;
+                                        if (!ok) f = dx = dy = dz = 0.0;
+                                    };
+                                    rare(e1.w, q1, dx1, dy1, dz1, f1, ok1);
+                                    rare(e2.w, q2, dx2, dy2, dz2, f2, ok2);
+                                }
+                                ok2 = ok2 && both;
+                                f2 = both ? f2 : 0.0;
+                                s.ax = __builtin_fma(f2, dx2, __builtin_fma(f1, dx1, s.ax));
+                                s.ay = __builtin_fma(f2, dy2, __builtin_fma(f1, dy1, s.ay));
+                                s.az = __builtin_fma(f2, dz2, __builtin_fma(f1, dz1, s.az));
+                                lnint += (ok1 ? 1u : 0u) + (ok2 ? 1u : 0u);
+                                if (decltype(spotting)::value) {
+                                    hit[h] |= ok1 && q1 < lim64 ? 1u << j1 : 0u;
+                                    hit[h] |= ok2 && q2 < lim64 ? 1u << j2 : 0u;
+                                }
+                            };
+                            // (in groups of 64; with fewer targets the loop's
+                            // registers spill)
+                            if (TPG < 64 || part) {
+                                bit_pairs(word[h], two);
+                            } else if (mine) {
+                                int j = 0;
+                                const int je = cnt - 32 * h < 32 ? cnt - 32 * h : 32;
+                                for (; j + 2 <= je; j += 2) two(j, j + 1, true);
+                                if (j < je) two(j, j, false);
+                            }
                         }
                     };
                     if (!part && !mine) word[0] = word[kHalves - 1] = 0u;
@@ -1099,14 +1147,17 @@ __device__ inline int wave_group() {
 // targets give eight or four times the waves, each with a smaller box (fewer
 // nodes) and its sweep split over the 64 / TPG lanes of a target; the whole
 // walk does more traversal work (2.1 and 1.3 times the node tests per lane of
-// a SIMD), which costs once the SIMDs have waves to overlap.  Walk kernel,
-// microseconds, 8 / 16 / 64 targets: Plummer 10,000 FP32 39 / 51 / 130, FP64
-// 44 / 64 / 184; disk 33,333 FP32 89 / 84 / 170; disk 100,003 FP32 180 / 157 /
-// 226, FP64 - / 193 / 305; disk 200,000 FP32 - / 256 / 243, FP64 - / 330 /
-// 366; disk 1 M FP32 - / 1014 / 759, FP64 - / 1340 / 1239.  The choice
-// depends on the set alone, so a job of a batched walk has the arithmetic of
-// a walk of its own.
-constexpr int kTpg8Max = 24576, kTpg16Max32 = 150000, kTpg16Max64 = 280000;
+// a SIMD), which costs once the SIMDs have waves to overlap: groups of 8 up to
+// the 4,096 waves the chip holds at once.  Walk kernel, microseconds, groups
+// of 8 / 16 / 64: Plummer 10,000 FP32 39 / 51 / 130; 24,576 FP32 54 / 64 / -;
+// 32,768 FP32 57 / 62 / -, FP64 60 / 68 / -; 33,333 FP64 69 / 69 / -; disk
+// 28,000 FP32 67 / 79 / -; 32,768 FP32 75 / 84 / -, FP64 76 / 86 / -; 100,000
+// FP64 - / 167 / 254; 150,000 FP32 - / 180 / 229; 200,000 FP32 - / 228 / 248,
+// FP64 - / 273 / 307; 400,000 FP64 - / 495 / 503; 450,000 FP64 - / 552 / 542;
+// 1 M FP32 - / 1014 / 710, FP64 - / 1147 / 991.  The choice depends on the
+// set alone, so a job of a batched walk has the arithmetic of a walk of its
+// own.
+constexpr int kTpg8Max = 32768, kTpg16Max32 = 200000, kTpg16Max64 = 400000;
 inline int walk_tpg(int64_t n, bool f32) {
     return n <= kTpg8Max ? 8 : n <= (f32 ? kTpg16Max32 : kTpg16Max64) ? 16 : 64;
 }

@@ -56,7 +56,7 @@ def test_gas_free_sphere(ag2, orc, precision):
     check(ag2, orc, ag2.ics.config1_plummer(3001, seed=5), 0.4, precision)
 
 
-@pytest.mark.parametrize("n,precision", [(24576, 0), (24577, 1), (150000, 1), (150001, 1), (280000, 0), (280001, 0)])
+@pytest.mark.parametrize("n,precision", [(32768, 0), (32769, 1), (200000, 1), (200001, 1), (400000, 0), (400001, 0)])
 def test_group_size_limits(ag2, orc, n, precision):
     """Either side of the particle counts where the walk's groups change size
     (8, 16, 64 targets)."""
@@ -64,7 +64,7 @@ def test_group_size_limits(ag2, orc, n, precision):
     check(ag2, orc, ag2.ics.disk_galaxy(nh, nd, n - nh - nd, seed=2), 0.5, precision)
 
 
-@pytest.mark.parametrize("n", [3000, 25000, 280001])
+@pytest.mark.parametrize("n", [3000, 33000, 400001])
 def test_potential_in_every_group_size(ag2, n):
     """The tree potential with every node opened is the direct sum's: 0.5 sum
     m phi, all terms of one sign, so both are within n 2^-53 of it (each target
@@ -91,3 +91,29 @@ def test_long_sph_lists(ag2, orc, n, precision):
     assert da["sph_overflow"] > 0
     for f in ("ax", "ay", "az", "dUdt"):
         assert np.array_equal(getattr(a, f), getattr(b, f)), f
+
+
+@pytest.mark.parametrize("n,power", [(500, 0), (500, 300), (500, -330), (40000, -330)])
+def test_fp64_forces_at_any_scale(ag2, orc, n, power):
+    """Radii near 2^66, 2^366 (r^2 (r^2 + e^2)^2 of the one-root form
+    overflows) and 2^-264 metres (the softening branch is live), with a
+    coincident pair."""
+    E, U = ag2.engine, ag2.units
+    ps = ag2.ics.plummer(n, 1e10, 1.0, 20.0, seed=n)
+    s = 2.0 ** power
+    for a in (ps.x, ps.y, ps.z):
+        a *= s
+    ps.x[1], ps.y[1], ps.z[1] = ps.x[0], ps.y[0], ps.z[0]   # one coincident pair
+    e0 = 0.1 * U.KPC * s
+    with E.Engine(E.make_params(theta=0.5, e0=e0, split_threshold=100), n) as eng:
+        eng.upload(ps)
+        eng.init_forces()
+        got = eng.download(ps.copy())
+        d = eng.diagnostics()
+    want = ps.copy()
+    st = orc.force_step(want, orc.params(0.5, e0, 1.0, 100))
+    assert d["interactions"] == st["interactions"]
+    unit = max(np.abs(getattr(want, f)).max() for f in ("ax", "ay", "az"))
+    assert 0 < unit < np.inf
+    err = vec_rel_err(*[getattr(p, f) / unit for p in (got, want) for f in ("ax", "ay", "az")])
+    assert err.max() < 1e-10
