@@ -282,7 +282,9 @@ constexpr int kMsThreads = 1024;
 constexpr int kMsWaves = kMsThreads / 64;
 // Sort phase in microseconds (first build after an upload, in caller order;
 // later builds are 1-5 us below), radix passes / merge with tiles of 2048 /
-// of 4096 / sample sort:
+// of 4096 / sample sort (merge with tiles of 1024: 10,000 30, 15,000 30 for
+// 36, 20,000 40 for 37 -- past the 16 tiles a key's four lanes take in one
+// round):
 //    10,000   69 / 33 / 36 / 51        100,003   89 / 142 / 95 / 58
 //    20,000   73 / 36 / 43 / 51        200,000   94 / 467 / 273 / 69
 //    33,333   86 / 42 / 46 / 52        520,000  112 / - / - / 84
@@ -290,7 +292,8 @@ constexpr int kMsWaves = kMsThreads / 64;
 //    65,000   87 / 66 / 55 / 53      1,500,000  178 / - / - / 185
 // The merge's searches grow with the tiles' number for every key; the sample
 // sort runs out of CUs above 256 tiles (a workgroup's sort fills one).
-constexpr int kMsSmall = 40000, kMsMax = 60000;       // merge: up to here kMsTile0, kMsTile1
+constexpr int kMsTiny = 16384, kMsSmall = 40000, kMsMax = 60000;   // merge: up to here kMsTiny0, kMsTile0, kMsTile1
+constexpr int kMsTiny0 = 1024;
 constexpr int kMsTile0 = 2048, kMsTile1 = 4096;
 constexpr int kBsMax = 256 * kMsTile1;                // sample sort up to here, radix passes above
 constexpr int kBsTiles = kBsMax / kMsTile0;           // most tiles of a set (a thread each)
@@ -2013,6 +2016,14 @@ static void radix_pairs(Ctx &c, int n, uint64_t *kin, uint64_t *kout, uint32_t *
     }
 }
 
+template <int TILE>
+static void merge_sort(Ctx &c, int n) {
+    hipLaunchKernelGGL(k_ms_tile<TILE>, dim3(grid_for(n, TILE)), dim3(kMsThreads), 0, c.stream, n, c.key, c.idx,
+                       c.key_alt, c.idx_alt, c.sort_lo, (uint64_t *)nullptr, 0);
+    hipLaunchKernelGGL(k_ms_merge<TILE>, dim3(grid_for(n, kMsPer)), dim3(256), 0, c.stream, n, c.key_alt, c.idx_alt,
+                       c.key, c.idx, c.sort_lo);
+}
+
 template <int TILE, int ITEMS>
 static void sample_sort(Ctx &c, int n, int step) {
     // samples and splitters in key2, which is written after the sort
@@ -2030,16 +2041,9 @@ static void radix_sort(Ctx &c, int n) {
     uint64_t *kin = c.key, *kout = c.key_alt;
     uint32_t *vin = c.idx, *vout = c.idx_alt;
     if (n <= kMsMax) {
-        const dim3 gt(grid_for(n, n <= kMsSmall ? kMsTile0 : kMsTile1)), gm(grid_for(n, kMsPer));
-        if (n <= kMsSmall) {
-            hipLaunchKernelGGL(k_ms_tile<kMsTile0>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo,
-                               (uint64_t *)nullptr, 0);
-            hipLaunchKernelGGL(k_ms_merge<kMsTile0>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
-        } else {
-            hipLaunchKernelGGL(k_ms_tile<kMsTile1>, gt, dim3(kMsThreads), 0, c.stream, n, kin, vin, kout, vout, c.sort_lo,
-                               (uint64_t *)nullptr, 0);
-            hipLaunchKernelGGL(k_ms_merge<kMsTile1>, gm, dim3(256), 0, c.stream, n, kout, vout, kin, vin, c.sort_lo);
-        }
+        if (n <= kMsTiny) merge_sort<kMsTiny0>(c, n);
+        else if (n <= kMsSmall) merge_sort<kMsTile0>(c, n);
+        else merge_sort<kMsTile1>(c, n);
         return;
     }
     if (n <= kBsMax) {
@@ -2165,6 +2169,12 @@ void build_tree_a(Ctx &c) {
 
 size_t sort_job_bytes() { return sizeof(SortJob); }
 
+template <int TILE>
+static void merge_batch(int tiles, const SortJob *dj, int nc, int lo, hipStream_t st) {
+    hipLaunchKernelGGL(k_msb_tile<TILE>, dim3(tiles), dim3(kMsThreads), 0, st, dj, nc, lo, 0);
+    hipLaunchKernelGGL(k_msb_merge<TILE>, dim3((unsigned)(tiles * (TILE / kMsPer))), dim3(256), 0, st, dj, nc, lo);
+}
+
 void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void *scratch_host) {
     if (nc <= 0) return;
     SortJob *hj = (SortJob *)scratch_host;
@@ -2176,7 +2186,10 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
         lo = cs[k]->sort_lo < lo ? cs[k]->sort_lo : lo;
         most = cs[k]->n > most ? cs[k]->n : most;
     }
-    const int tile = most > kBsMax ? kSortTile : most > kMsMax || most <= kMsSmall ? kMsTile0 : kMsTile1;
+    const int tile = most > kBsMax                         ? kSortTile
+                     : most <= kMsTiny                     ? kMsTiny0
+                     : most > kMsMax || most <= kMsSmall ? kMsTile0
+                                                           : kMsTile1;
     int total = 0;
     for (int k = 0; k < nc; k++) {
         Ctx &c = *cs[k];
@@ -2189,14 +2202,9 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
     SortJob *dj = (SortJob *)scratch_dev;
     AG2_HIP(hipMemcpyAsync(dj, hj, sizeof(SortJob) * (size_t)nc, hipMemcpyHostToDevice, st));
     if (most <= kMsMax) {
-        const dim3 gm((unsigned)(total * (tile / kMsPer)));
-        if (tile == kMsTile0) {
-            hipLaunchKernelGGL(k_msb_tile<kMsTile0>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo, 0);
-            hipLaunchKernelGGL(k_msb_merge<kMsTile0>, gm, dim3(256), 0, st, dj, nc, lo);
-        } else {
-            hipLaunchKernelGGL(k_msb_tile<kMsTile1>, dim3(total), dim3(kMsThreads), 0, st, dj, nc, lo, 0);
-            hipLaunchKernelGGL(k_msb_merge<kMsTile1>, gm, dim3(256), 0, st, dj, nc, lo);
-        }
+        if (tile == kMsTiny0) merge_batch<kMsTiny0>(total, dj, nc, lo, st);
+        else if (tile == kMsTile0) merge_batch<kMsTile0>(total, dj, nc, lo, st);
+        else merge_batch<kMsTile1>(total, dj, nc, lo, st);
         AG2_HIP(hipGetLastError());
         return;
     }

@@ -53,9 +53,10 @@ def test_order(ag2, n):
             check_order(ag2, eng, n)
 
 
-@pytest.mark.parametrize("n", [59999, 60000, 60001, 262144, 262145, 524288, 524289, 1048576, 1048577])
-def test_order_sample_sort(ag2, n):
-    """Either side of the sample sort's range and of its steps."""
+@pytest.mark.parametrize("n", [1024, 1025, 16384, 16385, 59999, 60000, 60001, 262144, 262145, 524288, 524289, 1048576, 1048577])
+def test_order_at_limits(ag2, n):
+    """Either side of the merge sort's tiles, the sample sort's range and its
+    steps."""
     E = ag2.engine
     ps = ag2.ics.shuffled(ag2.ics.hernquist(n, seed=n), n)
     with E.Engine(E.make_params(theta=0.7, e0=0.05 * ag2.units.KPC, split_threshold=800), n) as eng:
