@@ -1320,7 +1320,6 @@ __device__ inline void leaf_fold(int nb, const int32_t *part, DevState *ds) {
 constexpr int kSumSmall = 32;
 constexpr int kBlk1 = 64;
 constexpr int kBlk2 = 4096;
-constexpr int kStage = 256 + kSumSmall;   // particles a workgroup of 256 nodes stages
 
 struct PVals {
     const double *sx, *sy, *sz, *sm, *svx, *svy, *svz;
@@ -1528,15 +1527,18 @@ __device__ inline void load_piece(double (&f)[8], const Cover &c, int k, const P
 // counts the particles outside its cube, Node.cpp:477-499), centre of mass,
 // gas-weighted velocity, and the walk record at the node's layout place.
 //
-// 256 nodes per workgroup, in XCD ranges (neighbours in pre-order share
+// PER nodes per workgroup, in XCD ranges (neighbours in pre-order share
 // particles and blocks).  The particles of the workgroup's small nodes and
 // leaves are staged in LDS once; the internal nodes are listed as small (up
 // to kSumTiny particles, or more) and wide, so that the lanes of a wave loop
 // over nodes of like size and the four waves share the wide ones; the sums
 // pass to the nodes' own threads through LDS.  At 1,000,000 particles this is
-// bound by memory (the node arrays and records, 230 bytes a node): sums and
+// bound by memory (the node arrays and records, 150 to 210 bytes a node): sums and
 // moments as two kernels, every node's lane looping over its own particles,
-// took 65 + 110 us (17 + 5 us at 10,000), this one 107 (11).
+// took 65 + 110 us (17 + 5 us at 10,000), this one 91.
+// A small tree takes 64 nodes per workgroup, whose wide nodes four waves then
+// share: 14,800 nodes 9.2 us against 10.9 with 256, 48,000 11.1 against 12.0;
+// 148,000 21.0 against 18.8, 1.48 M 119 against 92.
 //
 // Zero masses (zm, set when any particle has m == 0): the serial insert's
 // running centre of mass (Node.cpp:692-697) divides by the node's mass after
@@ -1545,7 +1547,9 @@ __device__ inline void load_piece(double (&f)[8], const Cover &c, int k, const P
 // is 0/0 and the node's centre stays NaN for good.  Such a node is never
 // accepted (radius / NaN < theta is false), so the walk opens it.
 constexpr int kSumTiny = 8;
+constexpr int kMomentsSpread = 65536;   // up to this many nodes, 64 per workgroup
 
+template <int PER>
 __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, int proot, int64_t thr, int zm,
                                                       const uint32_t *rid, DevState *ds,
                                                       const int32_t *first, const int32_t *count,
@@ -1557,19 +1561,21 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, in
                                                       const int32_t *cstart, double *gas_mass,
                                                       core::TreeNode *tree, core::SphNode *tsph,
                                                       int32_t *group_first, uint8_t *group_fired) {
+    constexpr int kStage = PER + kSumSmall;   // particles staged
     __shared__ double st_m[kStage], st_x[kStage], st_y[kStage], st_z[kStage];
     __shared__ double st_vx[kStage], st_vy[kStage], st_vz[kStage];
     __shared__ uint8_t st_g[kStage];
-    __shared__ double sum[8][256];
-    __shared__ int l_first[256], l_count[256];
-    __shared__ uint8_t list[3][256];   // tiny, small and wide nodes of this workgroup
+    __shared__ double sum[8][PER];
+    __shared__ int l_first[PER], l_count[PER];
+    __shared__ uint8_t list[3][PER];   // tiny, small and wide nodes of this workgroup
     __shared__ int part[3][4];
-    const int nd0 = xcd_block(blockIdx.x, gridDim.x) * 256;
-    const int last = nd0 + 255 < nn ? nd0 + 255 : nn - 1;
+    const int nd0 = xcd_block(blockIdx.x, gridDim.x) * PER;
+    const int last = nd0 + PER - 1 < nn ? nd0 + PER - 1 : nn - 1;
     const int lane = lane_id(), wv = threadIdx.x >> 6;
-    const int nd = nd0 + (int)threadIdx.x;
+    // PER < 256: the threads past PER own no node, and help with the sums
+    const int nd = (int)threadIdx.x < PER ? nd0 + (int)threadIdx.x : nn;
     // every particle between the first particles of two nodes has its leaf
-    // between them in pre-order, so the span is at most 255 + kSumSmall
+    // between them in pre-order, so the span is at most PER - 1 + kSumSmall
     const int P0 = first[nd0];
     int P1 = first[last] + kSumSmall;
     P1 = P1 < nin ? P1 : nin;
@@ -1591,8 +1597,10 @@ __global__ __launch_bounds__(256) void k_node_moments(int nn, int nin, int n, in
     const bool tiny = inner && !wide && cn <= kSumTiny;
     const unsigned long long bal[3] = {__ballot(tiny), __ballot(inner && !wide && !tiny), __ballot(wide)};
     if (lane < 3) part[lane][wv] = __popcll(lane == 0 ? bal[0] : lane == 1 ? bal[1] : bal[2]);
-    l_first[threadIdx.x] = s;
-    l_count[threadIdx.x] = cn;
+    if ((int)threadIdx.x < PER) {
+        l_first[threadIdx.x] = s;
+        l_count[threadIdx.x] = cn;
+    }
     __syncthreads();
     int len[3];
 #pragma unroll
@@ -2423,12 +2431,17 @@ void build_tree_b(Ctx &c) {
         tile_sum_buffers(c, &blk1, &blk2);
         hipLaunchKernelGGL(k_iscan_apply, dim3(nbn), dim3(256), 0, st, nn, c.n_nchild, c.n_bsum, c.n_cstart,
                            (nin + kLevTile - 1) / kLevTile, c.leaf_part, c.ds);
-        hipLaunchKernelGGL(k_node_moments, dim3(gn), dim3(256), 0, st, nn, nin, n, proot, c.p.split_threshold,
-                           c.zero_mass > 0 ? 1 : 0, c.rid, c.ds,
-                           c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_level, blk1, blk2, c.gas_table,
-                           c.gas_equal, c.gas_count, pv,
-                           c.n_nchild, c.n_rank, c.n_cstart, c.n_gas, c.tnode,
-                           c.sph_active ? c.tsph : nullptr, c.g_first, c.g_fired);
+        auto moments = [&](auto per) {
+            constexpr int kPer = decltype(per)::value;
+            hipLaunchKernelGGL(k_node_moments<kPer>, dim3(grid_for(nn, kPer)), dim3(256), 0, st, nn, nin, n, proot, c.p.split_threshold,
+                               c.zero_mass > 0 ? 1 : 0, c.rid, c.ds,
+                               c.n_first, c.n_count, c.n_parent, c.n_pidx, c.n_level, blk1, blk2, c.gas_table,
+                               c.gas_equal, c.gas_count, pv,
+                               c.n_nchild, c.n_rank, c.n_cstart, c.n_gas, c.tnode,
+                               c.sph_active ? c.tsph : nullptr, c.g_first, c.g_fired);
+        };
+        if (nn <= kMomentsSpread) moments(std::integral_constant<int, 64>{});
+        else moments(std::integral_constant<int, 256>{});
         c.groups_cleared = true;
         if (deep && nin > 0) {
             // the walk's stack bound comes from the branching depth here
