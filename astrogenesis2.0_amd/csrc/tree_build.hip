@@ -601,9 +601,17 @@ __device__ __forceinline__ void bs_bucket(int n, int step, const uint64_t *__res
     // one tile per thread
     int l = 0, h = 0;
     if (tid < tiles) {
-        h = n - tid * TILE < TILE ? n - tid * TILE : TILE;
-        if (b > 0) l = split_tile<TILE>(kin, n, tid, split[b - 1], shift);
-        if (b < buckets - 1) h = split_tile<TILE>(kin, n, tid, split[b], shift);
+        // both ends searched side by side: a chain of log2(TILE) reads, not two
+        const Splitter sl = split[b > 0 ? b - 1 : 0], sh = split[b < buckets - 1 ? b : 0];
+        const int len = n - tid * TILE < TILE ? n - tid * TILE : TILE;
+        const uint64_t *k = kin + (size_t)tid * TILE;
+        for (int d = TILE; d; d >>= 1) {
+            const uint64_t kl = k[l + d <= len ? l + d - 1 : 0] >> shift, kh = k[h + d <= len ? h + d - 1 : 0] >> shift;
+            l += l + d <= len && before(kl, sl.q, tid < sl.tile) ? d : 0;
+            h += h + d <= len && before(kh, sh.q, tid < sh.tile) ? d : 0;
+        }
+        l = b == 0 ? 0 : tid == sl.tile ? sl.pos : l;
+        h = b == buckets - 1 ? len : tid == sh.tile ? sh.pos : h;
     }
     const int inc = wave_incl_scan(h - l);
     int lsum = l;
@@ -621,16 +629,14 @@ __device__ __forceinline__ void bs_bucket(int n, int step, const uint64_t *__res
     // element i of the bucket: the last tile whose piece starts at or before it
     int top = 1;
     while (top < tiles) top <<= 1;
-    auto source = [&](int i) -> int {
-        int t = 0;
-        for (int d = top >> 1; d; d >>= 1)
-            if (t + d < tiles && off[t + d] <= i) t += d;
-        return from[t] + (i - off[t]);
-    };
+    auto source = [&](int i, int t) -> int { return from[t] + (i - off[t]); };
     if (size > ITEMS * kMsThreads) {
         // larger than the room: every key's place by searches in all tiles
         for (int i = tid; i < size; i += kMsThreads) {
-            const int g = source(i);
+            int t = 0;
+            for (int d = top >> 1; d; d >>= 1)
+                if (t + d < tiles && off[t + d] <= i) t += d;
+            const int g = source(i, t);
             const uint64_t k = kin[g];
             const Splitter me{k >> shift, g / TILE, g % TILE};
             int r = 0;
@@ -644,12 +650,19 @@ __device__ __forceinline__ void bs_bucket(int n, int step, const uint64_t *__res
     const int base = w * (64 * it) + lane;
     uint64_t k[ITEMS];
     uint32_t v[ITEMS];
+    int t[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) t[j] = 0;
+    for (int d = top >> 1; d; d >>= 1)
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++)
+            if (j < it && t[j] + d < tiles && off[t[j] + d] <= base + j * 64) t[j] += d;
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         k[j] = 0ull;
         v[j] = 0u;
         if (j < it && base + j * 64 < size) {
-            const int g = source(base + j * 64);
+            const int g = source(base + j * 64, t[j]);
             k[j] = kin[g];
             v[j] = vin[g];
         }
