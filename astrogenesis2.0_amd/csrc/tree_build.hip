@@ -285,7 +285,7 @@ constexpr int kMsWaves = kMsThreads / 64;
 // of 4096 / sample sort (merge with tiles of 1024: 10,000 30, 15,000 30 for
 // 36, 20,000 40 for 37 -- past the 16 tiles a key's four lanes take in one
 // round):
-//    10,000   69 / 33 / 36 / 51        100,003   89 / 142 / 95 / 58
+//    10,000   69 / 33 / 36 / 51        100,003   89 / 142 / 95 / 56
 //    20,000   73 / 36 / 43 / 51        200,000   94 / 467 / 273 / 69
 //    33,333   86 / 42 / 46 / 52        520,000  112 / - / - / 84
 //    45,000   87 / 52 / 48 / 52      1,000,000  146 / - / - / 108
