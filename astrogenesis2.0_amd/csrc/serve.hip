@@ -14,7 +14,7 @@
 //      admission stream, and steps from the next round.  A pool with no
 //      running job does this first, and its admitted jobs step at once;
 //   2. every resident job: time steps, first kick and drift, tree width and
-//      keys, on its side stream (job k on stream k mod 8); one batched radix
+//      keys, on its side stream (job k on stream k mod 8); one batched
 //      sort of all jobs' keys on the pool stream; then each job's ordering,
 //      state permutation and node count on its side stream;
 //   3. each job's node counts reach the host (an event per job);
@@ -533,7 +533,7 @@ int ag2_pool_step(void *pool, int32_t *n_stepped) {
                 ag2::build_keys(c);
             }
         });
-        // one batched radix sort of every job's keys on the pool stream
+        // one batched sort of every job's keys on the pool stream
         for (int k = 0; k < Pool::kSide; k++) {
             AG2_HIP(hipEventRecord(P->ev_side[k], P->side[k]));
             AG2_HIP(hipStreamWaitEvent(P->stream, P->ev_side[k], 0));

@@ -34,9 +34,11 @@ constexpr int kRing = 8;        // pieces of a large transfer's ring
 // may be off the CPU for milliseconds: below 64 MB the caller alone is as
 // fast (20 MB: 1.1 ms) and never waits (3.8 ms with helpers on a busy host).  A
 // download of 13 MB takes 0.57 ms with three helpers, 0.82 ms without, one of
-// 146 MB 3.5 and 7.8 ms.
+// 146 MB 3.5 and 7.8 ms; but on a busy host the small one may wait as well
+// (ten steps of 100,000 particles with a download 4.2 ms without helpers, 4.0
+// to 7 with), so below 32 MB the caller copies alone there too.
 constexpr int kHelpers = 3;
-constexpr size_t kHelpDown = (size_t)8 << 20, kHelpUp = (size_t)64 << 20;
+constexpr size_t kHelpDown = (size_t)32 << 20, kHelpUp = (size_t)64 << 20;
 constexpr int kMaxDev = 64;
 constexpr int kMaxFields = 20;
 

@@ -1,7 +1,9 @@
-// Octree build on the device: root half-width, 42-level octant keys,
-// LSD radix sort, tie refinement, linear-octree topology and bottom-up
-// moments.  Replaces Tree::buildTree / Node::insert (Tree.cpp:24-55,
-// Node.cpp:405-699).  All passes are HBM-bound integer/FP64 streaming work.
+// Octree build on the device: root half-width, octant keys, a key sort chosen
+// by size (merge, sample or LSD radix), tie refinement, linear-octree topology
+// from the levels that neighbouring keys share, node sums over each node's own
+// particle range.  Replaces Tree::buildTree / Node::insert (Tree.cpp:24-55,
+// Node.cpp:405-699).  Integer and FP64 streaming work: bound by HBM in the
+// millions, by launches and chains of dependent reads below.
 #include "ag2_internal.h"
 
 namespace ag2 {

@@ -213,6 +213,8 @@ struct NodeOut {
 };
 
 // Internal node of pair i at level l (L[i-1] < l <= L[i]); returns its parent.
+// (The CPU build's form, by searches over the keys; the device kernels find
+// ends, children and parents from the levels alone.)
 AG2_HD int make_internal(const KeyWords &k, const int8_t *L, const int32_t *base,
                          int i, int l, int nin, int n_nodes, NodeOut o) {
     int lp = lcp_prev(L, i);
@@ -231,7 +233,7 @@ AG2_HD int make_internal(const KeyWords &k, const int8_t *L, const int32_t *base
     return par;
 }
 
-// Leaf node of particle i; returns its parent.
+// Leaf node of particle i; returns its parent (CPU build).
 AG2_HD int make_leaf(const KeyWords &k, const int8_t *L, const int8_t *Lk, const int32_t *base,
                      const int32_t *c, int i, NodeOut o, int *leaf_level) {
     int lp = lcp_prev(L, i), li = L[i];
@@ -444,7 +446,7 @@ AG2_HD uint64_t octant_word(double px, double py, double pz, double R, int w, in
 }
 
 // ------------------------------------------------------------ FP64 walk
-// Node record read by the gravity walk: 64 bytes.
+// Node record of the CPU build's walk: 64 bytes.
 struct alignas(64) WalkNode {
     double cx, cy, cz;   // centre of mass
     double mass;

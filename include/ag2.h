@@ -132,7 +132,7 @@ int ag2_upload(void *ctx, const ag2_particles *host);
 int ag2_download(void *ctx, ag2_particles *host);
 
 /* Tree::buildTree (Tree.cpp:24-55): root half-width (Tree::calcTreeWidth,
- * Tree.cpp:86-117), 42-level Morton keys, LSD radix sort, linear octree and
+ * Tree.cpp:86-117), 42-level Morton keys, a key sort chosen by size, linear octree and
  * bottom-up moments. */
 int ag2_build_tree(void *ctx);
 /* Tree::calcGasDensity (Tree.cpp:119-150, Node.cpp:722-796). */
