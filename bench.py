@@ -644,8 +644,8 @@ def profiled_traffic(kernel, form):
 # out: its averages are dominated by the first build after upload, which
 # gathers from caller order, and the two summaries hold different numbers
 # of such builds).
-HBM_KERNELS = ("k_node_moments", "k_sums_direct", "k_tile_sums", "k_make_leaf", "k_make_internal", "k_keygen",
-               "k_rs_scatter", "k_kick_drift", "k_kick2", "k_sph_pairs", "k_group_rho")
+HBM_KERNELS = ("k_node_moments", "k_tile_sums", "k_make_leaf", "k_make_internal", "k_keygen", "k_ms_tile",
+               "k_bs_bucket", "k_kick_drift", "k_kick2", "k_sph_pairs", "k_group_rho")
 HBM_PEAK_GBS = 8000.0
 
 
