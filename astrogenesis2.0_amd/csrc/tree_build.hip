@@ -291,14 +291,19 @@ constexpr int kMsWaves = kMsThreads / 64;
 //    20,000   73 / 36 / 43 / 51        200,000   94 / 467 / 273 / 69
 //    33,333   86 / 42 / 46 / 52        520,000  112 / - / - / 84
 //    45,000   87 / 52 / 48 / 52      1,000,000  146 / - / - / 108
-//    65,000   87 / 66 / 55 / 53      1,500,000  178 / - / - / 185
+//    65,000   87 / 66 / 55 / 53      1,500,000  181 / - / - / 182
+//                                    2,000,000  217 / - / - / 211
+//                                    3,000,000  288 / - / - / 366
 // The merge's searches grow with the tiles' number for every key; the sample
-// sort runs out of CUs above 256 tiles (a workgroup's sort fills one).
+// sort fills a CU with each workgroup, and past two rounds of 256 tiles the
+// ranks of the samples cost too (later builds: 1,500,000 178 against 167,
+// 2,000,000 216 against 190, 3,000,000 287 against 317).
 constexpr int kMsTiny = 16384, kMsSmall = 40000, kMsMax = 60000;   // merge: up to here kMsTiny0, kMsTile0, kMsTile1
 constexpr int kMsTiny0 = 1024;
 constexpr int kMsTile0 = 2048, kMsTile1 = 4096;
-constexpr int kBsMax = 256 * kMsTile1;                // sample sort up to here, radix passes above
-constexpr int kBsTiles = kBsMax / kMsTile0;           // most tiles of a set (a thread each)
+constexpr int kBsTiles = 512;                         // most tiles of a set (a thread each)
+constexpr int kBsMax = kBsTiles * kMsTile1;           // sample sort up to here, radix passes above
+constexpr int kBsBatchMax = kBsTiles * kMsTile0;      // ... in a batch, whose tiles are the smaller ones
 
 // The first sample of a tile: its number's bits reversed, within the step.
 __device__ inline int sample_phase(int tile, int step) {
@@ -2209,7 +2214,7 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
         lo = cs[k]->sort_lo < lo ? cs[k]->sort_lo : lo;
         most = cs[k]->n > most ? cs[k]->n : most;
     }
-    const int tile = most > kBsMax                         ? kSortTile
+    const int tile = most > kBsBatchMax                         ? kSortTile
                      : most <= kMsTiny                     ? kMsTiny0
                      : most > kMsMax || most <= kMsSmall ? kMsTile0
                                                            : kMsTile1;
@@ -2231,7 +2236,7 @@ void sort_batch(Ctx *const *cs, int nc, hipStream_t st, void *scratch_dev, void 
         AG2_HIP(hipGetLastError());
         return;
     }
-    if (most <= kBsMax) {
+    if (most <= kBsBatchMax) {
         const dim3 g(total), b(kMsThreads);
         hipLaunchKernelGGL(k_msb_tile<kMsTile0>, g, b, 0, st, dj, nc, lo, kMsTile0 / kBsPer);
         hipLaunchKernelGGL(k_bsb_split<kMsTile0>, g, b, 0, st, dj, nc);

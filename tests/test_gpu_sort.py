@@ -53,7 +53,7 @@ def test_order(ag2, n):
             check_order(ag2, eng, n)
 
 
-@pytest.mark.parametrize("n", [1024, 1025, 16384, 16385, 59999, 60000, 60001, 262144, 262145, 524288, 524289, 1048576, 1048577])
+@pytest.mark.parametrize("n", [1024, 1025, 16384, 16385, 59999, 60000, 60001, 262144, 262145, 524288, 524289, 1048576, 1048577, 2097152, 2097153])
 def test_order_at_limits(ag2, n):
     """Either side of the merge sort's tiles, the sample sort's range and its
     steps."""
