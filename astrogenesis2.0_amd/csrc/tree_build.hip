@@ -928,20 +928,32 @@ struct StateSet {
 // out, for a build whose force phase writes every one of them.  zero_gas_h:
 // field kHField (h) becomes 0 for gas, for a build whose density phase
 // follows (it starts so, Tree.cpp:121-130).
+// PARTS: the fields shared by so many workgroups of the grid's second
+// dimension.  Up to 131,072 particles the chip is not full and a thread's
+// nineteen gathers are what it waits for: five parts of four fields take 4.8
+// us against 7.7 at 10,000, 5.7 against 8.4 at 33,333, 6.5 against 8.3 at
+// 100,000; 10.1 against 10.3 at 150,000, 14.3 against 13.8 at 200,000, and
+// more above (1,000,000: 60 against 52).
 constexpr int kAccField = 9;
 constexpr int kHField = 12;
+constexpr int kPermuteParts = 5, kPermuteSplit = 131072;
 
+template <int PARTS>
 __global__ __launch_bounds__(256) void k_permute(int n, const uint32_t *__restrict__ idx, StateSet in, StateSet out,
                                                  int skip_acc, int zero_gas_h) {
     int k = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     if (k >= n) return;
     uint32_t q = idx[k];
     const uint8_t ty = in.type[q];
+    constexpr int kPer = (kStateD + PARTS - 1) / PARTS;
+    const int j0 = PARTS > 1 ? (int)blockIdx.y * kPer : 0;
 #pragma unroll
-    for (int j = 0; j < kStateD; j++) {
-        if (skip_acc && j >= kAccField && j < kAccField + 3) continue;
+    for (int u = 0; u < kPer; u++) {
+        const int j = j0 + u;
+        if (j >= kStateD || (skip_acc && j >= kAccField && j < kAccField + 3)) continue;
         out.d[j][k] = (j == kHField && zero_gas_h && ty == 2) ? 0.0 : in.d[j][q];
     }
+    if (PARTS > 1 && blockIdx.y > 0) return;
     out.type[k] = ty;
     out.active[k] = in.active[q];
     out.rid[k] = in.rid[q];
@@ -2002,8 +2014,12 @@ static void launch_permute(Ctx &c, int n) {
     const int skip_acc = c.acc_overwritten && !c.p.graph_launch ? 1 : 0;
     const int zero_gas_h = c.density_follows && !c.p.graph_launch ? 1 : 0;
     c.h_cleared = zero_gas_h != 0;
-    hipLaunchKernelGGL(k_permute, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n, c.idx_alt, in, out, skip_acc,
-                       zero_gas_h);
+    const unsigned g = grid_for(n, 256);
+    if (n <= kPermuteSplit)
+        hipLaunchKernelGGL(k_permute<kPermuteParts>, dim3(g, kPermuteParts), dim3(256), 0, c.stream, n, c.idx_alt, in,
+                           out, skip_acc, zero_gas_h);
+    else
+        hipLaunchKernelGGL(k_permute<1>, dim3(g), dim3(256), 0, c.stream, n, c.idx_alt, in, out, skip_acc, zero_gas_h);
 }
 
 static void swap_state(Ctx &c) {
