@@ -2085,13 +2085,12 @@ template <int TILE>
 static void merge_sort(Ctx &c, int n) {
     hipLaunchKernelGGL(k_ms_tile<TILE>, dim3(grid_for(n, TILE)), dim3(kMsThreads), 0, c.stream, n, c.key, c.idx,
                        c.key_alt, c.idx_alt, c.sort_lo, (uint64_t *)nullptr, 0);
-    if (TILE == kMsTiny0) {
+    if constexpr (TILE == kMsTiny0)
         hipLaunchKernelGGL(k_ms_merge_lds, dim3(grid_for(n, kMsThreads / kMsLanes)), dim3(kMsThreads), 0, c.stream, n,
                            c.key_alt, c.idx_alt, c.key, c.idx, c.sort_lo);
-        return;
-    }
-    hipLaunchKernelGGL(k_ms_merge<TILE>, dim3(grid_for(n, kMsPer)), dim3(256), 0, c.stream, n, c.key_alt, c.idx_alt,
-                       c.key, c.idx, c.sort_lo);
+    else
+        hipLaunchKernelGGL(k_ms_merge<TILE>, dim3(grid_for(n, kMsPer)), dim3(256), 0, c.stream, n, c.key_alt, c.idx_alt,
+                           c.key, c.idx, c.sort_lo);
 }
 
 template <int TILE, int ITEMS>
