@@ -1133,10 +1133,12 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     }
     double ox, oy, oz;
     if (F32) {
+        // (a full chunk's sweep knows no mask: lanes whose target takes no part,
+        // a massless one among them, have summed what was not theirs)
         const double scale = a.nn > 0 ? a.wp.G * a.tree[0].mass * invL * invL : 0.0;
-        ox = (double)sumx * scale;
-        oy = (double)sumy * scale;
-        oz = (double)sumz * scale;
+        ox = mine ? (double)sumx * scale : 0.0;
+        oy = mine ? (double)sumy * scale : 0.0;
+        oz = mine ? (double)sumz * scale : 0.0;
     } else {
         ox = s.ax; oy = s.ay; oz = s.az;
     }
