@@ -397,7 +397,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
     double near_b2 = 0.0;   // uniform: see the full-queue test
     unsigned lnint = 0u;    // interactions counted per lane
     int nrec = 0;           // uniform: near pairs recorded for k_near_pass
-    bool dfmode = false;    // uniform: this group's partial chunks carry the offsets' remainders
+    bool dfmode = false;    // uniform: this group's chunks carry the offsets' remainders
     float sumx = 0.f, sumy = 0.f, sumz = 0.f, cmpx = 0.f, cmpy = 0.f, cmpz = 0.f;
     const double theta = a.wp.theta, th2 = a.wp.theta * a.wp.theta;
     const double th2lo = th2 * (1.0 - 1e-10), th2hi = th2 * (1.0 + 1e-10);   // group-box accept / open margins
@@ -723,7 +723,8 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                     word[0] = half0 ? thi : tlo;
                     if (kHalves == 2) word[kHalves - 1] = thi;
                 } else {   // a full chunk: every entry of the lane's field
-                    const unsigned long long all = (cnt == 64 ? ~0ull : (1ull << cnt) - 1) & (kAll << (TPG * sub & 63));
+                    unsigned long long all = (cnt == 64 ? ~0ull : (1ull << cnt) - 1) & (kAll << (TPG * sub & 63));
+                    if (!mine) all = 0ull;
                     word[0] = (unsigned)(all >> (32 * half0));
                     if (kHalves == 2) word[kHalves - 1] = (unsigned)(all >> 32);
                 }
@@ -736,17 +737,19 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                 const bool spot = KIND == 1 && candB != 0ull;   // uniform
                 unsigned hit[kHalves] = {};
                 unsigned long long hb = 0ull;
-                const bool dfc = F32 && part && dfmode;
+                const bool dfc = F32 && dfmode;
                 if (KIND == 2) {
                     // no gravity
                 } else if (F32) {
                     // Three sweeps, counted from the masks at staging:
-                    //  - full: every lane interacts (r2 > r2min > 0 for each);
+                    //  - full: every lane interacts (r2 > r2min > 0 for each), under
+                    //    no mask, lanes whose target takes no part included;
                     //  - partial: lanes within r2min of an entry (FP32
                     //    offsets cannot resolve the direction) are left out;
-                    //  - dfmode (a group that has met such lanes): offsets with
-                    //    their FP32 remainders (48 bits; the difference of the
-                    //    high parts is exact for close pairs), down to r2df.
+                    //  - dfmode (a group that has met such lanes, every later
+                    //    chunk): offsets with their FP32 remainders (48 bits; the
+                    //    difference of the high parts is exact for close pairs),
+                    //    down to r2df.
                     // Left-out lanes are found again after the sweep: resolved
                     // with the remainders where they can be, else recorded for
                     // the FP64 pass (and dropped from the count).
@@ -898,7 +901,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                 if (KIND == 1 && in_mask(Z & sphB)) hb |= 1ull << jj;
                             }
                         }
-                        dfmode = true;   // the rest of this group's partial chunks carry the remainders
+                        dfmode = true;   // the rest of this group's chunks carry the remainders
                     }
                     float y = cx - cmpx, tt = sumx + y; cmpx = (tt - sumx) - y; sumx = tt;
                     y = cy - cmpy; tt = sumy + y; cmpy = (tt - sumy) - y; sumy = tt;
@@ -986,7 +989,6 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                             }
                         }
                     };
-                    if (!part && !mine) word[0] = word[kHalves - 1] = 0u;
                     if (spot) sweep(std::integral_constant<bool, KIND == 1>{});
                     else sweep(std::false_type{});
                 }
