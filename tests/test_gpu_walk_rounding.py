@@ -58,6 +58,17 @@ def errors(ag2, ps, e0, precision, sample):
             ((off * want).sum(0) / (size * size)).astype(float))
 
 
+@pytest.mark.parametrize("n", [33333, 150001, 410001])
+def test_fp64_pairs_have_no_bias(ag2, n):
+    """Every step of a pair rounds to nearest: over a thousand targets the
+    errors along the force cancel (half of 2^-53 allowed), and the sums, formed
+    in chunks of at most 64 entries, keep the median error below 2^-52."""
+    ps = ag2.ics.plummer(n, 1e10, 1.0, 20.0, seed=n)
+    err, along = errors(ag2, ps, 0.05 * ag2.units.KPC, ag2.engine.AG2_FP64, 1000)
+    assert abs(np.median(along)) < 2.0 ** -54, np.median(along)
+    assert np.median(err) < 2.0 ** -52, np.median(err)
+
+
 # median relative errors of the same targets with every chunk's entries summed
 # under their masks, about 26 of 64 at a time
 MASKED = {410001: 5.842e-8, 700001: 6.031e-8}
