@@ -9,14 +9,20 @@
 // their coordinates are read through the scalar cache: a source's index is
 // the same for the whole wave, so a pair needs no LDS and no barrier.  The
 // pair's 1/r and 1/(r^2 + e0^2) come from one reciprocal square root of
-// r^2 (r^2 + e0^2)^2 (normal range: r from 1e-48 to 1e51 m), about 21 issue
-// slots with it, and the angle of the potential from fp64_math.h, where the
-// correctly rounded square root and quotient and the library's atan took ten
-// times that.  The parts of a target are added in source order.  1 M sources,
-// 16,384 targets with the potential: 374 ms before, 25.4 ms; 65,536 targets
-// without: 214 ms before, 44 ms.  Against 64-bit array sums: 2.7e-14 before (a
-// million terms one by one), 6.6e-16.
+// r^2 (r^2 + e0^2)^2, about 21 issue slots with it, and the angle of the
+// potential from fp64_math.h, where the correctly rounded square root and
+// quotient and the library's atan took ten times that.  The parts of a target
+// are added in source order.  1 M sources, 16,384 targets with the potential:
+// 374 ms before, 25.4 ms; 65,536 targets without: 214 ms before, 44 ms.
+// Against 64-bit array sums: 2.7e-14 before (a million terms one by one),
+// 6.6e-16.
+//
+// The fast pair holds for softening lengths between 2^42 and 2^150 m: there
+// no pair's r^2 (r^2 + e0^2)^2 is too small, and one that is too large makes
+// its part's sums no numbers, which are formed again with every pair checked.
+// Other softening lengths check every pair.
 #include <mutex>
+#include <type_traits>
 
 #include "ag2_internal.h"
 #include "fp64_math.h"
@@ -28,8 +34,9 @@ constexpr int kDirectBlock = 256;
 
 // Targets: lane k of the grid's first dimension; sources [split * per, ...).
 // part: column c of split s at (c * splits + s) * nt, unscaled sums.
-template <bool POT>
-__global__ __launch_bounds__(kDirectBlock) void k_direct(int n, const double *__restrict__ x,
+// ANY: the softening length is outside the fast pair's range.
+template <bool POT, bool ANY>
+__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(int n, const double *__restrict__ x,
                                                          const double *__restrict__ y, const double *__restrict__ z,
                                                          const double *__restrict__ m, int nt,
                                                          const int64_t *__restrict__ targets,
@@ -41,31 +48,61 @@ __global__ __launch_bounds__(kDirectBlock) void k_direct(int n, const double *__
     const int64_t i = valid ? inv[targets[k]] : 0;   // caller index -> resident slot
     const double px = x[i], py = y[i], pz = z[i];
     const double e02 = e0 * e0;
+    // (all of a target's pairs are long ones, where it is far away itself)
+    const bool far = !(fabs(px) < 0x1p150 && fabs(py) < 0x1p150 && fabs(pz) < 0x1p150);
     double gx = 0.0, gy = 0.0, gz = 0.0, ph = 0.0;
     const int j0 = split * per, j1 = n - j0 < per ? n : j0 + per;
-    auto pair = [&](int j) {
+    // checked: whatever the pair's scale
+    auto pair = [&](int j, auto checked) {
+        constexpr bool CHECK = decltype(checked)::value;
         const double dx = x[j] - px, dy = y[j] - py, dz = z[j] - pz;
         // (a pair at r == 0 has d == 0: only its finite factor matters)
         const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
         const double s2 = r2 + e02;
+        const double mj = r2 != 0.0 ? m[j] : 0.0;
+        double f, r = 0.0, ir = 0.0;
+        bool ok = true;
         if (!POT) {
-            const double f = m[j] * rsq_full(__builtin_fma(r2 * s2, s2, 1e-290));
-            gx = __builtin_fma(f, dx, gx);
-            gy = __builtin_fma(f, dy, gy);
-            gz = __builtin_fma(f, dz, gz);
+            f = m[j] * rsq_full(__builtin_fma(r2 * s2, s2, CHECK ? 0.0 : 1e-290));
+            if (CHECK) ok = r2 * s2 * s2 > 0x1p-900 && fabs(f) < 0x1p1000;
         } else {
-            const double ir = rsq_full(fmax(r2, 1e-290));
-            const double mj = r2 != 0.0 ? m[j] : 0.0;
-            const double f = mj * ir * rcp_full(fmax(s2, 1e-290));
-            gx = __builtin_fma(f, dx, gx);
-            gy = __builtin_fma(f, dy, gy);
-            gz = __builtin_fma(f, dz, gz);
-            ph = __builtin_fma(mj, softened_angle(e0, r2 * ir, ir), ph);
+            ir = rsq_full(fmax(r2, 0x1p-1074));
+            r = r2 * ir;
+            f = mj * ir * rcp_full(s2);
+            if (CHECK) ok = r2 > 0x1p-900 && s2 > 0x1p-900 && s2 < 0x1p300 && fabs(f) < 0x1p1000;
         }
+        double ux = dx, uy = dy, uz = dz;
+        if (CHECK && __any(!ok)) {
+            // the direction first: r^3 alone may leave the range
+            const double root = sqrt(r2), inv = r2 != 0.0 ? 1.0 / root : 0.0;
+            r = ok ? r : root;
+            ir = ok ? ir : inv;
+            f = ok ? f : r2 != 0.0 ? mj / s2 : 0.0;
+            ux = ok ? dx : dx * inv;
+            uy = ok ? dy : dy * inv;
+            uz = ok ? dz : dz * inv;
+        }
+        gx = __builtin_fma(f, ux, gx);
+        gy = __builtin_fma(f, uy, gy);
+        gz = __builtin_fma(f, uz, gz);
+        if (POT) ph = __builtin_fma(mj, softened_angle(e0, r, ir), ph);
     };
+    const std::integral_constant<bool, ANY> form;
     int j = j0;
-    for (; j + 4 <= j1; j += 4) { pair(j); pair(j + 1); pair(j + 2); pair(j + 3); }
-    for (; j < j1; j++) pair(j);
+    for (; j + 4 <= j1; j += 4) { pair(j, form); pair(j + 1, form); pair(j + 2, form); pair(j + 3, form); }
+    for (; j < j1; j++) pair(j, form);
+    if (!ANY) {
+        const bool bad = far || gx != gx || gy != gy || gz != gz || ph != ph;
+        if (__any(bad)) {
+            const double ox = gx, oy = gy, oz = gz, op = ph;
+            gx = gy = gz = ph = 0.0;
+            for (int u = j0; u < j1; u++) pair(u, std::true_type{});
+            gx = bad ? gx : ox;
+            gy = bad ? gy : oy;
+            gz = bad ? gz : oz;
+            ph = bad ? ph : op;
+        }
+    }
     if (!valid) return;
     const size_t col = (size_t)gridDim.y * nt;
     double *out = part + (size_t)split * nt + k;
@@ -91,6 +128,7 @@ __global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, const d
 void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, double *scratch, size_t room, double *ax,
                    double *ay, double *az, double *pot) {
     const int n = (int)c.n, cols = with_pot ? 4 : 3;
+    const bool any = !(c.p.e0 >= 0x1p42 && c.p.e0 <= 0x1p150);
     int at = 0;
     while (at < nt) {
         const size_t fit = room / (size_t)cols;
@@ -105,12 +143,12 @@ void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, doubl
         const int per = (int)((n + splits - 1) / splits);
         splits = (n + per - 1) / per;
         const dim3 grid(grid_for(here, kDirectBlock), (unsigned)splits), block(kDirectBlock);
-        if (with_pot)
-            hipLaunchKernelGGL(k_direct<true>, grid, block, 0, c.stream, n, c.x, c.y, c.z, c.m, here, d_targets + at,
-                               c.inv, c.p.e0, per, scratch);
-        else
-            hipLaunchKernelGGL(k_direct<false>, grid, block, 0, c.stream, n, c.x, c.y, c.z, c.m, here, d_targets + at,
-                               c.inv, c.p.e0, per, scratch);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, c.stream, n, c.x, c.y, c.z, c.m, here, d_targets + at, c.inv,
+                               c.p.e0, per, scratch);
+        };
+        if (with_pot) any ? go(k_direct<true, true>) : go(k_direct<true, false>);
+        else any ? go(k_direct<false, true>) : go(k_direct<false, false>);
         hipLaunchKernelGGL(k_direct_fold, dim3(grid_for(here, 256), cols), dim3(256), 0, c.stream, here, (int)splits,
                            scratch, c.p.G, c.p.e0, ax + at, ay + at, az + at, pot ? pot + at : nullptr);
         AG2_HIP(hipGetLastError());
