@@ -11,16 +11,22 @@
 // pair's 1/r and 1/(r^2 + e0^2) come from one reciprocal square root of
 // r^2 (r^2 + e0^2)^2, about 21 issue slots with it, and the angle of the
 // potential from fp64_math.h, where the correctly rounded square root and
-// quotient and the library's atan took ten times that.  The parts of a target
-// are added in source order.  1 M sources, 16,384 targets with the potential:
-// 374 ms before, 25.4 ms; 65,536 targets without: 214 ms before, 44 ms.
-// Against 64-bit array sums: 2.7e-14 before (a million terms one by one),
-// 6.6e-16.
+// quotient and the library's atan took ten times that.
 //
 // The fast pair holds for softening lengths between 2^42 and 2^150 m: there
 // no pair's r^2 (r^2 + e0^2)^2 is too small, and one that is too large makes
-// its part's sums no numbers, which are formed again with every pair checked.
-// Other softening lengths check every pair.
+// its block's sums no numbers, which are formed again with a root and
+// quotients of their own.  Other softening lengths test every pair.
+//
+// A target's sum depends on the sources alone, bit for bit, not on the other
+// targets asked for: sources are summed in blocks of fixed length, blocks
+// sixteen at a time, those in (at most) four parts of the set, and the parts
+// in order, however many of these one wave sums (SumPlan).
+//
+// 1 M sources, 16,384 targets: with the potential 372 ms one workgroup per 256
+// targets, now 26.1; without 212, now 10.5; 300 targets 1.5 and 0.85 ms.
+// Against sums in extended precision 2.9e-14 then (a million terms one by one;
+// the potential 4.2e-14), now 1.5e-16.
 #include <mutex>
 #include <type_traits>
 
@@ -31,16 +37,24 @@ namespace ag2 {
 namespace {
 
 constexpr int kDirectBlock = 256;
+constexpr int kMid = 16;   // blocks of sources summed at a time
 
-// Targets: lane k of the grid's first dimension; sources [split * per, ...).
-// part: column c of split s at (c * splits + s) * nt, unscaled sums.
+// The order of a target's sum over n sources: blocks of `len` sources, kMid
+// blocks at a time, `top` of those at a time, all of them.  A wave sums `per`
+// blocks (1, kMid or kMid top): its part of the sum.
+struct SumPlan {
+    int n, len, blocks, top, per;
+};
+
+// Targets: lane k of the grid's first dimension; blocks of sources [split *
+// per, ...).  part: column c of split s at (c * splits + s) * nt, unscaled sums.
 // ANY: the softening length is outside the fast pair's range.
 template <bool POT, bool ANY>
-__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(int n, const double *__restrict__ x,
+__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(SumPlan p, const double *__restrict__ x,
                                                          const double *__restrict__ y, const double *__restrict__ z,
                                                          const double *__restrict__ m, int nt,
                                                          const int64_t *__restrict__ targets,
-                                                         const int32_t *__restrict__ inv, double e0, int per,
+                                                         const int32_t *__restrict__ inv, double e0,
                                                          double *__restrict__ part) {
     const int k = blockIdx.x * kDirectBlock + threadIdx.x;
     const int split = blockIdx.y;
@@ -51,7 +65,6 @@ __global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4)
     // (all of a target's pairs are long ones, where it is far away itself)
     const bool far = !(fabs(px) < 0x1p150 && fabs(py) < 0x1p150 && fabs(pz) < 0x1p150);
     double gx = 0.0, gy = 0.0, gz = 0.0, ph = 0.0;
-    const int j0 = split * per, j1 = n - j0 < per ? n : j0 + per;
     // checked: whatever the pair's scale
     auto pair = [&](int j, auto checked) {
         constexpr bool CHECK = decltype(checked)::value;
@@ -88,68 +101,106 @@ __global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4)
         if (POT) ph = __builtin_fma(mj, softened_angle(e0, r, ir), ph);
     };
     const std::integral_constant<bool, ANY> form;
-    int j = j0;
-    for (; j + 4 <= j1; j += 4) { pair(j, form); pair(j + 1, form); pair(j + 2, form); pair(j + 3, form); }
-    for (; j < j1; j++) pair(j, form);
-    if (!ANY) {
-        const bool bad = far || gx != gx || gy != gy || gz != gz || ph != ph;
-        if (__any(bad)) {
-            const double ox = gx, oy = gy, oz = gz, op = ph;
-            gx = gy = gz = ph = 0.0;
-            for (int u = j0; u < j1; u++) pair(u, std::true_type{});
-            gx = bad ? gx : ox;
-            gy = bad ? gy : oy;
-            gz = bad ? gz : oz;
-            ph = bad ? ph : op;
+    double mx = 0.0, my = 0.0, mz = 0.0, mp = 0.0;   // of up to kMid blocks
+    double tx = 0.0, ty = 0.0, tz = 0.0, tp = 0.0;   // of those
+    const int b1 = (split + 1) * p.per < p.blocks ? (split + 1) * p.per : p.blocks;
+    for (int b = split * p.per; b < b1; b++) {
+        const int j0 = b * p.len, j1 = p.n - j0 < p.len ? p.n : j0 + p.len;
+        gx = gy = gz = ph = 0.0;
+        int j = j0;
+        for (; j + 4 <= j1; j += 4) { pair(j, form); pair(j + 1, form); pair(j + 2, form); pair(j + 3, form); }
+        for (; j < j1; j++) pair(j, form);
+        if (!ANY) {
+            const bool bad = far || gx != gx || gy != gy || gz != gz || ph != ph;
+            if (__any(bad)) {
+                const double ox = gx, oy = gy, oz = gz, op = ph;
+                gx = gy = gz = ph = 0.0;
+                for (int u = j0; u < j1; u++) pair(u, std::true_type{});
+                gx = bad ? gx : ox;
+                gy = bad ? gy : oy;
+                gz = bad ? gz : oz;
+                ph = bad ? ph : op;
+            }
+        }
+        mx += gx; my += gy; mz += gz; mp += ph;
+        if ((b + 1) % kMid == 0 || b + 1 == b1) {
+            tx += mx; ty += my; tz += mz; tp += mp;
+            mx = my = mz = mp = 0.0;
         }
     }
     if (!valid) return;
     const size_t col = (size_t)gridDim.y * nt;
     double *out = part + (size_t)split * nt + k;
-    out[0] = gx; out[col] = gy; out[2 * col] = gz;
-    if (POT) out[3 * col] = ph;
+    out[0] = tx; out[col] = ty; out[2 * col] = tz;
+    if (POT) out[3 * col] = tp;
 }
 
-// Column c of the result: its parts in source order, scaled.
-__global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, const double *__restrict__ part, double G,
-                                                     double e0, double *ax, double *ay, double *az, double *pot) {
+// Column c of the result: its parts in the plan's order, scaled.
+__global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, SumPlan p, const double *__restrict__ part,
+                                                     double G, double e0, double *ax, double *ay, double *az,
+                                                     double *pot) {
     const int k = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
     if (k >= nt) return;
-    const double *p = part + (size_t)c * splits * nt + k;
-    double s = 0.0;
-    for (int u = 0; u < splits; u++) s += p[(size_t)u * nt];
+    const double *q = part + (size_t)c * splits * nt + k;
+    double s = 0.0, t = 0.0, mid = 0.0;
+    for (int u0 = 0; u0 < splits; u0 += kMid) {
+        double v[kMid];   // every load before the first sum
+#pragma unroll
+        for (int k = 0; k < kMid; k++) v[k] = u0 + k < splits ? q[(size_t)(u0 + k) * nt] : 0.0;
+#pragma unroll
+        for (int k = 0; k < kMid; k++) {
+            if (u0 + k >= splits) break;
+            const int done = (u0 + k + 1) * p.per;   // blocks so far
+            const bool last = u0 + k + 1 == splits;
+            mid += v[k];
+            if (done % kMid == 0 || last) { t += mid; mid = 0.0; }
+            if (done % (kMid * p.top) == 0 || last) { s += t; t = 0.0; }
+        }
+    }
     double *out = c == 0 ? ax : c == 1 ? ay : c == 2 ? az : pot;
     out[k] = c < 3 ? G * s : -(G / e0) * s;
 }
 
-// Targets [0, nt) in slices whose parts fit `room` doubles of scratch.
-// Splits: enough for about four waves on each SIMD with sources left over
-// (16 * 1024 waves), at least 256 sources each.
+// Blocks of n / 256 sources (a multiple of four, 32 to 256 of them), and at
+// most four parts of the whole.
+SumPlan sum_plan(int n) {
+    SumPlan p;
+    p.n = n;
+    p.len = ((n + 255) / 256 + 3) / 4 * 4;
+    p.len = p.len < 32 ? 32 : p.len > 256 ? 256 : p.len;
+    p.blocks = (n + p.len - 1) / p.len;
+    p.top = ((p.blocks + kMid - 1) / kMid + 3) / 4;
+    p.per = 1;
+    return p;
+}
+
+// Targets [0, nt) in slices whose parts fit `room` doubles of scratch.  A wave
+// takes as many blocks as leave four waves for each of 1,024 SIMDs, or, where
+// the scratch holds no more parts, as have to be.
 void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, double *scratch, size_t room, double *ax,
                    double *ay, double *az, double *pot) {
-    const int n = (int)c.n, cols = with_pot ? 4 : 3;
+    const int cols = with_pot ? 4 : 3;
+    SumPlan p = sum_plan((int)c.n);
+    const int64_t waves = (nt + 63) / 64;
+    const int pers[3] = {kMid * p.top, kMid, 1};
+    auto parts = [&](int per) { return (int64_t)(p.blocks + per - 1) / per; };
+    p.per = pers[0];
+    for (int per : pers)
+        if (per < p.per && waves * parts(p.per) < 4096 && (int64_t)nt * cols * parts(per) <= (int64_t)room) p.per = per;
+    const int splits = (int)parts(p.per);
+    const int64_t fit = (int64_t)room / ((int64_t)cols * splits);
+    if (fit < 1) throw HipError("no scratch for the direct sum");
     const bool any = !(c.p.e0 >= 0x1p42 && c.p.e0 <= 0x1p150);
-    int at = 0;
-    while (at < nt) {
-        const size_t fit = room / (size_t)cols;
-        const int here = (size_t)(nt - at) < fit ? nt - at : (int)fit;
-        if (here < 1) throw HipError("no scratch for the direct sum");
-        const int64_t waves = (here + 63) / 64;
-        int64_t splits = (16384 + waves - 1) / waves;
-        if (splits > (n + 255) / 256) splits = (n + 255) / 256;
-        if (splits > (int64_t)(fit / (size_t)here)) splits = (int64_t)(fit / (size_t)here);
-        if (splits > 65535) splits = 65535;
-        if (splits < 1) splits = 1;
-        const int per = (int)((n + splits - 1) / splits);
-        splits = (n + per - 1) / per;
+    for (int at = 0; at < nt;) {
+        const int here = nt - at < fit ? nt - at : (int)fit;
         const dim3 grid(grid_for(here, kDirectBlock), (unsigned)splits), block(kDirectBlock);
         auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, block, 0, c.stream, n, c.x, c.y, c.z, c.m, here, d_targets + at, c.inv,
-                               c.p.e0, per, scratch);
+            hipLaunchKernelGGL(kernel, grid, block, 0, c.stream, p, c.x, c.y, c.z, c.m, here, d_targets + at, c.inv,
+                               c.p.e0, scratch);
         };
         if (with_pot) any ? go(k_direct<true, true>) : go(k_direct<true, false>);
         else any ? go(k_direct<false, true>) : go(k_direct<false, false>);
-        hipLaunchKernelGGL(k_direct_fold, dim3(grid_for(here, 256), cols), dim3(256), 0, c.stream, here, (int)splits,
+        hipLaunchKernelGGL(k_direct_fold, dim3(grid_for(here, 256), cols), dim3(256), 0, c.stream, here, splits, p,
                            scratch, c.p.G, c.p.e0, ax + at, ay + at, az + at, pot ? pot + at : nullptr);
         AG2_HIP(hipGetLastError());
         at += here;
