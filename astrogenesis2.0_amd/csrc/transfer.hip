@@ -6,23 +6,20 @@
 // from pageable memory goes through the runtime's own staging on one thread
 // (measured here: 7 GB/s into the caller's arrays, against 57 GB/s into
 // pinned memory).  A block of up to one piece (4 MiB) is a single copy.  A
-// larger one goes piece by piece through a ring of pinned slots, and a few
-// host threads move the pieces between the ring and the caller's arrays while
-// the next ones are under way.  Download of eleven fields of 1 M particles:
+// larger one goes piece by piece through a ring of pinned slots (ring.h), and
+// a few host threads move the pieces between the ring and the caller's arrays
+// while the next ones are under way.  Download of eleven fields of 1 M particles:
 // 10-13 ms before, 2.35 ms; the whole state (18 arrays) 9.4-16 ms, 3.5 ms;
 // upload of 150,001 particles 1.1 ms.
 //
 // Pinned buffers are kept for later transfers of any context of the device,
 // a few at most, and freed with the device's last context.
-#include <atomic>
-#include <chrono>
-#include <cstring>
 #include <functional>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "ag2_internal.h"
+#include "ring.h"
 
 namespace ag2 {
 namespace {
@@ -109,107 +106,21 @@ class Lease {
     bool large_;
 };
 
-// The caller's side of a flat block: consecutive runs of bytes.
-struct Run {
-    char *host;
-    size_t bytes;
-};
-
-// Copies [at, at + len) of the block between `buf` and the runs.
-void move_runs(const std::vector<Run> &runs, size_t at, size_t len, char *buf, bool to_runs) {
-    size_t lo = 0;
-    for (const Run &r : runs) {
-        const size_t hi = lo + r.bytes;
-        if (hi > at && lo < at + len) {
-            const size_t a = lo > at ? lo : at, b = hi < at + len ? hi : at + len;
-            if (to_runs) std::memcpy(r.host + (a - lo), buf + (a - at), b - a);
-            else std::memcpy(buf + (a - at), r.host + (a - lo), b - a);
-        }
-        lo = hi;
-        if (lo >= at + len) break;
-    }
-}
-
-// The pieces of a block through the ring.  The caller's thread issues the
-// device copies in order, is the only one to wait on the device, and takes
-// host-side pieces itself where it would wait for a helper.  Helpers sleep
-// while there is no piece to take (a spinning one would compete with the
-// caller's program for its share of the host), and every loop ends on `bad`.
-struct Ring {
+// The device's side of a ring (ring.h): copies on one stream, an event a slot.
+struct RingStream {
     Stage &s;
-    const std::vector<Run> &runs;
-    const size_t bytes;
-    const bool down;
-    const int pieces;
-    std::vector<std::atomic<int>> done;   // the host side of the piece is finished
-    std::atomic<int> next{0};             // pieces taken for their host side
-    std::atomic<int> open{0};             // pieces whose host side may start
-    std::atomic<int> bad{0};
-    std::vector<std::thread> th;
-
-    Ring(Stage &stage, const std::vector<Run> &r, size_t total, bool to_host)
-        : s(stage), runs(r), bytes(total), down(to_host), pieces((int)((total + kPiece - 1) / kPiece)),
-          done((size_t)pieces) {
-        open = down ? 0 : (pieces < kRing ? pieces : kRing);
-        const int n = total < (down ? kHelpDown : kHelpUp) ? 0 : kHelpers;
-        for (int k = 0; k < n; k++) th.emplace_back([this] { help(); });
+    hipStream_t st;
+    std::function<void(int)> copy;   // queue piece p's copy
+    void issue(int p) {
+        copy(p);
+        AG2_HIP(hipEventRecord(s.ev[p % kRing], st));
     }
-    ~Ring() {
-        if (next < pieces) bad = 1;   // left by an error
-        for (auto &t : th) t.join();
-    }
-    size_t off(int p) const { return (size_t)p * kPiece; }
-    size_t len(int p) const { return bytes - off(p) < kPiece ? bytes - off(p) : kPiece; }
-    char *slot(int p) const { return s.host + (size_t)(p % kRing) * kPiece; }
-    // The host side of one open piece, if there is one to take.
-    bool take() {
-        int p = next;
-        while (p < open)
-            if (next.compare_exchange_weak(p, p + 1)) {
-                move_runs(runs, off(p), len(p), slot(p), down);
-                done[(size_t)p] = 1;
-                return true;
-            }
-        return false;
-    }
-    void help() {
-        while (!bad && next < pieces)
-            if (!take()) std::this_thread::sleep_for(std::chrono::microseconds(20));
-    }
-    void take_or_spin() {
-        if (!take()) __builtin_ia32_pause();
-    }
-    // issue(p): queue piece p's device copy on st.
-    void run(hipStream_t st, const std::function<void(int)> &issue) {
-        int issued = 0, landed = 0;
-        auto send = [&](int p) {
-            issue(p);
-            AG2_HIP(hipEventRecord(s.ev[p % kRing], st));
-            issued = p + 1;
-        };
-        if (down) {
-            while (landed < pieces) {
-                while (issued < pieces && (issued < kRing || done[(size_t)(issued - kRing)])) send(issued);
-                if (landed < issued) {
-                    AG2_HIP(hipEventSynchronize(s.ev[landed % kRing]));
-                    open = ++landed;
-                } else {
-                    take_or_spin();
-                }
-            }
-        } else {
-            while (issued < pieces) {
-                if (done[(size_t)issued]) send(issued);
-                else take_or_spin();
-                // slots whose copy has left are open again
-                while (landed < issued && hipEventQuery(s.ev[landed % kRing]) == hipSuccess) landed++;
-                const int o = landed + kRing < pieces ? landed + kRing : pieces;
-                if (o > open) open = o;
-            }
-        }
-        while (next < pieces) take_or_spin();
-        for (auto &t : th) t.join();
-        th.clear();
+    void wait(int p) { AG2_HIP(hipEventSynchronize(s.ev[p % kRing])); }
+    bool left(int p) {
+        const hipError_t e = hipEventQuery(s.ev[p % kRing]);
+        if (e == hipErrorNotReady) return false;
+        AG2_HIP(e);
+        return true;
     }
 };
 
@@ -299,12 +210,13 @@ void fields_to_host(Ctx &c, int nf, const double *const *src, double *const *hos
         move_runs(runs, 0, bytes, s.host, true);
         return;
     }
-    Ring ring(s, runs, bytes, true);
+    RingStream dev{s, c.stream, {}};
+    Ring<RingStream> ring(dev, s.host, kRing, kPiece, runs, bytes, true, bytes < kHelpDown ? 0 : kHelpers);
     // a few fields at a time, so that the first pieces leave early
     const int per = (int)(n * 8 >= 4 * kPiece ? 1 : 4 * kPiece / (n * 8));
     int packed = 0;
     bool tpacked = !htype;
-    ring.run(c.stream, [&](int p) {
+    dev.copy = [&](int p) {
         const size_t end = ring.off(p) + ring.len(p);
         while ((packed < nf && (size_t)packed * n * 8 < end) || (packed == nf && !tpacked)) {
             const int k = nf - packed < per ? nf - packed : per;
@@ -314,14 +226,14 @@ void fields_to_host(Ctx &c, int nf, const double *const *src, double *const *hos
         }
         AG2_HIP(hipMemcpyAsync(ring.slot(p), (const char *)flat + ring.off(p), ring.len(p), hipMemcpyDeviceToHost,
                                c.stream));
-    });
+    };
+    ring.run();
     AG2_HIP(hipStreamSynchronize(c.stream));
 }
 
 // The caller's columns to the state arrays: dst[f] from host[f], or filled
 // with dflt[f] where host[f] is null; types (1 where htype is null), every
-// particle active, resident order = caller order.  The copies are queued on
-// the context's stream when this returns, and the caller's arrays read.
+// particle active, resident order = caller order.  Synchronous.
 void fields_to_device(Ctx &c, int nf, double *const *dst, const double *const *host, const double *dflt,
                       const uint8_t *htype) {
     const size_t n = (size_t)c.n;
@@ -355,11 +267,13 @@ void fields_to_device(Ctx &c, int nf, double *const *dst, const double *const *h
         move_runs(runs, 0, bytes, s.host, false);
         AG2_HIP(hipMemcpyAsync(flat, s.host, bytes, hipMemcpyHostToDevice, c.stream));
     } else {
-        Ring ring(s, runs, bytes, false);
-        ring.run(c.stream, [&](int p) {
+        RingStream dev{s, c.stream, {}};
+        Ring<RingStream> ring(dev, s.host, kRing, kPiece, runs, bytes, false, bytes < kHelpUp ? 0 : kHelpers);
+        dev.copy = [&](int p) {
             AG2_HIP(hipMemcpyAsync((char *)flat + ring.off(p), ring.slot(p), ring.len(p), hipMemcpyHostToDevice,
                                    c.stream));
-        });
+        };
+        ring.run();
     }
     unpack();
     AG2_HIP(hipStreamSynchronize(c.stream));   // the pinned buffer goes back
