@@ -41,8 +41,9 @@ inline void move_runs(const std::vector<Run> &runs, size_t at, size_t len, char 
 //   left(p)   has it completed?
 // The caller's thread takes host-side pieces itself where it would wait for a
 // helper.  Helpers sleep while there is no piece to take (a spinning one would
-// compete with the caller's program for its share of the host).  An error of
-// the device goes up from run(), and the destructor then stops the helpers.
+// compete with the caller's program for its share of the host).  The caller
+// alone is enough: where a thread cannot be had, those that were do.  An error
+// of the device goes up from run(), and the destructor then stops the helpers.
 template <class Device>
 class Ring {
   public:
@@ -54,7 +55,11 @@ class Ring {
         : dev_(device), slots_(slots), ring_(n_slots), piece_(piece), runs_(r), bytes_(total), down_(to_host),
           pieces_((int)((total + piece - 1) / piece)), done_((size_t)pieces_) {
         open_ = down_ ? 0 : (pieces_ < ring_ ? pieces_ : ring_);
-        for (int k = 0; k < helpers; k++) th_.push_back(start([this] { help(); }));
+        try {
+            th_.reserve((size_t)helpers);
+            for (int k = 0; k < helpers; k++) th_.push_back(start([this] { help(); }));
+        } catch (...) {
+        }
     }
     ~Ring() {
         if (next_ < pieces_) bad_ = 1;   // left by an error

@@ -1,7 +1,7 @@
 """The ring of a large transfer (csrc/ring.h) on the CPU, its device one of
-memory copies: whole blocks both ways with and without helpers, and errors of
-the device, each of which has to come up (and not leave the caller waiting, or a
-thread behind)."""
+memory copies: whole blocks both ways with any number of helpers, threads that
+cannot be had, and errors of the device, each of which has to come up (and not
+leave the caller waiting, or a thread behind)."""
 import ctypes as C
 import os
 import subprocess
@@ -35,8 +35,9 @@ def ring(tmp_path_factory):
 
 @pytest.mark.parametrize("down", [0, 1])
 @pytest.mark.parametrize("runs,each", [(1, 4097), (3, 1000), (11, 8000), (19, 24593), (2, 200000)])
-@pytest.mark.parametrize("helpers,threads", [(0, 0), (3, 3)])
+@pytest.mark.parametrize("helpers,threads", [(0, 0), (3, 0), (3, 1), (3, 2), (3, 3)])
 def test_whole_blocks(ring, runs, each, down, helpers, threads):
+    """... with fewer threads than asked for the rest of them and the caller do."""
     for late in (0, 3):
         rc, had, same = ring(runs, each, down, helpers, threads, late)
         assert rc == 0 and same
@@ -50,6 +51,6 @@ def test_whole_blocks(ring, runs, each, down, helpers, threads):
 @pytest.mark.parametrize("threads", [0, 3])
 def test_errors_come_up(ring, down, how, fail, threads):
     before = threading.active_count(), len(os.listdir("/proc/self/task"))
-    rc, _, _ = ring(16, 16384, down, threads, threads, 2, fail, how)   # 64 pieces
+    rc, _, _ = ring(16, 16384, down, 3, threads, 2, fail, how)   # 64 pieces
     assert rc == -1
     assert (threading.active_count(), len(os.listdir("/proc/self/task"))) == before
