@@ -35,6 +35,33 @@ inline void move_runs(const std::vector<Run> &runs, size_t at, size_t len, char 
     }
 }
 
+// A staging buffer, taken for a transfer and given back after it.  A transfer
+// that ends early (no call of whole()) may leave copies under way in the
+// buffer: those are waited for, and the buffer is not kept for others.
+//   take()      a buffer (may throw)
+//   drain()     wait for the copies queued so far, whatever became of them
+//   keep(b)     keep it for a later transfer, if there is room
+//   destroy(b)
+template <class Buffer, class Ops>
+class Lease {
+  public:
+    explicit Lease(Ops ops) : ops_(ops), buffer(ops_.take()) {}
+    ~Lease() {
+        if (!whole_) ops_.drain();
+        if (!whole_ || !ops_.keep(buffer)) ops_.destroy(buffer);
+    }
+    void whole() { whole_ = true; }   // every copy of the transfer has completed
+    Lease(const Lease &) = delete;
+    Lease &operator=(const Lease &) = delete;
+
+  private:
+    Ops ops_;
+    bool whole_ = false;
+
+  public:
+    Buffer buffer;
+};
+
 // The device's side, called by the caller's thread alone; each may throw.
 //   issue(p)  queue the copy of piece p between the block and its slot
 //   wait(p)   return when it has completed

@@ -52,29 +52,45 @@ void stage_free(Stage &s) {
     s = Stage{};
 }
 
+// Buffers kept for later transfers: up to N of one size.
+template <int N>
+struct Shelf {
+    Stage at[N];
+    int n = 0;
+    bool take(Stage &s) {
+        if (n == 0) return false;
+        s = at[--n];
+        return true;
+    }
+    bool give(const Stage &s) {
+        if (n == N) return false;
+        at[n++] = s;
+        return true;
+    }
+};
+
 struct Kept {
     std::mutex mu;
     int contexts = 0;
-    std::vector<Stage> small, large;
+    Shelf<4> small;
+    Shelf<2> large;
 };
 Kept &kept(int device) {
     static Kept k[kMaxDev];
     return k[device >= 0 && device < kMaxDev ? device : 0];
 }
 
-// One pinned buffer, taken for a transfer and given back after it.
-class Lease {
-  public:
-    Lease(int device, bool large) : dev_(device), large_(large) {
+// The device's pinned buffers for transfers on a stream (Lease, ring.h).
+struct Pinned {
+    int device;
+    bool large;
+    hipStream_t stream;
+    Stage take() {
         Kept &k = kept(device);
+        Stage s;
         {
             std::lock_guard<std::mutex> hold(k.mu);
-            auto &v = large ? k.large : k.small;
-            if (!v.empty()) {
-                s = v.back();
-                v.pop_back();
-                return;
-            }
+            if (large ? k.large.take(s) : k.small.take(s)) return s;
         }
         s.slots = large ? kRing : 1;
         try {
@@ -84,26 +100,15 @@ class Lease {
             stage_free(s);
             throw;
         }
+        return s;
     }
-    ~Lease() {
-        Kept &k = kept(dev_);
-        {
-            std::lock_guard<std::mutex> hold(k.mu);
-            auto &v = large_ ? k.large : k.small;
-            if (k.contexts > 0 && v.size() < (large_ ? 2u : 4u)) {
-                v.push_back(s);
-                return;
-            }
-        }
-        stage_free(s);
+    void drain() { (void)hipStreamSynchronize(stream); }
+    bool keep(const Stage &s) {
+        Kept &k = kept(device);
+        std::lock_guard<std::mutex> hold(k.mu);
+        return k.contexts > 0 && (large ? k.large.give(s) : k.small.give(s));
     }
-    Lease(const Lease &) = delete;
-    Lease &operator=(const Lease &) = delete;
-    Stage s;
-
-  private:
-    int dev_;
-    bool large_;
+    void destroy(Stage &s) { stage_free(s); }
 };
 
 // The device's side of a ring (ring.h): copies on one stream, an event a slot.
@@ -168,15 +173,16 @@ void transfer_ref(int device) {
 
 void transfer_unref(int device) {
     Kept &k = kept(device);
-    std::vector<Stage> dead;
+    Shelf<4> small;
+    Shelf<2> large;
     {
         std::lock_guard<std::mutex> hold(k.mu);
         if (--k.contexts > 0) return;
-        dead.swap(k.small);
-        dead.insert(dead.end(), k.large.begin(), k.large.end());
-        k.large.clear();
+        std::swap(small, k.small);
+        std::swap(large, k.large);
     }
-    for (Stage &s : dead) stage_free(s);
+    Stage dead;
+    while (small.take(dead) || large.take(dead)) stage_free(dead);
 }
 
 // Columns src[0 .. nf) (n values each, in resident order) and optionally the
@@ -201,12 +207,13 @@ void fields_to_host(Ctx &c, int nf, const double *const *src, double *const *hos
                            last ? tflat : nullptr);
         AG2_HIP(hipGetLastError());
     };
-    Lease lease(c.device, bytes > kPiece);
-    Stage &s = lease.s;
+    Lease<Stage, Pinned> lease(Pinned{c.device, bytes > kPiece, c.stream});
+    Stage &s = lease.buffer;
     if (bytes <= kPiece) {
         pack(0, nf, true);
         AG2_HIP(hipMemcpyAsync(s.host, flat, bytes, hipMemcpyDeviceToHost, c.stream));
         AG2_HIP(hipStreamSynchronize(c.stream));
+        lease.whole();
         move_runs(runs, 0, bytes, s.host, true);
         return;
     }
@@ -229,6 +236,7 @@ void fields_to_host(Ctx &c, int nf, const double *const *src, double *const *hos
     };
     ring.run();
     AG2_HIP(hipStreamSynchronize(c.stream));
+    lease.whole();
 }
 
 // The caller's columns to the state arrays: dst[f] from host[f], or filled
@@ -261,8 +269,8 @@ void fields_to_device(Ctx &c, int nf, double *const *dst, const double *const *h
         AG2_HIP(hipGetLastError());
     };
     if (bytes == 0) return unpack();
-    Lease lease(c.device, bytes > kPiece);
-    Stage &s = lease.s;
+    Lease<Stage, Pinned> lease(Pinned{c.device, bytes > kPiece, c.stream});
+    Stage &s = lease.buffer;
     if (bytes <= kPiece) {
         move_runs(runs, 0, bytes, s.host, false);
         AG2_HIP(hipMemcpyAsync(flat, s.host, bytes, hipMemcpyHostToDevice, c.stream));
@@ -276,7 +284,8 @@ void fields_to_device(Ctx &c, int nf, double *const *dst, const double *const *h
         ring.run();
     }
     unpack();
-    AG2_HIP(hipStreamSynchronize(c.stream));   // the pinned buffer goes back
+    AG2_HIP(hipStreamSynchronize(c.stream));
+    lease.whole();
 }
 
 }  // namespace ag2

@@ -30,6 +30,7 @@ def ring(tmp_path_factory):
         rc = lib.ring_copy(runs, C.c_int64(each), p(host), p(block), int(down), C.c_int64(piece), slots, helpers,
                                threads, late, fail, how, C.byref(had))
         return rc, had.value, np.array_equal(dst, data)
+    run.lib = lib
     return run
 
 
@@ -54,3 +55,11 @@ def test_errors_come_up(ring, down, how, fail, threads):
     rc, _, _ = ring(16, 16384, down, 3, threads, 2, fail, how)   # 64 pieces
     assert rc == -1
     assert (threading.active_count(), len(os.listdir("/proc/self/task"))) == before
+
+
+def test_a_buffer_left_early_is_not_kept(ring):
+    """Copies may still be under way in the buffer of a transfer that failed."""
+    assert ring.lib.lease_steps(1, 1) == 13
+    assert ring.lib.lease_steps(1, 0) == 14
+    assert ring.lib.lease_steps(0, 1) == 124
+    assert ring.lib.lease_steps(0, 0) == 124

@@ -66,3 +66,27 @@ extern "C" int ring_copy(int runs, int64_t each, char *host, char *block, int do
     }
     return 0;
 }
+
+// A lease that ends whole or early, with room on the shelf or not: what became
+// of its buffer, as decimal digits in order (1 taken, 2 drained, 3 kept, 4 destroyed).
+extern "C" int lease_steps(int whole, int room) {
+    struct Ops {
+        int *log, room;
+        void note(int d) { *log = *log * 10 + d; }
+        int take() { note(1); return 7; }
+        void drain() { note(2); }
+        bool keep(int) {
+            if (room) note(3);
+            return room != 0;
+        }
+        void destroy(int) { note(4); }
+    };
+    int log = 0;
+    try {
+        ag2::Lease<int, Ops> lease(Ops{&log, room});
+        if (!whole) throw std::runtime_error("a copy failed");
+        lease.whole();
+    } catch (const std::runtime_error &) {
+    }
+    return log;
+}
