@@ -1556,13 +1556,39 @@ __global__ void k_zero_job_counters(const JobWalk *jobs, int nj) {
     ds->near_redo = 0ull;
 }
 
+// Spill chunks for n_gas targets at this opening angle.  Within 2h a target
+// meets about 75 gas nodes at theta 0.5, 570 at 0.15 (the 200,000 disk), and
+// their number grows as theta^-1.75 up to the particles themselves; half as
+// many again are provided, over three quarters of the list (so from theta
+// 0.37 down: noting the chunks costs the walk 3 % where no list needs them).
+// At theta 0.15 the overflow walk of the lists that did not fit took 5.26 ms
+// of a force evaluation of 9.1 ms; with the chunks it has nothing to do, and
+// the evaluation takes 3.9 ms.
+int64_t sph_spill_chunks(int64_t n_gas, double theta) {
+    const double t = theta > 0.05 ? theta : 0.05;
+    double per = 1.5 * 75.0 * pow(0.5 / t, 1.75) / kSphK - 0.75;
+    if (!(per > 0.0) || n_gas <= 0) return 0;
+    if (per > kSphMore) per = kSphMore;
+    const double want = per * (double)n_gas + 64.0;
+    return want < 0x7fffffff ? (int64_t)want : 0x7fffffff;
+}
+
+// The chunks a context's targets may take: those of its own gas and opening
+// angle, however many more a context sized for larger sets holds (which lists
+// run past them, and so the rounding of the SPH sums, is then a matter of the
+// set alone), or none where it holds fewer.
+int64_t spill_usable(const Ctx &c) {
+    const int64_t own = sph_spill_chunks(c.gas_count, c.p.theta);
+    return c.spill_cap >= own ? own : 0;
+}
+
 WalkArgs walk_args(Ctx &c) {
     WalkArgs a;
     a.n = (int)c.n; a.nin = c.nin; a.nn = c.n_nodes;
     a.tree = c.tnode;
     a.tsph = c.tsph;
     a.gslot = c.gslot; a.sph_list = c.sph_list; a.sph_cnt = c.sph_cnt; a.gover = c.gover;
-    a.sph_spill = c.sph_spill; a.sph_more = c.sph_more; a.spill_cap = (int)c.spill_cap;
+    a.sph_spill = c.sph_spill; a.sph_more = c.sph_more; a.spill_cap = (int)spill_usable(c);
     a.sx = c.x; a.sy = c.y; a.sz = c.z; a.sm = c.m; a.stype = c.type;
     a.svx = c.vx; a.svy = c.vy; a.svz = c.vz;
     a.h = c.h; a.rho = c.rho; a.P = c.P; a.active = c.active;
@@ -1609,23 +1635,6 @@ void fold_counters(Ctx &c) {
     static_assert(kCountBins == 256, "k_fold_counters runs one thread per bin");
     hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(256), 0, c.stream, c.cbins, c.ds);
     AG2_HIP(hipGetLastError());
-}
-
-// Spill chunks for n_gas targets at this opening angle.  Within 2h a target
-// meets about 75 gas nodes at theta 0.5, 570 at 0.15 (the 200,000 disk), and
-// their number grows as theta^-1.75 up to the particles themselves; half as
-// many again are provided, over three quarters of the list (so from theta
-// 0.37 down: noting the chunks costs the walk 3 % where no list needs them).
-// At theta 0.15 the overflow walk of the lists that did not fit took 5.26 ms
-// of a force evaluation of 9.1 ms; with the chunks it has nothing to do, and
-// the evaluation takes 3.9 ms.
-int64_t sph_spill_chunks(int64_t n_gas, double theta) {
-    const double t = theta > 0.05 ? theta : 0.05;
-    double per = 1.5 * 75.0 * pow(0.5 / t, 1.75) / kSphK - 0.75;
-    if (!(per > 0.0) || n_gas <= 0) return 0;
-    if (per > kSphMore) per = kSphMore;
-    const double want = per * (double)n_gas + 64.0;
-    return want < 0x7fffffff ? (int64_t)want : 0x7fffffff;
 }
 
 int64_t sph_spill_bytes(int64_t n_gas, double theta) {
@@ -1675,7 +1684,7 @@ void sph_finish(Ctx &c) {
     WalkArgs a = walk_args(c);
     int64_t lanes = c.gas_count * kPairLanes;
     int nb = (int)((lanes + 255) / 256);
-    if (nb > 0 && c.spill_cap > 0) hipLaunchKernelGGL(k_sph_pairs<true>, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
+    if (nb > 0 && a.spill_cap > 0) hipLaunchKernelGGL(k_sph_pairs<true>, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
     else if (nb > 0) hipLaunchKernelGGL(k_sph_pairs<false>, dim3(nb), dim3(256), 0, st, a, c.gidx, c.sph_cnt);
     const int groups = (int)((c.n + 63) / 64);
     hipLaunchKernelGGL(k_walk_sph_overflow, dim3((groups + kWaves - 1) / kWaves), dim3(64 * kWaves), 0, st, a);
