@@ -155,6 +155,8 @@ struct Ctx {
     // (allocated for small opening angles, sph_spill_chunks)
     int32_t *sph_spill = nullptr, *sph_more = nullptr;
     int64_t spill_cap = 0, spill_refused = 0;
+    int64_t spill_room = -1;   // bytes they may take (a pool's share; -1: any)
+    int64_t charged = 0;       // bytes a pool counts for this context
     // split-precision walk: (node, lane mask) pairs whose targets lie within
     // the FP32 offsets' resolution, evaluated in FP64 after the walk
     // (kNearRecs per group; a group with more is walked again in FP64)

@@ -1642,10 +1642,13 @@ int64_t sph_spill_bytes(int64_t n_gas, double theta) {
     return chunks > 0 ? chunks * kSphK * 4 + n_gas * kSphMore * 4 : 0;
 }
 
-// Where there is no memory for the chunks the overflow walk does their work.
+// Where there is no memory for the chunks, or a pool allows none, the overflow
+// walk does their work.
 void reserve_spill(Ctx &c) {
     const int64_t want = sph_spill_chunks(c.sph_cap, c.p.theta);
     if (!c.sph_active || c.spill_cap >= want || c.spill_refused == want) return;
+    const int64_t bytes = sph_spill_bytes(c.sph_cap, c.p.theta);
+    if (c.spill_room >= 0 && bytes > c.spill_room) return;
     AG2_HIP(hipStreamSynchronize(c.stream));
     if (c.sph_spill) { (void)hipFree(c.sph_spill); c.sph_spill = nullptr; }
     if (c.sph_more) { (void)hipFree(c.sph_more); c.sph_more = nullptr; }

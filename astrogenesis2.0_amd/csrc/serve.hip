@@ -215,6 +215,31 @@ int64_t spill_bytes(const Ctx &c) {
     return c.spill_cap > 0 ? c.spill_cap * ag2::kSphListLen * 4 + c.sph_cap * ag2::kSphMore * 4 : 0;
 }
 
+// What a context takes of the budget.
+int64_t ctx_bytes(const Ctx &c) { return ag2::ctx_footprint(c.cap, c.sph_cap) + spill_bytes(c); }
+
+void drop_spare(Pool &P) {
+    Ctx *c = P.spare.back();
+    P.spare.pop_back();
+    P.used -= c->charged;
+    ag2::ctx_delete(c);
+}
+
+// Counts the spill chunks that job j's opening angle asks for in context c (of
+// gcap gas targets), where the budget has room for them, spare contexts
+// dropped if need be; without, its long SPH lists are left to the overflow walk.
+void allow_spill(Pool &P, Ctx &c, const Job &j, int64_t gcap) {
+    const int64_t want = j.n_gas > 0 ? ag2::sph_spill_bytes(gcap, j.p.theta) : 0;
+    const int64_t have = spill_bytes(c), more = want - have;
+    c.spill_room = have;
+    if (more <= 0) return;
+    while (P.used + more > P.budget && !P.spare.empty()) drop_spare(P);
+    if (P.used + more > P.budget) return;
+    P.used += more;
+    c.charged += more;
+    c.spill_room = want;
+}
+
 // A context for job j: the smallest spare one that is large enough, else a
 // new one if the budget allows (dropping spare contexts to make room).  New
 // contexts are sized in classes (particles and gas targets rounded up to a
@@ -225,36 +250,32 @@ Ctx *take_context(Pool &P, Job &j, hipStream_t st) {
     Ctx *best = nullptr;
     size_t bi = 0;
     for (size_t i = 0; i < P.spare.size(); i++)
-        if (P.spare[i]->cap >= j.n && P.spare[i]->sph_cap >= j.n_gas &&
-            spill_bytes(*P.spare[i]) >= ag2::sph_spill_bytes(j.n_gas > 0 ? P.spare[i]->sph_cap : 0, j.p.theta) &&
-            (!best || P.spare[i]->cap < best->cap)) {
+        if (P.spare[i]->cap >= j.n && P.spare[i]->sph_cap >= j.n_gas && (!best || P.spare[i]->cap < best->cap)) {
             best = P.spare[i];
             bi = i;
         }
     if (best) {
         P.spare.erase(P.spare.begin() + (ptrdiff_t)bi);
         best->p = j.p;
+        allow_spill(P, *best, j, best->sph_cap);
         return best;
     }
     int64_t cap = pow2_at_least(j.n > (1 << 14) ? j.n : (1 << 14));
     int64_t gcap = j.n_gas > 0 ? pow2_at_least(j.n_gas > (1 << 12) ? j.n_gas : (1 << 12)) : 0;
-    int64_t need = ag2::ctx_footprint(cap, gcap) + ag2::sph_spill_bytes(gcap, j.p.theta);
+    int64_t need = ag2::ctx_footprint(cap, gcap);
     if (P.used + need > P.budget) {
         cap = j.n;
         gcap = j.n_gas;
-        need = ag2::ctx_footprint(cap, gcap) + ag2::sph_spill_bytes(gcap, j.p.theta);
+        need = ag2::ctx_footprint(cap, gcap);
     }
-    while (P.used + need > P.budget && !P.spare.empty()) {
-        Ctx *c = P.spare.back();
-        P.spare.pop_back();
-        P.used -= ag2::ctx_footprint(c->cap, c->sph_cap) + spill_bytes(*c);
-        ag2::ctx_delete(c);
-    }
+    while (P.used + need > P.budget && !P.spare.empty()) drop_spare(P);
     if (P.used + need > P.budget) return nullptr;
     Ctx *c = ag2::ctx_new(j.p, cap, st);
     c->sph_reserve = gcap;
     c->timing = 0;
     P.used += need;
+    c->charged = need;
+    allow_spill(P, *c, j, gcap);
     return c;
 }
 
@@ -271,6 +292,9 @@ void admit(Pool &P, int slots, hipStream_t st, std::vector<Job *> &into, const s
         c->stream = st;
         ag2_particles h = view(*j);
         ag2::ctx_upload(*c, h);
+        // (chunks that were allowed may not have been had)
+        P.used += ctx_bytes(*c) - c->charged;
+        c->charged = ctx_bytes(*c);
         ag2::fill_active(*c, 1);
         {
             ag2::StepBuild sb(*c, true);   // every particle active
@@ -439,7 +463,7 @@ int ag2_job_submit(void *pool, const ag2_params *params, const ag2_particles *h,
         if (h->n < 1) return pfail(P, AG2_ERR_ARG, "n must be >= 1");
         if (h->n > 0x7fffff00LL / 2) return pfail(P, AG2_ERR_CAPACITY, "n too large");
         if (steps < 0) return pfail(P, AG2_ERR_ARG, "steps must be >= 0");
-        if (ag2::ctx_footprint(h->n, ngas_of(*h)) + ag2::sph_spill_bytes(ngas_of(*h), params->theta) > P->budget) return pfail(P, AG2_ERR_CAPACITY, "job exceeds the pool's memory budget");
+        if (ag2::ctx_footprint(h->n, ngas_of(*h)) > P->budget) return pfail(P, AG2_ERR_CAPACITY, "job exceeds the pool's memory budget");
         Job *j = new Job();
         j->id = P->next_id++;
         j->p = *params;

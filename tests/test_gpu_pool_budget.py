@@ -1,9 +1,10 @@
-"""The SPH spill chunks of small opening angles in a pool: a job's result does
-not depend on the size of the context it got."""
+"""The pool's memory budget and the SPH spill chunks of small opening angles:
+they are taken where the budget has room, refuse no job, balance when they go,
+and a job's result does not depend on the size of the context it got."""
 import numpy as np
 import pytest
 
-from test_gpu_serving import solo
+from test_gpu_serving import close, solo
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,32 @@ def run(ag2, pool, jobs, steps=2):
         pool.step()
         used.append(pool.stats()["hbm_used"])
     return [pool.result(i, ag2.ics.ParticleSet(ps.n)) for i, (ps, _) in zip(ids, jobs)], used
+
+
+def context_bytes(ag2, ps):
+    return ag2.engine.load_library().ag2_context_bytes(ps.n, int((ps.type == 2).sum()))
+
+
+def test_a_job_of_the_budgets_size_is_taken_at_any_angle(ag2):
+    """Without room for chunks its long lists are left to the overflow walk."""
+    ps, prm = job(ag2, 20000, 0.15)
+    budget = context_bytes(ag2, ps)
+    with ag2.engine.Pool(max_jobs=2, hbm_budget=budget) as pool:
+        (got,), used = run(ag2, pool, [(ps, prm)])
+    assert max(used) <= budget
+    assert close(got, solo(ag2, ps, prm, 2)) is None
+
+
+def test_what_is_used_balances(ag2):
+    """One context serves jobs of any angle one after another: what is used does
+    not grow after the smallest angle, and stays within the budget."""
+    with ag2.engine.Pool(max_jobs=1, hbm_budget=1 << 30) as pool:
+        last = []
+        for theta in (0.5, 0.15, 0.5, 0.2, 0.15, 0.7, 0.15):
+            _, used = run(ag2, pool, [job(ag2, 16000, theta)], 1)
+            last.append(used[-1])
+    assert last[0] < last[1] and set(last[1:]) == {last[1]}
+    assert last[1] <= 1 << 30
 
 
 def test_chunks_run_out_for_the_set_alone(ag2):
