@@ -1642,8 +1642,9 @@ int64_t sph_spill_bytes(int64_t n_gas, double theta) {
     return chunks > 0 ? chunks * kSphK * 4 + n_gas * kSphMore * 4 : 0;
 }
 
-// Where there is no memory for the chunks, or a pool allows none, the overflow
-// walk does their work.
+// Where there is no memory for the chunks the overflow walk does their work:
+// past the share a pool allows, or half of what is free on the device (later
+// buffers of the context, and other contexts, need theirs).
 void reserve_spill(Ctx &c) {
     const int64_t want = sph_spill_chunks(c.sph_cap, c.p.theta);
     if (!c.sph_active || c.spill_cap >= want || c.spill_refused == want) return;
@@ -1653,7 +1654,9 @@ void reserve_spill(Ctx &c) {
     if (c.sph_spill) { (void)hipFree(c.sph_spill); c.sph_spill = nullptr; }
     if (c.sph_more) { (void)hipFree(c.sph_more); c.sph_more = nullptr; }
     c.spill_cap = 0;
-    if (hipMalloc(&c.sph_spill, (size_t)want * kSphK * 4) != hipSuccess ||
+    size_t avail = 0, all = 0;
+    AG2_HIP(hipMemGetInfo(&avail, &all));
+    if ((size_t)bytes > avail / 2 || hipMalloc(&c.sph_spill, (size_t)want * kSphK * 4) != hipSuccess ||
         hipMalloc(&c.sph_more, (size_t)c.sph_cap * kSphMore * 4) != hipSuccess) {
         (void)hipGetLastError();
         if (c.sph_spill) { (void)hipFree(c.sph_spill); c.sph_spill = nullptr; }
