@@ -19,14 +19,14 @@
 // quotients of their own.  Other softening lengths test every pair.
 //
 // A target's sum depends on the sources alone, bit for bit, not on the other
-// targets asked for: sources are summed in blocks of fixed length, blocks
-// sixteen at a time, those in (at most) four parts of the set, and the parts
-// in order, however many of these one wave sums (SumPlan).
-//
-// 1 M sources, 16,384 targets: with the potential 372 ms one workgroup per 256
-// targets, now 26.1; without 212, now 10.5; 300 targets 1.5 and 0.85 ms.
+// targets asked for: sources are summed in blocks of fixed length, and the
+// blocks in a binary tree (pairs of neighbours, pairs of those, a node without
+// a right half being its left one), of which a wave takes an aligned power of
+// two, as many as the targets leave it.
+// 1 M sources, 16,384 targets: 372 ms with the potential and 212 without by one
+// workgroup per 256 targets, now 27.7 and 11.5; 300 targets 1.0 and 0.5 ms.
 // Against sums in extended precision 2.9e-14 then (a million terms one by one;
-// the potential 4.2e-14), now 1.5e-16.
+// the potential 4.2e-14), now 1.1e-16.
 #include <mutex>
 #include <type_traits>
 
@@ -37,25 +37,21 @@ namespace ag2 {
 namespace {
 
 constexpr int kDirectBlock = 256;
-constexpr int kMid = 16;   // blocks of sources summed at a time
+constexpr int kLevels = 24;   // of the tree over blocks
 
-// The order of a target's sum over n sources: blocks of `len` sources, kMid
-// blocks at a time, `top` of those at a time, all of them.  A wave sums `per`
-// blocks (1, kMid or kMid top): its part of the sum.
+// Sources in blocks of `len`; a wave sums 2^level of them.
 struct SumPlan {
-    int n, len, blocks, top, per;
+    int n, len, blocks, level;
 };
 
-// Targets: lane k of the grid's first dimension; blocks of sources [split *
-// per, ...).  part: column c of split s at (c * splits + s) * nt, unscaled sums.
+// Targets: lane k of the grid's first dimension; blocks of sources from split
+// 2^level on.  part: column c of split s at (c * splits + s) * nt, unscaled sums.
 // ANY: the softening length is outside the fast pair's range.
 template <bool POT, bool ANY>
-__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(SumPlan p, const double *__restrict__ x,
-                                                         const double *__restrict__ y, const double *__restrict__ z,
-                                                         const double *__restrict__ m, int nt,
-                                                         const int64_t *__restrict__ targets,
-                                                         const int32_t *__restrict__ inv, double e0,
-                                                         double *__restrict__ part) {
+__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void
+k_direct(SumPlan p, const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+         const double *__restrict__ m, int nt, const int64_t *__restrict__ targets, const int32_t *__restrict__ inv,
+         double e0, double *__restrict__ part) {
     const int k = blockIdx.x * kDirectBlock + threadIdx.x;
     const int split = blockIdx.y;
     const bool valid = k < nt;
@@ -98,13 +94,12 @@ __global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4)
         gx = __builtin_fma(f, ux, gx);
         gy = __builtin_fma(f, uy, gy);
         gz = __builtin_fma(f, uz, gz);
-        if (POT) ph = __builtin_fma(mj, softened_angle(e0, r, ir), ph);
+        if (POT) ph = __builtin_fma(mj, softened_angle_own(e0, r, ir), ph);
     };
     const std::integral_constant<bool, ANY> form;
-    double mx = 0.0, my = 0.0, mz = 0.0, mp = 0.0;   // of up to kMid blocks
-    double tx = 0.0, ty = 0.0, tz = 0.0, tp = 0.0;   // of those
-    const int b1 = (split + 1) * p.per < p.blocks ? (split + 1) * p.per : p.blocks;
-    for (int b = split * p.per; b < b1; b++) {
+    double node[kLevels][4];   // left halves that wait for their right ones, by level
+    const int b0 = split << p.level, b1 = b0 + (1 << p.level) < p.blocks ? b0 + (1 << p.level) : p.blocks;
+    for (int b = b0; b < b1; b++) {
         const int j0 = b * p.len, j1 = p.n - j0 < p.len ? p.n : j0 + p.len;
         gx = gy = gz = ph = 0.0;
         int j = j0;
@@ -122,77 +117,92 @@ __global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4)
                 ph = bad ? ph : op;
             }
         }
-        mx += gx; my += gy; mz += gz; mp += ph;
-        if ((b + 1) % kMid == 0 || b + 1 == b1) {
-            tx += mx; ty += my; tz += mz; tp += mp;
-            mx = my = mz = mp = 0.0;
+        int l = 0;
+        for (; (b - b0) >> l & 1; l++) {
+            gx = node[l][0] + gx;
+            gy = node[l][1] + gy;
+            gz = node[l][2] + gz;
+            if (POT) ph = node[l][3] + ph;
         }
+        node[l][0] = gx; node[l][1] = gy; node[l][2] = gz;
+        if (POT) node[l][3] = ph;
     }
+    // what is left of the set's last, incomplete part
+    const int done = b1 - b0;
+    int l = __builtin_ctz(done);
+    gx = node[l][0]; gy = node[l][1]; gz = node[l][2];
+    if (POT) ph = node[l][3];
+    for (l++; done >> l; l++)
+        if (done >> l & 1) {
+            gx = node[l][0] + gx;
+            gy = node[l][1] + gy;
+            gz = node[l][2] + gz;
+            if (POT) ph = node[l][3] + ph;
+        }
     if (!valid) return;
     const size_t col = (size_t)gridDim.y * nt;
     double *out = part + (size_t)split * nt + k;
-    out[0] = tx; out[col] = ty; out[2 * col] = tz;
-    if (POT) out[3 * col] = tp;
+    out[0] = gx; out[col] = gy; out[2 * col] = gz;
+    if (POT) out[3 * col] = ph;
 }
 
-// Column c of the result: its parts in the plan's order, scaled.
-__global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, SumPlan p, const double *__restrict__ part,
-                                                     double G, double e0, double *ax, double *ay, double *az,
-                                                     double *pot) {
+// Column c of the result: its parts up the rest of the tree, scaled.
+__global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, const double *__restrict__ part, double G,
+                                                     double e0, double *ax, double *ay, double *az, double *pot) {
+    constexpr int kAt = 16;   // parts read at a time
     const int k = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
     if (k >= nt) return;
     const double *q = part + (size_t)c * splits * nt + k;
-    double s = 0.0, t = 0.0, mid = 0.0;
-    for (int u0 = 0; u0 < splits; u0 += kMid) {
-        double v[kMid];   // every load before the first sum
+    double node[kLevels];
+    const int all = (splits + kAt - 1) / kAt;
+    double s = 0.0;
+    for (int b = 0; b < all; b++) {
+        const int have = splits - b * kAt;
+        double v[kAt];
 #pragma unroll
-        for (int k = 0; k < kMid; k++) v[k] = u0 + k < splits ? q[(size_t)(u0 + k) * nt] : 0.0;
+        for (int u = 0; u < kAt; u++) v[u] = u < have ? q[(size_t)(b * kAt + u) * nt] : 0.0;
 #pragma unroll
-        for (int k = 0; k < kMid; k++) {
-            if (u0 + k >= splits) break;
-            const int done = (u0 + k + 1) * p.per;   // blocks so far
-            const bool last = u0 + k + 1 == splits;
-            mid += v[k];
-            if (done % kMid == 0 || last) { t += mid; mid = 0.0; }
-            if (done % (kMid * p.top) == 0 || last) { s += t; t = 0.0; }
-        }
+        for (int d = 1; d < kAt; d *= 2)
+#pragma unroll
+            for (int u = 0; u < kAt; u += 2 * d) v[u] = u + d < have ? v[u] + v[u + d] : v[u];
+        s = v[0];
+        int l = 0;
+        for (; b >> l & 1; l++) s = node[l] + s;
+        node[l] = s;
     }
+    int l = __builtin_ctz(all);
+    s = node[l];
+    for (l++; all >> l; l++)
+        if (all >> l & 1) s = node[l] + s;
     double *out = c == 0 ? ax : c == 1 ? ay : c == 2 ? az : pot;
     out[k] = c < 3 ? G * s : -(G / e0) * s;
 }
 
-// Blocks of n / 256 sources (a multiple of four, 32 to 256 of them), and at
-// most four parts of the whole.
-SumPlan sum_plan(int n) {
-    SumPlan p;
-    p.n = n;
-    p.len = ((n + 255) / 256 + 3) / 4 * 4;
-    p.len = p.len < 32 ? 32 : p.len > 256 ? 256 : p.len;
-    p.blocks = (n + p.len - 1) / p.len;
-    p.top = ((p.blocks + kMid - 1) / kMid + 3) / 4;
-    p.per = 1;
-    return p;
-}
-
-// Targets [0, nt) in slices whose parts fit `room` doubles of scratch.  A wave
-// takes as many blocks as leave four waves for each of 1,024 SIMDs, or, where
-// the scratch holds no more parts, as have to be.
+// Targets [0, nt) in slices whose parts fit `room` doubles of scratch.  Blocks
+// of n / 256 sources (a multiple of four, 32 to 256 of them).  Parts: up to 64
+// waves for each of 1,024 SIMDs, of at least 256 sources (with 16 waves a SIMD,
+// four rounds of them, 16,384 targets wait 30.3 ms for the last, with 64 27.7).
 void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, double *scratch, size_t room, double *ax,
                    double *ay, double *az, double *pot) {
     const int cols = with_pot ? 4 : 3;
-    SumPlan p = sum_plan((int)c.n);
-    const int64_t waves = (nt + 63) / 64;
-    const int pers[3] = {kMid * p.top, kMid, 1};
-    auto parts = [&](int per) { return (int64_t)(p.blocks + per - 1) / per; };
-    p.per = pers[0];
-    for (int per : pers)
-        if (per < p.per && waves * parts(p.per) < 4096 && (int64_t)nt * cols * parts(per) <= (int64_t)room) p.per = per;
-    const int splits = (int)parts(p.per);
-    const int64_t fit = (int64_t)room / ((int64_t)cols * splits);
-    if (fit < 1) throw HipError("no scratch for the direct sum");
+    SumPlan p;
+    p.n = (int)c.n;
+    p.len = ((p.n + 255) / 256 + 3) / 4 * 4;
+    p.len = p.len < 32 ? 32 : p.len > 256 ? 256 : p.len;
+    p.blocks = (p.n + p.len - 1) / p.len;
     const bool any = !(c.p.e0 >= 0x1p42 && c.p.e0 <= 0x1p150);
     for (int at = 0; at < nt;) {
-        const int here = nt - at < fit ? nt - at : (int)fit;
+        const size_t fit = room / (size_t)cols;
+        const int here = (size_t)(nt - at) < fit ? nt - at : (int)fit;
+        if (here < 1) throw HipError("no scratch for the direct sum");
+        const int64_t waves = (here + 63) / 64;
+        int64_t most = (65536 + waves - 1) / waves;
+        if (most > (p.n + 255) / 256) most = (p.n + 255) / 256;
+        if (most > (int64_t)(fit / (size_t)here)) most = (int64_t)(fit / (size_t)here);
+        if (most > 65535) most = 65535;
+        p.level = 0;
+        while (((p.blocks - 1) >> p.level) + 1 > most) p.level++;
+        const int splits = ((p.blocks - 1) >> p.level) + 1;
         const dim3 grid(grid_for(here, kDirectBlock), (unsigned)splits), block(kDirectBlock);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, block, 0, c.stream, p, c.x, c.y, c.z, c.m, here, d_targets + at, c.inv,
@@ -200,7 +210,7 @@ void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, doubl
         };
         if (with_pot) any ? go(k_direct<true, true>) : go(k_direct<true, false>);
         else any ? go(k_direct<false, true>) : go(k_direct<false, false>);
-        hipLaunchKernelGGL(k_direct_fold, dim3(grid_for(here, 256), cols), dim3(256), 0, c.stream, here, splits, p,
+        hipLaunchKernelGGL(k_direct_fold, dim3(grid_for(here, 256), cols), dim3(256), 0, c.stream, here, splits,
                            scratch, c.p.G, c.p.e0, ax + at, ay + at, az + at, pot ? pot + at : nullptr);
         AG2_HIP(hipGetLastError());
         at += here;

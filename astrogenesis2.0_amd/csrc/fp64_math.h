@@ -52,14 +52,30 @@ __device__ __forceinline__ double atan_poly_small(double w) {
 }
 
 // pi/2 - atan(r / e) = atan(e / r) for r, e >= 0 (not both 0), ir = 1 / r, by
-// the quotient: up to 1/16 and up to tan(pi/8) the series alone (8 and 14 issue
-// slots); else, with a <= b the smaller and larger of r and e, atan(a / b) =
-// pi/4 + atan((a - b) / (a + b)) above tan(pi/8), and the complement where r is
-// the smaller (42 slots).  The wave takes the branches that some lane needs (a
-// tree walk or a direct sum mostly the series), and a lane's value is that of
-// its own branch, whatever the others need: it costs the direct sum of 16,384
-// targets 2 % (25.5 -> 26.1 ms); one series of 14 slots for both, 5 %.
+// the largest quotient in the wave: up to 1/16 and up to tan(pi/8) the series
+// alone (8 and 14 issue slots; most waves of a tree walk or a direct sum);
+// else, with a <= b the smaller and larger of r and e, atan(a / b) = pi/4 +
+// atan((a - b) / (a + b)) above tan(pi/8), and the complement where r is the
+// smaller (42 slots).
 __device__ __forceinline__ double softened_angle(double e, double r, double ir) {
+    const double u = e * ir;
+    if (__any(!(u <= 0.41421356237309503))) {
+        const double a = r < e ? r : e, b = r < e ? e : r;
+        const bool up = a > 0.41421356237309503 * b;
+        const double num = up ? a - b : a, den = up ? a + b : b;
+        const double x = num * rcp_full(den);
+        const double t = (up ? 0.78539816339744828 : 0.0) + x * atan_poly(x * x);
+        return r < e ? 1.5707963267948966 - t : t;
+    }
+    if (__any(u > 0.0625)) return u * atan_poly(u * u);
+    return u * atan_poly_small(u * u);
+}
+
+// The same, a lane's value that of its own branch whatever the wave's others
+// need: the wave takes every branch that some lane needs.  (The direct sum of
+// 16,384 targets takes 27.7 ms with it, 26.6 with the wave's branch; 29.2 with
+// one series of 14 slots up to tan(pi/8).)
+__device__ __forceinline__ double softened_angle_own(double e, double r, double ir) {
     const double u = e * ir;
     const bool far = u <= 0.41421356237309503, small = u <= 0.0625;
     double t = 0.0;

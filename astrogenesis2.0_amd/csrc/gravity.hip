@@ -916,9 +916,9 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                                 const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
                                 if (KIND == 4) {
                                     // -(G / e0) m (pi/2 - atan(r / e0)), scaled at the end
-                                    // (nothing is left of it beyond 2^500 m, and where
-                                    // r^2 overflows it has no root)
-                                    if (r2 != 0.0 && !(r2 > 0x1p1000) && on) {
+                                    // (neither 0 nor inf: where r^2 overflows nothing is
+                                    // left of the pair, and it has no root)
+                                    if (__builtin_amdgcn_class(r2, 0x183) && on) {
                                         const double ir = rsq_full(r2);
                                         s.pot = __builtin_fma(e.w, softened_angle(a.wp.e0, r2 * ir, ir), s.pot);
                                         lnint++;
