@@ -1189,12 +1189,15 @@ __device__ inline int wave_group() {
 // of 8 / 16 / 64: Plummer 10,000 FP32 39 / 51 / 130; 24,576 FP32 54 / 64 / -;
 // 32,768 FP32 57 / 62 / -, FP64 60 / 68 / -; 33,333 FP64 69 / 69 / -; disk
 // 28,000 FP32 67 / 79 / -; 32,768 FP32 75 / 84 / -, FP64 76 / 86 / -; 100,000
-// FP64 - / 167 / 254; 150,000 FP32 - / 180 / 229; 200,000 FP32 - / 228 / 248,
+// FP64 - / 167 / 254; 150,000 FP32 - / 181 / 224; 200,000 FP32 - / 231 / 246,
 // FP64 - / 273 / 307; 400,000 FP64 - / 495 / 503; 450,000 FP64 - / 552 / 542;
-// 1 M FP32 - / 1014 / 710, FP64 - / 1147 / 991.  The choice depends on the
-// set alone, so a job of a batched walk has the arithmetic of a walk of its
-// own.
-constexpr int kTpg8Max = 32768, kTpg16Max32 = 200000, kTpg16Max64 = 400000;
+// 1 M FP32 - / 1014 / 710, FP64 - / 1147 / 991.  In FP32 the two draw level
+// above: 250,000 disk 265 / 295, Hernquist 226 / 246, Plummer 216 / 206 (at
+// opening angle 0.15 2,610 / 3,325, 2,500 / 3,085, 2,295 / 2,545); 275,000 291 /
+// 269, 242 / 242, 238 / 254; 400,000 393 / 391, 325 / 329, 322 / 310.  The
+// choice depends on the set alone, so a job of a batched walk has the
+// arithmetic of a walk of its own.
+constexpr int kTpg8Max = 32768, kTpg16Max32 = 262144, kTpg16Max64 = 400000;
 inline int walk_tpg(int64_t n, bool f32) {
     return n <= kTpg8Max ? 8 : n <= (f32 ? kTpg16Max32 : kTpg16Max64) ? 16 : 64;
 }
