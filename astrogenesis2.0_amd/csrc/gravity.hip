@@ -2,8 +2,8 @@
 // Tree::calculateForces (Tree.cpp:57-83) -> Node::calculateGravityForce
 // (Node.cpp:247-399) -> Node::calcSPHForce (Node.cpp:88-172).
 //
-// k_walk_block: one wavefront per group of 64 targets that are consecutive in
-// key order (spatial neighbours).  The wave walks a child-contiguous copy of
+// walk_block: one wavefront per group of 8, 16 or 64 targets (walk_tpg) that are
+// consecutive in key order (spatial neighbours).  The wave walks a child-contiguous copy of
 // the tree together.  Each iteration pops up to eight sibling blocks (64
 // nodes, one per lane) from an LDS stack of (first child, count, lane mask)
 // and classifies every node against the group's bounding box:
@@ -164,8 +164,9 @@ __device__ inline void sph_pair(double dx, double dy, double dz, double r2, doub
 
 // The same term, value for value, with the square root and the four quotients
 // in short correctly rounded forms: one estimate and its Newton steps serve
-// the root and the quotient by r, 1 / h (ih) is formed once per target, and
-// each quotient ends with one step on its exact remainder.  The compiler's
+// the root and the quotient by r (Goldschmidt's iteration, two corrections by
+// the root's remainder), 1 / h (ih) is formed once per target, and each
+// quotient ends with one step on its exact remainder (Markstein).  The compiler's
 // general forms scale their operands against overflow and fix up special
 // values on every call; plain_support and plain_pair stand for that here
 // (every intermediate and remainder far inside the normal range), and what
@@ -325,11 +326,11 @@ __device__ inline bool list_overflowed(const WalkArgs &a, int cnt) {
 //    LDS.  The loop ends with the busiest lane: on the 1 M disk the partial
 //    masks hold a fifth of the lanes on average, and a lane meets at most
 //    two fifths of a chunk, where a sweep under the masks ran over all of it.
-// The walk is bound by VALU issue (76 % of the SIMDs' cycles): with the two
+// The walk is bound by VALU issue (82 % of the SIMDs' cycles): with the two
 // queues, the SPH margin tested in the sweep and two entries in flight per
-// lane it issues 22.6 k vector instructions per wave where one masked sweep
+// lane it issues 22.4 k vector instructions per wave where one masked sweep
 // issued 28.4 k (1 M disk, FP32), and the kernel takes 0.69 ms against
-// 1.00 ms; the FP64 form 0.99 ms against 1.90 ms.
+// 1.00 ms; the FP64 form 1.00 ms against 1.90 ms.
 template <bool F32, int KIND, int TPG>
 __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *lds) {
     static_assert(TPG == 64 || TPG == 16 || TPG == 8, "targets per group");
@@ -939,7 +940,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, int g, BlockLds *l
                             // them but the rare case: f = m / ((r^2 + e^2) r) as
                             // one reciprocal root of r^2 (r^2 + e^2)^2.  (A root
                             // and a quotient took half as many instructions
-                            // again: the 1 M disk's walk 1,192 us, now 991; one
+                            // again: the 1 M disk's walk 1,192 us, now 1,000; one
                             // entry at a time, with the rare case between
                             // two, 1,236.)
                             auto two = [&](int j1, int j2, bool both) {
@@ -1191,7 +1192,7 @@ __device__ inline int wave_group() {
 // 28,000 FP32 67 / 79 / -; 32,768 FP32 75 / 84 / -, FP64 76 / 86 / -; 100,000
 // FP64 - / 167 / 254; 150,000 FP32 - / 181 / 224; 200,000 FP32 - / 231 / 246,
 // FP64 - / 273 / 307; 400,000 FP64 - / 495 / 503; 450,000 FP64 - / 552 / 542;
-// 1 M FP32 - / 1014 / 710, FP64 - / 1147 / 991.  In FP32 the two draw level
+// 1 M FP32 - / 1014 / 690, FP64 - / 1147 / 1000.  In FP32 the two draw level
 // above: 250,000 disk 265 / 295, Hernquist 226 / 246, Plummer 216 / 206 (at
 // opening angle 0.15 2,610 / 3,325, 2,500 / 3,085, 2,295 / 2,545); 275,000 291 /
 // 269, 242 / 242, 238 / 254; 400,000 393 / 391, 325 / 329, 322 / 310.  The

@@ -805,14 +805,7 @@ __global__ __launch_bounds__(256) void k_rsb_scatter(const SortJob *jobs, int nj
 
 // ------------------------------------------------------------ after sort
 
-// Tie runs (equal word 0) in key order get their order by (word 1, caller
-// index): the reference inserts a run's particles in array order
-// (Tree.cpp:44-48) whatever resident order they were sorted from.  Each
-// particle of a run of k counts the members before it (k steps per thread),
-// and everything goes to the alternate buffers: word 1 to w1, the sort
-// permutation to ord (particles outside runs keep their place).  Runs longer
-// than kTieRankMax are left in order and flagged in ds->tie_big; the build
-// then sorts them with the general segmented sort (refine_ties).
+// Longest run of particles sharing the sorted bits that k_tie_rank orders.
 constexpr int kTieRankMax = 1024;
 
 // First and last particle of the run sharing k[i] >> shift (galloping).

@@ -115,8 +115,8 @@ typedef struct ag2_diag {
     int64_t near_pairs;      /* AG2_FP32_SPLIT: (target, node) pairs of the last
                                 forces closer than the FP32 offsets resolve,
                                 evaluated in FP64 instead                        */
-    int64_t near_redo_groups; /* AG2_FP32_SPLIT: groups of 64 targets with more
-                                such pairs than recorded (32 nodes), whose
+    int64_t near_redo_groups; /* AG2_FP32_SPLIT: groups of targets (8, 16 or 64) with
+                                more such pairs than recorded (32 nodes), whose
                                 gravity came from an FP64 walk instead           */
 } ag2_diag;
 
@@ -180,7 +180,8 @@ int ag2_walk_kernel_ms(void *ctx, double *ms);
 
 /* FP64 direct summation over all particles with the same softened law, for
  * the listed targets (caller indices): accuracy diagnostic of the tree forces.
- * pot may be NULL.  Synchronous. */
+ * A target's sums are the same bit for bit whatever other targets are listed.
+ * Pairs of any scale that FP64 holds.  pot may be NULL.  Synchronous. */
 int ag2_direct_sum(void *ctx, int64_t nt, const int64_t *targets, double *ax, double *ay, double *az,
                    double *pot);
 

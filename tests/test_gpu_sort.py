@@ -1,6 +1,6 @@
-"""The key sort either side of the particle counts where it changes (one launch
-pair over tiles of 2048 and 4096 keys, radix passes), on the first build after
-an upload (caller order) and on builds after steps (nearly sorted): particles
+"""The key sort either side of the particle counts where it changes (merge sort
+over tiles of 1024, 2048 and 4096 keys, sample sort, radix passes), on the first
+build after an upload (caller order) and on builds after steps (nearly sorted): particles
 stand in the order of their octant paths, coincident ones by caller index."""
 import numpy as np
 import pytest
