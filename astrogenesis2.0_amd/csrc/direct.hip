@@ -21,10 +21,13 @@
 // A target's sum depends on the sources alone, bit for bit, not on the other
 // targets asked for: sources are summed in blocks of fixed length, and the
 // blocks in a binary tree (pairs of neighbours, pairs of those, a node without
-// a right half being its left one), of which a wave takes an aligned power of
-// two, as many as the targets leave it.
+// a right half being its left one), of which a workgroup takes a node of any
+// level, as the number of targets and the scratch for the nodes' sums leave it.
+// Its four waves take a quarter of the node each, for the same 64 targets.
 // 1 M sources, 16,384 targets: 372 ms with the potential and 212 without by one
-// workgroup per 256 targets, now 26.0 and 10.4; 256 targets 0.87 and 0.48 ms.
+// workgroup per 256 targets, now 26.1 and 10.5; 256 targets 0.71 and 0.30 ms.
+// (A node per wave, four times the parts: 40,000 sources, 16,384 targets, whose
+// parts the scratch bounds, 1.69 ms, now 1.35.)
 // Against sums in extended precision 2.9e-14 then (a million terms one by one;
 // the potential 4.2e-14), now 1.1e-16.
 #include <mutex>
@@ -36,23 +39,26 @@
 namespace ag2 {
 namespace {
 
-constexpr int kDirectBlock = 256;
+constexpr int kDirectWaves = 4;
 constexpr int kLevels = 24;   // of the tree over blocks
 
-// Sources in blocks of `len`; a wave sums 2^level of them.
+// Sources in blocks of `len`; a workgroup sums 2^level (level >= 2) of them.
 struct SumPlan {
     int n, len, blocks, level;
 };
 
-// Targets: lane k of the grid's first dimension; blocks of sources from split
-// 2^level on.  part: column c of split s at (c * splits + s) * nt, unscaled sums.
+// Targets: 64 per workgroup of the grid's first dimension, a lane each; blocks of
+// sources from split 2^level on, a quarter of them per wave.  part: column c of
+// split s at (c * splits + s) * nt, unscaled sums.
 // ANY: the softening length is outside the fast pair's range.
 template <bool POT, bool ANY>
-__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void
+__global__ __launch_bounds__(64 * kDirectWaves) __attribute__((amdgpu_waves_per_eu(4))) void
 k_direct(SumPlan p, const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
          const double *__restrict__ m, int nt, const int64_t *__restrict__ targets, const int32_t *__restrict__ inv,
          double e0, double *__restrict__ part) {
-    const int k = blockIdx.x * kDirectBlock + threadIdx.x;
+    __shared__ double quarter[kDirectWaves][4][64];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int k = blockIdx.x * 64 + lane;
     const int split = blockIdx.y;
     const bool valid = k < nt;
     const int64_t i = valid ? inv[targets[k]] : 0;   // caller index -> resident slot
@@ -98,7 +104,8 @@ k_direct(SumPlan p, const double *__restrict__ x, const double *__restrict__ y, 
     };
     const std::integral_constant<bool, ANY> form;
     double node[kLevels][4];   // left halves that wait for their right ones, by level
-    const int b0 = split << p.level, b1 = b0 + (1 << p.level) < p.blocks ? b0 + (1 << p.level) : p.blocks;
+    const int size = 1 << (p.level - 2);   // blocks of a quarter
+    const int b0 = (split << p.level) + wave * size, b1 = b0 + size < p.blocks ? b0 + size : p.blocks;
     for (int b = b0; b < b1; b++) {
         const int j0 = b * p.len, j1 = p.n - j0 < p.len ? p.n : j0 + p.len;
         gx = gy = gz = ph = 0.0;
@@ -127,23 +134,32 @@ k_direct(SumPlan p, const double *__restrict__ x, const double *__restrict__ y, 
         node[l][0] = gx; node[l][1] = gy; node[l][2] = gz;
         if (POT) node[l][3] = ph;
     }
-    // what is left of the set's last, incomplete part
-    const int done = b1 - b0;
-    int l = __builtin_ctz(done);
-    gx = node[l][0]; gy = node[l][1]; gz = node[l][2];
-    if (POT) ph = node[l][3];
-    for (l++; done >> l; l++)
-        if (done >> l & 1) {
-            gx = node[l][0] + gx;
-            gy = node[l][1] + gy;
-            gz = node[l][2] + gz;
-            if (POT) ph = node[l][3] + ph;
-        }
-    if (!valid) return;
-    const size_t col = (size_t)gridDim.y * nt;
-    double *out = part + (size_t)split * nt + k;
-    out[0] = gx; out[col] = gy; out[2 * col] = gz;
-    if (POT) out[3 * col] = ph;
+    if (b0 < b1) {
+        // what is left of an incomplete node, the set's last
+        const int done = b1 - b0;
+        int l = __builtin_ctz(done);
+        gx = node[l][0]; gy = node[l][1]; gz = node[l][2];
+        if (POT) ph = node[l][3];
+        for (l++; done >> l; l++)
+            if (done >> l & 1) {
+                gx = node[l][0] + gx;
+                gy = node[l][1] + gy;
+                gz = node[l][2] + gz;
+                if (POT) ph = node[l][3] + ph;
+            }
+    }
+    quarter[wave][0][lane] = gx;
+    quarter[wave][1][lane] = gy;
+    quarter[wave][2][lane] = gz;
+    if (POT) quarter[wave][3][lane] = ph;
+    __syncthreads();
+    // wave c: column c of the quarters that there are
+    if (!valid || wave >= (POT ? 4 : 3)) return;
+    const int rest = p.blocks - (split << p.level);
+    const double lo = quarter[0][wave][lane], hi = quarter[2][wave][lane];
+    double sum = rest > size ? lo + quarter[1][wave][lane] : lo;
+    if (rest > 2 * size) sum = sum + (rest > 3 * size ? hi + quarter[3][wave][lane] : hi);
+    part[((size_t)wave * gridDim.y + split) * nt + k] = sum;
 }
 
 // Column c of the result: its parts up the rest of the tree, scaled.
@@ -180,8 +196,8 @@ __global__ __launch_bounds__(256) void k_direct_fold(int nt, int splits, const d
 
 // Targets [0, nt) in slices whose parts fit `room` doubles of scratch.  Blocks
 // of n / 256 sources (a multiple of four, 32 to 256 of them).  Parts: up to 64
-// waves for each of 1,024 SIMDs, of at least 256 sources (with 16 waves a SIMD,
-// four rounds of them, 16,384 targets wait 30.3 ms for the last, with 64 27.7).
+// waves for each of 1,024 SIMDs (with 16, four rounds of them, 16,384 targets
+// waited 30.3 ms for the last, with 64 27.7), of at least 1,024 sources.
 void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, double *scratch, size_t room, double *ax,
                    double *ay, double *az, double *pot) {
     const int cols = with_pot ? 4 : 3;
@@ -195,15 +211,15 @@ void launch_direct(Ctx &c, int nt, const int64_t *d_targets, int with_pot, doubl
         const size_t fit = room / (size_t)cols;
         const int here = (size_t)(nt - at) < fit ? nt - at : (int)fit;
         if (here < 1) throw HipError("no scratch for the direct sum");
-        const int64_t waves = (here + 63) / 64;
+        const int64_t waves = (here + 63) / 64 * kDirectWaves;
         int64_t most = (65536 + waves - 1) / waves;
-        if (most > (p.n + 255) / 256) most = (p.n + 255) / 256;
+        if (most > (p.n + 1023) / 1024) most = (p.n + 1023) / 1024;
         if (most > (int64_t)(fit / (size_t)here)) most = (int64_t)(fit / (size_t)here);
         if (most > 65535) most = 65535;
-        p.level = 0;
+        p.level = 2;
         while (((p.blocks - 1) >> p.level) + 1 > most) p.level++;
         const int splits = ((p.blocks - 1) >> p.level) + 1;
-        const dim3 grid(grid_for(here, kDirectBlock), (unsigned)splits), block(kDirectBlock);
+        const dim3 grid(grid_for(here, 64), (unsigned)splits), block(64 * kDirectWaves);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, block, 0, c.stream, p, c.x, c.y, c.z, c.m, here, d_targets + at, c.inv,
                                c.p.e0, scratch);
